@@ -1,0 +1,97 @@
+// Host-side choices of the GEMM family that do not depend on the storage type's kernels: which
+// operands the matrix-core kernels take, and when a product is split along K.
+#pragma once
+
+#include "gemm_mfma.h"
+#include "gemm_f32.h"
+
+namespace tmb {
+
+static inline bool mfma_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b) {
+  if (trans_a) return false;
+  if (g.k % 8 != 0 || g.lda % 8 != 0 || g.ldb % 8 != 0) return false;
+  if (!aligned16(g.a) || !aligned16(g.b)) return false;
+  if (batch > 1 && (g.stride_a % 8 != 0 || g.stride_b % 8 != 0)) return false;
+  if (g.m < 1 || g.n < 1 || g.k < 8) return false;
+  // the kernel addresses operands with 32-bit byte offsets from their base
+  const int64_t a_span = g.m * g.lda * 2, b_span = (trans_b ? g.n : g.k) * g.ldb * 2;
+  if (a_span >= (int64_t{1} << 32) || b_span >= (int64_t{1} << 32)) return false;
+  (void)trans_b;
+  return true;
+}
+
+// Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
+// leave most CUs idle. K is cut into `splits` runs of whole stages (equal to within one stage)
+// that run as the y dimension of one launch of a ring kernel and store fp32 partials
+// [splits][M][N] into a workspace; a second kernel adds them in split order and applies bias,
+// epilogue and the one cast, so the result is still "fp32 accumulation, one rounding" and depends
+// on the shape only.
+//
+// Tile and split count come from a small cost model (all in microseconds): the 256 x 256 x 64
+// kernel sustains about 1240 TFLOP/s over 256 one-per-CU workgroups, the 128 x 128 x 32 kernel
+// about 900 TFLOP/s over 512 two-per-CU workgroups; the launch takes ceil(units / slots) rounds of
+// one unit's time, the reduction reads splits * M * N * 4 bytes at about 4 TB/s.
+struct SplitKPlan {
+  int splits;  // 0: not used
+  int tile;    // 128 or 256
+  int64_t k_chunk;  // fp32 kernel only: equal chunks
+};
+static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  SplitKPlan p{0, 0, 0};
+  if (batch != 1 || k < 2048 || k % 32 != 0 || n <= 64 || m < 1) return p;
+  const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128);
+  if (t128 >= 256) return p;  // at least one tile per CU: no split
+  const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256);
+  double best = 0.0;
+  for (int tile = 128; tile <= 256; tile += 128) {
+    const int bk = tile == 128 ? 32 : 64;
+    if (k % bk != 0) continue;
+    if (tile == 256 && (m <= 128 || n <= 128)) continue;
+    const int64_t tiles = tile == 128 ? t128 : t256;
+    const int64_t slots = tile == 128 ? 512 : 256;
+    const double unit_rate = tile == 128 ? 900e6 / 512 : 1240e6 / 256;  // FLOP per us per workgroup
+    for (int64_t splits = 2; splits <= 16; ++splits) {
+      if (k / bk / splits < 8) break;  // at least 8 stages per split
+      const double chunk = static_cast<double>(k) / splits;
+      // (a 128-tile workgroup that has its CU to itself runs about 1.7 times faster than one of
+      // two: 768 x 768 x 16384 in 5 splits of 36 tiles takes 32 us)
+      const double alone = (tile == 128 && tiles * splits <= 256) ? 1.7 : 1.0;
+      const double unit = 2.0 * tile * tile * chunk / (unit_rate * alone);
+      const double rounds = static_cast<double>((tiles * splits + slots - 1) / slots);
+      const double reduce = 3.0 + static_cast<double>(splits) * m * n * 4.0 / 4e6;
+      const double cost = rounds * unit + reduce;
+      if (p.splits == 0 || cost < best) {
+        best = cost;
+        p.splits = static_cast<int>(splits);
+        p.tile = tile;
+      }
+    }
+  }
+  return p;
+}
+
+// fp32 products run 16 times slower on the matrix cores than 16-bit ones, so a 128 x 128 tile
+// with a few hundred K already takes tens of microseconds and the split pays from much shorter K.
+// Chunks are whole 16-byte groups of K so that every chunk keeps the operands' alignment.
+static inline SplitKPlan splitk_plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  SplitKPlan p{0, 0, 0};
+  if (batch != 1 || k < 128 || m < 1 || n < 1) return p;
+  const int64_t tiles = ((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN);
+  if (tiles >= 256) return p;
+  int64_t splits = 512 / tiles;
+  if (splits > 16) splits = 16;
+  if (splits > k / 64) splits = k / 64;
+  while (splits >= 2 && k % (splits * 4) != 0) --splits;
+  if (splits < 2) return p;
+  p.splits = static_cast<int>(splits);
+  p.tile = 128;
+  p.k_chunk = k / splits;
+  return p;
+}
+
+// The typed half of the entry point (gemm_typed.h), one translation unit per storage type.
+template <typename T>
+int gemm_epi(const GemmArgs& g, int64_t batch, int ta, int tb, int epilogue, hipStream_t stream, void* ws,
+             size_t ws_bytes);
+
+}  // namespace tmb

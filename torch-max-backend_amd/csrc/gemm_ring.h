@@ -647,7 +647,7 @@ void gemm_ring_kernel(GemmArgs g) {
 // longer than the ring's two stages of lookahead cover. 16384 x 50257 x 768 behind other work:
 // 1.69-1.87 ms as it is, 1.14-1.19 ms behind a 22 us pass over the 77 MB of B (which is also what
 // the same launch takes when it runs twice in a row).
-__global__ __launch_bounds__(256) void warm_lines_kernel(const uint32_t* __restrict__ p, int64_t lines,
+static __global__ __launch_bounds__(256) void warm_lines_kernel(const uint32_t* __restrict__ p, int64_t lines,
                                                          int64_t last_dword) {
   uint32_t seen = 0;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < lines;
