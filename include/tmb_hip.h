@@ -180,6 +180,9 @@ int tmb_gemm(void* c, const void* a, const void* b, const void* bias, int64_t ba
  * (eager_kernels/matmul_ops.mojo:1040-1049, `multistage_gemm_kernel`); here the caller owns it,
  * as with every other buffer. */
 size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int dtype);
+/* The same for a known operand layout: 0 also where a kernel that needs no scratch takes the product. */
+size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a,
+                                       int trans_b, int dtype);
 int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch, int64_t m,
                 int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, int64_t stride_a,
                 int64_t stride_b, int64_t stride_c, int trans_a, int trans_b, int dtype,
@@ -204,6 +207,14 @@ int tmb_gemm_residual(void* c, const void* a, const void* b, const void* bias,
                       int64_t stride_b, int64_t stride_c, int64_t stride_r, int trans_a,
                       int trans_b, int dtype, int residual_dtype, int out_dtype, int epilogue,
                       void* stream);
+
+/* tmb_gemm_residual with a workspace (tmb_gemm_layout_workspace_bytes): a product that is split along K adds its
+ * residual in the kernel that sums the partials. NULL or too small: as tmb_gemm_residual. */
+int tmb_gemm_residual_ws(void* c, const void* a, const void* b, const void* bias, const void* residual,
+                         int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc,
+                         int64_t ldr, int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_r,
+                         int trans_a, int trans_b, int dtype, int residual_dtype, int out_dtype, int epilogue,
+                         void* workspace, size_t workspace_bytes, void* stream);
 
 /* Fused attention forward: out[b,t,h,:] = softmax_j(scale * q[b,h,t,:] . k[b,h,j,:]) v[b,h,j,:],
  * with `causal` != 0 only keys j <= t take part. The [batch, heads, q_len, kv_len] scores never

@@ -119,6 +119,14 @@ extern "C" size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, 
   return static_cast<size_t>(plan.splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
 }
 
+extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a,
+                                                  int trans_b, int dtype) {
+  // the kernel for small products needs none (operands it cannot take run unsplit then)
+  if (dtype != TMB_F32 && !trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k))
+    return 0;
+  return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
+}
+
 extern "C" int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch,
                            int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc,
                            int64_t stride_a, int64_t stride_b, int64_t stride_c, int trans_a,
@@ -135,9 +143,20 @@ extern "C" int tmb_gemm_residual(void* c, const void* a, const void* b, const vo
                                  int64_t stride_a, int64_t stride_b, int64_t stride_c,
                                  int64_t stride_r, int trans_a, int trans_b, int dtype,
                                  int residual_dtype, int out_dtype, int epilogue, void* stream) {
+  return tmb_gemm_residual_ws(c, a, b, bias, residual, batch, m, n, k, lda, ldb, ldc, ldr, stride_a, stride_b,
+                              stride_c, stride_r, trans_a, trans_b, dtype, residual_dtype, out_dtype, epilogue,
+                              nullptr, 0, stream);
+}
+
+extern "C" int tmb_gemm_residual_ws(void* c, const void* a, const void* b, const void* bias, const void* residual,
+                                    int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                                    int64_t ldc, int64_t ldr, int64_t stride_a, int64_t stride_b, int64_t stride_c,
+                                    int64_t stride_r, int trans_a, int trans_b, int dtype, int residual_dtype,
+                                    int out_dtype, int epilogue, void* workspace, size_t workspace_bytes,
+                                    void* stream) {
   if (residual == nullptr) return TMB_ERR_INVALID_ARGUMENT;
   if (residual_dtype < 0 || out_dtype < 0) return TMB_ERR_INVALID_ARGUMENT;
   return gemm_entry(c, a, b, bias, residual, batch, m, n, k, lda, ldb, ldc, ldr, stride_a,
-                    stride_b, stride_c, stride_r, trans_a, trans_b, dtype, epilogue, stream, nullptr,
-                    0, residual_dtype, out_dtype);
+                    stride_b, stride_c, stride_r, trans_a, trans_b, dtype, epilogue, stream, workspace,
+                    workspace_bytes, residual_dtype, out_dtype);
 }

@@ -602,7 +602,7 @@ __device__ __forceinline__ void store_wave_tile16(f32x4v_t (&acc)[AM][AN], lds_b
 
 // The batch entry's epilogue description out of the launch arguments.
 template <typename T>
-__device__ __forceinline__ EpilogueArgs epilogue_args(const GemmArgs& g, int64_t batch) {
+__host__ __device__ __forceinline__ EpilogueArgs epilogue_args(const GemmArgs& g, int64_t batch) {
   const void* r = nullptr;
   if (g.residual != nullptr) {
     r = g.resid_f32 ? static_cast<const void*>(static_cast<const float*>(g.residual) + batch * g.stride_r)
@@ -669,18 +669,27 @@ __device__ __forceinline__ void store_wave_tile16_f32(f32x4v_t (&acc)[AM][AN], f
   }
 }
 
-// c[m, n] = epilogue(sum over the splits (in order) of partial[s][m][n] + bias[n]), one cast.
-// VEC = 4: four consecutive columns per thread (n % 4 == 0 keeps them in one row).
+// c[m, n] = epilogue(sum over the splits (in order) of partial[s][m][n] + bias[n]) [+ residual], one
+// cast (or rounded step by step: see EpilogueArgs). VEC = 4: four consecutive columns per thread
+// (n % 4 == 0 keeps them in one row).
 template <typename T, int EPI, int VEC>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(T* __restrict__ c,
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(void* __restrict__ c,
                                                             const float* __restrict__ partial,
                                                             const T* __restrict__ bias, int64_t m,
                                                             int64_t n, int64_t ldc, int splits,
-                                                            bool twice) {
+                                                            EpilogueArgs ep) {
   const int64_t total = m * n;
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * VEC;
   if (i >= total) return;
-  float sum[VEC];
+  const int64_t row = i / n, col = i - row * n;
+  float sum[VEC], resid[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    const int64_t at = row * ep.ldr + col + e;
+    resid[e] = ep.residual == nullptr ? 0.0f
+               : ep.resid_f32         ? static_cast<const float*>(ep.residual)[at]
+                                      : to_f32(static_cast<const T*>(ep.residual)[at]);
+  }
   if constexpr (VEC == 4) {
     typedef float f32x4_aligned_t __attribute__((ext_vector_type(4)));
     f32x4_aligned_t v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_aligned_t*>(partial + i));
@@ -695,27 +704,35 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(T* __restrict__ c,
     sum[0] = partial[i];
     for (int s = 1; s < splits; ++s) sum[0] += partial[s * total + i];
   }
-  const int64_t row = i / n, col = i - row * n;
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
     if (bias != nullptr) sum[e] += to_f32(bias[col + e]);
-    c[row * ldc + col + e] = finish<T, EPI>(sum[e], twice);
+    const int64_t at = row * ldc + col + e;
+    if (EPI == TMB_EPI_NONE && ep.wide()) {
+      const float v = sum[e] + resid[e];
+      if (ep.out_f32) static_cast<float*>(c)[at] = v;
+      else static_cast<T*>(c)[at] = from_f32<T>(v);
+    } else {
+      T v = finish<T, EPI>(sum[e], ep.twice);
+      if (ep.residual != nullptr) v = from_f32<T>(pin_f32(to_f32(v) + resid[e]));
+      static_cast<T*>(c)[at] = v;
+    }
   }
 }
 
 // Launches the reduction over `splits` partials (workspace is 16-byte aligned or the scalar form runs).
 template <typename T, int EPI>
-static inline void launch_splitk_reduce(T* c, const float* partial, const T* bias, int64_t m,
-                                        int64_t n, int64_t ldc, int splits, bool twice,
+static inline void launch_splitk_reduce(void* c, const float* partial, const T* bias, int64_t m,
+                                        int64_t n, int64_t ldc, int splits, const EpilogueArgs& ep,
                                         hipStream_t stream) {
   const int64_t total = m * n;
   if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(partial) & 15) == 0) {
     const int64_t threads = total / 4;
     splitk_reduce_kernel<T, EPI, 4><<<dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream>>>(
-        c, partial, bias, m, n, ldc, splits, twice);
+        c, partial, bias, m, n, ldc, splits, ep);
   } else {
     splitk_reduce_kernel<T, EPI, 1><<<dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, stream>>>(
-        c, partial, bias, m, n, ldc, splits, twice);
+        c, partial, bias, m, n, ldc, splits, ep);
   }
 }
 

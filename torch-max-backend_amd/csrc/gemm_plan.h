@@ -2,6 +2,8 @@
 // operands the matrix-core kernels take, and when a product is split along K.
 #pragma once
 
+#include <cmath>
+
 #include "gemm_mfma.h"
 #include "gemm_f32.h"
 
@@ -19,6 +21,53 @@ static inline bool mfma_eligible(const GemmArgs& g, int64_t batch, int trans_a, 
   (void)trans_b;
   return true;
 }
+
+// Tiles of the kernel for products that leave most of the chip idle (gemm_small.h), and what a
+// launch with one of them takes, in microseconds: a start, then per tile its operands' bytes at the
+// rate one workgroup's loads sustain and the way of its partial tiles through LDS. A CU that gets a
+// second workgroup of the tiles that fit it twice (up to 32 x 32) loads faster than one alone,
+// hence the power; the two large ones take a CU's LDS and run in whole rounds. The constants are a
+// fit to 720 shapes (1 .. 2048 rows, 256 .. 8192 columns, K 64 .. 4096, both layouts of B), within
+// 15 % of them.
+struct SmallTile {
+  int bm, bn, waves;
+  double start, bytes_per_us, lds;
+  bool alone;
+};
+constexpr SmallTile kSmallTiles[] = {{16, 16, 8, 2.8, 60e3, 0.4, false}, {16, 32, 8, 2.8, 70e3, 0.7, false},
+                                     {32, 32, 8, 2.8, 80e3, 1.0, false}, {32, 32, 4, 3.0, 70e3, 0.4, false},
+                                     {32, 64, 8, 2.8, 90e3, 1.5, true},  {64, 64, 8, 3.0, 90e3, 2.0, true}};
+constexpr int kSmallTileCount = sizeof(kSmallTiles) / sizeof(kSmallTiles[0]);
+
+static inline int small_tile(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < kSmallTileCount; ++i) {
+    const SmallTile& t = kSmallTiles[i];
+    const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch;
+    double rounds = 1.0;
+    if (tiles > 256) rounds = t.alone ? static_cast<double>((tiles + 255) / 256) : std::pow(tiles / 256.0, 0.9);
+    const double cost = t.start + rounds * ((t.bm + t.bn) * 2.0 * k / t.bytes_per_us + t.lds);
+    if (i == 0 || cost < least) {
+      least = cost;
+      best = i;
+    }
+  }
+  return best;
+}
+
+// Which products that kernel takes (16-bit operands, A row-major): those whose 64 x 64 tiles fit one
+// round of the 256 CUs, up to K = 4096 (at K = 8192 the split-K launch is level with it), and 16 rows
+// or fewer against any number of columns, which is a pass over B. Measured over the 600 such shapes
+// of the sweep above it is 1.8 times as fast as what ran before (128 x 768 x 768 8.9 -> 3.6 us,
+// 32 x 2304 x 768 11.5 -> 4.0, 128 x 768 x 3072 13.4 -> 6.2, 1024 x 768 x 3072 19.9 -> 14.3 us; two
+// N-major shapes of 600 run 5-10 % longer), and over what lies outside on average slower.
+static inline bool small_applies(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  if (k > 4096 || k < 8 || m < 1 || n < 1) return false;
+  if (m <= 16 && batch == 1) return true;
+  return ((m + 63) / 64) * ((n + 63) / 64) * batch <= 256;
+}
+int gemm_small(const GemmArgs& g, int64_t batch, int trans_b, bool bf16, int epilogue, hipStream_t stream);
 
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
 // leave most CUs idle. K is cut into `splits` runs of whole stages (equal to within one stage)

@@ -7,7 +7,7 @@
 // (BM x BN, 16 .. 64 each way) and its WAVES waves share K between them: wave w multiplies the
 // 64-deep slices w, w + WAVES, ... of the whole tile, so a wave has all its operands in flight at
 // once and no barrier stands between a load and its MFMAs. The fp32 partial tiles meet in LDS once,
-// are added in wave order (the result depends on the shape only) and leave through one epilogue
+// are added pairwise in wave order (the result depends on the shape only) and leave through one epilogue
 // (bias, GELU, residual), which also spares these shapes the second launch of a split-K product.
 //
 // A wave brings its slices in as whole 128-byte lines (eight lanes to a line), lays them into a
@@ -234,13 +234,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_small_kernel(GemmArgs g) {
     const int r = idx / (BN / 4), c = (idx % (BN / 4)) * 4;
     const int64_t row = m0 + r, col = n0 + c;
     if (row >= M || col >= N) continue;
-    float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // pairwise: a short chain of adds, and the rounding of log2(WAVES) of them instead of WAVES
+    f32x4v_t v[WAVES];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const f32x4v_t v = *reinterpret_cast<const f32x4v_t*>(all + w * (BM * RP) + r * RP + c);
+    for (int w = 0; w < WAVES; ++w) v[w] = *reinterpret_cast<const f32x4v_t*>(all + w * (BM * RP) + r * RP + c);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum[e] += v[e];
-    }
+    for (int step = 1; step < WAVES; step *= 2)
+#pragma unroll
+      for (int w = 0; w < WAVES; w += 2 * step)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[w][e] += v[w + step][e];
+    const float sum[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
     small_epilogue4<T, EPI>(sum, g, ep, batch, row, col);
   }
 #endif
@@ -267,33 +271,6 @@ static int launch_small(const GemmArgs& base, int64_t batch, hipStream_t stream)
   if (tiles >= (int64_t{1} << 31) || batch > 65535) return TMB_ERR_UNSUPPORTED;
   kernel<<<dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(batch)), dim3(WAVES * 64), SMEM, stream>>>(g);
   return check_launch();
-}
-
-struct SmallTile {
-  int bm, bn, waves;
-};
-constexpr SmallTile kSmallTiles[] = {{16, 16, 8}, {16, 32, 8}, {32, 32, 8}, {32, 32, 4}, {32, 64, 8}, {64, 64, 8}};
-
-// Microseconds a launch takes with one of the tiles: 3 us to start and end, then per round of one
-// workgroup on each CU what its operands take at the 80 GB/s a CU's loads sustain and what the
-// partial tiles take on their way through LDS. Within 10 % of the measured times from 1 x 768 x 768
-// (3.1 us) to 1024 x 768 x 3072 (14.3 us).
-static inline double small_cost(const SmallTile& t, int64_t batch, int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * batch;
-  const double rounds = static_cast<double>((tiles + 255) / 256);
-  return 3.0 + rounds * ((t.bm + t.bn) * 2.0 * k / 80e3 + t.waves * t.bm * t.bn * 8.0 / 200e3);
-}
-static inline int small_pick(int64_t batch, int64_t m, int64_t n, int64_t k, double* cost) {
-  int best = 0;
-  *cost = 0.0;
-  for (int i = 0; i < static_cast<int>(sizeof(kSmallTiles) / sizeof(kSmallTiles[0])); ++i) {
-    const double c = small_cost(kSmallTiles[i], batch, m, n, k);
-    if (i == 0 || c < *cost) {
-      *cost = c;
-      best = i;
-    }
-  }
-  return best;
 }
 
 }  // namespace tmb

@@ -219,8 +219,8 @@ static int launch_splitk(const GemmArgs& g, const SplitKPlan& plan, int trans_a,
     rc = launch_ring<T, 128, 128, 32, 2, 2, 4, false, TMB_EPI_NONE, false, true>(part, plan.splits, stream);
   }
   if (rc != 0) return rc;
-  launch_splitk_reduce<T, EPI>(static_cast<T*>(g.c), workspace, static_cast<const T*>(g.bias), g.m,
-                               g.n, g.ldc, plan.splits, g.round_like_unfused != 0, stream);
+  launch_splitk_reduce<T, EPI>(g.c, workspace, static_cast<const T*>(g.bias), g.m, g.n, g.ldc, plan.splits,
+                               epilogue_args<T>(g, 0), stream);
   return check_launch();
 }
 
@@ -237,9 +237,8 @@ static int launch_splitk_f32(const GemmArgs& g, const SplitKPlan& plan, int tran
   part.stride_b = trans_b ? plan.k_chunk : plan.k_chunk * g.ldb;
   const int rc = launch_f32_mfma<TMB_EPI_NONE>(part, plan.splits, trans_a, trans_b, stream);
   if (rc != 0) return rc;
-  launch_splitk_reduce<float, EPI>(static_cast<float*>(g.c), workspace,
-                                   static_cast<const float*>(g.bias), g.m, g.n, g.ldc, plan.splits,
-                                   false, stream);
+  launch_splitk_reduce<float, EPI>(g.c, workspace, static_cast<const float*>(g.bias), g.m, g.n, g.ldc,
+                                   plan.splits, epilogue_args<float>(g, 0), stream);
   return check_launch();
 }
 
@@ -247,7 +246,10 @@ template <typename T, int EPI>
 static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, bool half,
                       hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
   if constexpr (!__is_same(T, float)) {
-    if (half && workspace != nullptr && g.residual == nullptr) {
+    if (half && small_applies(batch, g.m, g.n, g.k) && mfma_eligible(g, batch, trans_a, trans_b) &&
+        (trans_b || g.n % 8 == 0))
+      return gemm_small(g, batch, trans_b, __is_same(T, bf16_t), EPI, stream);
+    if (half && workspace != nullptr) {
       const SplitKPlan plan = splitk_plan(batch, g.m, g.n, g.k);
       const bool operands_ok =
           trans_a ? mfma_transposed_a_eligible(g, batch, trans_a, trans_b, TMB_EPI_NONE)

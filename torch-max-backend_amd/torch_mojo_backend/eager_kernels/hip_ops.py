@@ -334,10 +334,11 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         return out
     lib = _ek.lib()
     # few output tiles and a long K: the library splits K when it is handed scratch memory
-    key = (batch, m, n, k, a.dtype)
+    key = (batch, m, n, k, la[0], lb[0], a.dtype)
     ws_bytes = _GEMM_WS_BYTES.get(key)
-    if ws_bytes is None:  # a pure function of the shape: asked once per shape
-        ws_bytes = _GEMM_WS_BYTES[key] = lib.tmb_gemm_workspace_bytes(batch, m, n, k, code_of(a.dtype))
+    if ws_bytes is None:  # a pure function of shape and layout: asked once for each
+        ws_bytes = _GEMM_WS_BYTES[key] = lib.tmb_gemm_layout_workspace_bytes(batch, m, n, k, la[0], lb[0],
+                                                                             code_of(a.dtype))
 
     def unfused_residual():
         # no kernel carries this epilogue for these operands: product first, then the add.
@@ -347,21 +348,21 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
             return (prod.float() + residual.float()).to(result_dtype)
         return prod + residual
 
-    if residual is not None and (ws_bytes or (epilogue != _ek.EPI_NONE and not round_like_unfused)):
-        # the split kernels have no residual step; a GELU in front of a float32 add neither
-        return unfused_residual()
+    if residual is not None and epilogue != _ek.EPI_NONE and not round_like_unfused:
+        return unfused_residual()   # no kernel has a GELU in front of a float32 add
     if residual is not None:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
         res = residual if residual.stride(-1) == 1 and residual.stride(-2) >= n else residual.contiguous()
-        rc = lib.tmb_gemm_residual(
+        rc = lib.tmb_gemm_residual_ws(
             out.data_ptr(), a.data_ptr(), b.data_ptr(), None if bias is None else bias.data_ptr(),
             res.data_ptr(), batch, m, n, k, la[1], lb[1], n, res.stride(-2),
             a.stride(0) if batched else 0, b.stride(0) if batched else 0, m * n,
             res.stride(0) if batched else 0,
             la[0], lb[0], code_of(a.dtype), code_of(res.dtype), code_of(result_dtype), epi_flags,
-            _stream())
+            None if ws is None else ws.data_ptr(), ws_bytes, _stream())
         if rc == _ek.ERR_UNSUPPORTED:
             return unfused_residual()
-        _check("tmb_gemm_residual", rc)
+        _check("tmb_gemm_residual_ws", rc)
         return out
     if key is not None and a is a_in and b is b_in and bias is bias_in and out_dtype is None:
         # operands are consumed in place: remember the launch arguments for this layout
