@@ -76,7 +76,7 @@ static int gemm_entry(void* c, const void* a, const void* b, const void* bias,
   if (out_f32 && residual == nullptr) return TMB_ERR_UNSUPPORTED;  // fp32 C exists for the residual form only
   if (residual != nullptr) {
     // only the MFMA kernels carry the second epilogue step; the caller adds separately otherwise
-    if (dtype == TMB_F32 || k == 0 || ldr < n || !mfma_eligible(g, batch, trans_a, trans_b))
+    if (k == 0 || ldr < n || (dtype != TMB_F32 && !mfma_eligible(g, batch, trans_a, trans_b)))
       return TMB_ERR_UNSUPPORTED;
     // fp32 operands of the epilogue and an epilogue that stays in fp32 exist without GELU only
     if ((resid_f32 || out_f32 || !twice) && epilogue != TMB_EPI_NONE) return TMB_ERR_UNSUPPORTED;
@@ -124,6 +124,10 @@ extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int6
   // the kernel for small products needs none (operands it cannot take run unsplit then)
   if (dtype != TMB_F32 && !trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k))
     return 0;
+  if (dtype == TMB_F32) {
+    if (batch < 1 || m < 1 || n < 1 || k < 1 || tmb::f32_wide_pays(batch, m, n, k) || m * n >= (int64_t{1} << 31)) return 0;
+    return static_cast<size_t>(tmb::f32_plan(batch, m, n, k).splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
+  }
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
 }
 

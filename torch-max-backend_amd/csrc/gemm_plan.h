@@ -5,7 +5,7 @@
 #include <cmath>
 
 #include "gemm_mfma.h"
-#include "gemm_f32.h"
+#include "gemm_f32_wide.h"
 
 namespace tmb {
 
@@ -119,9 +119,8 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
   return p;
 }
 
-// fp32 products run 16 times slower on the matrix cores than 16-bit ones, so a 128 x 128 tile
-// with a few hundred K already takes tens of microseconds and the split pays from much shorter K.
-// Chunks are whole 16-byte groups of K so that every chunk keeps the operands' alignment.
+// What tmb_gemm_workspace_bytes answers for fp32: room for the splits of a long K over few 128 x 128
+// tiles, as many as any plan below asks for on such shapes.
 static inline SplitKPlan splitk_plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
   SplitKPlan p{0, 0, 0};
   if (batch != 1 || k < 128 || m < 1 || n < 1) return p;
@@ -136,6 +135,73 @@ static inline SplitKPlan splitk_plan_f32(int64_t batch, int64_t m, int64_t n, in
   p.tile = 128;
   p.k_chunk = k / splits;
   return p;
+}
+
+// fp32: tile and split count. A launch of the kernel whose waves share K takes about 7 us (start, first
+// operands, the partial tiles' way through LDS, stores) and, per round of tiles, the matrix cores' time
+// for one (2 FLOP per 256 and cycle at 2.4 GHz) stretched by what L1, L2 and LDS cost at that tile size;
+// 32 x 32 tiles share a CU and are not bound to whole rounds. Within 8-9 % (rms) of 2000 measured
+// shapes (1 .. 4096 rows, 64 .. 4096 columns, K 64 .. 12564, 1 .. 48 batches). A split adds the reduction:
+// a launch and its bytes at 4 TB/s.
+struct F32Tile {
+  int bm, bn;
+  double stretch, per_tile;
+};
+constexpr F32Tile kF32Tiles[] = {{32, 32, 2.0, 0.5}, {32, 64, 1.6, 1.0}, {64, 64, 1.4, 2.0}, {64, 128, 1.3, 4.0}};
+constexpr int kF32TileCount = sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+struct F32Plan {
+  int tile;    // index into kF32Tiles
+  int splits;  // 0: not split
+};
+static inline double f32_cost(const F32Tile& t, double batch, int64_t m, int64_t n, double k) {
+  const double tiles = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * batch;
+  double rounds = std::ceil(tiles / 256.0);
+  if (t.bm * t.bn == 1024) {
+    if (tiles > 1536.0) return 1e30;  // (far slower than the larger tiles there: L1 and L2 traffic)
+    const double r = tiles / 256.0;
+    rounds = r <= 1.0 ? 1.0 : (0.5 + 0.5 * rounds / r) * std::pow(r, 0.9);
+  }
+  return 7.0 + rounds * (2.0 * t.bm * t.bn * k / 256.0 / 2400.0 * t.stretch + t.per_tile);
+}
+static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  F32Plan p{kF32TileCount - 1, 0};
+  double best = 0.0;
+  for (int i = 0; i < kF32TileCount; ++i) {
+    const double c = f32_cost(kF32Tiles[i], static_cast<double>(batch), m, n, static_cast<double>(k));
+    if (i == 0 || c < best) {
+      best = c;
+      p.tile = i;
+    }
+  }
+  if (batch != 1) return p;
+  best *= 0.92;  // a second launch and a workspace have to pay for themselves
+  for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
+    if (k < 96 * s) break;
+    for (int i = 0; i < kF32TileCount; ++i) {
+      const double c = f32_cost(kF32Tiles[i], s, m, n, static_cast<double>(k) / s) + 5.5 + 1e-6 * s * m * n;
+      if (c < best) {
+        best = c;
+        p.tile = i;
+        p.splits = s;
+      }
+    }
+  }
+  return p;
+}
+// The 128 x 128 kernel (16-byte aligned operands): where its tiles fill at least two rounds well (4096^3
+// level, 1332 x 50257 x 768 870 against 930 us, 4096 x 4096 x 768 225 against 248), and short K, whose tiles
+// are all prologue, from 176 of them on (4096 x 768 x 64 15.1 against 17 us).
+static inline bool f32_wide_pays(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN) * batch;
+  const int64_t slots = (tiles + 255) / 256 * 256;
+  return (tiles >= 512 && tiles * 20 >= slots * 17) || (k <= 256 && tiles >= 176);
+}
+// What the kernel whose waves share K asks of its operands: at least four elements along each
+// contiguous direction, and lane offsets within a tile that fit 32 bits.
+static inline bool f32_shared_eligible(const GemmArgs& g, int trans_a, int trans_b) {
+  if (g.m < 1 || g.n < 1 || g.k < 1) return false;
+  if ((trans_a ? g.m : g.k) < 4 || (trans_b ? g.k : g.n) < 4) return false;
+  return g.lda < (int64_t{1} << 23) && g.ldb < (int64_t{1} << 23);
 }
 
 // The typed half of the entry point (gemm_typed.h), one translation unit per storage type.

@@ -225,20 +225,45 @@ static int launch_splitk(const GemmArgs& g, const SplitKPlan& plan, int trans_a,
 }
 
 template <int EPI>
-static int launch_splitk_f32(const GemmArgs& g, const SplitKPlan& plan, int trans_a, int trans_b,
-                             float* workspace, hipStream_t stream) {
+static int launch_f32_shared(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, hipStream_t stream) {
+  switch (tile) {
+    case 0: return launch_f32_tile<32, 32, 4, EPI>(g, batch, trans_a, trans_b, stream);
+    case 1: return launch_f32_tile<32, 64, 4, EPI>(g, batch, trans_a, trans_b, stream);
+    case 2: return launch_f32_tile<64, 64, 4, EPI>(g, batch, trans_a, trans_b, stream);
+    default: return launch_f32_tile<64, 128, 4, EPI>(g, batch, trans_a, trans_b, stream);
+  }
+}
+
+template <int EPI>
+static int gemm_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, hipStream_t stream, void* workspace,
+                    size_t workspace_bytes) {
+  if (g.residual == nullptr && f32_wide_pays(batch, g.m, g.n, g.k) && f32_mfma_eligible(g, batch, trans_a, trans_b))
+    return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
+  F32Plan plan = f32_plan(batch, g.m, g.n, g.k);
+  if (plan.splits > 0 && (workspace == nullptr || g.m * g.n >= (int64_t{1} << 31) ||
+                          workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4)) {
+    plan.splits = 0;
+    double best = 0.0;
+    for (int i = 0; i < kF32TileCount; ++i) {
+      const double c = f32_cost(kF32Tiles[i], static_cast<double>(batch), g.m, g.n, static_cast<double>(g.k));
+      if (i == 0 || c < best) {
+        best = c;
+        plan.tile = i;
+      }
+    }
+  }
+  if (plan.splits == 0) return launch_f32_shared<EPI>(g, batch, plan.tile, trans_a, trans_b, stream);
   GemmArgs part = g;
   part.c = workspace;
   part.bias = nullptr;
-  part.k = plan.k_chunk;
+  part.residual = nullptr;
   part.ldc = g.n;
   part.stride_c = g.m * g.n;
-  part.stride_a = trans_a ? plan.k_chunk * g.lda : plan.k_chunk;
-  part.stride_b = trans_b ? plan.k_chunk : plan.k_chunk * g.ldb;
-  const int rc = launch_f32_mfma<TMB_EPI_NONE>(part, plan.splits, trans_a, trans_b, stream);
+  part.splits = plan.splits;
+  const int rc = launch_f32_shared<TMB_EPI_NONE>(part, plan.splits, plan.tile, trans_a, trans_b, stream);
   if (rc != 0) return rc;
-  launch_splitk_reduce<float, EPI>(g.c, workspace, static_cast<const float*>(g.bias), g.m, g.n, g.ldc,
-                                   plan.splits, epilogue_args<float>(g, 0), stream);
+  launch_splitk_reduce<float, EPI>(g.c, static_cast<const float*>(workspace), static_cast<const float*>(g.bias), g.m,
+                                   g.n, g.ldc, plan.splits, epilogue_args<float>(g, 0), stream);
   return check_launch();
 }
 
@@ -271,14 +296,9 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
     }
   }
   if constexpr (__is_same(T, float)) {
-    if (g.residual == nullptr && f32_mfma_eligible(g, batch, trans_a, trans_b)) {
-      const SplitKPlan plan = splitk_plan_f32(batch, g.m, g.n, g.k);
-      if (plan.splits > 0 && workspace != nullptr && g.m * g.n < (int64_t{1} << 31) &&
-          workspace_bytes >= static_cast<size_t>(plan.splits) * g.m * g.n * 4)
-        return launch_splitk_f32<EPI>(g, plan, trans_a, trans_b, static_cast<float*>(workspace),
-                                      stream);
-      return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
-    }
+    if (f32_shared_eligible(g, trans_a, trans_b))
+      return gemm_f32<EPI>(g, batch, trans_a, trans_b, stream, workspace, workspace_bytes);
+    if (g.residual != nullptr) return TMB_ERR_UNSUPPORTED;
   }
   return launch_simt<T, EPI>(g, batch, trans_a, trans_b, stream);
 }
