@@ -343,7 +343,8 @@ class _GraphFactory:
         """Grows a fused masked softmax into a fused attention when it sits in
             bmm(flat(q), flat(k^T)) -> view -> [mul, masked_fill, _softmax] -> expand -> view
               -> bmm(., flat(v)) -> view -> transpose(1, 2) -> clone(contiguous)
-        with flat(x) = _unsafe_view(clone(expand(x))) and every link used once. The clone at the
+        with flat(x) = _unsafe_view(clone(expand(x))), or view(expand(x)) for a batch of one, whose
+        heads need no copy to be flattened, and every link used once. The clone at the
         end becomes the fused step over (q, k, v, scale, mask buffer, slices) and returns the
         [batch, tokens, heads, head_dim] tensor; everything in between is skipped. The plan of
         the _softmax node is replaced in place. Returns {fused clone node: every node the fused
@@ -358,20 +359,21 @@ class _GraphFactory:
                     and node.target in targets and len(node.users) == 1)
 
         def unflatten(node):
-            """_unsafe_view/view(clone(expand(x))) -> (x, [nodes])"""
+            """_unsafe_view/view([clone](expand(x))) -> (x, [nodes])"""
             if not single(node, aten._unsafe_view.default, aten.view.default):
                 return None
-            c = node.args[0]
-            if not single(c, aten.clone.default):
-                return None
-            e = c.args[0]
+            links = [node]
+            e = node.args[0]
+            if single(e, aten.clone.default):
+                links.append(e)
+                e = e.args[0]
             if not single(e, aten.expand.default):
                 return None
             src = e.args[0]
             val, eval_ = (src.meta.get("val") if isinstance(src, torch.fx.Node) else None), e.meta.get("val")
             if val is None or eval_ is None or tuple(val.shape) != tuple(eval_.shape) or val.dim() != 4:
                 return None  # the expand really broadcasts: not this pattern
-            return src, [node, c, e]
+            return src, [*links, e]
 
         for sm_node, plan in list(softmax_rewrites.items()):
             if plan is None or plan[0] != "softmax":
