@@ -277,6 +277,21 @@ int tmb_attention_decode(void* out, const void* q, const void* k, const void* v,
                          const int64_t* mask_strides, float scale, int causal, int dtype,
                          void* stream);
 
+/* One decode step over a growing key/value cache in one pass: k_out = [k_past ; k_new], v_out = [v_past ; v_new]
+ * along the token dimension, and out = softmax(scale * q k_out^T) v_out for the one query per (batch,
+ * head). k_past / v_past [batch, heads, past_len >= 1, head_dim] and the single rows q, k_new, v_new, out
+ * [batch, heads, 1, head_dim] are addressed through three element strides {batch, head, token} (16-byte
+ * aligned, multiples of 8); k_out and v_out are contiguous [batch, heads, past_len + 1, head_dim]. head_dim
+ * 64 or 128, fp16 / bf16. Returns TMB_ERR_UNSUPPORTED for anything else (the caller then concatenates and
+ * attends apart). Replaces `Cat2` (aten_fast.py:2203-2228) twice and
+ * `fast_aten_scaled_dot_product_attention` (aten_fast.py:5177-5285) on decode shapes. */
+int tmb_attention_decode_append(void* out, void* k_out, void* v_out, const void* q, const void* k_past,
+                                const void* v_past, const void* k_new, const void* v_new, int64_t batch,
+                                int64_t heads, int64_t past_len, int64_t head_dim, const int64_t* q_strides,
+                                const int64_t* k_strides, const int64_t* v_strides, const int64_t* k_new_strides,
+                                const int64_t* v_new_strides, const int64_t* out_strides, float scale, int dtype,
+                                void* stream);
+
 /* Embedding lookup: out[i, :] = table[indices[i], :] for a contiguous [num_rows, row_len] table of
  * type `dtype` and `num_indices` contiguous indices of type `index_dtype` (TMB_I64 or TMB_I32).
  * Replaces `Gather0(out, table, indices, idx_dtype, num_indices, row_len, dtype, ctx)`

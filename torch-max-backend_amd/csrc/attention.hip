@@ -279,12 +279,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 }
 
 // ---------------------------------------------------------------------------
-// Few queries per (batch, head): the decode step of a generation loop. One wave per query row;
-// the work is reading K and V once, so there is no MFMA: D/8 lanes share a key (16 bytes of the
-// row each), a wave covers 64/(D/8) keys per step with whole-row loads, every key group keeps its
-// own running maximum, sum and output chunk (online softmax), and the groups are merged at the
-// end. An optional boolean mask (broadcastable, True = takes part) and the top-left aligned
-// causal rule are applied to the scores; a row without any key comes out as NaN, as in ATen.
+// Few queries per (batch, head): the decode step of a generation loop. The work is reading K and V
+// once, so there is no MFMA: D/8 lanes share a key (16 bytes of the row each), a wave covers
+// 64/(D/8) keys per step with whole-row loads, every key group keeps its own running maximum, sum and
+// output chunk (online softmax), and the groups are merged at the end. An optional boolean mask
+// (broadcastable, True = takes part) and the top-left aligned causal rule are applied to the scores; a
+// row without any key comes out as NaN, as in ATen.
+//
+// What bounds it is how many loads are in flight: WPR waves share a query row (each takes every WPR-th
+// group of four steps, and their results meet in LDS in wave order), chosen so that a few thousand
+// waves run whatever the batch (one wave per row left 32 x 12 heads on 96 workgroups and 12 heads of a
+// single sequence on three), and a wave requests four steps of K and V at once.
+//
+// APPEND: the keys are a cache [batch, heads, kv_len - 1, D] plus one new row, and the pass that reads
+// them writes the grown caches [batch, heads, kv_len, D] on its way: a generation loop that
+// concatenates its cache and then attends to it moves the cache once in and once out instead of twice
+// in and once out.
 // ---------------------------------------------------------------------------
 struct AttnDecodeArgs {
   void* out;
@@ -301,15 +311,25 @@ struct AttnDecodeArgs {
   int heads, q_len, kv_len;
   float scale;
   int causal;
+  // APPEND only: the new rows and the grown caches (contiguous)
+  const void* k_new;
+  const void* v_new;
+  void* k_out;
+  void* v_out;
+  int64_t kn_sb, kn_sh, vn_sb, vn_sh;
 };
 
-template <typename T, int D>
-__global__ __launch_bounds__(256) void attention_decode_kernel(AttnDecodeArgs a) {
+template <typename T, int D, int WPR, bool APPEND>
+__global__ __launch_bounds__(WPR < 4 ? 256 : WPR * 64) void attention_decode_kernel(AttnDecodeArgs a) {
   constexpr int LPK = D / 8;        // lanes per key
   constexpr int KPI = kWave / LPK;  // keys per step of a wave
-  const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= a.rows) return;  // whole waves leave; no barriers below
+  constexpr int U = 4;              // steps in flight
+  constexpr int RPB = WPR < 4 ? 4 / WPR : 1;  // rows per workgroup
+  __shared__ float merged[WPR > 1 ? RPB * WPR * (D + 2) : 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int part = wave % WPR;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + wave / WPR;
+  if (WPR == 1 && row >= a.rows) return;  // whole waves leave; no barriers below (RPB is 1 otherwise)
   const int t = static_cast<int>(row % a.q_len);
   const int64_t bh = row / a.q_len;
   const int h = static_cast<int>(bh % a.heads);
@@ -321,6 +341,16 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnDecodeArgs a)
   const T* vbase = static_cast<const T*>(a.v) + b * a.v_sb + h * a.v_sh + sub * 8;
   const unsigned char* mrow =
       a.mask == nullptr ? nullptr : a.mask + b * a.m_sb + h * a.m_sh + t * a.m_st;
+  const T* knew = nullptr;
+  const T* vnew = nullptr;
+  T* kout = nullptr;
+  T* vout = nullptr;
+  if constexpr (APPEND) {
+    knew = static_cast<const T*>(a.k_new) + b * a.kn_sb + h * a.kn_sh + sub * 8;
+    vnew = static_cast<const T*>(a.v_new) + b * a.vn_sb + h * a.vn_sh + sub * 8;
+    kout = static_cast<T*>(a.k_out) + bh * a.kv_len * D + sub * 8;
+    vout = static_cast<T*>(a.v_out) + bh * a.kv_len * D + sub * 8;
+  }
 
   const float c = a.scale * 1.44269504088896340736f;  // scores in the log2 domain
   float qf[8];
@@ -335,26 +365,46 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnDecodeArgs a)
   for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
 
   const int last = a.causal ? (t < a.kv_len - 1 ? t : a.kv_len - 1) : a.kv_len - 1;
-  for (int s0 = 0; s0 <= last; s0 += KPI) {
-    const int s = s0 + kg;
-    bool valid = s <= last;
-    if (valid && mrow != nullptr) valid = mrow[s * a.m_ss] != 0;
-    const int sr = s <= last ? s : last;  // a readable row for lanes without a key
-    const Vec16<T> kv = load_vec16_stream(kbase + static_cast<int64_t>(sr) * a.k_st);
-    const Vec16<T> vv = load_vec16_stream(vbase + static_cast<int64_t>(sr) * a.v_st);
-    float x = 0.0f;
+  for (int s0 = part * (U * KPI); s0 <= last; s0 += WPR * (U * KPI)) {
+    Vec16<T> kv[U], vv[U];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x = __builtin_fmaf(qf[e], to_f32(kv.v[e]), x);
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * KPI + kg;
+      const int sr = s <= last ? s : last;  // a readable row for lanes without a key
+      const T* kp = kbase + static_cast<int64_t>(sr) * a.k_st;
+      const T* vp = vbase + static_cast<int64_t>(sr) * a.v_st;
+      if constexpr (APPEND) {
+        kp = sr == a.kv_len - 1 ? knew : kp;
+        vp = sr == a.kv_len - 1 ? vnew : vp;
+      }
+      kv[u] = load_vec16_stream(kp);
+      vv[u] = load_vec16_stream(vp);
+    }
 #pragma unroll
-    for (int w = 1; w < LPK; w <<= 1) x += __shfl_xor(x, w, kWave);
-    if (valid) {
-      const float m_new = fmaxf(m, x);
-      const float corr = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the first key (m = -inf)
-      const float p = __builtin_amdgcn_exp2f(x - m_new);
-      l = l * corr + p;
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * KPI + kg;
+      bool valid = s <= last;
+      if constexpr (APPEND) {
+        if (valid) {
+          store_vec16_stream(kout + static_cast<int64_t>(s) * D, kv[u]);
+          store_vec16_stream(vout + static_cast<int64_t>(s) * D, vv[u]);
+        }
+      }
+      if (valid && mrow != nullptr) valid = mrow[s * a.m_ss] != 0;
+      float x = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = acc[e] * corr + p * to_f32(vv.v[e]);
-      m = m_new;
+      for (int e = 0; e < 8; ++e) x = __builtin_fmaf(qf[e], to_f32(kv[u].v[e]), x);
+#pragma unroll
+      for (int w = 1; w < LPK; w <<= 1) x += __shfl_xor(x, w, kWave);
+      if (valid) {
+        const float m_new = fmaxf(m, x);
+        const float corr = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the first key (m = -inf)
+        const float p = __builtin_amdgcn_exp2f(x - m_new);
+        l = l * corr + p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = acc[e] * corr + p * to_f32(vv[u].v[e]);
+        m = m_new;
+      }
     }
   }
   // merge the key groups (lanes with equal `sub`)
@@ -371,6 +421,34 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnDecodeArgs a)
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], w, kWave);
   }
+  if constexpr (WPR > 1) {  // then the waves of the row, in wave order
+    float* mine = merged + wave * (D + 2);
+    if (kg == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mine[sub * 8 + e] = acc[e];
+      if (sub == 0) {
+        mine[D] = big;
+        mine[D + 1] = l;
+      }
+    }
+    __syncthreads();
+    if (part != 0 || kg != 0) return;
+    const float* all = merged + (wave / WPR) * WPR * (D + 2);
+    float top = neg_inf;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) top = fmaxf(top, all[w * (D + 2) + D]);
+    l = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) {
+      const float mw = all[w * (D + 2) + D];
+      const float f = mw == neg_inf ? 0.0f : __builtin_amdgcn_exp2f(mw - top);
+      l += f * all[w * (D + 2) + D + 1];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += f * all[w * (D + 2) + sub * 8 + e];
+    }
+  }
   if (kg == 0) {
     float r[8];
 #pragma unroll
@@ -378,6 +456,22 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnDecodeArgs a)
     T* dst = static_cast<T*>(a.out) + b * a.o_sb + h * a.o_sh + t * a.o_st + sub * 8;
     store_converted<T, 8>(dst, r);
   }
+}
+
+// Waves per row: enough that about four thousand run, and at least one group of steps for each.
+template <typename T, int D, bool APPEND>
+static int launch_decode(const AttnDecodeArgs& a, hipStream_t s) {
+  constexpr int kGroup = 4 * kWave / (D / 8);  // keys a wave requests at once
+  const int64_t groups = (a.kv_len + kGroup - 1) / kGroup;
+  const unsigned rows = static_cast<unsigned>(a.rows);
+  if (a.rows > 2048 || groups < 2) {
+    attention_decode_kernel<T, D, 1, APPEND><<<dim3(static_cast<unsigned>((a.rows + 3) / 4)), dim3(256), 0, s>>>(a);
+  } else if (a.rows > 512 || groups < 8) {
+    attention_decode_kernel<T, D, 4, APPEND><<<dim3(rows), dim3(256), 0, s>>>(a);
+  } else {
+    attention_decode_kernel<T, D, 16, APPEND><<<dim3(rows), dim3(1024), 0, s>>>(a);
+  }
+  return check_launch();
 }
 
 }  // namespace tmb
@@ -471,14 +565,48 @@ extern "C" int tmb_attention_decode(void* out, const void* q, const void* k, con
                    mask ? mask_strides[2] : 0, mask ? mask_strides[3] : 0,
                    batch * heads * q_len, static_cast<int>(heads), static_cast<int>(q_len),
                    static_cast<int>(kv_len), scale, causal ? 1 : 0};
-  const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define TMB_AD(T, D) attention_decode_kernel<T, D><<<grid, dim3(256), 0, s>>>(a)
-  if (dtype == TMB_BF16) {
-    if (head_dim == 64) TMB_AD(bf16_t, 64); else TMB_AD(bf16_t, 128);
-  } else {
-    if (head_dim == 64) TMB_AD(f16_t, 64); else TMB_AD(f16_t, 128);
-  }
-#undef TMB_AD
-  return check_launch();
+  if (dtype == TMB_BF16) return head_dim == 64 ? launch_decode<bf16_t, 64, false>(a, s) : launch_decode<bf16_t, 128, false>(a, s);
+  return head_dim == 64 ? launch_decode<f16_t, 64, false>(a, s) : launch_decode<f16_t, 128, false>(a, s);
+}
+
+extern "C" int tmb_attention_decode_append(void* out, void* k_out, void* v_out, const void* q, const void* k_past,
+                                           const void* v_past, const void* k_new, const void* v_new, int64_t batch,
+                                           int64_t heads, int64_t past_len, int64_t head_dim,
+                                           const int64_t* q_strides, const int64_t* k_strides,
+                                           const int64_t* v_strides, const int64_t* k_new_strides,
+                                           const int64_t* v_new_strides, const int64_t* out_strides, float scale,
+                                           int dtype, void* stream) {
+  using namespace tmb;
+  if (batch < 0 || heads < 0 || past_len < 0) return TMB_ERR_INVALID_ARGUMENT;
+  if (dtype != TMB_F16 && dtype != TMB_BF16) return TMB_ERR_UNSUPPORTED;
+  if (head_dim != 64 && head_dim != 128) return TMB_ERR_UNSUPPORTED;
+  if (!(scale == scale)) return TMB_ERR_INVALID_ARGUMENT;
+  if (batch == 0 || heads == 0) return TMB_OK;
+  if (past_len == 0) return TMB_ERR_UNSUPPORTED;
+  if (!out || !k_out || !v_out || !q || !k_past || !v_past || !k_new || !v_new || !q_strides || !k_strides ||
+      !v_strides || !k_new_strides || !v_new_strides || !out_strides)
+    return TMB_ERR_INVALID_ARGUMENT;
+  if (heads >= (int64_t{1} << 31) || past_len >= (int64_t{1} << 30) || batch * heads >= (int64_t{1} << 31))
+    return TMB_ERR_UNSUPPORTED;
+  auto aligned = [](const void* p, const int64_t* s) {
+    return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0 &&
+           s[0] >= 0 && s[1] >= 0 && s[2] >= 0;
+  };
+  if (!aligned(q, q_strides) || !aligned(k_past, k_strides) || !aligned(v_past, v_strides) ||
+      !aligned(k_new, k_new_strides) || !aligned(v_new, v_new_strides) || !aligned(out, out_strides) ||
+      !aligned16(k_out) || !aligned16(v_out))
+    return TMB_ERR_UNSUPPORTED;
+  AttnDecodeArgs a{out, q, k_past, v_past, nullptr,
+                   q_strides[0], q_strides[1], q_strides[2],
+                   k_strides[0], k_strides[1], k_strides[2],
+                   v_strides[0], v_strides[1], v_strides[2],
+                   out_strides[0], out_strides[1], out_strides[2],
+                   0, 0, 0, 0,
+                   batch * heads, static_cast<int>(heads), 1, static_cast<int>(past_len + 1), scale, 0,
+                   k_new, v_new, k_out, v_out,
+                   k_new_strides[0], k_new_strides[1], v_new_strides[0], v_new_strides[1]};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == TMB_BF16) return head_dim == 64 ? launch_decode<bf16_t, 64, true>(a, s) : launch_decode<bf16_t, 128, true>(a, s);
+  return head_dim == 64 ? launch_decode<f16_t, 64, true>(a, s) : launch_decode<f16_t, 128, true>(a, s);
 }

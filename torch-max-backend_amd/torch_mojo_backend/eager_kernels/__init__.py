@@ -49,6 +49,7 @@ SIGNATURES = {
     "tmb_attention_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "tmb_attention_bwd": (_ci, [_vp] * 10 + [_i64] * 5 + [_vp] * 8 + [_flt, _ci, _ci, _vp]),
     "tmb_attention_decode": (_ci, [_vp] * 5 + [_i64] * 5 + [_vp] * 5 + [_flt, _ci, _ci, _vp]),
+    "tmb_attention_decode_append": (_ci, [_vp] * 8 + [_i64] * 4 + [_vp] * 6 + [_flt, _ci, _vp]),
     "tmb_gelu": (_ci, [_vp, _vp, _i64, _ci, _ci, _vp]),
     "tmb_gather_rows": (_ci, [_vp, _vp, _vp, _i64, _i64, _i64, _ci, _ci, _vp]),
     "tmb_gelu_backward": (_ci, [_vp, _vp, _vp, _i64, _ci, _ci, _vp]),

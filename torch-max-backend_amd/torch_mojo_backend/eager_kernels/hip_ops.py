@@ -600,16 +600,20 @@ def attention_decode_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
 
 def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                      causal: bool, attn_mask: Optional[torch.Tensor] = None,
-                     checked: bool = False) -> torch.Tensor:
+                     checked: bool = False, token_major: bool = False) -> torch.Tensor:
     """softmax(scale q kᵀ [masked]) v for a few queries per head in one launch; returns
-    [batch, heads, tokens, head_dim] contiguous. `checked`: the caller has just seen
+    [batch, heads, tokens, head_dim] contiguous, or with `token_major` the transposed view of a
+    [batch, tokens, heads, head_dim] tensor. `checked`: the caller has just seen
     `attention_decode_supported` accept exactly these operands."""
     if not checked:
         require_hip(q, k, v, attn_mask)
         if not attention_decode_supported(q, k, v, attn_mask):
             raise ValueError("attention_decode: unsupported operands (see attention_decode_supported)")
     b, h, t, d = q.shape
-    out = torch.empty((b, h, t, d), dtype=q.dtype, device=q.device)
+    if token_major:
+        out = torch.empty((b, t, h, d), dtype=q.dtype, device=q.device).transpose(1, 2)
+    else:
+        out = torch.empty((b, h, t, d), dtype=q.dtype, device=q.device)
     i64x3 = _I64X3
     mask_ptr, mask_strides = None, None
     if attn_mask is not None:
@@ -619,10 +623,35 @@ def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     rc = _ek.lib().tmb_attention_decode(
         out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), mask_ptr, b, h, t, k.shape[2], d,
         i64x3(qs[0], qs[1], qs[2]), i64x3(ks[0], ks[1], ks[2]), i64x3(vs[0], vs[1], vs[2]),
-        i64x3(h * t * d, t * d, d), mask_strides, float(scale), int(bool(causal)),
+        i64x3(*out.stride()[:3]), mask_strides, float(scale), int(bool(causal)),
         _CODES[q.dtype], _stream())
     _check("tmb_attention_decode", rc)
     return out
+
+
+def attention_decode_append(q, k_past, v_past, k_new, v_new, scale: float):
+    """One decode step over a growing cache: (out [batch, heads, 1, head_dim], k, v) with
+    k = cat([k_past, k_new], 2), v likewise and out = softmax(scale q kᵀ) v, in one pass over the
+    cache. None when the kernel does not take these tensors."""
+    if not attention_decode_supported(q, k_past, v_past, None) or q.shape[2] != 1:
+        return None
+    b, h, _, d = q.shape
+    for x in (k_new, v_new):
+        if not x.is_cuda or x.dtype != q.dtype or tuple(x.shape) != (b, h, 1, d) or x.stride(3) != 1 \
+                or any(s % 8 or s < 0 for s in x.stride()[:3]) or x.data_ptr() % 16:
+            return None
+    past = k_past.shape[2]
+    out = torch.empty((b, h, 1, d), dtype=q.dtype, device=q.device)
+    k = torch.empty((b, h, past + 1, d), dtype=q.dtype, device=q.device)
+    v = torch.empty_like(k)
+    st = [_I64X3(*x.stride()[:3]) for x in (q, k_past, v_past, k_new, v_new, out)]
+    rc = _ek.lib().tmb_attention_decode_append(
+        out.data_ptr(), k.data_ptr(), v.data_ptr(), q.data_ptr(), k_past.data_ptr(), v_past.data_ptr(),
+        k_new.data_ptr(), v_new.data_ptr(), b, h, past, d, *st, float(scale), _CODES[q.dtype], _stream())
+    if rc == _ek.ERR_UNSUPPORTED:
+        return None
+    _check("tmb_attention_decode_append", rc)
+    return out, k, v
 
 
 def attention_composed(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,

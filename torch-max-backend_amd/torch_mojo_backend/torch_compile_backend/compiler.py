@@ -595,6 +595,53 @@ class _GraphFactory:
         return out
 
     @staticmethod
+    def _fuse_decode_append(graph: torch.fx.Graph) -> dict:
+        """The attention of one decode step over a cache that grows by concatenation:
+        cat([k_past, k_new], 2) and cat([v_past, v_new], 2), one new token each, ->
+        _scaled_dot_product_flash_attention of one query per head, of whose results only the first
+        is used. The attention node becomes one step that also writes the two grown caches
+        (`hip_ops.attention_decode_append`), which take the place of the cat nodes; every other
+        user of those comes later. Returns {node: None (its value comes from the fused step) |
+        ("decode_append", q, k_past, v_past, k_new, v_new, scale, k cat, v cat)}."""
+        plans: dict = {}
+        flash = aten._scaled_dot_product_flash_attention
+        if MAPPING_TORCH_ATEN_TO_MOJO.get(flash) is not _BUILTIN_FLASH or \
+                MAPPING_TORCH_ATEN_TO_MOJO.get(aten.cat) is not _BUILTIN_CAT:
+            return plans
+        order = {n: i for i, n in enumerate(graph.nodes)}
+        for node in graph.nodes:
+            if node.op != "call_function" or node.target is not flash.default or len(node.args) < 3:
+                continue
+            rest = list(node.args[3:]) + [0.0, False, False][len(node.args) - 3:]
+            if rest != [0.0, False, False] or set(node.kwargs) - {"scale"} or \
+                    not isinstance(node.kwargs.get("scale"), (int, float, type(None))) or \
+                    any(u.target is not operator.getitem or u.args[1] != 0 for u in node.users):
+                continue
+            q, pairs = node.args[0], []
+            for x in node.args[1:3]:
+                if not (isinstance(x, torch.fx.Node) and x.op == "call_function"
+                        and x.target is aten.cat.default and len(x.args) == 2 and x.args[1] in (2, -2)
+                        and isinstance(x.args[0], (list, tuple)) and len(x.args[0]) == 2):
+                    break
+                past, new = x.args[0]
+                vals = [n.meta.get("val") for n in (q, past, new)]
+                if any(v is None or v.dim() != 4 for v in vals) or \
+                        any(v.dtype not in (torch.bfloat16, torch.float16) for v in vals) or \
+                        any(not isinstance(v.shape[2], int) or v.shape[2] != 1 for v in (vals[0], vals[2])) or \
+                        any(order[u] < order[node] for u in x.users) or x in plans:
+                    break
+                pairs.append((past, new, x))
+            if len(pairs) != 2 or pairs[0][2] is pairs[1][2]:
+                continue
+            (kp, kn, kc), (vp, vn, vc) = pairs
+            scale = node.kwargs.get("scale")
+            if scale is None:
+                scale = 1.0 / float(q.meta["val"].shape[3]) ** 0.5
+            plans[node] = ("decode_append", q, kp, vp, kn, vn, float(scale), kc, vc)
+            plans[kc] = plans[vc] = None
+        return plans
+
+    @staticmethod
     def _widen_residual_stream(plans: dict) -> None:
         """A fused residual step of a 16-bit graph whose result only feeds other fused residual
         steps (as their residual operand) and native_layer_norm nodes (as their input) hands that
@@ -686,6 +733,22 @@ class _GraphFactory:
             except Exception:  # noqa: BLE001 - without a verdict the step runs its ops unfused
                 pass
 
+    def _emit(self, fn, key, args, kwargs, node: torch.fx.Node, idx: int) -> None:
+        """Appends a step that computes `node`'s value; `idx` is the position it runs at."""
+        step = _Step()
+        step.fn = fn
+        step.key = key
+        step.args = self._convert(args)
+        step.kwargs = self._convert(kwargs)
+        step.dynamic_args = _has_slot(step.args)
+        step.dynamic_kwargs = _has_slot(step.kwargs)
+        step.flat = _flat_plan(step.args) if step.dynamic_args else None
+        step.out = self.slots.setdefault(node.name, len(self.slots))
+        step.node = node
+        step.node_idx = idx
+        step.release = ()
+        self.steps.append(step)
+
     def create_graph(self, graph: torch.fx.Graph):
         rewrites = self._fuse_bias_gelu(graph) if _fusion_enabled() else {}
         softmax_rewrites = self._fuse_masked_softmax(graph) if _fusion_enabled() else {}
@@ -699,6 +762,7 @@ class _GraphFactory:
                 self._widen_residual_stream(softmax_rewrites)
             softmax_rewrites.update(self._fuse_loss_backward(graph))
             softmax_rewrites.update(self._fuse_norm_backward_add(graph))
+            softmax_rewrites.update(self._fuse_decode_append(graph))
         nodes = list(graph.nodes)
         # what each node reads after the rewrites (liveness must follow the rewritten program)
         reads: dict = {}
@@ -719,6 +783,8 @@ class _GraphFactory:
                     reads[node] = list(node.all_input_nodes) + ([plan[1]] if plan[1] is not None else [])
                 elif plan[0] in ("take", "colsum"):
                     reads[node] = [plan[1]]
+                elif plan[0] == "decode_append":
+                    reads[node] = list(plan[1:6])
                 else:
                     reads[node] = [plan[1], plan[2], plan[3], plan[5]]
             else:
@@ -765,6 +831,8 @@ class _GraphFactory:
                         fn, args, kwargs = _identity, (plan[1],), {}
                     elif plan[0] == "colsum":
                         fn, args, kwargs = _TAKE_COLUMN_SUMS, (plan[1], plan[2]), {}
+                    elif plan[0] == "decode_append":
+                        fn, args, kwargs = _fused_decode_append, plan[1:7], {}
                     else:
                         fn, kwargs = _FUSED_ATTENTION, {}
                         args = plan[1:]
@@ -781,20 +849,11 @@ class _GraphFactory:
                     # no step at all: a fused step later does this node's work
                     self.slots[node.name] = len(self.slots)
                     continue
-                step = _Step()
-                step.fn = fn
-                step.key = key
-                step.args = self._convert(args)
-                step.kwargs = self._convert(kwargs)
-                step.dynamic_args = _has_slot(step.args)
-                step.dynamic_kwargs = _has_slot(step.kwargs)
-                step.flat = _flat_plan(step.args) if step.dynamic_args else None
-                self.slots[node.name] = len(self.slots)
-                step.out = self.slots[node.name]
-                step.node = node
-                step.node_idx = idx
-                step.release = ()
-                self.steps.append(step)
+                self._emit(fn, key, args, kwargs, node, idx)
+                plan = softmax_rewrites.get(node)
+                if plan is not None and plan[0] == "decode_append":
+                    for i, grown in enumerate(plan[7:9], start=1):   # the grown caches
+                        self._emit(operator.getitem, operator.getitem, (node, i), {}, grown, idx)
             elif node.op == "output":
                 self.output_template = self._convert(node.args[0])
             else:
@@ -1021,6 +1080,16 @@ def _fused_norm_backward_add(grad_out, input, normalized_shape, mean, rstd, weig
     return dx, dw, db, sums
 
 
+def _fused_decode_append(q, k_past, v_past, k_new, v_new, scale):
+    """(attention of the one query per head over the grown caches, k, v)."""
+    from ..eager_kernels import hip_ops
+    done = hip_ops.attention_decode_append(q, k_past, v_past, k_new, v_new, scale)
+    if done is not None:
+        return done
+    k, v = _BUILTIN_CAT([k_past, k_new], 2), _BUILTIN_CAT([v_past, v_new], 2)
+    return _BUILTIN_FLASH(q, k, v, scale=scale)[0], k, v
+
+
 def _take_column_sums(backward_result, shape):
     return backward_result[3].view(shape)
 
@@ -1175,6 +1244,8 @@ _BUILTIN_LOG_SOFTMAX_BACKWARD = MAPPING_TORCH_ATEN_TO_MOJO.get(aten._log_softmax
 _BUILTIN_NLL_LOSS_BACKWARD = MAPPING_TORCH_ATEN_TO_MOJO.get(aten.nll_loss_backward)
 _BUILTIN_LAYER_NORM_BACKWARD = MAPPING_TORCH_ATEN_TO_MOJO.get(aten.native_layer_norm_backward)
 _BUILTIN_SUM = MAPPING_TORCH_ATEN_TO_MOJO.get(aten.sum)
+_BUILTIN_CAT = MAPPING_TORCH_ATEN_TO_MOJO.get(aten.cat)
+_BUILTIN_FLASH = MAPPING_TORCH_ATEN_TO_MOJO.get(aten._scaled_dot_product_flash_attention)
 _FUSED_ADDMM_GELU = _fused_addmm_gelu
 _FUSED_MASKED_SOFTMAX = _fused_masked_softmax
 _FUSED_ATTENTION = _fused_attention
