@@ -177,41 +177,55 @@ def _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, plain_epilogue=True) -> boo
     """Whether the matrix-core kernels take these operands as they lie (mirrors the library's
     own checks; when it says no, the library would run its any-layout kernel, which is one to two
     orders of magnitude slower on large products)."""
-    if a.element_size() == 4:   # the fp32 kernel takes any alignment and extent
-        return True
-    if la[1] % 8 or lb[1] % 8 or a.data_ptr() % 16 or b.data_ptr() % 16:
+    unit = 16 // a.element_size()  # elements per 16-byte vector: 8 (16-bit) or 4 (fp32)
+    if la[1] % unit or lb[1] % unit or a.data_ptr() % 16 or b.data_ptr() % 16:
         return False
-    if batched and a.shape[0] > 1 and (a.stride(0) % 8 or b.stride(0) % 8):
+    if batched and a.shape[0] > 1 and (a.stride(0) % unit or b.stride(0) % unit):
         return False
+    if a.element_size() == 4:
+        return (m if la[0] else k) % 4 == 0 and (k if lb[0] else n) % 4 == 0
     if la[0]:  # A stored [K, M]: the weight-gradient form, with B stored [K, N] and no epilogue
         return plain_epilogue and not lb[0] and k % 32 == 0 and k >= 256 and m % 8 == 0 \
             and n % 8 == 0 and n > 64
     return k % 8 == 0
 
 
+def _f32_in_place(a, la, lb, m, n, k) -> bool:
+    """Whether the fp32 kernel reads these operands where they lie, whatever their alignment (mirrors
+    the library's check): four elements along each contiguous direction."""
+    return a.element_size() == 4 and (m if la[0] else k) >= 4 and (k if lb[0] else n) >= 4 \
+        and la[1] < 1 << 23 and lb[1] < 1 << 23
+
+
 def _relayout_for_mfma(a, b, la, lb, m, n, k, batched, plain=True):
-    """Re-lays the 16-bit operands of a large product so that the matrix-core kernels take it. A
+    """Re-lays the operands of a large product so that the matrix-core kernels take it. A
     contraction length or pitch that is not whole 16-byte vectors (a 50257-wide vocabulary as K)
     is zero-padded; B becomes K-major where its own pitch is the obstacle; a transposed A with an
     odd M in the weight-gradient form keeps its form and gets zero columns (the product then has
     a few extra rows, which the caller drops); any other transposed A becomes row-major.
     `plain`: no epilogue and no residual. Returns (a, b, la, lb, k, rows of the launch)."""
+    unit = 16 // a.element_size()
     if la[0]:
-        keep_form = plain and not batched and lb[1] % 8 == 0 and b.data_ptr() % 16 == 0 and not lb[0] \
-            and k % 32 == 0 and k >= 256 and n % 8 == 0 and n > 64
+        b_fits = lb[1] % unit == 0 and b.data_ptr() % 16 == 0
+        if a.element_size() == 2:
+            keep_form = plain and not batched and b_fits and not lb[0] and k % 32 == 0 \
+                and k >= 256 and n % 8 == 0 and n > 64
+        else:
+            keep_form = not batched and b_fits and (k if lb[0] else n) % 4 == 0
         if keep_form:
             # (the same width as a contraction length of m gets below, so that one padded copy
             # can serve both products of a backward pass)
-            mp = m if m % 8 == 0 else (m + 63) // 64 * 64
+            mp = m if m % unit == 0 else (m + 63) // 64 * 64
             stored = _pad_last(a.transpose(-1, -2), mp)          # [K, mp], zero columns
             return stored.transpose(-1, -2), b, (1, mp), lb, k, mp
         a = a.contiguous()                      # [.., M, K] row-major (a transposing copy)
-    kp = k if k % 8 == 0 else (k + 63) // 64 * 64
-    if a.shape[-1] != kp or a.stride(-2) % 8 or a.data_ptr() % 16 or not a.is_contiguous():
+    kp = k if k % unit == 0 else (k + 63) // 64 * 64
+    if a.shape[-1] != kp or a.stride(-2) % unit or a.data_ptr() % 16 or not a.is_contiguous():
         a = _pad_last(a, kp)
     bt = b.transpose(-1, -2)                    # [.., N, K]
-    n_major_ok = not lb[0] and lb[1] % 8 == 0 and b.data_ptr() % 16 == 0
-    k_major_ok = bool(lb[0]) and lb[1] % 8 == 0 and b.data_ptr() % 16 == 0 and kp == k
+    n_major_ok = not lb[0] and lb[1] % unit == 0 and b.data_ptr() % 16 == 0 and \
+        (a.element_size() == 2 or n % 4 == 0)
+    k_major_ok = bool(lb[0]) and lb[1] % unit == 0 and b.data_ptr() % 16 == 0 and kp == k
     if n_major_ok:
         if kp != k:                             # rows of zeros below the last k
             grown = torch.empty(tuple(b.shape[:-2]) + (kp, n), dtype=b.dtype, device=b.device)
@@ -309,8 +323,8 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         b = b.contiguous()
         lb = (0, max(n, 1))
     m_given = m
-    if batch * m * n * k >= _RELAYOUT_MIN_WORK and not _mfma_layouts_ok(
-            a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE):
+    if batch * m * n * k >= _RELAYOUT_MIN_WORK and not _f32_in_place(a, la, lb, m, n, k) \
+            and not _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE):
         a, b, la, lb, k, m = _relayout_for_mfma(a, b, la, lb, m, n, k, batched,
                                                 epilogue == _ek.EPI_NONE and residual is None)
     out_shape = (batch, m, n) if batched else (m, n)
