@@ -183,6 +183,14 @@ size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, 
 /* The same for a known operand layout: 0 also where a kernel that needs no scratch takes the product. */
 size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a,
                                        int trans_b, int dtype);
+/* 16-bit operands that are not whole aligned 16-byte vectors (lda, ldb or k no multiple of eight, a base
+ * or batch stride off a 16-byte boundary: a_aligned / b_aligned 0), or a transposed A the aligned kernels do
+ * not take: the bytes of workspace with which multiplying them where they lie is fastest (0: none), or -1
+ * where zero-padding them into aligned buffers first is faster, or where only the any-layout kernel takes
+ * them. `plain`: no epilogue and no residual. tmb_gemm* take such operands either way. */
+int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda,
+                                          int64_t ldb, int a_aligned, int b_aligned, int trans_a, int trans_b,
+                                          int plain, int dtype);
 int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch, int64_t m,
                 int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, int64_t stride_a,
                 int64_t stride_b, int64_t stride_c, int trans_a, int trans_b, int dtype,

@@ -16,7 +16,7 @@ if [ -n "$TMB_VARIANT" ]; then
 fi
 HIPCC="${HIPCC:-/opt/rocm/bin/hipcc}"
 FLAGS="--offload-arch=gfx950 -O3 -std=c++17 -fPIC -Wno-inline-asm -Xclang -target-feature -Xclang -packed-fp32-ops"
-units="gemm_bf16 gemm_f16 gemm_f32 gemm_small softmax layer_norm reduce reduce_cols gemm attention attention_bwd backward misc"
+units="gemm_bf16 gemm_f16 gemm_f32 gemm_small gemm_any softmax layer_norm reduce reduce_cols gemm attention attention_bwd backward misc"
 objs=""
 pids=""
 for f in $units; do

@@ -12,6 +12,8 @@
 // Workgroups are numbered so that the 32 tiles resident on one XCD form a compact patch of
 // C and share A/B panels through that XCD's L2.
 //
+// 16-bit operands that are not whole aligned 16-byte vectors: gemm_any.h.
+//
 // Fallback path: a 64x64 SIMT tile kernel that takes any dtype, strides and alignment.
 //
 // Arithmetic contract: fp32 accumulate, bias added in fp32 before the single down-cast
@@ -76,7 +78,8 @@ static int gemm_entry(void* c, const void* a, const void* b, const void* bias,
   if (out_f32 && residual == nullptr) return TMB_ERR_UNSUPPORTED;  // fp32 C exists for the residual form only
   if (residual != nullptr) {
     // only the MFMA kernels carry the second epilogue step; the caller adds separately otherwise
-    if (k == 0 || ldr < n || (dtype != TMB_F32 && !mfma_eligible(g, batch, trans_a, trans_b)))
+    if (k == 0 || ldr < n || (dtype != TMB_F32 && !mfma_eligible(g, batch, trans_a, trans_b) &&
+                              !any_eligible(m, n, k, lda, ldb, trans_a, trans_b)))
       return TMB_ERR_UNSUPPORTED;
     // fp32 operands of the epilogue and an epilogue that stays in fp32 exist without GELU only
     if ((resid_f32 || out_f32 || !twice) && epilogue != TMB_EPI_NONE) return TMB_ERR_UNSUPPORTED;
@@ -129,6 +132,18 @@ extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int6
     return static_cast<size_t>(tmb::f32_plan(batch, m, n, k).splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
   }
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
+}
+
+extern "C" int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda,
+                                                     int64_t ldb, int a_aligned, int b_aligned, int trans_a,
+                                                     int trans_b, int plain, int dtype) {
+  if ((dtype != TMB_F16 && dtype != TMB_BF16) || batch < 1 || batch > 65535) return -1;
+  if (!tmb::any_eligible(m, n, k, lda, ldb, trans_a, trans_b)) return -1;
+  const tmb::AnyPlan plan = tmb::any_plan(batch, m, n, k, true);
+  if (plan.cost > tmb::padded_cost(batch, m, n, k, lda, ldb, a_aligned != 0, b_aligned != 0, trans_a, trans_b,
+                                   plain != 0))
+    return -1;
+  return static_cast<int64_t>(plan.splits) * m * n * 4;
 }
 
 extern "C" int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch,

@@ -69,6 +69,77 @@ static inline bool small_applies(int64_t batch, int64_t m, int64_t n, int64_t k)
 }
 int gemm_small(const GemmArgs& g, int64_t batch, int trans_b, bool bf16, int epilogue, hipStream_t stream);
 
+// 16-bit operands in any layout and at any alignment (gemm_any.h): tile and split count. A launch takes,
+// in microseconds, a start and per round of tiles their operands' bytes at the rate a workgroup's
+// unaligned pieces arrive (half of the aligned kernel's above) and the partial tiles' way through LDS;
+// several workgroups share a CU, hence the power instead of whole rounds. Fitted to 70 shapes of 8 .. 8192
+// rows, 64 .. 50257 columns and K 64 .. 30001 in all layouts, within 15-20 % (rms) of each tile; the tile
+// it picks takes 3 % longer than the best one on average. A split adds its reduction.
+struct AnyTile {
+  int bm, bn;
+  double start, bytes_per_us, lds, power;
+};
+constexpr AnyTile kAnyTiles[] = {{16, 16, 3.4, 38e3, 0.3, 1.08}, {16, 32, 3.1, 44e3, 0.9, 1.0},
+                                 {32, 32, 3.1, 49e3, 1.0, 1.02}, {32, 32, 3.5, 41e3, 0.5, 0.96},
+                                 {64, 64, 2.6, 43e3, 3.7, 0.88}};
+struct AnyPlan {
+  int tile;    // index into kAnyTiles
+  int splits;  // 0: not split
+  double cost;
+};
+static inline AnyPlan any_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool may_split) {
+  AnyPlan p{0, 0, 0.0};
+  auto consider = [&](int splits) {
+    const int64_t runs = splits > 0 ? splits : batch;
+    const double depth = static_cast<double>(k) / (splits > 0 ? splits : 1);
+    for (int i = 0; i < static_cast<int>(sizeof(kAnyTiles) / sizeof(kAnyTiles[0])); ++i) {
+      const AnyTile& t = kAnyTiles[i];
+      const double tiles = static_cast<double>((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * runs;
+      const double rounds = tiles <= 256.0 ? 1.0 : std::pow(tiles / 256.0, t.power);
+      double cost = t.start + rounds * ((t.bm + t.bn) * 2.0 * depth / t.bytes_per_us + t.lds);
+      if (splits > 0) cost += 5.5 + 1e-6 * splits * m * n;
+      if (p.cost == 0.0 || cost < p.cost) p = AnyPlan{i, splits, cost};
+    }
+  };
+  consider(0);
+  if (may_split && batch == 1 && m * n < (int64_t{1} << 31))
+    for (const int s : {2, 3, 4, 6, 8, 12, 16})
+      if (k >= 192 * s) consider(s);
+  return p;
+}
+// What that kernel asks of its operands: eight elements along each contiguous direction, and lane
+// offsets within a tile that fit 32 bits.
+static inline bool any_eligible(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int trans_a, int trans_b) {
+  if (m < 1 || n < 1 || k < 1) return false;
+  if ((trans_a ? m : k) < 8 || (trans_b ? k : n) < 8) return false;
+  return lda < (int64_t{1} << 23) && ldb < (int64_t{1} << 23);
+}
+// Microseconds of the other way for the same operands: copy what the ring kernels cannot read into padded
+// buffers (3 us and the bytes at 4 TB/s each; a transposing copy at 1 TB/s), then multiply at 900
+// TFLOP/s in rounds of 128 x 128 tiles, two per CU. Within 15 % of the measured sum for products from
+// 10 GFLOP on (4099^3 198 against 197, 4383 x 1568 x 1228 38 against 38, 1829 x 3429 x 4716 147 against 156).
+static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool a_ok,
+                                 bool b_ok, int trans_a, int trans_b, bool plain) {
+  const double tiles = static_cast<double>((m + 127) / 128) * ((n + 127) / 128) * batch;
+  double cost = 6.0 + (tiles <= 256.0 ? 0.011 * k : std::ceil(tiles / 512.0) * 0.0186 * k);
+  auto copy = [&](int64_t elements, bool transposing) {
+    return 3.0 + static_cast<double>(elements) * batch * 4.0 / (transposing ? 1e6 : 4e6);
+  };
+  const bool b_fits = b_ok && ldb % 8 == 0;
+  if (trans_a) {
+    const bool keeps_form = plain && batch == 1 && b_fits && !trans_b && k % 32 == 0 && k >= 256 && n % 8 == 0 && n > 64;
+    if (keeps_form) return cost + copy(m * k, false);
+    cost += copy(m * k, true) + (k % 8 != 0 ? copy(m * k, false) : 0.0);
+  } else if (k % 8 != 0 || lda % 8 != 0 || !a_ok) {
+    cost += copy(m * k, false);
+  }
+  if (trans_b ? !b_fits || k % 8 != 0 : b_fits && k % 8 != 0) cost += copy(n * k, false);
+  else if (!trans_b && !b_fits) cost += copy(n * k, true);
+  return cost;
+}
+int gemm_any(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, bool bf16, int epilogue,
+             hipStream_t stream);
+
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
 // leave most CUs idle. K is cut into `splits` runs of whole stages (equal to within one stage)
 // that run as the y dimension of one launch of a ring kernel and store fp32 partials

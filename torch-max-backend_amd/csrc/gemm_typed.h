@@ -267,6 +267,30 @@ static int gemm_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, 
   return check_launch();
 }
 
+// Operands that the kernels above cannot read, where they lie.
+template <typename T, int EPI>
+static int gemm_unaligned(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, hipStream_t stream, void* workspace,
+                          size_t workspace_bytes) {
+  AnyPlan plan = any_plan(batch, g.m, g.n, g.k, true);
+  if (plan.splits > 0 &&
+      (workspace == nullptr || workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
+    plan = any_plan(batch, g.m, g.n, g.k, false);
+  constexpr bool BF16 = __is_same(T, bf16_t);
+  if (plan.splits == 0) return gemm_any(g, batch, plan.tile, trans_a, trans_b, BF16, EPI, stream);
+  GemmArgs part = g;
+  part.c = workspace;
+  part.bias = nullptr;
+  part.residual = nullptr;
+  part.ldc = g.n;
+  part.stride_c = g.m * g.n;
+  part.splits = plan.splits;
+  const int rc = gemm_any(part, plan.splits, plan.tile, trans_a, trans_b, BF16, TMB_EPI_NONE, stream);
+  if (rc != 0) return rc;
+  launch_splitk_reduce<T, EPI>(g.c, static_cast<const float*>(workspace), static_cast<const T*>(g.bias), g.m, g.n,
+                               g.ldc, plan.splits, epilogue_args<T>(g, 0), stream);
+  return check_launch();
+}
+
 template <typename T, int EPI>
 static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, bool half,
                       hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
@@ -284,8 +308,12 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
         return launch_splitk<T, EPI>(g, plan, trans_a, trans_b, static_cast<float*>(workspace),
                                      stream);
     }
-    if (half && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, EPI))
+    if (half && g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, EPI))
       return mfma_transposed_a<T>(g, batch, stream);
+    if (half && !mfma_eligible(g, batch, trans_a, trans_b) &&
+        any_eligible(g.m, g.n, g.k, g.lda, g.ldb, trans_a, trans_b))
+      return gemm_unaligned<T, EPI>(g, batch, trans_a, trans_b, stream, workspace, workspace_bytes);
+    if (g.residual != nullptr && !mfma_eligible(g, batch, trans_a, trans_b)) return TMB_ERR_UNSUPPORTED;
     if (half && !trans_a && stream64_eligible(g, batch, trans_b, EPI)) {
       return trans_b ? launch_stream64<T, true>(g, batch, stream)
                      : launch_stream64<T, false>(g, batch, stream);

@@ -237,7 +237,29 @@ def _relayout_for_mfma(a, b, la, lb, m, n, k, batched, plain=True):
     return a, b, _matrix_layout(a), _matrix_layout(b), kp, m
 
 
+def _in_place_workspace(a, b, la, lb, batch, m, n, k, batched, plain) -> Optional[int]:
+    """Scratch bytes of the product on the kernel that reads 16-bit operands of any alignment where they
+    lie, or None where it does not take them or padded copies and the aligned kernels are faster."""
+    if a.element_size() != 2 or m < 1 or n < 1 or k < 1:
+        return None
+    reuse = getattr(_PAD_STATE, "reuse", None)
+    if reuse is not None and a.numel() * 2 >= _PAD_REUSE_MIN_BYTES:
+        return None   # a running graph may hold the padded copy already, or pad once for two products
+    rows_ok = not (batched and batch > 1)
+    key = (batch, m, n, k, la, lb, a.dtype, plain,
+           a.data_ptr() % 16 == 0 and (rows_ok or a.stride(0) % 8 == 0),
+           b.data_ptr() % 16 == 0 and (rows_ok or b.stride(0) % 8 == 0))
+    ws = _IN_PLACE_WS.get(key)
+    if ws is None:   # a pure function of shape, layout and alignment: asked once for each
+        if len(_IN_PLACE_WS) >= 4096:
+            _IN_PLACE_WS.clear()
+        ws = _IN_PLACE_WS[key] = _ek.lib().tmb_gemm_in_place_workspace_bytes(
+            batch, m, n, k, la[1], lb[1], key[8], key[9], la[0], lb[0], plain, _CODES[a.dtype])
+    return None if ws < 0 else ws
+
+
 _I64X3 = ctypes.c_int64 * 3
+_IN_PLACE_WS: dict = {}
 _GEMM_WS_BYTES: dict = {}
 _GEMM_PLANS: dict = {}
 
@@ -323,8 +345,11 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         b = b.contiguous()
         lb = (0, max(n, 1))
     m_given = m
-    if batch * m * n * k >= _RELAYOUT_MIN_WORK and not _f32_in_place(a, la, lb, m, n, k) \
-            and not _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE):
+    fits = _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE)
+    in_place_ws = None if fits else _in_place_workspace(a, b, la, lb, batch, m, n, k, batched,
+                                                        epilogue == _ek.EPI_NONE and residual is None)
+    if not fits and in_place_ws is None and batch * m * n * k >= _RELAYOUT_MIN_WORK \
+            and not _f32_in_place(a, la, lb, m, n, k):
         a, b, la, lb, k, m = _relayout_for_mfma(a, b, la, lb, m, n, k, batched,
                                                 epilogue == _ek.EPI_NONE and residual is None)
     out_shape = (batch, m, n) if batched else (m, n)
@@ -342,7 +367,7 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
     lib = _ek.lib()
     # few output tiles and a long K: the library splits K when it is handed scratch memory
     key = (batch, m, n, k, la[0], lb[0], a.dtype)
-    ws_bytes = _GEMM_WS_BYTES.get(key)
+    ws_bytes = _GEMM_WS_BYTES.get(key) if in_place_ws is None else in_place_ws
     if ws_bytes is None:  # a pure function of shape and layout: asked once for each
         ws_bytes = _GEMM_WS_BYTES[key] = lib.tmb_gemm_layout_workspace_bytes(batch, m, n, k, la[0], lb[0],
                                                                              code_of(a.dtype))
