@@ -56,6 +56,19 @@ def test_append_and_attend_in_one_pass(case, dtype, head_dim):
     assert hip_ops.attention_decode_append(q.float(), kp.float(), vp.float(), kn.float(), vn.float(), 0.125) is None
 
 
+@pytest.mark.parametrize("keys", [40, 300])
+def test_scores_of_minus_infinity_weigh_nothing(keys):
+    """Every first key of a wave's share scores -inf: the others decide, as in ATen."""
+    from torch_mojo_backend.eager_kernels import hip_ops
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    q, k, v = (_rand(g, 1, 2, n, 64, dtype=torch.bfloat16) for n in (1, keys, keys))
+    q[..., 0] = 1.0
+    k[:, :, :keys // 2, 0] = -float("inf")
+    want = _exact(q, k, v, 0.125)
+    got = hip_ops.attention_decode(q, k, v, 0.125, False)
+    assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("dynamic", [False, True])
 def test_a_compiled_decode_step_appends_while_it_attends(dynamic):
     import torch.nn.functional as F

@@ -396,7 +396,7 @@ __global__ __launch_bounds__(WPR < 4 ? 256 : WPR * 64) void attention_decode_ker
       for (int e = 0; e < 8; ++e) x = __builtin_fmaf(qf[e], to_f32(kv[u].v[e]), x);
 #pragma unroll
       for (int w = 1; w < LPK; w <<= 1) x += __shfl_xor(x, w, kWave);
-      if (valid) {
+      if (valid && x != neg_inf) {  // (a score of -inf weighs nothing, and must not be a first maximum)
         const float m_new = fmaxf(m, x);
         const float corr = __builtin_amdgcn_exp2f(m - m_new);  // 0 on the first key (m = -inf)
         const float p = __builtin_amdgcn_exp2f(x - m_new);
