@@ -396,7 +396,9 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
             return unfused_residual()
         _check("tmb_gemm_residual_ws", rc)
         return out
-    if key is not None and a is a_in and b is b_in and bias is bias_in and out_dtype is None:
+    # (scratch for operands that only their addresses keep from the aligned kernels is not for others)
+    any_address = in_place_ws is None or (a.data_ptr() | b.data_ptr()) % 16 == 0
+    if key is not None and a is a_in and b is b_in and bias is bias_in and out_dtype is None and any_address:
         # operands are consumed in place: remember the launch arguments for this layout
         if len(_GEMM_PLANS) >= 4096:
             _GEMM_PLANS.clear()
