@@ -76,6 +76,18 @@ def test_attention_backward_matches_float64_autograd_and_oracle(btsh, dtype, cau
         assert np.abs(as64(got) - as64(orc)).max() <= TOL[dtype] * big, f"d{name} vs oracle"
 
 
+@pytest.mark.parametrize("ts", [(96, 192), (192, 96), (256, 256), (191, 193), (320, 63)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_backward_where_masked_and_unmasked_blocks_meet(ts, causal):
+    """Blocks of 64 that the diagonal or an end crosses beside blocks that neither does; a scale that is
+    no power of two."""
+    q, k, v, dout = _inputs(1, 2, *ts, torch.bfloat16, seed=sum(ts))
+    _, _, got = _run(q, k, v, dout, 0.21, causal)
+    _, _, *want = _float64_reference(q, k, v, dout, 0.21, causal)
+    for g, w in zip(got, want):
+        assert np.abs(as64(g) - w.numpy()).max() <= TOL[torch.bfloat16] * max(w.abs().max().item(), 1e-2)
+
+
 def test_attention_backward_special_cases():
     # one key: p == 1, dS == 0 up to the summation order of dout . v against dout . out:
     # dq = dk = 0 and dv = sum of the queries' dout

@@ -5,10 +5,10 @@
 //
 //   1. attention_bwd_dq_kernel: one workgroup = 128 queries of one (batch, head), 32 per wave, a
 //      lane owning one query (as in the forward kernel). It first forms
-//      delta = rowsum(dout * out) and lse * log2(e) for its queries and stores both for the second
+//      delta = scale * rowsum(dout * out) and lse * log2(e) for its queries and stores both for the second
 //      launch, then walks the keys in blocks of 64 through an LDS ring:
 //        S^T  = K Q^T, dP^T = V dout^T              (keys as MFMA rows, the query as the column)
-//        P^T  = exp2(S^T * scale * log2 e - lse2),  dS^T = P^T (dP^T - delta) * scale
+//        P^T  = exp2(S^T * scale * log2 e - lse2),  dS^T = P^T (dP^T * scale - delta)
 //        dQ^T += K^T dS^T                           (K^T by transposed LDS reads)
 //   2. attention_bwd_dkv_kernel: one workgroup = 128 keys, 32 per wave, a lane owning one key
 //      (K and V rows stay in registers); queries stream through the LDS ring in blocks of 64
@@ -21,10 +21,21 @@
 // in exchange there is no float32 dq accumulator to zero, add into and convert. P and dS are
 // rounded to the storage type before they enter a product, as the forward kernel rounds P.
 //
+// Vector instructions bound both launches (per 16 products of a wave 80 to 90 of them, 16 exponentials
+// among them), so a block that neither the diagonal nor the end of a sequence crosses runs a body without
+// masks, and the scale rides in one multiply-add. Three waves per SIMD: left to itself the compiler took
+// two (one for dk/dv) and moved the accumulators between its two register files around every product. The
+// dk/dv body is not unrolled over its two halves, which keeps it within 168 registers (unrolled it spills
+// 16 and takes 159 us below instead of 143). [batch, heads, tokens] causal, both launches: [16, 12, 1024]
+// 212 -> 143 us, [32, 12, 1024] 365 -> 262, [4, 12, 1024] 96 -> 67, [16, 12, 500] 77 -> 65, [3, 12, 250]
+// 40 -> 34. Two waves per SIMD for dk/dv: 150, 268, 62, 63 and 33 us.
+//
 // Replaces the backward of the reference's fused attention
 // (eager_kernels/aten_fast.py:4089-4170 `fast_fa4_bf16_d64_causal_backward`, which needs the same
 // inputs and two float32 statistics buffers; registered as
 // aten::_scaled_dot_product_flash_attention_backward, mojo_device/mojo_device_aten_ops.py:881).
+#include <type_traits>
+
 #include "attention_tiles.h"
 
 namespace tmb {
@@ -39,7 +50,7 @@ struct AttnBwdArgs {
   const void* v;
   const void* out;
   const float* lse;  // [batch, heads, q_len]
-  float* delta;      // [batch, heads, q_len] rowsum(dout * out), written by the dq launch
+  float* delta;      // [batch, heads, q_len] scale * rowsum(dout * out), written by the dq launch
   float* lse2;       // [batch, heads, q_len] lse * log2(e), written by the dq launch
   int64_t q_sb, q_sh, q_st;  // element strides: batch, head, token (head_dim is contiguous)
   int64_t k_sb, k_sh, k_st;
@@ -82,7 +93,7 @@ __device__ __forceinline__ void store_row(T* dst, const f32x16_t (&acc)[2], int 
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void attention_bwd_dq_kernel(AttnBwdArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void attention_bwd_dq_kernel(AttnBwdArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kAttnStages * kBwdKvBuf];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
@@ -147,7 +158,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(AttnBwdArgs a) {
           delta = __builtin_fmaf(g0, o0, delta);
           delta = __builtin_fmaf(g1, o1, delta);
         }
-      delta += other_half(delta, lane);
+      delta = (delta + other_half(delta, lane)) * a.scale;
     }
     const float lse2 = a.lse[stat] * kLog2e;
     if (half == 0 && qi < a.q_len) {
@@ -190,48 +201,55 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(AttnBwdArgs a) {
       attn_lds_u8* k_tile = (attn_lds_u8*)lds + cur_off;
       attn_lds_u8* v_tile = k_tile + kAttnTile;
 
-      uint32_t dsf[2][8];
+      // (blocks that no edge crosses take a body without the compares and selects)
+      auto add_block = [&](auto edge) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        f32x16_t acc_s, acc_dp;
+        for (int kt = 0; kt < 2; ++kt) {
+          f32x16_t acc_s, acc_dp;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc_s[e] = acc_dp[e] = 0.0f;
+          for (int e = 0; e < 16; ++e) acc_s[e] = acc_dp[e] = 0.0f;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const u32x4_t kf = *(const attn_lds_u32x4_t*)(k_tile + row_off[s] + kt * 32 * kAttnRow);
-          acc_s = Mfma<T>::run(kf, qf[s], acc_s);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const u32x4_t vf = *(const attn_lds_u32x4_t*)(v_tile + row_off[s] + kt * 32 * kAttnRow);
-          acc_dp = Mfma<T>::run(vf, dof[s], acc_dp);
-        }
-        // register r is key kb + 32 kt + 8 (r / 4) + 4 half + r % 4 of query qi
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          float ds[2];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int key = kb + kt * 32 + ((r + i) >> 2) * 8 + half * 4 + ((r + i) & 3);
-            const bool hidden = (a.causal && key > qi) || key >= a.kv_len;
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(acc_s[r + i], c, -lse2));
-            ds[i] = hidden ? 0.0f : p * (acc_dp[r + i] - delta) * a.scale;
+          for (int s = 0; s < 4; ++s) {
+            const u32x4_t kf = *(const attn_lds_u32x4_t*)(k_tile + row_off[s] + kt * 32 * kAttnRow);
+            acc_s = Mfma<T>::run(kf, qf[s], acc_s);
           }
-          dsf[kt][r >> 1] = pack2<T>(ds[0], ds[1]);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const u32x4_t vf = *(const attn_lds_u32x4_t*)(v_tile + row_off[s] + kt * 32 * kAttnRow);
+            acc_dp = Mfma<T>::run(vf, dof[s], acc_dp);
+          }
+          // register r is key kb + 32 kt + 8 (r / 4) + 4 half + r % 4 of query qi
+          uint32_t dsf[8];
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            float ds[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(acc_s[r + i], c, -lse2));
+              ds[i] = p * __builtin_fmaf(acc_dp[r + i], a.scale, -delta);
+              if constexpr (decltype(edge)::value) {
+                const int key = kb + kt * 32 + ((r + i) >> 2) * 8 + half * 4 + ((r + i) & 3);
+                ds[i] = (a.causal && key > qi) || key >= a.kv_len ? 0.0f : ds[i];
+              }
+            }
+            dsf[r >> 1] = pack2<T>(ds[0], ds[1]);
+          }
+          // dQ^T += K^T dS^T over these 32 keys, k-step s = keys 16 s .. 16 s + 15 in register order
+#pragma unroll
+          for (int s = 2 * kt; s < 2 * kt + 2; ++s) {
+            u32x4_t dsb;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dsb[e] = dsf[4 * (s & 1) + e];
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) {
+              const u32x4_t kt_op = attn_tr_operand(k_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
+              acc_dq[dt] = Mfma<T>::run(kt_op, dsb, acc_dq[dt]);
+            }
+          }
         }
-      }
-      // dQ^T += K^T dS^T over the 64 keys, k-step s = keys 16 s .. 16 s + 15 in register order
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        u32x4_t dsb;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dsb[e] = dsf[s >> 1][4 * (s & 1) + e];
-#pragma unroll
-        for (int dt = 0; dt < 2; ++dt) {
-          const u32x4_t kt_op = attn_tr_operand(k_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
-          acc_dq[dt] = Mfma<T>::run(kt_op, dsb, acc_dq[dt]);
-        }
-      }
+      };
+      if ((a.causal && kb + kAttnBKV - 1 > qw0) || kb + kAttnBKV > a.kv_len) add_block(std::true_type{});
+      else add_block(std::false_type{});
     }
     if (qi < a.q_len)
       store_row<T>(static_cast<T*>(a.dq) + b * a.dq_sb + h * a.dq_sh + static_cast<int64_t>(qi) * a.dq_st,
@@ -246,7 +264,7 @@ __global__ __launch_bounds__(256) void attention_bwd_dq_kernel(AttnBwdArgs a) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(AttnBwdArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void attention_bwd_dkv_kernel(AttnBwdArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kAttnStages * kBwdQBuf];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
@@ -340,60 +358,69 @@ __global__ __launch_bounds__(256) void attention_bwd_dkv_kernel(AttnBwdArgs a) {
       attn_lds_u8* do_tile = q_tile + kAttnTile;
       attn_lds_u8* stats = q_tile + 2 * kAttnTile;
 
-      uint32_t pf[2][8], dsf[2][8];
+      // (blocks that no edge crosses take a body without the compares and selects)
+      auto add_block = [&](auto edge) {
+#pragma unroll 1
+        for (int qt = 0; qt < 2; ++qt) {
+          f32x16_t acc_s, acc_dp;
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        f32x16_t acc_s, acc_dp;
+          for (int e = 0; e < 16; ++e) acc_s[e] = acc_dp[e] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc_s[e] = acc_dp[e] = 0.0f;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const u32x4_t qf = *(const attn_lds_u32x4_t*)(q_tile + row_off[s] + qt * 32 * kAttnRow);
-          acc_s = Mfma<T>::run(qf, kf[s], acc_s);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const u32x4_t dof = *(const attn_lds_u32x4_t*)(do_tile + row_off[s] + qt * 32 * kAttnRow);
-          acc_dp = Mfma<T>::run(dof, vf[s], acc_dp);
-        }
-        // register r is query q0 + 32 qt + 8 (r / 4) + 4 half + r % 4 against key ki
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int qoff = qt * 32 + g * 8 + half * 4;
-          const attn_f32x4_t l4 = *(const attn_lds_f32x4_t*)(stats + qoff * 4);
-          const attn_f32x4_t d4 = *(const attn_lds_f32x4_t*)(stats + 256 + qoff * 4);
-          float p[4], ds[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int query = q0 + qoff + i;
-            const bool hidden = (a.causal && ki > query) || query >= a.q_len;
-            const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(acc_s[4 * g + i], c, -l4[i]));
-            p[i] = hidden ? 0.0f : e;
-            ds[i] = hidden ? 0.0f : e * (acc_dp[4 * g + i] - d4[i]) * a.scale;
+          for (int s = 0; s < 4; ++s) {
+            const u32x4_t qf = *(const attn_lds_u32x4_t*)(q_tile + row_off[s] + qt * 32 * kAttnRow);
+            acc_s = Mfma<T>::run(qf, kf[s], acc_s);
           }
-          pf[qt][2 * g] = pack2<T>(p[0], p[1]);
-          pf[qt][2 * g + 1] = pack2<T>(p[2], p[3]);
-          dsf[qt][2 * g] = pack2<T>(ds[0], ds[1]);
-          dsf[qt][2 * g + 1] = pack2<T>(ds[2], ds[3]);
-        }
-      }
-      // dV^T += dout^T P and dK^T += Q^T dS over the 64 queries, k-step s = queries 16 s .. 16 s + 15
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        u32x4_t pb, dsb;
+          for (int s = 0; s < 4; ++s) {
+            const u32x4_t dof = *(const attn_lds_u32x4_t*)(do_tile + row_off[s] + qt * 32 * kAttnRow);
+            acc_dp = Mfma<T>::run(dof, vf[s], acc_dp);
+          }
+          // register r is query q0 + 32 qt + 8 (r / 4) + 4 half + r % 4 against key ki
+          uint32_t pf[8], dsf[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          pb[e] = pf[s >> 1][4 * (s & 1) + e];
-          dsb[e] = dsf[s >> 1][4 * (s & 1) + e];
-        }
+          for (int g = 0; g < 4; ++g) {
+            const int qoff = qt * 32 + g * 8 + half * 4;
+            const attn_f32x4_t l4 = *(const attn_lds_f32x4_t*)(stats + qoff * 4);
+            const attn_f32x4_t d4 = *(const attn_lds_f32x4_t*)(stats + 256 + qoff * 4);
+            float p[4], ds[4];
 #pragma unroll
-        for (int dt = 0; dt < 2; ++dt) {
-          const u32x4_t dot_op = attn_tr_operand(do_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
-          acc_dv[dt] = Mfma<T>::run(dot_op, pb, acc_dv[dt]);
-          const u32x4_t qt_op = attn_tr_operand(q_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
-          acc_dk[dt] = Mfma<T>::run(qt_op, dsb, acc_dk[dt]);
+            for (int i = 0; i < 4; ++i) {
+              p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(acc_s[4 * g + i], c, -l4[i]));
+              ds[i] = p[i] * __builtin_fmaf(acc_dp[4 * g + i], a.scale, -d4[i]);
+              if constexpr (decltype(edge)::value) {
+                const int query = q0 + qoff + i;
+                const bool hidden = (a.causal && ki > query) || query >= a.q_len;
+                p[i] = hidden ? 0.0f : p[i];
+                ds[i] = hidden ? 0.0f : ds[i];
+              }
+            }
+            pf[2 * g] = pack2<T>(p[0], p[1]);
+            pf[2 * g + 1] = pack2<T>(p[2], p[3]);
+            dsf[2 * g] = pack2<T>(ds[0], ds[1]);
+            dsf[2 * g + 1] = pack2<T>(ds[2], ds[3]);
+          }
+          // dV^T += dout^T P and dK^T += Q^T dS over these 32 queries, k-step s = queries 16 s .. 16 s + 15
+#pragma unroll
+          for (int s1 = 0; s1 < 2; ++s1) {
+            const int s = 2 * qt + s1;
+            u32x4_t pb, dsb;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              pb[e] = pf[4 * s1 + e];
+              dsb[e] = dsf[4 * s1 + e];
+            }
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt) {
+              const u32x4_t dot_op = attn_tr_operand(do_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
+              acc_dv[dt] = Mfma<T>::run(dot_op, pb, acc_dv[dt]);
+              const u32x4_t qt_op = attn_tr_operand(q_tile + s * 16 * kAttnRow, tr_off[dt][0], tr_off[dt][1]);
+              acc_dk[dt] = Mfma<T>::run(qt_op, dsb, acc_dk[dt]);
+            }
+          }
         }
-      }
+      };
+      if ((a.causal && kw0 + 31 > q0) || q0 + kAttnBKV > a.q_len) add_block(std::true_type{});
+      else add_block(std::false_type{});
     }
     if (ki < a.kv_len) {
       store_row<T>(static_cast<T*>(a.dk) + b * a.dk_sb + h * a.dk_sh + static_cast<int64_t>(ki) * a.dk_st,
