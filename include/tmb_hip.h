@@ -191,6 +191,25 @@ size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int6
 int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda,
                                           int64_t ldb, int a_aligned, int b_aligned, int trans_a, int trans_b,
                                           int plain, int dtype);
+/* The kernels of tmb_gemm*. */
+typedef enum tmb_gemm_kernel {
+  TMB_GEMM_SIMT = 0,         /* any layout, vector instructions */
+  TMB_GEMM_RING = 1,         /* 16-bit, aligned, A row-major: direct-to-LDS rings and register-staged tiles */
+  TMB_GEMM_TRANSPOSED_A = 2, /* 16-bit, aligned, A stored [K, M] and B [K, N] */
+  TMB_GEMM_SPLITK = 3,       /* the two above with K split over workgroups; tile 128 or 256 */
+  TMB_GEMM_SMALL = 4,        /* 16-bit, aligned, few tiles: waves share K; tile 0 .. 5 */
+  TMB_GEMM_ANY = 5,          /* 16-bit, any layout and alignment; tile 0 .. 4 */
+  TMB_GEMM_STREAM64 = 6,     /* 16-bit, K = 64 on whole 128 x 128 tiles */
+  TMB_GEMM_F32 = 7,          /* fp32, any layout and alignment; tile 0 .. 3 */
+  TMB_GEMM_F32_WIDE = 8      /* fp32, aligned, 128 x 128 tiles */
+} tmb_gemm_kernel;
+/* What a product of such operands runs on: kernel | tile << 8 | splits << 16 (a tmb_gemm_kernel, an index into
+ * its tiles, 0 splits where K is not split), or a negative status where tmb_gemm* answers that. The launch follows
+ * the same choice. a_aligned / b_aligned: the base lies on a 16-byte boundary; with_residual: as by tmb_gemm_residual*;
+ * workspace_bytes: what the call would be handed. Sizes, pitches and flags as for tmb_gemm_ws (k >= 1). */
+int64_t tmb_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                       int64_t stride_a, int64_t stride_b, int a_aligned, int b_aligned, int trans_a, int trans_b,
+                       int dtype, int epilogue, int with_residual, size_t workspace_bytes);
 int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch, int64_t m,
                 int64_t n, int64_t k, int64_t lda, int64_t ldb, int64_t ldc, int64_t stride_a,
                 int64_t stride_b, int64_t stride_c, int trans_a, int trans_b, int dtype,

@@ -129,7 +129,7 @@ extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int6
     return 0;
   if (dtype == TMB_F32) {
     if (batch < 1 || m < 1 || n < 1 || k < 1 || tmb::f32_wide_pays(batch, m, n, k) || m * n >= (int64_t{1} << 31)) return 0;
-    return static_cast<size_t>(tmb::f32_plan(batch, m, n, k).splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
+    return static_cast<size_t>(tmb::f32_plan(batch, m, n, k, true).splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
   }
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
 }
@@ -144,6 +144,31 @@ extern "C" int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, i
                                    plain != 0))
     return -1;
   return static_cast<int64_t>(plan.splits) * m * n * 4;
+}
+
+extern "C" int64_t tmb_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
+                                  int64_t stride_a, int64_t stride_b, int a_aligned, int b_aligned, int trans_a,
+                                  int trans_b, int dtype, int epilogue_flags, int with_residual,
+                                  size_t workspace_bytes) {
+  using namespace tmb;
+  if (batch < 1 || m < 1 || n < 1 || k < 1 || lda < (trans_a ? m : k) || ldb < (trans_b ? k : n))
+    return TMB_ERR_INVALID_ARGUMENT;
+  if ((dtype != TMB_F32 && dtype != TMB_F16 && dtype != TMB_BF16) || batch > 65535) return TMB_ERR_UNSUPPORTED;
+  // addresses that are never read: only their alignment is looked at
+  auto at = [](int aligned) { return reinterpret_cast<const void*>(static_cast<uintptr_t>(aligned ? 16 : 18)); };
+  GemmArgs g{};
+  g.a = at(a_aligned);
+  g.b = at(b_aligned);
+  g.m = m, g.n = n, g.k = k, g.lda = lda, g.ldb = ldb, g.ldc = n;
+  g.stride_a = stride_a, g.stride_b = stride_b, g.stride_c = m * n;
+  g.residual = with_residual ? at(1) : nullptr;
+  g.ldr = n;
+  g.round_like_unfused = (epilogue_flags & TMB_EPI_ROUND_LIKE_UNFUSED) != 0;
+  const GemmRoute r = dtype == TMB_F32
+                          ? route_f32(g, batch, trans_a, trans_b, workspace_bytes)
+                          : route_16bit(g, batch, trans_a, trans_b, epilogue_flags & 0xff, workspace_bytes);
+  if (r.kernel < 0) return r.kernel;
+  return r.kernel | static_cast<int64_t>(r.tile) << 8 | static_cast<int64_t>(r.splits) << 16;
 }
 
 extern "C" int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t batch,

@@ -22,6 +22,32 @@ static inline bool mfma_eligible(const GemmArgs& g, int64_t batch, int trans_a, 
   return true;
 }
 
+// A stored [K, M] with B stored [K, N] (the weight-gradient product) on the ring kernels: whole 16-byte
+// chunks along m and n, whole stages of K and enough of them for the ring.
+static inline bool mfma_transposed_a_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
+                                              int epilogue) {
+  if (!trans_a || trans_b || epilogue != TMB_EPI_NONE) return false;
+  if (g.k % 32 != 0 || g.k < 256 || g.m % 8 != 0 || g.n % 8 != 0 || g.n <= 64) return false;
+  if (g.lda % 8 != 0 || g.ldb % 8 != 0 || !aligned16(g.a) || !aligned16(g.b)) return false;
+  if (batch > 1 && (g.stride_a % 8 != 0 || g.stride_b % 8 != 0)) return false;
+  const int64_t a_span = g.k * g.lda * 2, b_span = g.k * g.ldb * 2;
+  return a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32);
+}
+
+// Shapes the stream kernel takes: K = 64, whole 128 x 128 tiles, 16-byte aligned operands whose
+// rows are whole 16-byte chunks, no epilogue beyond the bias, no residual.
+static inline bool stream64_eligible(const GemmArgs& g, int64_t batch, int trans_b, int epilogue) {
+  if (g.k != 64 || g.m % 128 != 0 || g.n % 128 != 0 || epilogue != TMB_EPI_NONE) return false;
+  if (g.residual != nullptr || g.out_f32) return false;
+  if (g.lda % 8 != 0 || g.ldb % 8 != 0 || !aligned16(g.a) || !aligned16(g.b)) return false;
+  if (batch > 1 && (g.stride_a % 8 != 0 || g.stride_b % 8 != 0)) return false;
+  // lane offsets are 32-bit byte offsets inside one tile's rows
+  const int64_t a_span = 128 * g.lda * 2, b_span = (trans_b ? 128 : 64) * g.ldb * 2;
+  if (a_span >= (int64_t{1} << 32) || b_span >= (int64_t{1} << 32)) return false;
+  const int64_t tiles = (g.m / 128) * (g.n / 128) * batch;
+  return tiles >= 512 && tiles < (int64_t{1} << 40);
+}
+
 // Tiles of the kernel for products that leave most of the chip idle (gemm_small.h), and what a
 // launch with one of them takes, in microseconds: a start, then per tile its operands' bytes at the
 // rate one workgroup's loads sustain and the way of its partial tiles through LDS. A CU that gets a
@@ -67,7 +93,7 @@ static inline bool small_applies(int64_t batch, int64_t m, int64_t n, int64_t k)
   if (m <= 16 && batch == 1) return true;
   return ((m + 63) / 64) * ((n + 63) / 64) * batch <= 256;
 }
-int gemm_small(const GemmArgs& g, int64_t batch, int trans_b, bool bf16, int epilogue, hipStream_t stream);
+int gemm_small(const GemmArgs& g, int64_t batch, int tile, int trans_b, bool bf16, int epilogue, hipStream_t stream);
 
 // 16-bit operands in any layout and at any alignment (gemm_any.h): tile and split count. A launch takes,
 // in microseconds, a start and per round of tiles their operands' bytes at the rate a workgroup's
@@ -234,7 +260,7 @@ static inline double f32_cost(const F32Tile& t, double batch, int64_t m, int64_t
   }
   return 7.0 + rounds * (2.0 * t.bm * t.bn * k / 256.0 / 2400.0 * t.stretch + t.per_tile);
 }
-static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
+static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool may_split) {
   F32Plan p{kF32TileCount - 1, 0};
   double best = 0.0;
   for (int i = 0; i < kF32TileCount; ++i) {
@@ -244,7 +270,7 @@ static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
       p.tile = i;
     }
   }
-  if (batch != 1) return p;
+  if (batch != 1 || !may_split) return p;
   best *= 0.92;  // a second launch and a workspace have to pay for themselves
   for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
     if (k < 96 * s) break;
@@ -273,6 +299,57 @@ static inline bool f32_shared_eligible(const GemmArgs& g, int trans_a, int trans
   if (g.m < 1 || g.n < 1 || g.k < 1) return false;
   if ((trans_a ? g.m : g.k) < 4 || (trans_b ? g.k : g.n) < 4) return false;
   return g.lda < (int64_t{1} << 23) && g.ldb < (int64_t{1} << 23);
+}
+
+// Which kernel takes a product, with its tile (an index into the kernel's own list; 128 or 256 for SplitK) and
+// its number of splits (0: not split). The launch follows it (gemm_typed.h), and tmb_gemm_route answers it.
+struct GemmRoute {
+  int kernel;  // TMB_GEMM_*, or TMB_ERR_UNSUPPORTED
+  int tile;
+  int splits;
+};
+
+static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int epilogue,
+                                    size_t workspace_bytes) {
+  const bool aligned = mfma_eligible(g, batch, trans_a, trans_b);
+  const bool whole_columns = trans_b || g.n % 8 == 0;
+  if (aligned && whole_columns && small_applies(batch, g.m, g.n, g.k))
+    return {TMB_GEMM_SMALL, small_tile(batch, g.m, g.n, g.k), 0};
+  if (workspace_bytes > 0) {
+    const SplitKPlan plan = splitk_plan(batch, g.m, g.n, g.k);
+    const bool operands_ok = trans_a ? mfma_transposed_a_eligible(g, batch, trans_a, trans_b, TMB_EPI_NONE)
+                                     : aligned && whole_columns;
+    if (plan.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
+        workspace_bytes >= static_cast<size_t>(plan.splits) * g.m * g.n * 4)
+      return {TMB_GEMM_SPLITK, plan.tile, plan.splits};
+  }
+  if (g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue))
+    return {TMB_GEMM_TRANSPOSED_A, 0, 0};
+  if (!aligned && any_eligible(g.m, g.n, g.k, g.lda, g.ldb, trans_a, trans_b)) {
+    AnyPlan plan = any_plan(batch, g.m, g.n, g.k, true);
+    if (plan.splits > 0 && workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4)
+      plan = any_plan(batch, g.m, g.n, g.k, false);
+    return {TMB_GEMM_ANY, plan.tile, plan.splits};
+  }
+  if (aligned) {
+    if (stream64_eligible(g, batch, trans_b, epilogue)) return {TMB_GEMM_STREAM64, 0, 0};
+    return {TMB_GEMM_RING, 0, 0};
+  }
+  if (g.residual != nullptr) return {TMB_ERR_UNSUPPORTED, 0, 0};
+  return {TMB_GEMM_SIMT, 0, 0};
+}
+
+static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
+                                  size_t workspace_bytes) {
+  if (!f32_shared_eligible(g, trans_a, trans_b))
+    return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
+  if (g.residual == nullptr && f32_wide_pays(batch, g.m, g.n, g.k) && f32_mfma_eligible(g, batch, trans_a, trans_b))
+    return {TMB_GEMM_F32_WIDE, 0, 0};
+  F32Plan plan = f32_plan(batch, g.m, g.n, g.k, true);
+  if (plan.splits > 0 && (g.m * g.n >= (int64_t{1} << 31) ||
+                          workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
+    plan = f32_plan(batch, g.m, g.n, g.k, false);
+  return {TMB_GEMM_F32, plan.tile, plan.splits};
 }
 
 // The typed half of the entry point (gemm_typed.h), one translation unit per storage type.

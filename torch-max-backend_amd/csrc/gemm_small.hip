@@ -5,8 +5,8 @@
 namespace tmb {
 
 template <typename T, bool B_KMAJOR, int EPI>
-static int small_launch(const GemmArgs& g, int64_t batch, hipStream_t stream) {
-  switch (small_tile(batch, g.m, g.n, g.k)) {
+static int small_launch(const GemmArgs& g, int64_t batch, int tile, hipStream_t stream) {
+  switch (tile) {
     case 0: return launch_small<T, 16, 16, 8, B_KMAJOR, EPI>(g, batch, stream);
     case 1: return launch_small<T, 16, 32, 8, B_KMAJOR, EPI>(g, batch, stream);
     case 2: return launch_small<T, 32, 32, 8, B_KMAJOR, EPI>(g, batch, stream);
@@ -17,20 +17,20 @@ static int small_launch(const GemmArgs& g, int64_t batch, hipStream_t stream) {
 }
 
 template <typename T, bool B_KMAJOR>
-static int small_epi(const GemmArgs& g, int64_t batch, int epilogue, hipStream_t stream) {
+static int small_epi(const GemmArgs& g, int64_t batch, int tile, int epilogue, hipStream_t stream) {
   switch (epilogue) {
-    case TMB_EPI_NONE: return small_launch<T, B_KMAJOR, TMB_EPI_NONE>(g, batch, stream);
-    case TMB_EPI_GELU_TANH: return small_launch<T, B_KMAJOR, TMB_EPI_GELU_TANH>(g, batch, stream);
-    case TMB_EPI_GELU_ERF: return small_launch<T, B_KMAJOR, TMB_EPI_GELU_ERF>(g, batch, stream);
+    case TMB_EPI_NONE: return small_launch<T, B_KMAJOR, TMB_EPI_NONE>(g, batch, tile, stream);
+    case TMB_EPI_GELU_TANH: return small_launch<T, B_KMAJOR, TMB_EPI_GELU_TANH>(g, batch, tile, stream);
+    case TMB_EPI_GELU_ERF: return small_launch<T, B_KMAJOR, TMB_EPI_GELU_ERF>(g, batch, tile, stream);
     default: return TMB_ERR_INVALID_ARGUMENT;
   }
 }
 
-int gemm_small(const GemmArgs& g, int64_t batch, int trans_b, bool bf16, int epilogue, hipStream_t stream) {
-  if (bf16) return trans_b ? small_epi<bf16_t, true>(g, batch, epilogue, stream)
-                           : small_epi<bf16_t, false>(g, batch, epilogue, stream);
-  return trans_b ? small_epi<f16_t, true>(g, batch, epilogue, stream)
-                 : small_epi<f16_t, false>(g, batch, epilogue, stream);
+int gemm_small(const GemmArgs& g, int64_t batch, int tile, int trans_b, bool bf16, int epilogue, hipStream_t stream) {
+  if (bf16) return trans_b ? small_epi<bf16_t, true>(g, batch, tile, epilogue, stream)
+                           : small_epi<bf16_t, false>(g, batch, tile, epilogue, stream);
+  return trans_b ? small_epi<f16_t, true>(g, batch, tile, epilogue, stream)
+                 : small_epi<f16_t, false>(g, batch, tile, epilogue, stream);
 }
 
 }  // namespace tmb

@@ -175,20 +175,6 @@ __global__ __launch_bounds__(256, BUFS == 2 ? 2 : 4) void gemm_k64_stream_kernel
 #endif
 }
 
-// Shapes the stream kernel takes: K = 64, whole 128 x 128 tiles, 16-byte aligned operands whose
-// rows are whole 16-byte chunks, no epilogue beyond the bias, no residual.
-inline bool stream64_eligible(const GemmArgs& g, int64_t batch, int trans_b, int epilogue) {
-  if (g.k != 64 || g.m % 128 != 0 || g.n % 128 != 0 || epilogue != TMB_EPI_NONE) return false;
-  if (g.residual != nullptr || g.out_f32) return false;
-  if (g.lda % 8 != 0 || g.ldb % 8 != 0 || !aligned16(g.a) || !aligned16(g.b)) return false;
-  if (batch > 1 && (g.stride_a % 8 != 0 || g.stride_b % 8 != 0)) return false;
-  // lane offsets are 32-bit byte offsets inside one tile's rows
-  const int64_t a_span = 128 * g.lda * 2, b_span = (trans_b ? 128 : 64) * g.ldb * 2;
-  if (a_span >= (int64_t{1} << 32) || b_span >= (int64_t{1} << 32)) return false;
-  const int64_t tiles = (g.m / 128) * (g.n / 128) * batch;
-  return tiles >= 512 && tiles < (int64_t{1} << 40);
-}
-
 template <typename T, bool B_KMAJOR, int BUFS = 2, int BM = 128, int BN = 128, int WAVES_M = 2>
 static int launch_stream64(const GemmArgs& base, int64_t batch, hipStream_t stream,
                            int64_t grid_override = 0, int stream_override = -1) {

@@ -180,16 +180,6 @@ static int mfma_transposed_a(const GemmArgs& g, int64_t batch, hipStream_t strea
   return launch_ring<T, 128, 128, 32, 2, 2, 4, false, TMB_EPI_NONE, true>(g, batch, stream);
 }
 
-static bool mfma_transposed_a_eligible(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
-                                       int epilogue) {
-  if (!trans_a || trans_b || epilogue != TMB_EPI_NONE) return false;
-  if (g.k % 32 != 0 || g.k < 256 || g.m % 8 != 0 || g.n % 8 != 0 || g.n <= 64) return false;
-  if (g.lda % 8 != 0 || g.ldb % 8 != 0 || !aligned16(g.a) || !aligned16(g.b)) return false;
-  if (batch > 1 && (g.stride_a % 8 != 0 || g.stride_b % 8 != 0)) return false;
-  const int64_t a_span = g.k * g.lda * 2, b_span = g.k * g.ldb * 2;
-  return a_span < (int64_t{1} << 32) && b_span < (int64_t{1} << 32);
-}
-
 template <typename T, int EPI>
 static int launch_splitk(const GemmArgs& g, const SplitKPlan& plan, int trans_a, int trans_b,
                          float* workspace, hipStream_t stream) {
@@ -234,110 +224,70 @@ static int launch_f32_shared(const GemmArgs& g, int64_t batch, int tile, int tra
   }
 }
 
-template <int EPI>
-static int gemm_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, hipStream_t stream, void* workspace,
-                    size_t workspace_bytes) {
-  if (g.residual == nullptr && f32_wide_pays(batch, g.m, g.n, g.k) && f32_mfma_eligible(g, batch, trans_a, trans_b))
-    return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
-  F32Plan plan = f32_plan(batch, g.m, g.n, g.k);
-  if (plan.splits > 0 && (workspace == nullptr || g.m * g.n >= (int64_t{1} << 31) ||
-                          workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4)) {
-    plan.splits = 0;
-    double best = 0.0;
-    for (int i = 0; i < kF32TileCount; ++i) {
-      const double c = f32_cost(kF32Tiles[i], static_cast<double>(batch), g.m, g.n, static_cast<double>(g.k));
-      if (i == 0 || c < best) {
-        best = c;
-        plan.tile = i;
-      }
-    }
-  }
-  if (plan.splits == 0) return launch_f32_shared<EPI>(g, batch, plan.tile, trans_a, trans_b, stream);
+// A split launch of `launch` into `workspace` and the reduction that adds bias, epilogue and residual.
+template <typename T, int EPI, typename Launch>
+static int launch_split(const GemmArgs& g, int splits, hipStream_t stream, void* workspace, const Launch& launch) {
   GemmArgs part = g;
   part.c = workspace;
   part.bias = nullptr;
   part.residual = nullptr;
   part.ldc = g.n;
   part.stride_c = g.m * g.n;
-  part.splits = plan.splits;
-  const int rc = launch_f32_shared<TMB_EPI_NONE>(part, plan.splits, plan.tile, trans_a, trans_b, stream);
-  if (rc != 0) return rc;
-  launch_splitk_reduce<float, EPI>(g.c, static_cast<const float*>(workspace), static_cast<const float*>(g.bias), g.m,
-                                   g.n, g.ldc, plan.splits, epilogue_args<float>(g, 0), stream);
-  return check_launch();
-}
-
-// Operands that the kernels above cannot read, where they lie.
-template <typename T, int EPI>
-static int gemm_unaligned(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, hipStream_t stream, void* workspace,
-                          size_t workspace_bytes) {
-  AnyPlan plan = any_plan(batch, g.m, g.n, g.k, true);
-  if (plan.splits > 0 &&
-      (workspace == nullptr || workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
-    plan = any_plan(batch, g.m, g.n, g.k, false);
-  constexpr bool BF16 = __is_same(T, bf16_t);
-  if (plan.splits == 0) return gemm_any(g, batch, plan.tile, trans_a, trans_b, BF16, EPI, stream);
-  GemmArgs part = g;
-  part.c = workspace;
-  part.bias = nullptr;
-  part.residual = nullptr;
-  part.ldc = g.n;
-  part.stride_c = g.m * g.n;
-  part.splits = plan.splits;
-  const int rc = gemm_any(part, plan.splits, plan.tile, trans_a, trans_b, BF16, TMB_EPI_NONE, stream);
+  part.splits = splits;
+  const int rc = launch(part);
   if (rc != 0) return rc;
   launch_splitk_reduce<T, EPI>(g.c, static_cast<const float*>(workspace), static_cast<const T*>(g.bias), g.m, g.n,
-                               g.ldc, plan.splits, epilogue_args<T>(g, 0), stream);
+                               g.ldc, splits, epilogue_args<T>(g, 0), stream);
   return check_launch();
 }
 
 template <typename T, int EPI>
-static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, bool half,
-                      hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0) {
-  if constexpr (!__is_same(T, float)) {
-    if (half && small_applies(batch, g.m, g.n, g.k) && mfma_eligible(g, batch, trans_a, trans_b) &&
-        (trans_b || g.n % 8 == 0))
-      return gemm_small(g, batch, trans_b, __is_same(T, bf16_t), EPI, stream);
-    if (half && workspace != nullptr) {
-      const SplitKPlan plan = splitk_plan(batch, g.m, g.n, g.k);
-      const bool operands_ok =
-          trans_a ? mfma_transposed_a_eligible(g, batch, trans_a, trans_b, TMB_EPI_NONE)
-                  : (mfma_eligible(g, batch, trans_a, trans_b) && (trans_b || g.n % 8 == 0));
-      if (plan.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
-          workspace_bytes >= static_cast<size_t>(plan.splits) * g.m * g.n * 4)
-        return launch_splitk<T, EPI>(g, plan, trans_a, trans_b, static_cast<float*>(workspace),
-                                     stream);
-    }
-    if (half && g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, EPI))
-      return mfma_transposed_a<T>(g, batch, stream);
-    if (half && !mfma_eligible(g, batch, trans_a, trans_b) &&
-        any_eligible(g.m, g.n, g.k, g.lda, g.ldb, trans_a, trans_b))
-      return gemm_unaligned<T, EPI>(g, batch, trans_a, trans_b, stream, workspace, workspace_bytes);
-    if (g.residual != nullptr && !mfma_eligible(g, batch, trans_a, trans_b)) return TMB_ERR_UNSUPPORTED;
-    if (half && !trans_a && stream64_eligible(g, batch, trans_b, EPI)) {
-      return trans_b ? launch_stream64<T, true>(g, batch, stream)
-                     : launch_stream64<T, false>(g, batch, stream);
-    }
-    if (half && mfma_eligible(g, batch, trans_a, trans_b)) {
-      return trans_b ? mfma_pick_tile<T, true, EPI>(g, batch, stream)
-                     : mfma_pick_tile<T, false, EPI>(g, batch, stream);
-    }
-  }
+static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, hipStream_t stream, void* workspace,
+                      size_t workspace_bytes) {
+  const size_t scratch = workspace != nullptr ? workspace_bytes : 0;
   if constexpr (__is_same(T, float)) {
-    if (f32_shared_eligible(g, trans_a, trans_b))
-      return gemm_f32<EPI>(g, batch, trans_a, trans_b, stream, workspace, workspace_bytes);
-    if (g.residual != nullptr) return TMB_ERR_UNSUPPORTED;
+    const GemmRoute r = route_f32(g, batch, trans_a, trans_b, scratch);
+    switch (r.kernel) {
+      case TMB_GEMM_F32_WIDE: return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
+      case TMB_GEMM_F32:
+        if (r.splits == 0) return launch_f32_shared<EPI>(g, batch, r.tile, trans_a, trans_b, stream);
+        return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](const GemmArgs& part) {
+          return launch_f32_shared<TMB_EPI_NONE>(part, r.splits, r.tile, trans_a, trans_b, stream);
+        });
+      case TMB_GEMM_SIMT: return launch_simt<T, EPI>(g, batch, trans_a, trans_b, stream);
+      default: return TMB_ERR_UNSUPPORTED;
+    }
+  } else {
+    constexpr bool BF16 = __is_same(T, bf16_t);
+    const GemmRoute r = route_16bit(g, batch, trans_a, trans_b, EPI, scratch);
+    switch (r.kernel) {
+      case TMB_GEMM_SMALL: return gemm_small(g, batch, r.tile, trans_b, BF16, EPI, stream);
+      case TMB_GEMM_SPLITK:
+        return launch_splitk<T, EPI>(g, SplitKPlan{r.splits, r.tile, 0}, trans_a, trans_b,
+                                     static_cast<float*>(workspace), stream);
+      case TMB_GEMM_TRANSPOSED_A: return mfma_transposed_a<T>(g, batch, stream);
+      case TMB_GEMM_ANY:
+        if (r.splits == 0) return gemm_any(g, batch, r.tile, trans_a, trans_b, BF16, EPI, stream);
+        return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](const GemmArgs& part) {
+          return gemm_any(part, r.splits, r.tile, trans_a, trans_b, BF16, TMB_EPI_NONE, stream);
+        });
+      case TMB_GEMM_STREAM64:
+        return trans_b ? launch_stream64<T, true>(g, batch, stream) : launch_stream64<T, false>(g, batch, stream);
+      case TMB_GEMM_RING:
+        return trans_b ? mfma_pick_tile<T, true, EPI>(g, batch, stream) : mfma_pick_tile<T, false, EPI>(g, batch, stream);
+      case TMB_GEMM_SIMT: return launch_simt<T, EPI>(g, batch, trans_a, trans_b, stream);
+      default: return TMB_ERR_UNSUPPORTED;
+    }
   }
-  return launch_simt<T, EPI>(g, batch, trans_a, trans_b, stream);
 }
 
 template <typename T>
 int gemm_epi(const GemmArgs& g, int64_t batch, int ta, int tb, int epilogue,
                     hipStream_t stream, void* ws, size_t ws_bytes) {
   switch (epilogue) {
-    case TMB_EPI_NONE: return gemm_typed<T, TMB_EPI_NONE>(g, batch, ta, tb, true, stream, ws, ws_bytes);
-    case TMB_EPI_GELU_TANH: return gemm_typed<T, TMB_EPI_GELU_TANH>(g, batch, ta, tb, true, stream, ws, ws_bytes);
-    case TMB_EPI_GELU_ERF: return gemm_typed<T, TMB_EPI_GELU_ERF>(g, batch, ta, tb, true, stream, ws, ws_bytes);
+    case TMB_EPI_NONE: return gemm_typed<T, TMB_EPI_NONE>(g, batch, ta, tb, stream, ws, ws_bytes);
+    case TMB_EPI_GELU_TANH: return gemm_typed<T, TMB_EPI_GELU_TANH>(g, batch, ta, tb, stream, ws, ws_bytes);
+    case TMB_EPI_GELU_ERF: return gemm_typed<T, TMB_EPI_GELU_ERF>(g, batch, ta, tb, stream, ws, ws_bytes);
     default: return TMB_ERR_INVALID_ARGUMENT;
   }
 }
