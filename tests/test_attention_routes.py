@@ -1,0 +1,103 @@
+"""Which kernel the fused attention ops of a compiled graph run on and how their result is laid out: on
+the host with a library that only records its launches, and compiled on the GPU."""
+
+import operator
+import types
+
+import pytest
+import torch
+
+
+class RecordingLibrary:
+    """Answers sizes and routes like the library; launches are noted and succeed."""
+
+    def __init__(self, real):
+        self.real, self.launched = real, []
+
+    def __getattr__(self, name):
+        if name.endswith("_bytes") or name == "tmb_gemm_route":
+            return getattr(self.real, name)
+        return lambda *args: (self.launched.append((name, args)), 0)[1]
+
+
+@pytest.fixture()
+def recorded(monkeypatch):
+    """Launchers on host tensors, which count as device tensors here."""
+    from torch_mojo_backend import aten_functions
+    from torch_mojo_backend import eager_kernels as ek
+    from torch_mojo_backend.eager_kernels import hip_ops
+
+    lib = RecordingLibrary(ek.lib())
+    monkeypatch.setattr(ek, "lib", lambda: lib)
+    monkeypatch.setattr(hip_ops, "_stream", lambda: 0)
+    monkeypatch.setattr(hip_ops, "require_hip", lambda *a: None)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    node = types.SimpleNamespace(users=[types.SimpleNamespace(target=operator.getitem, args=(None, 0))])
+    token = aten_functions.CURRENT_FX_NODE.set(node)
+    yield lib
+    aten_functions.CURRENT_FX_NODE.reset(token)
+
+
+def _queries(b, h, t, d, layout):
+    if layout == "contiguous":
+        return torch.zeros(b, h, t, d, dtype=torch.bfloat16)
+    if layout == "token-major":
+        return torch.zeros(b, t, h, d, dtype=torch.bfloat16).transpose(1, 2)
+    if layout == "head-outermost":
+        return torch.zeros(h, b, t, d, dtype=torch.bfloat16).transpose(0, 1)
+    return torch.zeros(b, t, 3, h, d, dtype=torch.bfloat16)[:, :, 0].transpose(1, 2)    # out of a packed projection
+
+
+LAYOUTS = ["contiguous", "token-major", "head-outermost", "packed"]
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("t", [1, 2, 5, 16, 17])
+@pytest.mark.parametrize("d", [64, 128])
+def test_the_flash_result_is_laid_out_like_the_query(recorded, layout, t, d):
+    """Views that are legal for the layout the graph was traced with stay legal."""
+    from torch_mojo_backend.aten_functions import aten__scaled_dot_product_flash_attention as flash
+    if d == 128 and t == 17:
+        pytest.skip("PyTorch's own op")
+    q = _queries(2, 3, t, d, layout)
+    k = v = torch.zeros(2, 3, 300, d, dtype=torch.bfloat16)
+    out = flash(q, k, v)[0]
+    assert len(recorded.launched) == 1
+    assert out.shape == q.shape and out.stride() == torch.empty_like(q).stride()
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_the_appending_step_lays_its_result_out_like_the_query(recorded, layout):
+    from torch_mojo_backend.eager_kernels import hip_ops
+    q, past, new = _queries(2, 3, 1, 64, layout), torch.zeros(2, 3, 9, 64).bfloat16(), torch.zeros(2, 3, 1, 64).bfloat16()
+    out, _, _ = hip_ops.attention_decode_append(q, past, past, new, new, 0.125)
+    assert out.stride() == torch.empty_like(q).stride()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("t", [2, 5, 16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("token_major", [False, True])
+def test_compiled_attention_of_a_few_queries_is_viewed_and_multiplied(t, head_dim, token_major):
+    import torch.nn.functional as F
+    from torch_mojo_backend import mojo_backend
+
+    def step(q, k, v, w):
+        y = F.scaled_dot_product_attention(q, k, v)
+        return y @ w, y.reshape(6, t, head_dim) * 2.0, y.transpose(1, 2).reshape(2, t, 3 * head_dim)
+
+    g = torch.Generator(device="cuda").manual_seed(t)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device="cuda").bfloat16()
+
+    q = rand(2, t, 3, head_dim).transpose(1, 2) if token_major else rand(2, 3, t, head_dim)
+    k, v, w = rand(2, 3, 300, head_dim), rand(2, 3, 300, head_dim), rand(head_dim, 32)
+    with torch.no_grad():
+        got = torch.compile(step, backend=mojo_backend, fullgraph=True)(q, k, v, w)
+    scores = q.double() @ k.double().transpose(-1, -2).contiguous() / head_dim ** 0.5
+    y = (torch.softmax(scores, -1) @ v.double())
+    for x, want in zip(got, (y @ w.double(), y.reshape(6, t, head_dim) * 2.0,
+                             y.transpose(1, 2).reshape(2, t, 3 * head_dim))):
+        # P is rounded to bf16 in one of the kernels, y once, and the product sums head_dim of them
+        assert (x.double() - want).abs().max().item() <= 2.0 ** -7 * (1 + want.abs().max().item())

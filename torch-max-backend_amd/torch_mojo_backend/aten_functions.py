@@ -358,7 +358,7 @@ def aten__scaled_dot_product_flash_attention(query, key, value, dropout_p: float
             and query.shape[2] <= hip_ops.DECODE_MAX_QUERIES and _only_first_output_used() \
             and hip_ops.attention_decode_supported(query, key, value, None):
         # a few queries and no backward pass to hand statistics to: the memory-bound kernel
-        out = hip_ops.attention_decode(query, key, value, s, bool(is_causal), checked=True, token_major=True)
+        out = hip_ops.attention_decode(query, key, value, s, bool(is_causal), checked=True, like_query=True)
         return (out,) + (None,) * 8
     if dropout_p == 0.0 and not return_debug_mask and query.dim() == 4 and s > 0.0 \
             and hip_ops.attention_supported(query, key, value):

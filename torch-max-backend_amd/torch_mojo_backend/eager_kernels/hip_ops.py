@@ -534,8 +534,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, c
 
 
 def _gradient_like(x: torch.Tensor) -> torch.Tensor:
-    """A [batch, heads, tokens, 64] buffer laid out as `torch.empty_like(x)` when the kernels can
-    write that layout (rows of 64 contiguous, strides multiples of 4), token-major otherwise."""
+    """A [batch, heads, tokens, head_dim] buffer laid out as `torch.empty_like(x)` when the kernels can
+    write that layout (head_dim contiguous, strides multiples of 4), token-major otherwise."""
     like = torch.empty_like(x)
     if like.stride(3) == 1 and all(s % 4 == 0 and s >= 0 for s in like.stride()[:3]):
         return like
@@ -641,17 +641,21 @@ def attention_decode_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
 
 def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float,
                      causal: bool, attn_mask: Optional[torch.Tensor] = None,
-                     checked: bool = False, token_major: bool = False) -> torch.Tensor:
+                     checked: bool = False, token_major: bool = False,
+                     like_query: bool = False) -> torch.Tensor:
     """softmax(scale q kᵀ [masked]) v for a few queries per head in one launch; returns
-    [batch, heads, tokens, head_dim] contiguous, or with `token_major` the transposed view of a
-    [batch, tokens, heads, head_dim] tensor. `checked`: the caller has just seen
+    [batch, heads, tokens, head_dim] contiguous, with `token_major` the transposed view of a
+    [batch, tokens, heads, head_dim] tensor, with `like_query` laid out as `torch.empty_like(q)` (what
+    ATen's fused attention ops return). `checked`: the caller has just seen
     `attention_decode_supported` accept exactly these operands."""
     if not checked:
         require_hip(q, k, v, attn_mask)
         if not attention_decode_supported(q, k, v, attn_mask):
             raise ValueError("attention_decode: unsupported operands (see attention_decode_supported)")
     b, h, t, d = q.shape
-    if token_major:
+    if like_query:
+        out = _gradient_like(q)
+    elif token_major:
         out = torch.empty((b, t, h, d), dtype=q.dtype, device=q.device).transpose(1, 2)
     else:
         out = torch.empty((b, h, t, d), dtype=q.dtype, device=q.device)
@@ -671,7 +675,7 @@ def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
 
 
 def attention_decode_append(q, k_past, v_past, k_new, v_new, scale: float):
-    """One decode step over a growing cache: (out [batch, heads, 1, head_dim], k, v) with
+    """One decode step over a growing cache: (out [batch, heads, 1, head_dim] laid out like q, k, v) with
     k = cat([k_past, k_new], 2), v likewise and out = softmax(scale q kᵀ) v, in one pass over the
     cache. None when the kernel does not take these tensors."""
     if not attention_decode_supported(q, k_past, v_past, None) or q.shape[2] != 1:
@@ -682,7 +686,7 @@ def attention_decode_append(q, k_past, v_past, k_new, v_new, scale: float):
                 or any(s % 8 or s < 0 for s in x.stride()[:3]) or x.data_ptr() % 16:
             return None
     past = k_past.shape[2]
-    out = torch.empty((b, h, 1, d), dtype=q.dtype, device=q.device)
+    out = _gradient_like(q)
     k = torch.empty((b, h, past + 1, d), dtype=q.dtype, device=q.device)
     v = torch.empty_like(k)
     st = [_I64X3(*x.stride()[:3]) for x in (q, k_past, v_past, k_new, v_new, out)]
