@@ -101,3 +101,36 @@ def test_compiled_attention_of_a_few_queries_is_viewed_and_multiplied(t, head_di
                              y.transpose(1, 2).reshape(2, t, 3 * head_dim))):
         # P is rounded to bf16 in one of the kernels, y once, and the product sums head_dim of them
         assert (x.double() - want).abs().max().item() <= 2.0 ** -7 * (1 + want.abs().max().item())
+
+
+def _took(recorded):
+    return [name for name, _ in recorded.launched]
+
+
+@pytest.mark.parametrize("scale", [float("nan"), float("inf"), 0.0, -1.0])
+def test_scales_the_kernels_do_not_take_go_to_pytorchs_op(recorded, monkeypatch, scale):
+    from torch_mojo_backend import aten_functions
+    theirs = []
+    flash = aten_functions.aten__scaled_dot_product_flash_attention
+    monkeypatch.setattr(aten_functions, "aten", types.SimpleNamespace(
+        _scaled_dot_product_flash_attention=lambda *a, **k: (theirs.append(1), (None,) * 9)[1]))
+    q = torch.zeros(1, 2, 1, 128).bfloat16()
+    flash(q, q, q, scale=scale)
+    assert theirs == [1] and _took(recorded) == []
+
+
+@pytest.mark.parametrize("scale", [float("nan"), float("inf"), 0.0, -1.0, 0.5])
+def test_only_an_ordinary_scale_makes_a_step_that_appends(scale):
+    from torch_mojo_backend.torch_compile_backend.compiler import _GraphFactory
+    aten = torch.ops.aten
+    graph = torch.fx.Graph()
+
+    def value(node, tokens):
+        node.meta["val"] = torch.zeros(1, 2, tokens, 64, dtype=torch.bfloat16)
+        return node
+
+    q, past, new = (value(graph.placeholder(name), n) for name, n in (("q", 1), ("past", 8), ("new", 1)))
+    k, v = (value(graph.call_function(aten.cat.default, ([past, new], 2)), 9) for _ in range(2))
+    flash = graph.call_function(aten._scaled_dot_product_flash_attention.default, (q, k, v), {"scale": scale})
+    graph.output((graph.call_function(operator.getitem, (flash, 0)), k, v))
+    assert (flash in _GraphFactory._fuse_decode_append(graph)) == (scale == 0.5)

@@ -30,6 +30,7 @@ step bit-identical to the kernels it replaces).
 from __future__ import annotations
 
 import datetime as dt
+import math
 import operator
 import os
 import time
@@ -637,6 +638,8 @@ class _GraphFactory:
             scale = node.kwargs.get("scale")
             if scale is None:
                 scale = 1.0 / float(q.meta["val"].shape[3]) ** 0.5
+            if not 0.0 < scale < math.inf:
+                continue
             plans[node] = ("decode_append", q, kp, vp, kn, vn, float(scale), kc, vc)
             plans[kc] = plans[vc] = None
         return plans
