@@ -223,9 +223,10 @@ int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t
  * GEMM kernel followed by an add kernel would.
  * `residual_dtype` and `out_dtype` are `dtype` or TMB_F32: a 16-bit model may keep its residual
  * stream in fp32 (fp32 residual in, fp32 sum out, nothing rounded in between; not together
- * with TMB_EPI_ROUND_LIKE_UNFUSED). 16-bit A and B on the MFMA path only; TMB_ERR_UNSUPPORTED
- * otherwise (fp32 A/B, k == 0, transposed A, unaligned operands, a GELU epilogue unless
- * TMB_EPI_ROUND_LIKE_UNFUSED): the caller then launches tmb_gemm and adds separately.
+ * with TMB_EPI_ROUND_LIKE_UNFUSED). TMB_ERR_UNSUPPORTED, after which the caller launches tmb_gemm and
+ * adds separately: k == 0, operands with fewer than eight (fp32: four) elements along a contiguous direction,
+ * a GELU epilogue unless TMB_EPI_ROUND_LIKE_UNFUSED, and a transposed A of a size at which the two launches are
+ * faster (tmb_gemm_route answers the same).
  * Replaces `AddF32Bf16Spec` / the residual add of aten_fast.py:657-687 together with the GEMM
  * in front of it. */
 int tmb_gemm_residual(void* c, const void* a, const void* b, const void* bias,

@@ -59,3 +59,41 @@ def test_the_scratch_a_caller_is_told_of_is_what_the_launch_splits_with(dtype_na
         assert full[2] * m * n * 4 in (0, told)
         split += full[2] > 0
     assert split > 20
+
+
+def test_a_large_transposed_a_with_a_residual_is_multiplied_and_added():
+    """The rings take such a product without a residual only; the any-layout kernel, which takes it with
+    one, is behind the two launches once the product is large."""
+    ek = _ek()
+    for residual_step in (0, ek.EPI_ROUND_LIKE_UNFUSED):
+        large = dict(ta=1, residual=1, epilogue=residual_step, workspace=PLENTY)
+        assert route(4096, 4096, 4096, **large) == ek.ERR_UNSUPPORTED
+        assert route(50304, 768, 16384, **large) == ek.ERR_UNSUPPORTED
+        assert route(256, 256, 256, **large)[0] == ANY               # one launch instead of two
+        assert route(768, 3072, 16384, **large)[0] == SPLITK         # its reduction adds the residual
+        assert route(4097, 4096, 4096, **large)[0] == ANY            # the rings do not take it either way
+    rounded = dict(ta=1, residual=1, epilogue=ek.EPI_ROUND_LIKE_UNFUSED)
+    assert route(768, 3072, 1024, **rounded) == ek.ERR_UNSUPPORTED   # one cheap add
+    assert route(768, 3072, 1024, ta=1, residual=1)[0] == ANY        # an add in float32 is four launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(256, 256, 256), (2048, 2048, 512), (4096, 2048, 2048)])
+def test_transposed_a_with_a_residual_matches_float64(mnk):
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    m, n, k = mnk
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, w, bias, r = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((k, m), (k, n), (n,), (m, n)))
+    plain = hip_ops.gemm(x.t(), w, bias)
+    exact = x.double().t().contiguous() @ w.double() + bias.double()
+    slack = (k + 2) * 2.0 ** -24 * (x.double().abs().t().contiguous() @ w.double().abs() + exact.abs()) + 1e-6
+    step = hip_ops.gemm(x.t(), w, bias, residual=r, round_like_unfused=True)
+    # rounded after the product (2^-9 of it) and after the sum
+    exact_step = exact + r.double()
+    assert ((step.double() - exact_step).abs() <= 2 * slack + 2.0 ** -8 * (exact.abs() + exact_step.abs())).all()
+    if mnk != (256, 256, 256):
+        assert torch.equal(step, plain + r)      # the same product, added apart
+    for out_dtype in (None, torch.float32):
+        wide = hip_ops.gemm(x.t(), w, bias, residual=r.float(), out_dtype=out_dtype)
+        assert ((wide.double() - exact_step).abs() <= 2 * slack + 2.0 ** -8 * (exact.abs() + exact_step.abs())).all()

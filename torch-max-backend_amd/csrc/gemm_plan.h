@@ -140,14 +140,17 @@ static inline bool any_eligible(int64_t m, int64_t n, int64_t k, int64_t lda, in
   if ((trans_a ? m : k) < 8 || (trans_b ? k : n) < 8) return false;
   return lda < (int64_t{1} << 23) && ldb < (int64_t{1} << 23);
 }
+// Microseconds of a product on the ring kernels: 900 TFLOP/s in rounds of 128 x 128 tiles, two per CU.
+static inline double ring_cost(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const double tiles = static_cast<double>((m + 127) / 128) * ((n + 127) / 128) * batch;
+  return 6.0 + (tiles <= 256.0 ? 0.011 * k : std::ceil(tiles / 512.0) * 0.0186 * k);
+}
 // Microseconds of the other way for the same operands: copy what the ring kernels cannot read into padded
-// buffers (3 us and the bytes at 4 TB/s each; a transposing copy at 1 TB/s), then multiply at 900
-// TFLOP/s in rounds of 128 x 128 tiles, two per CU. Within 15 % of the measured sum for products from
+// buffers (3 us and the bytes at 4 TB/s each; a transposing copy at 1 TB/s), then multiply there. Within 15 % of the measured sum for products from
 // 10 GFLOP on (4099^3 198 against 197, 4383 x 1568 x 1228 38 against 38, 1829 x 3429 x 4716 147 against 156).
 static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool a_ok,
                                  bool b_ok, int trans_a, int trans_b, bool plain) {
-  const double tiles = static_cast<double>((m + 127) / 128) * ((n + 127) / 128) * batch;
-  double cost = 6.0 + (tiles <= 256.0 ? 0.011 * k : std::ceil(tiles / 512.0) * 0.0186 * k);
+  double cost = ring_cost(batch, m, n, k);
   auto copy = [&](int64_t elements, bool transposing) {
     return 3.0 + static_cast<double>(elements) * batch * 4.0 / (transposing ? 1e6 : 4e6);
   };
@@ -165,6 +168,17 @@ static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k,
 }
 int gemm_any(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, bool bf16, int epilogue,
              hipStream_t stream);
+
+// A transposed A with a residual that the rings would multiply without one: whether the any-layout kernel, which
+// takes the residual along, is faster than their product and the caller's add (one pass of three 16-bit tensors, or
+// four in float32 when only the sum is rounded; 5.8 TB/s). 4096^3: 241 us there against 122 and 193 apart, 768 x 3072 x
+// 1024 24 against 17 and 31, 2048^3 40 against 27 and 46, 1024^3 14 against 15 and 27, 8192 x 8192 x 1024 420 against
+// 204 and 492. The fifth is the models' own error.
+static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, double any_cost) {
+  const double elements = static_cast<double>(g.m) * g.n * batch;
+  const double add = g.round_like_unfused ? 3.0 + elements * 6.0 / 5.8e6 : 12.0 + elements * 30.0 / 5.8e6;
+  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add;
+}
 
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
 // leave most CUs idle. K is cut into `splits` runs of whole stages (equal to within one stage)
@@ -329,6 +343,9 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
     AnyPlan plan = any_plan(batch, g.m, g.n, g.k, true);
     if (plan.splits > 0 && workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4)
       plan = any_plan(batch, g.m, g.n, g.k, false);
+    if (g.residual != nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue) &&
+        !any_with_residual_pays(g, batch, plan.cost))
+      return {TMB_ERR_UNSUPPORTED, 0, 0};
     return {TMB_GEMM_ANY, plan.tile, plan.splits};
   }
   if (aligned) {
