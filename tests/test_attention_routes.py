@@ -134,3 +134,30 @@ def test_only_an_ordinary_scale_makes_a_step_that_appends(scale):
     flash = graph.call_function(aten._scaled_dot_product_flash_attention.default, (q, k, v), {"scale": scale})
     graph.output((graph.call_function(operator.getitem, (flash, 0)), k, v))
     assert (flash in _GraphFactory._fuse_decode_append(graph)) == (scale == 0.5)
+
+
+@pytest.mark.parametrize("case,decode", [
+    # (batch, heads, queries, keys, head size): one query, whatever the rest
+    ((1, 12, 1, 64, 64), True), ((64, 16, 1, 4096, 64), True), ((64, 16, 1, 1024, 128), True),
+    # a few queries on few rows, from the keys on where the prefill kernel's serial walk is longer
+    ((1, 12, 2, 256, 64), True), ((1, 12, 16, 4096, 64), True), ((4, 12, 4, 1024, 64), True), ((1, 256, 1, 256, 64), True),
+    ((1, 12, 2, 255, 64), False), ((4, 12, 4, 64, 128), True),
+    # more rows: K and V once per row against once per 128 queries
+    ((32, 12, 16, 1024, 64), False), ((32, 12, 2, 1024, 64), False), ((4, 12, 8, 1024, 64), False),
+    ((8, 12, 4, 512, 128), False), ((1, 257, 2, 4096, 64), False), ((1, 128, 2, 4096, 64), True)])
+def test_a_few_queries_take_the_decode_kernel_where_it_is_the_faster_one(recorded, monkeypatch, case, decode):
+    from torch_mojo_backend import aten_functions
+    theirs = []
+    flash = aten_functions.aten__scaled_dot_product_flash_attention
+    monkeypatch.setattr(aten_functions, "aten", types.SimpleNamespace(
+        _scaled_dot_product_flash_attention=lambda *a, **k: (theirs.append(1), (None,) * 9)[1]))
+    b, h, t, s, d = case
+    q = torch.zeros(d, dtype=torch.bfloat16).as_strided((b, h, t, d), (0, 0, 0, 1))    # (only sizes are looked at)
+    k = torch.zeros(d, dtype=torch.bfloat16).as_strided((b, h, s, d), (0, 0, 0, 1))
+    flash(q, k, k)
+    if decode:
+        assert _took(recorded) == ["tmb_attention_decode"] and not theirs
+    elif d == 64:
+        assert _took(recorded) == ["tmb_attention_fwd"] and not theirs
+    else:
+        assert theirs == [1] and _took(recorded) == []

@@ -355,7 +355,7 @@ def aten__scaled_dot_product_flash_attention(query, key, value, dropout_p: float
     Dropout, a debug mask, other head sizes: PyTorch-ROCm's own op."""
     s = _flash_scale(query, scale)
     if dropout_p == 0.0 and not return_debug_mask and query.dim() == 4 and 0.0 < s < math.inf \
-            and query.shape[2] <= hip_ops.DECODE_MAX_QUERIES and _only_first_output_used() \
+            and key.dim() == 4 and hip_ops.attention_decode_pays(query, key) and _only_first_output_used() \
             and hip_ops.attention_decode_supported(query, key, value, None):
         # a few queries and no backward pass to hand statistics to: the memory-bound kernel
         out = hip_ops.attention_decode(query, key, value, s, bool(is_causal), checked=True, like_query=True)

@@ -607,9 +607,22 @@ def attention_backward(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: 
     return dq, dk, dv
 
 
-# Queries per (batch, head) up to which the decode kernel (one wave per query row, K and V read
-# once per query) is used instead of the GEMM-based paths.
+# Queries per (batch, head) up to which the decode kernel (K and V read once per query row) is used
+# instead of the GEMM-based paths.
 DECODE_MAX_QUERIES = 16
+
+
+def attention_decode_pays(q: torch.Tensor, k: torch.Tensor) -> bool:
+    """Whether the decode kernel is faster than a prefill kernel, which reads K and V once per 128 queries
+    but walks the keys of a (batch, head) in one workgroup. One query per head: at every size but a few
+    short ones (microseconds of launches in a recorded graph, decode against prefill, bf16, head size 64:
+    12 heads x 4096 keys 24 / 59, 384 x 256 9.8 / 8.2, 384 x 1024 22 / 28, 1024 x 1024 45 / 53; head size 128
+    against PyTorch's op: 1024 x 1024 89 / 112). More queries: while each row has a CU of its own and the
+    walk is long enough to matter (192 rows in all x 256 keys 6.6 / 6.3, x 1024 12 / 17, x 4096 41 / 71; 384
+    rows x 1024 22 / 17, 1536 x 1024 63 / 28, 6144 x 1024 169 / 28; head size 128, whose other way is
+    PyTorch's op: 192 rows x 64 keys 4.6 / 6.0, x 1024 21 / 34, 384 rows x 512 22 / 21)."""
+    b, h, t, d = q.shape
+    return t == 1 or (t <= DECODE_MAX_QUERIES and b * h * t <= 256 and (k.shape[2] >= 256 or d == 128))
 
 
 def attention_decode_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
