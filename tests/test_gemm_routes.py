@@ -97,3 +97,66 @@ def test_transposed_a_with_a_residual_matches_float64(mnk):
     for out_dtype in (None, torch.float32):
         wide = hip_ops.gemm(x.t(), w, bias, residual=r.float(), out_dtype=out_dtype)
         assert ((wide.double() - exact_step).abs() <= 2 * slack + 2.0 ** -8 * (exact.abs() + exact_step.abs())).all()
+
+
+@pytest.fixture()
+def recorded(monkeypatch):
+    """The launchers on host tensors with empty plan tables and a library that notes its launches."""
+    import torch
+    from test_attention_routes import RecordingLibrary
+    from torch_mojo_backend.eager_kernels import hip_ops
+
+    lib = RecordingLibrary(_ek().lib())
+    monkeypatch.setattr(_ek(), "lib", lambda: lib)
+    monkeypatch.setattr(hip_ops, "_stream", lambda: 0)
+    monkeypatch.setattr(hip_ops, "require_hip", lambda *a: None)
+    monkeypatch.setattr(hip_ops, "_GEMM_PLANS", {})
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    return lib
+
+
+def _launch(recorded, *args, **kwargs):
+    """(entry, sizes and flags, scratch) of the product's launch and of the copies in front of it."""
+    from torch_mojo_backend.eager_kernels import hip_ops
+    recorded.launched.clear()
+    hip_ops.gemm(*args, **kwargs)
+    seen = []
+    for name, args in recorded.launched:
+        scratch = args[-2] if name == "tmb_gemm_ws" else 0
+        seen.append((name, args[4:18] if name.startswith("tmb_gemm") else (), scratch))
+    return seen
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 104, 4096), (300, 1024, 8192), (512, 2048, 8192), (2048, 2048, 2048)])
+def test_the_launch_of_a_product_does_not_depend_on_the_one_before(recorded, m, n, k):
+    """Same sizes and strides, once on a 16-byte boundary and once off it: whichever came first."""
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    store = torch.zeros(m * k + 8, dtype=torch.bfloat16)
+    assert store.data_ptr() % 16 == 0
+    on, off = store[:m * k].view(m, k), store[1:m * k + 1].view(m, k)
+    b = torch.zeros(k, n, dtype=torch.bfloat16)
+    fresh = []
+    for a in (on, off):
+        hip_ops._GEMM_PLANS.clear()
+        fresh.append(_launch(recorded, a, b))
+    assert fresh[0] != fresh[1]
+    for order in ((0, 1), (1, 0)):
+        hip_ops._GEMM_PLANS.clear()
+        for _ in range(2):
+            for i in order:
+                assert _launch(recorded, (on, off)[i], b) == fresh[i], (order, i)
+
+
+def test_the_launch_of_an_epilogue_does_not_depend_on_the_plain_product_before(recorded):
+    """A transposed A: the rings take it without an epilogue only."""
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    a, b = torch.zeros(2048, 2048).bfloat16().t(), torch.zeros(2048, 2048).bfloat16()
+    gelu = dict(epilogue=_ek().EPI_GELU_ERF)
+    alone = _launch(recorded, a, b, **gelu)
+    hip_ops._GEMM_PLANS.clear()
+    plain = _launch(recorded, a, b)
+    assert plain != alone
+    for _ in range(2):
+        assert _launch(recorded, a, b, **gelu) == alone and _launch(recorded, a, b) == plain

@@ -264,15 +264,19 @@ _GEMM_WS_BYTES: dict = {}
 _GEMM_PLANS: dict = {}
 
 
+def _gemm_plan_key(a, b, bias, epi_flags) -> tuple:
+    return (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device,
+            a.data_ptr() % 16 == 0, b.data_ptr() % 16 == 0, epi_flags,
+            None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+
+
 def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
                     epi_flags: int = _ek.EPI_NONE) -> Optional[torch.Tensor]:
-    """``gemm(a, b, bias)`` when exactly this operand layout (shapes, strides, dtypes, devices)
-    has been validated and launched before, else None: the plan holds the launch arguments, so a
+    """``gemm(a, b, bias)`` when exactly this operand layout (shapes, strides, dtypes, devices, bases
+    on a 16-byte boundary or not, epilogue) has been validated and launched before, else None: the plan holds the launch arguments, so a
     repeated call (every layer of every decode step) costs one dictionary lookup, one allocation
     and the launch."""
-    plan = _GEMM_PLANS.get(
-        (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device,
-         None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device)))
+    plan = _GEMM_PLANS.get(_gemm_plan_key(a, b, bias, epi_flags))
     if plan is None:
         return None
     out_shape, dims, ws_bytes = plan
@@ -396,18 +400,15 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
             return unfused_residual()
         _check("tmb_gemm_residual_ws", rc)
         return out
-    # (scratch for operands that only their addresses keep from the aligned kernels is not for others)
-    any_address = in_place_ws is None or (a.data_ptr() | b.data_ptr()) % 16 == 0
-    if key is not None and a is a_in and b is b_in and bias is bias_in and out_dtype is None and any_address:
+    # (an operand that a running graph would pad and share is multiplied in place outside of one only)
+    shared = in_place_ws is not None and a.numel() * 2 >= _PAD_REUSE_MIN_BYTES
+    if key is not None and a is a_in and b is b_in and bias is bias_in and out_dtype is None and not shared:
         # operands are consumed in place: remember the launch arguments for this layout
         if len(_GEMM_PLANS) >= 4096:
             _GEMM_PLANS.clear()
-        plan_key = (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device,
-                    None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
-        _GEMM_PLANS[plan_key] = (tuple(out.shape),
-                                 (batch, m, n, k, la[1], lb[1], n, a.stride(0) if batched else 0,
-                                  b.stride(0) if batched else 0, m * n, la[0], lb[0], code_of(a.dtype)),
-                                 ws_bytes)
+        _GEMM_PLANS[_gemm_plan_key(a, b, bias, epi_flags)] = (
+            tuple(out.shape), (batch, m, n, k, la[1], lb[1], n, a.stride(0) if batched else 0,
+                               b.stride(0) if batched else 0, m * n, la[0], lb[0], code_of(a.dtype)), ws_bytes)
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
         rc = lib.tmb_gemm_ws(
