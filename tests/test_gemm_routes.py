@@ -160,3 +160,28 @@ def test_the_launch_of_an_epilogue_does_not_depend_on_the_plain_product_before(r
     assert plain != alone
     for _ in range(2):
         assert _launch(recorded, a, b, **gelu) == alone and _launch(recorded, a, b) == plain
+
+
+def test_products_of_depth_64_stay_on_their_kernel_beyond_four_gigabytes():
+    """It addresses a tile at a time; the rings' 32-bit offsets from the base end there."""
+    for m in (8192, (1 << 25) - 128, 1 << 25, 1 << 26):
+        for tb in (0, 1):
+            assert route(m, 1024, 64, tb=tb)[0] == STREAM64, m
+    assert route(1 << 25, 1024, 64, lda=1 << 23)[0] == STREAM64
+    assert route(1 << 25, 1024, 64, residual=1)[0] == ANY
+
+
+@pytest.mark.gpu
+def test_depth_64_beyond_four_gigabytes_matches_float64():
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    m, n = 1 << 25, 128
+    g = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.randn(m // 64, 64, generator=g, device="cuda").bfloat16().repeat(64, 1)
+    a[-1000:] = torch.randn(1000, 64, generator=g, device="cuda").bfloat16()
+    b = torch.randn(64, n, generator=g, device="cuda").bfloat16()
+    got = hip_ops.gemm(a, b)
+    rows = torch.cat([torch.arange(0, 300), torch.arange(m // 2 - 200, m // 2 + 200), torch.arange(m - 1200, m)]).cuda()
+    want = a[rows].double() @ b.double()
+    bound = 66 * 2.0 ** -24 * (a[rows].double().abs() @ b.double().abs()) + 1e-6 + 2.0 ** -8 * want.abs()
+    assert ((got[rows].double() - want).abs() <= bound).all()

@@ -339,6 +339,8 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
   }
   if (g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue))
     return {TMB_GEMM_TRANSPOSED_A, 0, 0};
+  // (in front of the any-layout kernel: it takes operands beyond the rings' 4 GiB)
+  if (!trans_a && stream64_eligible(g, batch, trans_b, epilogue)) return {TMB_GEMM_STREAM64, 0, 0};
   if (!aligned && any_eligible(g.m, g.n, g.k, g.lda, g.ldb, trans_a, trans_b)) {
     AnyPlan plan = any_plan(batch, g.m, g.n, g.k, true);
     if (plan.splits > 0 && workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4)
@@ -348,10 +350,7 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
       return {TMB_ERR_UNSUPPORTED, 0, 0};
     return {TMB_GEMM_ANY, plan.tile, plan.splits};
   }
-  if (aligned) {
-    if (stream64_eligible(g, batch, trans_b, epilogue)) return {TMB_GEMM_STREAM64, 0, 0};
-    return {TMB_GEMM_RING, 0, 0};
-  }
+  if (aligned) return {TMB_GEMM_RING, 0, 0};
   if (g.residual != nullptr) return {TMB_ERR_UNSUPPORTED, 0, 0};
   return {TMB_GEMM_SIMT, 0, 0};
 }
