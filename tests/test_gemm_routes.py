@@ -185,3 +185,66 @@ def test_depth_64_beyond_four_gigabytes_matches_float64():
     want = a[rows].double() @ b.double()
     bound = 66 * 2.0 ** -24 * (a[rows].double().abs() @ b.double().abs()) + 1e-6 + 2.0 ** -8 * want.abs()
     assert ((got[rows].double() - want).abs() <= bound).all()
+
+
+def test_fp32_products_with_long_rows_stay_on_the_matrix_cores():
+    """Lane offsets are 32-bit within a tile: what counts is the tile's rows times the pitch, and beyond that the
+    aligned kernel, which addresses in 64 bits, takes the product."""
+    f32 = dict(dtype=_ek().F32, workspace=PLENTY)
+    for k in (1 << 23, (1 << 23) + 1, 1 << 26):
+        kernel, _, splits = route(4, 8, k, tb=1, **f32)
+        assert kernel == F32 and splits > 1, k
+    assert route(1 << 24, 64, 100, ta=1, a_aligned=0, **f32)[0] == F32
+    kernel, _, splits = route(64, 64, 1 << 25, tb=1, **f32)
+    assert kernel == F32_WIDE and splits > 1 and (1 << 25) % (4 * splits) == 0
+    assert route(64, 64, (1 << 25) + 4, tb=1, **f32)[0] == F32_WIDE
+    assert route(64, 64, 1 << 25, tb=1, dtype=_ek().F32) == (F32_WIDE, 0, 0)
+    assert route(1 << 26, 64, 64, ta=1, **f32)[0] == F32_WIDE
+    assert route(64, 64, 1 << 25, tb=1, residual=1, **f32) == _ek().ERR_UNSUPPORTED
+    assert route(64, 64, 1 << 25, tb=1, a_aligned=0, **f32)[0] == SIMT     # (the launcher pads it first)
+
+
+def test_the_launcher_pads_exactly_what_the_fp32_kernel_does_not_read():
+    import itertools
+    from torch_mojo_backend.eager_kernels import hip_ops
+
+    class Operand:
+        @staticmethod
+        def element_size():
+            return 4
+
+    for m, n, k, ta, tb, extra in itertools.product((3, 4, 64, 65, 1 << 24, 1 << 25), (3, 4, 128, 129, 1 << 23),
+                                                    (3, 4, 31, 33, 1 << 23, 1 << 26), (0, 1), (0, 1), (0, 1 << 23)):
+        lda, ldb = (m if ta else k) + extra, (k if tb else n) + extra
+        read = route(m, n, k, ta, tb, _ek().F32, lda=lda, ldb=ldb, a_aligned=0, b_aligned=0)[0] == F32
+        assert hip_ops._f32_in_place(Operand, (ta, lda), (tb, ldb), m, n, k) == read, (m, n, k, ta, tb, extra)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [
+    # (m, n, k, pitch of A, A stored [K, M])
+    (4, 8, (1 << 23) + 1, None, False),      # long rows, few of them
+    (64, 60, 4096, 1 << 25, False),          # rows out of reach: the wide kernel, K split as a batch
+    (130, 60, 100, 35651584, True)])         # k-rows out of reach
+def test_fp32_long_rows_match_float64(case):
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    m, n, k, pitch, ta = case
+    g = torch.Generator(device="cuda").manual_seed(m)
+    rows, cols = (k, m) if ta else (m, k)
+    if pitch is None:
+        stored = torch.randn(rows, cols, generator=g, device="cuda")
+    else:
+        stored = torch.empty((rows - 1) * pitch + cols, device="cuda").as_strided((rows, cols), (pitch, 1))
+        stored.copy_(torch.randn(rows, cols, generator=g, device="cuda"))
+    a = stored.t() if ta else stored
+    b = torch.randn(n, k, generator=g, device="cuda").t()
+    bias = torch.randn(n, generator=g, device="cuda")
+    got = hip_ops.gemm(a, b, bias)
+    exact, size = bias.double().expand(m, n).clone(), bias.double().abs().expand(m, n).clone()
+    for at in range(0, k, 1 << 18):
+        x, y = a[:, at:at + (1 << 18)].double().contiguous(), b[at:at + (1 << 18)].double().contiguous()
+        exact += x @ y
+        size += x.abs() @ y.abs()
+    # k roundings in a chain would be k 2^-24 of the sum of magnitudes; runs of at most 2^19 of them are chained
+    assert ((got.double() - exact).abs() <= (min(k, 1 << 19) + 40) * 2.0 ** -24 * size).all()

@@ -308,11 +308,14 @@ static inline bool f32_wide_pays(int64_t batch, int64_t m, int64_t n, int64_t k)
   return (tiles >= 512 && tiles * 20 >= slots * 17) || (k <= 256 && tiles >= 176);
 }
 // What the kernel whose waves share K asks of its operands: at least four elements along each
-// contiguous direction, and lane offsets within a tile that fit 32 bits.
+// contiguous direction, and lane offsets that fit 32 bits in its largest tile (64 x 128; 32 rows of k for an
+// operand stored K-outer).
 static inline bool f32_shared_eligible(const GemmArgs& g, int trans_a, int trans_b) {
   if (g.m < 1 || g.n < 1 || g.k < 1) return false;
   if ((trans_a ? g.m : g.k) < 4 || (trans_b ? g.k : g.n) < 4) return false;
-  return g.lda < (int64_t{1} << 23) && g.ldb < (int64_t{1} << 23);
+  auto reached = [](int64_t lines, int64_t ld) { return ld < ((int64_t{1} << 30) - 256) / (lines > 1 ? lines - 1 : 1); };
+  return reached(trans_a ? kF32KS : (g.m < 64 ? g.m : 64), g.lda) &&
+         reached(trans_b ? (g.n < 128 ? g.n : 128) : kF32KS, g.ldb);
 }
 
 // Which kernel takes a product, with its tile (an index into the kernel's own list; 128 or 256 for SplitK) and
@@ -357,15 +360,19 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
 
 static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
                                   size_t workspace_bytes) {
-  if (!f32_shared_eligible(g, trans_a, trans_b))
-    return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
-  if (g.residual == nullptr && f32_wide_pays(batch, g.m, g.n, g.k) && f32_mfma_eligible(g, batch, trans_a, trans_b))
-    return {TMB_GEMM_F32_WIDE, 0, 0};
+  const bool shared = f32_shared_eligible(g, trans_a, trans_b);
+  const bool wide = g.residual == nullptr && f32_mfma_eligible(g, batch, trans_a, trans_b);
+  if (!shared && !wide) return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
+  if (wide && f32_wide_pays(batch, g.m, g.n, g.k)) return {TMB_GEMM_F32_WIDE, 0, 0};
   F32Plan plan = f32_plan(batch, g.m, g.n, g.k, true);
   if (plan.splits > 0 && (g.m * g.n >= (int64_t{1} << 31) ||
                           workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
     plan = f32_plan(batch, g.m, g.n, g.k, false);
-  return {TMB_GEMM_F32, plan.tile, plan.splits};
+  if (shared) return {TMB_GEMM_F32, plan.tile, plan.splits};
+  // rows too long for 32-bit offsets: the wide kernel, a split as a batch of equal runs of whole 16-byte pieces
+  int splits = plan.splits;
+  while (splits > 0 && (splits == 1 || g.k % (4 * splits) != 0)) --splits;
+  return {TMB_GEMM_F32_WIDE, 0, splits};
 }
 
 // The typed half of the entry point (gemm_typed.h), one translation unit per storage type.

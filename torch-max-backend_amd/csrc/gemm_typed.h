@@ -248,7 +248,14 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
   if constexpr (__is_same(T, float)) {
     const GemmRoute r = route_f32(g, batch, trans_a, trans_b, scratch);
     switch (r.kernel) {
-      case TMB_GEMM_F32_WIDE: return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
+      case TMB_GEMM_F32_WIDE:
+        if (r.splits == 0) return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
+        return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](GemmArgs part) {
+          part.k = g.k / r.splits;
+          part.stride_a = trans_a ? part.k * g.lda : part.k;
+          part.stride_b = trans_b ? part.k : part.k * g.ldb;
+          return launch_f32_mfma<TMB_EPI_NONE>(part, r.splits, trans_a, trans_b, stream);
+        });
       case TMB_GEMM_F32:
         if (r.splits == 0) return launch_f32_shared<EPI>(g, batch, r.tile, trans_a, trans_b, stream);
         return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](const GemmArgs& part) {

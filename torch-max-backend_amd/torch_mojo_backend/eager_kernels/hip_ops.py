@@ -192,9 +192,11 @@ def _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, plain_epilogue=True) -> boo
 
 def _f32_in_place(a, la, lb, m, n, k) -> bool:
     """Whether the fp32 kernel reads these operands where they lie, whatever their alignment (mirrors
-    the library's check): four elements along each contiguous direction."""
+    the library's check): four elements along each contiguous direction, and a tile's rows within
+    reach of 32-bit offsets."""
     return a.element_size() == 4 and (m if la[0] else k) >= 4 and (k if lb[0] else n) >= 4 \
-        and la[1] < 1 << 23 and lb[1] < 1 << 23
+        and la[1] < ((1 << 30) - 256) // max((32 if la[0] else min(m, 64)) - 1, 1) \
+        and lb[1] < ((1 << 30) - 256) // max((min(n, 128) if lb[0] else 32) - 1, 1)
 
 
 def _relayout_for_mfma(a, b, la, lb, m, n, k, batched, plain=True):
