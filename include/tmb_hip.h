@@ -174,8 +174,9 @@ int tmb_gemm(void* c, const void* a, const void* b, const void* bias, int64_t ba
  * weight gradient dy^T x, narrow projections) then run split along K: fp32 partials
  * [splits][m][n] in the workspace, added in split order by a second kernel that applies bias,
  * epilogue and the one cast (still fp32 accumulation and one rounding; the result depends on the
- * shape only). tmb_gemm_workspace_bytes is 0 when the shape would not be split; with a NULL or
- * too small workspace the call behaves exactly like tmb_gemm.
+ * shape only). tmb_gemm_workspace_bytes is what a product of this shape is split with in the layout that
+ * asks for most (16-bit: aligned operands), 0 when none would be split; with a NULL or too small workspace
+ * the call behaves exactly like tmb_gemm.
  * The reference's GPU GEMM takes its split-K scratch from the MAX runtime
  * (eager_kernels/matmul_ops.mojo:1040-1049, `multistage_gemm_kernel`); here the caller owns it,
  * as with every other buffer. */

@@ -105,9 +105,10 @@ def test_workspace_plan_is_a_pure_function_of_the_shape():
     assert full == L.tmb_reduce_workspace_bytes(1, 65536 * 4096, ek.BF16)
     assert L.tmb_reduce_workspace_bytes(512, 50257, ek.F32) == 512 * 3 * 16
     assert L.tmb_reduce_workspace_bytes(0, 10, ek.F32) == 0
-    # split-K scratch: only for half-precision products with fewer tiles than CUs and a long K
+    # split-K scratch: only for products with fewer tiles than CUs and a long K
     assert L.tmb_gemm_workspace_bytes(1, 8192, 8192, 8192, ek.BF16) == 0
-    assert L.tmb_gemm_workspace_bytes(1, 1024, 768, 3072, ek.F32) == 8 * 1024 * 768 * 4
+    assert L.tmb_gemm_workspace_bytes(1, 1024, 768, 3072, ek.F32) == 0    # 32 x 32 tiles fill the chip unsplit
+    assert L.tmb_gemm_workspace_bytes(1, 128, 768, 3072, ek.F32) == 8 * 128 * 768 * 4
     assert L.tmb_gemm_workspace_bytes(1, 4096, 4096, 4096, ek.F32) == 0
     assert L.tmb_gemm_workspace_bytes(1, 1024, 768, 3072, ek.BF16) == 5 * 1024 * 768 * 4
     assert L.tmb_gemm_workspace_bytes(2, 1024, 768, 3072, ek.BF16) == 0

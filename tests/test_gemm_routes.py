@@ -61,6 +61,32 @@ def test_the_scratch_a_caller_is_told_of_is_what_the_launch_splits_with(dtype_na
     assert split > 20
 
 
+@pytest.mark.parametrize("seed", range(4))
+def test_scratch_for_an_unknown_layout_is_enough_for_every_layout(seed):
+    """fp32, whose splits do not depend on the layout: what tmb_gemm_workspace_bytes answers splits as far as any
+    amount does, and is no more than that."""
+    import math
+    import random
+    ek, rng = _ek(), random.Random(seed)
+    shapes = [(31, 67, 12565), (12, 1272, 1974), (245, 4220, 13614), (100, 72, 8200), (1024, 768, 3072), (2759, 3965, 26572)]
+    shapes += [tuple(round(math.exp(rng.uniform(math.log(4), math.log(30000)))) for _ in range(3)) for _ in range(300)]
+    split = 0
+    for m, n, k in shapes:
+        told = ek.lib().tmb_gemm_workspace_bytes(1, m, n, k, ek.F32)
+        most = 0
+        for ta, tb, aligned in itertools.product((0, 1), repeat=3):
+            form = dict(ta=ta, tb=tb, dtype=ek.F32, a_aligned=aligned)
+            full = route(m, n, k, workspace=PLENTY, **form)
+            assert route(m, n, k, workspace=told, **form) == full, (m, n, k, form)
+            most = max(most, full[2])
+            by_layout = ek.lib().tmb_gemm_layout_workspace_bytes(1, m, n, k, ta, tb, ek.F32)
+            if aligned or by_layout:
+                assert route(m, n, k, workspace=by_layout, **form) == full, (m, n, k, form)
+        assert told == most * m * n * 4, (m, n, k)
+        split += most > 0
+    assert split > 30
+
+
 def test_a_large_transposed_a_with_a_residual_is_multiplied_and_added():
     """The rings take such a product without a residual only; the any-layout kernel, which takes it with
     one, is behind the two launches once the product is large."""

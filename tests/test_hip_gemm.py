@@ -573,7 +573,7 @@ def test_split_k_is_reproducible_and_needs_scratch_only_when_it_pays():
     assert lib.tmb_gemm_workspace_bytes(4, 1024, 768, 4096, code) == 0       # batched
     f32 = _ops().code_of(torch.float32)
     assert lib.tmb_gemm_workspace_bytes(1, 4096, 4096, 4096, f32) == 0       # fp32: plenty of tiles
-    assert lib.tmb_gemm_workspace_bytes(1, 1024, 768, 4096, f32) == 8 * 1024 * 768 * 4
+    assert lib.tmb_gemm_workspace_bytes(1, 1024, 768, 4096, f32) == 0        # fp32: its smaller tiles fill the chip
     a = _dev(seeded((512, 4096), seed=31, dtype=torch.bfloat16))
     b = _dev(seeded((4096, 384), seed=32, dtype=torch.bfloat16))
     first = _ops().gemm(a, b)
@@ -632,7 +632,7 @@ def test_fp32_mfma_batched_strided_and_gelu():
 def test_fp32_split_k_is_reproducible_and_close_to_the_unsplit_kernel():
     m, n, k = 128, 768, 3072
     lib, ek = _ek().lib(), _ek()
-    assert lib.tmb_gemm_workspace_bytes(1, m, n, k, ek.F32) == 16 * m * n * 4
+    assert lib.tmb_gemm_workspace_bytes(1, m, n, k, ek.F32) == 8 * m * n * 4
     a = _dev(seeded((m, k), seed=51, dtype=torch.float32))
     w = _dev(seeded((n, k), seed=52, dtype=torch.float32))
     bias = _dev(seeded((n,), seed=53, dtype=torch.float32))

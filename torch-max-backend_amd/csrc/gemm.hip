@@ -115,21 +115,20 @@ extern "C" int tmb_gemm(void* c, const void* a, const void* b, const void* bias,
 
 extern "C" size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k,
                                            int dtype) {
+  using namespace tmb;
   if (dtype != TMB_F32 && dtype != TMB_F16 && dtype != TMB_BF16) return 0;
-  const tmb::SplitKPlan plan = dtype == TMB_F32 ? tmb::splitk_plan_f32(batch, m, n, k)
-                                                : tmb::splitk_plan(batch, m, n, k);
-  if (plan.splits == 0 || m * n >= (int64_t{1} << 31)) return 0;
-  return static_cast<size_t>(plan.splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
+  if (batch < 1 || m < 1 || n < 1 || k < 1 || m * n >= (int64_t{1} << 31)) return 0;
+  const int splits = dtype == TMB_F32 ? f32_plan(batch, m, n, k, true).splits : splitk_plan(batch, m, n, k).splits;
+  return static_cast<size_t>(splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
 }
 
 extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a,
                                                   int trans_b, int dtype) {
-  // the kernel for small products needs none (operands it cannot take run unsplit then)
-  if (dtype != TMB_F32 && !trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k))
-    return 0;
+  // the kernels for small and for wide products need none (operands they cannot take run unsplit then)
   if (dtype == TMB_F32) {
-    if (batch < 1 || m < 1 || n < 1 || k < 1 || tmb::f32_wide_pays(batch, m, n, k) || m * n >= (int64_t{1} << 31)) return 0;
-    return static_cast<size_t>(tmb::f32_plan(batch, m, n, k, true).splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
+    if ((trans_a ? m : k) % 4 == 0 && (trans_b ? k : n) % 4 == 0 && tmb::f32_wide_pays(batch, m, n, k)) return 0;
+  } else if (!trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k)) {
+    return 0;
   }
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
 }

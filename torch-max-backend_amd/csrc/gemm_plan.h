@@ -194,10 +194,9 @@ static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, doub
 struct SplitKPlan {
   int splits;  // 0: not used
   int tile;    // 128 or 256
-  int64_t k_chunk;  // fp32 kernel only: equal chunks
 };
 static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  SplitKPlan p{0, 0, 0};
+  SplitKPlan p{0, 0};
   if (batch != 1 || k < 2048 || k % 32 != 0 || n <= 64 || m < 1) return p;
   const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128);
   if (t128 >= 256) return p;  // at least one tile per CU: no split
@@ -227,24 +226,6 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
       }
     }
   }
-  return p;
-}
-
-// What tmb_gemm_workspace_bytes answers for fp32: room for the splits of a long K over few 128 x 128
-// tiles, as many as any plan below asks for on such shapes.
-static inline SplitKPlan splitk_plan_f32(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  SplitKPlan p{0, 0, 0};
-  if (batch != 1 || k < 128 || m < 1 || n < 1) return p;
-  const int64_t tiles = ((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN);
-  if (tiles >= 256) return p;
-  int64_t splits = 512 / tiles;
-  if (splits > 16) splits = 16;
-  if (splits > k / 64) splits = k / 64;
-  while (splits >= 2 && k % (splits * 4) != 0) --splits;
-  if (splits < 2) return p;
-  p.splits = static_cast<int>(splits);
-  p.tile = 128;
-  p.k_chunk = k / splits;
   return p;
 }
 
