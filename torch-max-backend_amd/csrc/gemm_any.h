@@ -186,6 +186,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_any_kernel(GemmArgs g, int ep
   for (int64_t s = first + wave; s < slices; s += WAVES) {
     sa.lay_down(la, K - s * KS, a_edge, lane);
     sb.lay_down(lb, K - s * KS, b_edge, lane);
+    wave_lds_point();
     if (s + WAVES < slices) load(s + WAVES);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -199,6 +200,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_any_kernel(GemmArgs g, int ep
         for (int i = 0; i < TM; ++i) acc[i][j] = Mfma16<T>::run(bf, af[i], acc[i][j]);
       }
     }
+    wave_lds_point();
   }
 
   // A lane holds row lane % 16 and four consecutive columns of each 16 x 16 result.

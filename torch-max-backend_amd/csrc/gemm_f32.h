@@ -173,6 +173,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
   for (int64_t s = first + wave; s < slices; s += WAVES) {
     sa.lay_down(la, K - s * kF32KS, a_edge, lane);
     sb.lay_down(lb, K - s * kF32KS, b_edge, lane);
+    wave_lds_point();
     if (s + WAVES < slices) load(s + WAVES);
 #pragma unroll
     for (int grp = 0; grp < kF32KS / 8; ++grp) {
@@ -189,6 +190,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
           for (int j = 0; j < TN; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[j][e], af[i][e], acc[i][j], 0, 0, 0);
     }
+    wave_lds_point();
   }
 
   // Lane holds row lr of each 32 x 32 result and columns 8q + 4 * lk + {0..3}.

@@ -21,6 +21,15 @@
 
 namespace tmb {
 
+// Between a wave's stores to LDS and its other lanes' reads of them, and again before the next stores: the hardware
+// keeps a wave's LDS accesses in order, this keeps the compiler from reordering accesses that only look unrelated
+// lane by lane. No instruction comes of it.
+__device__ __forceinline__ void wave_lds_point() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Bias has already been added in fp32. A GELU epilogue works on that fp32 sum and the result is
 // cast once (the reference's rule for everything it fuses into a GEMM: form the value in fp32,
 // cast exactly once, matmul_ops.mojo:2651-2657). With `twice` the sum is first rounded to the

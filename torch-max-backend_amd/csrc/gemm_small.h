@@ -12,7 +12,7 @@
 //
 // A wave brings its slices in as whole 128-byte lines (eight lanes to a line), lays them into a
 // wave-private part of LDS and reads the MFMA operands from there; the LDS works in order per wave,
-// so no workgroup barrier is needed. (Loading operand fragments straight into registers, 16 rows of
+// so no workgroup barrier is needed, only a point the compiler moves no LDS access across. (Loading operand fragments straight into registers, 16 rows of
 // 64 bytes per instruction, ran 20-25 % slower at K = 3072: half-line requests.) B stored [K, N] is
 // laid down as it lies in memory and read back transposed with ds_read_b64_tr_b16.
 #pragma once
@@ -212,8 +212,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_small_kernel(GemmArgs g) {
   if (wave < slices) load(wave);
   for (int64_t at = wave; at < slices; at += WAVES) {
     lay_down();
+    wave_lds_point();
     if (at + WAVES < slices) load(at + WAVES);
     multiply();
+    wave_lds_point();
   }
 
   // A lane holds row lane % 16 and four consecutive columns of each 16 x 16 result.
