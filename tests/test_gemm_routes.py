@@ -230,20 +230,66 @@ def test_fp32_products_with_long_rows_stay_on_the_matrix_cores():
     assert route(64, 64, 1 << 25, tb=1, a_aligned=0, **f32)[0] == SIMT     # (the launcher pads it first)
 
 
-def test_the_launcher_pads_exactly_what_the_fp32_kernel_does_not_read():
-    import itertools
-    from torch_mojo_backend.eager_kernels import hip_ops
-
-    class Operand:
-        @staticmethod
-        def element_size():
-            return 4
-
-    for m, n, k, ta, tb, extra in itertools.product((3, 4, 64, 65, 1 << 24, 1 << 25), (3, 4, 128, 129, 1 << 23),
-                                                    (3, 4, 31, 33, 1 << 23, 1 << 26), (0, 1), (0, 1), (0, 1 << 23)):
+def test_fp32_operands_that_no_matrix_kernel_reads_are_padded():
+    """Fewer than four contiguous elements, or rows out of reach of 32-bit offsets; and where padding is only the faster
+    way, the copies run on the kernel for which they are made."""
+    pays = 0
+    for m, n, k, ta, tb, extra in itertools.product((3, 4, 64, 65, 5000, 1 << 24, 1 << 25), (3, 4, 128, 129, 8000, 1 << 23),
+                                                    (3, 4, 31, 33, 200, 1 << 23, 1 << 26), (0, 1), (0, 1), (0, 1 << 23)):
         lda, ldb = (m if ta else k) + extra, (k if tb else n) + extra
-        read = route(m, n, k, ta, tb, _ek().F32, lda=lda, ldb=ldb, a_aligned=0, b_aligned=0)[0] == F32
-        assert hip_ops._f32_in_place(Operand, (ta, lda), (tb, ldb), m, n, k) == read, (m, n, k, ta, tb, extra)
+        pad = _ek().lib().tmb_gemm_f32_padding_pays(1, m, n, k, lda, ldb, 0, 0, ta, tb, 0)
+        lines, lanes = (32 if ta else min(m, 64)), (min(n, 128) if tb else 32)
+        reach = (1 << 30) - 256
+        read = (m if ta else k) >= 4 and (k if tb else n) >= 4 and lda < reach // max(lines - 1, 1) \
+            and ldb < reach // max(lanes - 1, 1)
+        if not read:
+            assert pad == 1, (m, n, k, ta, tb, extra)
+        elif pad and m * n < 1 << 31:
+            depth = k if k % 4 == 0 else (k + 63) // 64 * 64
+            assert route(m, n, depth, 0, 1, _ek().F32)[0] == F32_WIDE, (m, n, k, ta, tb, extra)
+            pays += 1
+    assert pays > 20
+
+
+FORMS_F32 = [dict(ta=ta, tb=tb, a_aligned=a, b_aligned=b) for ta, tb, a, b in itertools.product((0, 1), repeat=4)]
+
+
+@pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])
+def test_short_k_over_many_tiles_leaves_the_kernels_whose_waves_share_k(dtype_name):
+    """One slice of K or less for a workgroup's four waves and a launch of many tiles: the vector kernel or the 128 x 128
+    one, as before those kernels; few tiles or a longer K stay, whatever the form."""
+    dtype = getattr(_ek(), dtype_name)
+    waves = F32 if dtype_name == "F32" else ANY
+    many = [(48, 5222, 16, 8), (48, 402, 354, 8), (1, 6461, 1251, 9), (5, 2632, 758, 8)]
+    for (batch, m, n, k), form in itertools.product(many, FORMS_F32):
+        if dtype_name != "F32" and form["a_aligned"] and not form["ta"] and k % 8 == 0:
+            form = dict(form, a_aligned=0)      # (aligned 16-bit operands have kernels of their own)
+        got = route(m, n, k, batch=batch, dtype=dtype, **form)
+        assert got in ((SIMT, 0, 0), (F32_WIDE, 0, 0)), (batch, m, n, k, form)
+    for (batch, m, n, k), form in itertools.product([(1, 100, 200, 30), (1, 8, 8, 8), (1, 2000, 999, 150), (48, 401, 350, 130),
+                                                     (1, 333, 77, 50), (2, 5000, 3001, 333)], FORMS_F32):
+        form = dict(form, a_aligned=0)
+        assert route(m, n, k, batch=batch, dtype=dtype, **form)[0] == waves, (batch, m, n, k, form)
+    # the waves' kernels carry a residual, the others' product and the add apart where they are the faster way
+    off = dict(a_aligned=0, dtype=dtype, residual=1)
+    assert route(2000, 999, 150, **off)[0] == waves
+    if dtype_name == "F32":
+        for batch, m, n, k in ((1, 7016, 248, 12), (1, 840, 3000, 8), (5, 1696, 1848, 312)):
+            assert route(m, n, k, tb=1, batch=batch, dtype=dtype) == (F32_WIDE, 0, 0)
+        assert route(4104, 608, 8, tb=1, batch=48, **off) == _ek().ERR_UNSUPPORTED
+        assert route(112, 6216, 8, tb=1, batch=48, residual=1, dtype=dtype) == _ek().ERR_UNSUPPORTED
+        assert route(4096, 4096, 4096, residual=1, dtype=dtype)[0] == F32
+
+
+def test_the_launcher_pads_fp32_operands_of_short_k(recorded):
+    """Off a 16-byte boundary; the copies run without a residual, which is added apart."""
+    import torch
+    m, n, k = 6000, 7000, 96
+    store, b = torch.zeros(m * k + 4), torch.zeros(k, n)
+    off, residual = store[1:m * k + 1].view(m, k), torch.zeros(m, n)
+    for kw in ({}, {"residual": residual}):
+        assert [name for name, _, _ in _launch(recorded, off, b, **kw)] == ["tmb_pad_rows", "tmb_gemm"]
+    assert [name for name, _, _ in _launch(recorded, off[:300], b[:, :400])] == ["tmb_gemm"]
 
 
 @pytest.mark.gpu

@@ -133,6 +133,44 @@ static inline AnyPlan any_plan(int64_t batch, int64_t m, int64_t n, int64_t k, b
       if (k >= 192 * s) consider(s);
   return p;
 }
+// Short K over many tiles, against the vector kernel: the waves of a workgroup share 64-deep slices (32-deep in
+// fp32), so with one slice or less all but one of them idle, and a launch of many tiles takes what a tile's
+// way through LDS takes. The vector kernel's 64 x 64 tiles are then faster (bf16 7309 x 3268 x 2 31 against 70 us, 48 x
+// 402 x 354 x 8 14 against 26; fp32 48 x 5222 x 7 x 5 17 against 55). Microseconds of both, a start and rounds of tiles,
+// fitted to 1200 shapes a type of 2 .. 9000 in each extent, half of them K <= 128, 1 .. 48 batches; 12-17 % (rms). Over
+// those shapes, where one of the two was forced: 97 (fp32: 287) of 1200 were more than a tenth slower than before the
+// kernels whose waves share K, with these rules and f32_padded_cost below 4 (15) are.
+struct ManyTiles {
+  double start, per_k, per_tile, power;
+};
+constexpr ManyTiles kAnyMany[] = {{3.1, 0.00157, 0.585, 0.991}, {2.9, 0.00204, 1.11, 0.986}, {3.2, 0.00262, 1.355, 0.978},
+                                  {3.8, 0.00285, 0.637, 0.972}, {2.9, 0.00604, 3.21, 0.919}};
+static inline double many_tiles_cost(const ManyTiles& t, int bm, int bn, int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const double r = static_cast<double>(((m + bm - 1) / bm) * ((n + bn - 1) / bn)) * batch / 256.0;
+  return t.start + (r <= 1.0 ? 1.0 : std::pow(r, t.power)) * (t.per_k * k + t.per_tile);
+}
+static inline double simt_cost(bool f32, int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const double tiles = static_cast<double>(((m + 63) / 64) * ((n + 63) / 64)) * batch, r = tiles / 256.0;
+  const double filled = static_cast<double>(m) * n * batch / (tiles * 4096.0);
+  const double alone = f32 ? 0.17 * k - 1.9 : 0.15 * k - 0.5;
+  const double many = f32 ? r * (0.038 * k + 0.24 + 1.33 * filled) : r * (0.036 * k + 0.21 + 0.72 * filled);
+  return (f32 ? 5.2 : 5.1) + (alone > many ? alone : many);
+}
+// What a product costs beside itself when its residual is added apart: one pass of three tensors, or four launches in
+// float32 when only the sum of 16-bit operands is rounded; 5.8 TB/s.
+constexpr double kF32ResidualPerElement = 2e-6;  // what it costs in the fp32 kernel whose waves share K: about as much
+static inline double add_apart_cost(const GemmArgs& g, int64_t batch, bool f32) {
+  const double elements = static_cast<double>(g.m) * g.n * batch;
+  if (f32) return 3.0 + elements * 12.0 / 5.8e6;
+  return g.round_like_unfused ? 3.0 + elements * 6.0 / 5.8e6 : 12.0 + elements * 30.0 / 5.8e6;
+}
+static inline bool simt_instead_of_any(const GemmArgs& g, int64_t batch, const AnyPlan& plan) {
+  if (plan.splits > 0 || g.k > 32) return false;
+  const AnyTile& t = kAnyTiles[plan.tile];
+  const double apart = g.residual != nullptr ? add_apart_cost(g, batch, false) : 0.0;
+  return simt_cost(false, batch, g.m, g.n, g.k) + apart <
+         many_tiles_cost(kAnyMany[plan.tile], t.bm, t.bn, batch, g.m, g.n, g.k);
+}
 // What that kernel asks of its operands: eight elements along each contiguous direction, and lane
 // offsets within a tile that fit 32 bits.
 static inline bool any_eligible(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int trans_a, int trans_b) {
@@ -170,14 +208,11 @@ int gemm_any(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_
              hipStream_t stream);
 
 // A transposed A with a residual that the rings would multiply without one: whether the any-layout kernel, which
-// takes the residual along, is faster than their product and the caller's add (one pass of three 16-bit tensors, or
-// four in float32 when only the sum is rounded; 5.8 TB/s). 4096^3: 241 us there against 122 and 193 apart, 768 x 3072 x
-// 1024 24 against 17 and 31, 2048^3 40 against 27 and 46, 1024^3 14 against 15 and 27, 8192 x 8192 x 1024 420 against
-// 204 and 492. The fifth is the models' own error.
+// takes the residual along, is faster than their product and the caller's add. 4096^3: 241 us there against 122 and
+// 193 apart, 768 x 3072 x 1024 24 against 17 and 31, 2048^3 40 against 27 and 46, 1024^3 14 against 15 and 27, 8192 x
+// 8192 x 1024 420 against 204 and 492. The fifth is the models' own error.
 static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, double any_cost) {
-  const double elements = static_cast<double>(g.m) * g.n * batch;
-  const double add = g.round_like_unfused ? 3.0 + elements * 6.0 / 5.8e6 : 12.0 + elements * 30.0 / 5.8e6;
-  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add;
+  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add_apart_cost(g, batch, false);
 }
 
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
@@ -244,7 +279,10 @@ constexpr int kF32TileCount = sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
 struct F32Plan {
   int tile;    // index into kF32Tiles
   int splits;  // 0: not split
+  double cost;
 };
+constexpr ManyTiles kF32Many[] = {{2.9, 0.0075, 0.90, 0.933}, {2.8, 0.0129, 1.95, 0.939}, {3.6, 0.0211, 3.2, 0.969},
+                                  {0.0, 0.0368, 10.97, 0.953}};
 static inline double f32_cost(const F32Tile& t, double batch, int64_t m, int64_t n, double k) {
   const double tiles = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * batch;
   double rounds = std::ceil(tiles / 256.0);
@@ -256,7 +294,7 @@ static inline double f32_cost(const F32Tile& t, double batch, int64_t m, int64_t
   return 7.0 + rounds * (2.0 * t.bm * t.bn * k / 256.0 / 2400.0 * t.stretch + t.per_tile);
 }
 static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool may_split) {
-  F32Plan p{kF32TileCount - 1, 0};
+  F32Plan p{kF32TileCount - 1, 0, 0.0};
   double best = 0.0;
   for (int i = 0; i < kF32TileCount; ++i) {
     const double c = f32_cost(kF32Tiles[i], static_cast<double>(batch), m, n, static_cast<double>(k));
@@ -265,6 +303,7 @@ static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, b
       p.tile = i;
     }
   }
+  p.cost = many_tiles_cost(kF32Many[p.tile], kF32Tiles[p.tile].bm, kF32Tiles[p.tile].bn, batch, m, n, k);
   if (batch != 1 || !may_split) return p;
   best *= 0.92;  // a second launch and a workspace have to pay for themselves
   for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
@@ -273,8 +312,7 @@ static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, b
       const double c = f32_cost(kF32Tiles[i], s, m, n, static_cast<double>(k) / s) + 5.5 + 1e-6 * s * m * n;
       if (c < best) {
         best = c;
-        p.tile = i;
-        p.splits = s;
+        p = F32Plan{i, s, c};
       }
     }
   }
@@ -287,6 +325,46 @@ static inline bool f32_wide_pays(int64_t batch, int64_t m, int64_t n, int64_t k)
   const int64_t tiles = ((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN) * batch;
   const int64_t slots = (tiles + 255) / 256 * 256;
   return (tiles >= 512 && tiles * 20 >= slots * 17) || (k <= 256 && tiles >= 176);
+}
+// Microseconds on that kernel (fitted with the ones above), and whether aligned operands run there: also where these say
+// so (short K on fewer tiles: 7016 x 248 x 12 7 against 13 us, 840 x 3000 x 8 7 against 13; 5 x 1696 x 1848 x 312 122
+// against 159).
+static inline double f32_wide_cost(int64_t batch, int64_t m, int64_t n, int64_t k) {
+  const double rounds = static_cast<double>((((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN) * batch + 255) / 256);
+  const double tiles = std::pow(rounds, 0.923) * (0.078 * k + 3.09);
+  const double stores = static_cast<double>(batch) * m * n * 4.0 / 5.5e6;
+  return 3.2 + (tiles > stores ? tiles : stores);
+}
+static inline bool f32_wide_wins(int64_t batch, int64_t m, int64_t n, int64_t k, const F32Plan& plan) {
+  return f32_wide_pays(batch, m, n, k) || (plan.splits == 0 && f32_wide_cost(batch, m, n, k) < plan.cost);
+}
+// Unaligned operands: the other way is to copy what the 128 x 128 kernel cannot read into padded buffers (8 us a copy
+// with what the host does for it, and the bytes at 5.3 TB/s, 1.3 where it transposes) and to multiply there, a K that is no
+// whole number of 16-byte vectors as the next multiple of 64; infinite where the copies would not run on that kernel.
+// 7710 x 8280 x 8 60 against 317 us where it lies, 48 x 816 x 3664 x 16 175 against 721, 8051 x 6756 x 172 with a
+// residual 350 against 630.
+static inline double f32_padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool a_ok,
+                                     bool b_ok, int trans_a, int trans_b) {
+  double cost = 0.0;
+  auto copy = [&](int64_t elements, bool transposing) {
+    cost += 8.0 + static_cast<double>(elements) * batch * 8.0 / (transposing ? 1.3e6 : 5.3e6);
+  };
+  int64_t depth = k;
+  const bool b_fits = b_ok && ldb % 4 == 0;
+  if (trans_a && batch == 1 && b_fits && (trans_b ? k : n) % 4 == 0) {
+    copy(m * k, false);  // (zero columns; it stays transposed)
+  } else {
+    depth = k % 4 == 0 ? k : (k + 63) / 64 * 64;
+    if (trans_a) copy(m * k, true);
+    if (depth != k || (!trans_a && (lda % 4 != 0 || !a_ok))) copy(m * k, false);
+    if (!trans_b && b_fits && n % 4 == 0) {
+      if (depth != k) copy(n * k, false);
+    } else if (!(trans_b && b_fits && depth == k)) {
+      copy(n * k, !trans_b);
+    }
+  }
+  if (!f32_wide_wins(batch, m, n, depth, f32_plan(batch, m, n, depth, true))) return HUGE_VAL;
+  return cost + f32_wide_cost(batch, m, n, depth);
 }
 // What the kernel whose waves share K asks of its operands: at least four elements along each
 // contiguous direction, and lane offsets that fit 32 bits in its largest tile (64 x 128; 32 rows of k for an
@@ -332,6 +410,8 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
     if (g.residual != nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue) &&
         !any_with_residual_pays(g, batch, plan.cost))
       return {TMB_ERR_UNSUPPORTED, 0, 0};
+    if (simt_instead_of_any(g, batch, plan))
+      return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
     return {TMB_GEMM_ANY, plan.tile, plan.splits};
   }
   if (aligned) return {TMB_GEMM_RING, 0, 0};
@@ -342,14 +422,27 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
 static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
                                   size_t workspace_bytes) {
   const bool shared = f32_shared_eligible(g, trans_a, trans_b);
-  const bool wide = g.residual == nullptr && f32_mfma_eligible(g, batch, trans_a, trans_b);
+  const bool aligned = f32_mfma_eligible(g, batch, trans_a, trans_b);
+  const bool wide = g.residual == nullptr && aligned;
   if (!shared && !wide) return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
   if (wide && f32_wide_pays(batch, g.m, g.n, g.k)) return {TMB_GEMM_F32_WIDE, 0, 0};
   F32Plan plan = f32_plan(batch, g.m, g.n, g.k, true);
   if (plan.splits > 0 && (g.m * g.n >= (int64_t{1} << 31) ||
                           workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
     plan = f32_plan(batch, g.m, g.n, g.k, false);
-  if (shared) return {TMB_GEMM_F32, plan.tile, plan.splits};
+  if (shared) {
+    if (plan.splits == 0) {
+      // (neither of the two others carries a residual: the caller adds it then, which has to pay for itself)
+      const double apart = g.residual != nullptr ? add_apart_cost(g, batch, true) : 0.0;
+      const double cost =
+          g.residual != nullptr ? 0.95 * (plan.cost + kF32ResidualPerElement * g.m * g.n * batch) : plan.cost;
+      if (aligned && f32_wide_wins(batch, g.m, g.n, g.k, plan) && f32_wide_cost(batch, g.m, g.n, g.k) + apart < cost)
+        return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_F32_WIDE, 0, 0};
+      if (g.k <= 64 && simt_cost(true, batch, g.m, g.n, g.k) + apart < cost)
+        return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
+    }
+    return {TMB_GEMM_F32, plan.tile, plan.splits};
+  }
   // rows too long for 32-bit offsets: the wide kernel, a split as a batch of equal runs of whole 16-byte pieces
   int splits = plan.splits;
   while (splits > 0 && (splits == 1 || g.k % (4 * splits) != 0)) --splits;

@@ -190,15 +190,6 @@ def _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, plain_epilogue=True) -> boo
     return k % 8 == 0
 
 
-def _f32_in_place(a, la, lb, m, n, k) -> bool:
-    """Whether the fp32 kernel reads these operands where they lie, whatever their alignment (mirrors
-    the library's check): four elements along each contiguous direction, and a tile's rows within
-    reach of 32-bit offsets."""
-    return a.element_size() == 4 and (m if la[0] else k) >= 4 and (k if lb[0] else n) >= 4 \
-        and la[1] < ((1 << 30) - 256) // max((32 if la[0] else min(m, 64)) - 1, 1) \
-        and lb[1] < ((1 << 30) - 256) // max((min(n, 128) if lb[0] else 32) - 1, 1)
-
-
 def _relayout_for_mfma(a, b, la, lb, m, n, k, batched, plain=True):
     """Re-lays the operands of a large product so that the matrix-core kernels take it. A
     contraction length or pitch that is not whole 16-byte vectors (a 50257-wide vocabulary as K)
@@ -258,6 +249,21 @@ def _in_place_workspace(a, b, la, lb, batch, m, n, k, batched, plain) -> Optiona
         ws = _IN_PLACE_WS[key] = _ek.lib().tmb_gemm_in_place_workspace_bytes(
             batch, m, n, k, la[1], lb[1], key[8], key[9], la[0], lb[0], plain, _CODES[a.dtype])
     return None if ws < 0 else ws
+
+
+def _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched, residual) -> bool:
+    """Whether padded copies and the aligned kernel are faster than (or all that multiplies quickly) fp32
+    operands that are not whole aligned vectors."""
+    one = not (batched and batch > 1)
+    key = (batch, m, n, k, la, lb, residual, a.data_ptr() % 16 == 0 and (one or a.stride(0) % 4 == 0),
+           b.data_ptr() % 16 == 0 and (one or b.stride(0) % 4 == 0))
+    pays = _IN_PLACE_WS.get(key)
+    if pays is None:   # a pure function of shape, layout and alignment, as the above
+        if len(_IN_PLACE_WS) >= 4096:
+            _IN_PLACE_WS.clear()
+        pays = _IN_PLACE_WS[key] = _ek.lib().tmb_gemm_f32_padding_pays(
+            batch, m, n, k, la[1], lb[1], key[7], key[8], la[0], lb[0], residual)
+    return bool(pays)
 
 
 _I64X3 = ctypes.c_int64 * 3
@@ -354,10 +360,13 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
     fits = _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE)
     in_place_ws = None if fits else _in_place_workspace(a, b, la, lb, batch, m, n, k, batched,
                                                         epilogue == _ek.EPI_NONE and residual is None)
-    if not fits and in_place_ws is None and batch * m * n * k >= _RELAYOUT_MIN_WORK \
-            and not _f32_in_place(a, la, lb, m, n, k):
-        a, b, la, lb, k, m = _relayout_for_mfma(a, b, la, lb, m, n, k, batched,
-                                                epilogue == _ek.EPI_NONE and residual is None)
+    apart = False
+    if not fits and in_place_ws is None and batch * m * n * k >= _RELAYOUT_MIN_WORK and (
+            a.element_size() == 2 or _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched, residual is not None)):
+        apart = residual is not None and a.element_size() == 4   # (the kernel for the copies adds none)
+        if not apart:
+            a, b, la, lb, k, m = _relayout_for_mfma(a, b, la, lb, m, n, k, batched,
+                                                    epilogue == _ek.EPI_NONE and residual is None)
     out_shape = (batch, m, n) if batched else (m, n)
     if residual is not None and (residual.dtype not in (a.dtype, torch.float32)
                                  or tuple(residual.shape) != out_shape):
@@ -386,8 +395,9 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
             return (prod.float() + residual.float()).to(result_dtype)
         return prod + residual
 
-    if residual is not None and epilogue != _ek.EPI_NONE and not round_like_unfused:
-        return unfused_residual()   # no kernel has a GELU in front of a float32 add
+    if residual is not None and (apart or (epilogue != _ek.EPI_NONE and not round_like_unfused)):
+        # no kernel has a GELU in front of a float32 add, nor a residual on padded copies of fp32 operands
+        return unfused_residual()
     if residual is not None:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
         res = residual if residual.stride(-1) == 1 and residual.stride(-2) >= n else residual.contiguous()
