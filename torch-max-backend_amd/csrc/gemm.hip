@@ -140,6 +140,8 @@ extern "C" int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, i
   if (!tmb::any_eligible(m, n, k, lda, ldb, trans_a, trans_b)) return -1;
   const tmb::AnyPlan plan = tmb::any_plan(batch, m, n, k, true);
   double cost = plan.cost;
+  if (plan.splits == 0 && k > 2048)  // (runs of K this long no longer stay in L2: 597 x 5159 x 7235 166 us, not 131)
+    cost *= 1.0 + 0.1 * static_cast<double>(k - 2048) / 2048.0;
   tmb::GemmArgs g{};
   g.m = m, g.n = n, g.k = k;
   if (tmb::simt_instead_of_any(g, batch, plan)) cost = tmb::simt_cost(false, batch, m, n, k);

@@ -186,9 +186,18 @@ static inline double ring_cost(int64_t batch, int64_t m, int64_t n, int64_t k) {
 // Microseconds of the other way for the same operands: copy what the ring kernels cannot read into padded
 // buffers (3 us and the bytes at 4 TB/s each; a transposing copy at 1 TB/s), then multiply there. Within 15 % of the measured sum for products from
 // 10 GFLOP on (4099^3 198 against 197, 4383 x 1568 x 1228 38 against 38, 1829 x 3429 x 4716 147 against 156).
+struct SplitKPlan {
+  int splits;  // 0: not used
+  int tile;    // 128 or 256
+  double cost;
+};
+static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_t k);
 static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool a_ok,
                                  bool b_ok, int trans_a, int trans_b, bool plain) {
   double cost = ring_cost(batch, m, n, k);
+  const int64_t depth = k % 8 == 0 ? k : (k + 63) / 64 * 64;
+  const SplitKPlan split = splitk_plan(batch, m, n, depth);
+  if (split.splits > 0 && (trans_a || !small_applies(batch, m, n, depth))) cost = std::fmin(cost, split.cost + 6.0);  // (2336 x 512 x 8672 57 us so, 81 where it lies)
   auto copy = [&](int64_t elements, bool transposing) {
     return 3.0 + static_cast<double>(elements) * batch * 4.0 / (transposing ? 1e6 : 4e6);
   };
@@ -226,12 +235,8 @@ static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, doub
 // kernel sustains about 1240 TFLOP/s over 256 one-per-CU workgroups, the 128 x 128 x 32 kernel
 // about 900 TFLOP/s over 512 two-per-CU workgroups; the launch takes ceil(units / slots) rounds of
 // one unit's time, the reduction reads splits * M * N * 4 bytes at about 4 TB/s.
-struct SplitKPlan {
-  int splits;  // 0: not used
-  int tile;    // 128 or 256
-};
 static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  SplitKPlan p{0, 0};
+  SplitKPlan p{0, 0, 0.0};
   if (batch != 1 || k < 2048 || k % 32 != 0 || n <= 64 || m < 1) return p;
   const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128);
   if (t128 >= 256) return p;  // at least one tile per CU: no split
