@@ -231,12 +231,12 @@ def test_fp32_products_with_long_rows_stay_on_the_matrix_cores():
 
 
 def test_long_runs_of_k_are_padded_for_the_aligned_kernels():
-    """(m, n, k, transposed A, transposed B) off a 16-byte boundary whose padded copies measured 1.3 .. 1.6 times as fast as
+    """(m, n, k, transposed A, transposed B), A (the first two: and B) off a 16-byte boundary, whose padded copies measured 1.3 .. 1.6 times as fast as
     the operands where they lie, some of them on a split launch; and a shape that stays."""
     ek = _ek()
     for m, n, k, ta, tb in ((597, 5159, 7235, 0, 1), (2336, 512, 8672, 0, 1), (192, 7168, 4704, 1, 0)):
         ask = ek.lib().tmb_gemm_in_place_workspace_bytes
-        assert ask(1, m, n, k, m if ta else k, k if tb else n, 0, 0, ta, tb, 1, ek.BF16) == -1, (m, n, k)
+        assert ask(1, m, n, k, m if ta else k, k if tb else n, 0, ta, ta, tb, 1, ek.BF16) == -1, (m, n, k)
         assert ask(1, 1999, 1001, 1500, 1999 if ta else 1500, 1500 if tb else 1001, 0, 0, ta, tb, 1, ek.BF16) == 0
 
 
