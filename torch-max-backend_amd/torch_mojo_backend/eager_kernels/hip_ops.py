@@ -272,19 +272,20 @@ _GEMM_WS_BYTES: dict = {}
 _GEMM_PLANS: dict = {}
 
 
-def _gemm_plan_key(a, b, bias, epi_flags) -> tuple:
-    return (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device,
-            a.data_ptr() % 16 == 0, b.data_ptr() % 16 == 0, epi_flags,
-            None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+def _gemm_plan_key(a, b, bias, epi_flags, a_ptr, b_ptr) -> tuple:
+    # (the plan belongs to this alignment of the bases: other kernels and other scratch off a 16-byte boundary)
+    return (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device, a_ptr & 15, b_ptr & 15,
+            epi_flags, None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
 
 
 def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
                     epi_flags: int = _ek.EPI_NONE) -> Optional[torch.Tensor]:
-    """``gemm(a, b, bias)`` when exactly this operand layout (shapes, strides, dtypes, devices, bases
-    on a 16-byte boundary or not, epilogue) has been validated and launched before, else None: the plan holds the launch arguments, so a
-    repeated call (every layer of every decode step) costs one dictionary lookup, one allocation
-    and the launch."""
-    plan = _GEMM_PLANS.get(_gemm_plan_key(a, b, bias, epi_flags))
+    """``gemm(a, b, bias)`` when exactly this operand layout (shapes, strides, dtypes, devices, alignment of
+    the bases, epilogue) has been validated and launched before, else None: the plan holds the launch
+    arguments, so a repeated call (every layer of every decode step) costs one dictionary lookup, one
+    allocation and the launch."""
+    a_ptr, b_ptr = a.data_ptr(), b.data_ptr()
+    plan = _GEMM_PLANS.get(_gemm_plan_key(a, b, bias, epi_flags, a_ptr, b_ptr))
     if plan is None:
         return None
     out_shape, dims, ws_bytes = plan
@@ -292,10 +293,10 @@ def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tenso
     bias_ptr = None if bias is None else bias.data_ptr()
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
-        rc = _ek.lib().tmb_gemm_ws(out.data_ptr(), a.data_ptr(), b.data_ptr(), bias_ptr,
+        rc = _ek.lib().tmb_gemm_ws(out.data_ptr(), a_ptr, b_ptr, bias_ptr,
                                    *dims, epi_flags, ws.data_ptr(), ws_bytes, _stream())
     else:
-        rc = _ek.lib().tmb_gemm(out.data_ptr(), a.data_ptr(), b.data_ptr(), bias_ptr,
+        rc = _ek.lib().tmb_gemm(out.data_ptr(), a_ptr, b_ptr, bias_ptr,
                                 *dims, epi_flags, _stream())
     if rc:
         _check("tmb_gemm", rc)
@@ -418,7 +419,7 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         # operands are consumed in place: remember the launch arguments for this layout
         if len(_GEMM_PLANS) >= 4096:
             _GEMM_PLANS.clear()
-        _GEMM_PLANS[_gemm_plan_key(a, b, bias, epi_flags)] = (
+        _GEMM_PLANS[_gemm_plan_key(a, b, bias, epi_flags, a.data_ptr(), b.data_ptr())] = (
             tuple(out.shape), (batch, m, n, k, la[1], lb[1], n, a.stride(0) if batched else 0,
                                b.stride(0) if batched else 0, m * n, la[0], lb[0], code_of(a.dtype)), ws_bytes)
     if ws_bytes:
@@ -681,10 +682,11 @@ def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     b, h, t, d = q.shape
     if like_query:
         out = _gradient_like(q)
+        os = out.stride()
     elif token_major:
-        out = torch.empty((b, t, h, d), dtype=q.dtype, device=q.device).transpose(1, 2)
+        out, os = torch.empty((b, t, h, d), dtype=q.dtype, device=q.device).transpose(1, 2), (h * t * d, d, h * d)
     else:
-        out = torch.empty((b, h, t, d), dtype=q.dtype, device=q.device)
+        out, os = torch.empty((b, h, t, d), dtype=q.dtype, device=q.device), (h * t * d, t * d, d)
     i64x3 = _I64X3
     mask_ptr, mask_strides = None, None
     if attn_mask is not None:
@@ -694,7 +696,7 @@ def attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     rc = _ek.lib().tmb_attention_decode(
         out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), mask_ptr, b, h, t, k.shape[2], d,
         i64x3(qs[0], qs[1], qs[2]), i64x3(ks[0], ks[1], ks[2]), i64x3(vs[0], vs[1], vs[2]),
-        i64x3(*out.stride()[:3]), mask_strides, float(scale), int(bool(causal)),
+        i64x3(os[0], os[1], os[2]), mask_strides, float(scale), int(bool(causal)),
         _CODES[q.dtype], _stream())
     _check("tmb_attention_decode", rc)
     return out
