@@ -161,7 +161,7 @@ extern "C" int tmb_gemm_f32_padding_pays(int64_t batch, int64_t m, int64_t n, in
   const F32Plan plan = f32_plan(batch, m, n, k, true);
   const double apart = with_residual ? add_apart_cost(g, batch, true) : 0.0;
   double here = plan.cost + (with_residual ? kF32ResidualPerElement * m * n * batch : 0.0);
-  if (k <= 64 && plan.splits == 0) here = std::fmin(here, simt_cost(true, batch, m, n, k) + apart);
+  if (k <= 48 && plan.splits == 0) here = std::fmin(here, simt_cost(true, batch, m, n, k) + apart);
   return f32_padded_cost(batch, m, n, k, lda, ldb, a_aligned != 0, b_aligned != 0, trans_a, trans_b) + apart < here;
 }
 

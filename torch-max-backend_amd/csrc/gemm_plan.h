@@ -443,7 +443,7 @@ static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a,
           g.residual != nullptr ? 0.95 * (plan.cost + kF32ResidualPerElement * g.m * g.n * batch) : plan.cost;
       if (aligned && f32_wide_wins(batch, g.m, g.n, g.k, plan) && f32_wide_cost(batch, g.m, g.n, g.k) + apart < cost)
         return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_F32_WIDE, 0, 0};
-      if (g.k <= 64 && simt_cost(true, batch, g.m, g.n, g.k) + apart < cost)
+      if (g.k <= 48 && simt_cost(true, batch, g.m, g.n, g.k) + apart < cost)
         return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
     }
     return {TMB_GEMM_F32, plan.tile, plan.splits};
