@@ -272,12 +272,6 @@ _GEMM_WS_BYTES: dict = {}
 _GEMM_PLANS: dict = {}
 
 
-def _gemm_plan_key(a, b, bias, epi_flags, a_ptr, b_ptr) -> tuple:
-    # (the plan belongs to this alignment of the bases: other kernels and other scratch off a 16-byte boundary)
-    return (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device, a_ptr & 15, b_ptr & 15,
-            epi_flags, None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
-
-
 def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
                     epi_flags: int = _ek.EPI_NONE) -> Optional[torch.Tensor]:
     """``gemm(a, b, bias)`` when exactly this operand layout (shapes, strides, dtypes, devices, alignment of
@@ -285,7 +279,10 @@ def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tenso
     arguments, so a repeated call (every layer of every decode step) costs one dictionary lookup, one
     allocation and the launch."""
     a_ptr, b_ptr = a.data_ptr(), b.data_ptr()
-    plan = _GEMM_PLANS.get(_gemm_plan_key(a, b, bias, epi_flags, a_ptr, b_ptr))
+    # (`gemm` stores its plans under the same key; off a 16-byte boundary the kernels and the scratch are others)
+    plan = _GEMM_PLANS.get(
+        (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device, a_ptr & 15, b_ptr & 15,
+         epi_flags, None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device)))
     if plan is None:
         return None
     out_shape, dims, ws_bytes = plan
@@ -419,7 +416,10 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         # operands are consumed in place: remember the launch arguments for this layout
         if len(_GEMM_PLANS) >= 4096:
             _GEMM_PLANS.clear()
-        _GEMM_PLANS[_gemm_plan_key(a, b, bias, epi_flags, a.data_ptr(), b.data_ptr())] = (
+        plan_key = (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device,
+                    a.data_ptr() & 15, b.data_ptr() & 15, epi_flags,
+                    None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+        _GEMM_PLANS[plan_key] = (
             tuple(out.shape), (batch, m, n, k, la[1], lb[1], n, a.stride(0) if batched else 0,
                                b.stride(0) if batched else 0, m * n, la[0], lb[0], code_of(a.dtype)), ws_bytes)
     if ws_bytes:
