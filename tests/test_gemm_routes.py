@@ -32,6 +32,8 @@ def test_routes_of_known_products():
     assert route(128, 768, 768)[0] == SMALL
     assert route(8192, 3072, 16384, ta=1)[0] == TRANSPOSED_A
     assert route(768, 3072, 16384, ta=1, workspace=PLENTY)[0] == SPLITK
+    assert route(768, 768, 32768, ta=1, workspace=PLENTY) == (SPLITK, 0, 14)       # 128 x 128 tiles
+    assert route(3072, 768, 8192, ta=1, workspace=PLENTY) == (SPLITK, 1, 7)        # 256 x 256
     assert route(100, 77, 50, a_aligned=0)[0] == ANY
     assert route(8192, 4096, 64)[0] == STREAM64
     assert route(4, 4, 4, b_aligned=0)[0] == SIMT            # fewer than eight contiguous elements

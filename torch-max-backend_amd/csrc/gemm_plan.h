@@ -382,7 +382,7 @@ static inline bool f32_shared_eligible(const GemmArgs& g, int trans_a, int trans
          reached(trans_b ? (g.n < 128 ? g.n : 128) : kF32KS, g.ldb);
 }
 
-// Which kernel takes a product, with its tile (an index into the kernel's own list; 128 or 256 for SplitK) and
+// Which kernel takes a product, with its tile (an index into the kernel's own list) and
 // its number of splits (0: not split). The launch follows it (gemm_typed.h), and tmb_gemm_route answers it.
 struct GemmRoute {
   int kernel;  // TMB_GEMM_*, or TMB_ERR_UNSUPPORTED
@@ -402,7 +402,7 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
                                      : aligned && whole_columns;
     if (plan.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
         workspace_bytes >= static_cast<size_t>(plan.splits) * g.m * g.n * 4)
-      return {TMB_GEMM_SPLITK, plan.tile, plan.splits};
+      return {TMB_GEMM_SPLITK, plan.tile == 256 ? 1 : 0, plan.splits};
   }
   if (g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue))
     return {TMB_GEMM_TRANSPOSED_A, 0, 0};

@@ -270,7 +270,7 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
     switch (r.kernel) {
       case TMB_GEMM_SMALL: return gemm_small(g, batch, r.tile, trans_b, BF16, EPI, stream);
       case TMB_GEMM_SPLITK:
-        return launch_splitk<T, EPI>(g, SplitKPlan{r.splits, r.tile, 0.0}, trans_a, trans_b,
+        return launch_splitk<T, EPI>(g, SplitKPlan{r.splits, r.tile == 1 ? 256 : 128, 0.0}, trans_a, trans_b,
                                      static_cast<float*>(workspace), stream);
       case TMB_GEMM_TRANSPOSED_A: return mfma_transposed_a<T>(g, batch, stream);
       case TMB_GEMM_ANY:
