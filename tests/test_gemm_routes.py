@@ -45,6 +45,34 @@ def test_routes_of_known_products():
     assert route(4, 4, 0) == route(4, 0, 4) == route(4, 8, 8, lda=4) == ek.ERR_INVALID_ARGUMENT
 
 
+def test_the_shapes_of_the_gpu_tests_take_every_tile():
+    """One per tile of each kernel, in each layout: a refit of the models' constants must not drop one."""
+    import test_hip_gemm
+    import test_hip_gemm_any
+    import test_hip_gemm_f32_edges
+    import test_hip_gemm_small
+    from torch_mojo_backend.eager_kernels import hip_ops
+    ek = _ek()
+    off = dict(a_aligned=0, b_aligned=0, workspace=PLENTY)
+    for ta, tb in itertools.product((0, 1), repeat=2):
+        took = [route(*mnk, ta=ta, tb=tb, **off) for mnk in test_hip_gemm_any.SHAPES]
+        assert {t for kernel, t, _ in took if kernel == ANY} == set(range(5)) and max(t[2] for t in took) > 1
+        took = [route(*mnk, ta=ta, tb=tb, dtype=ek.F32, **off) for mnk in test_hip_gemm_f32_edges.SHAPES]
+        assert {t for kernel, t, _ in took if kernel == F32} == set(range(4)) and max(t[2] for t in took) > 1
+        assert ta or {route(*mnk, tb=tb) for mnk in test_hip_gemm_small.SHAPES} == {(SMALL, t, 0) for t in range(6)}
+    took = {(ta, tb, *route(m, n, k, int(ta), int(tb), workspace=PLENTY)[:2]) for m, n, k, ta, tb in test_hip_gemm.SPLITK}
+    assert took == {(ta, tb, SPLITK, t) for ta, tb in ((False, False), (False, True), (True, False)) for t in (0, 1)}
+    # which products of awkward layouts are copied first
+    for dtype, a, ta, b, tb, padded in test_hip_gemm.AWKWARD:
+        m, k = (a[-1], a[-2]) if ta else a[-2:]
+        n, batch = (b[-2] if tb else b[-1]), (a[0] if len(a) == 3 else 1)
+        form = (batch, m, n, k, m if ta else k, k if tb else n, 1, 1, int(ta), int(tb))
+        if dtype.itemsize == 4:
+            assert ek.lib().tmb_gemm_f32_padding_pays(*form, 0) == padded, form
+        else:
+            assert (ek.lib().tmb_gemm_in_place_workspace_bytes(*form, 1, hip_ops.code_of(dtype)) < 0) == padded, form
+
+
 @pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])
 def test_the_scratch_a_caller_is_told_of_is_what_the_launch_splits_with(dtype_name):
     ek = _ek()

@@ -528,17 +528,27 @@ def test_mm_transposed_a_batched_and_strided():
 
 
 # ---- split-K (few output tiles, long K) ----------------------------------------------------------
-SPLITK = [  # (m, n, k, trans_a, trans_b)
+# (m, n, k, trans_a, trans_b): row-major A with both layouts of B and transposed A, on both tiles of the split launch
+# (test_gemm_routes.py checks that), ragged rows and columns, the fewest and the most splits; the rest are products whose
+# K the waves of one small tile share (the comparison with the unsplit kernel is one of a kernel with itself there)
+SPLITK = [
+    (2000, 768, 3072, False, False), (2000, 768, 3072, False, True), (512, 2048, 8192, False, True),
+    (768, 3072, 4096, False, False), (3072, 768, 4096, False, True), (1800, 768, 8192, False, False),
+    (264, 136, 4160, False, False), (100, 72, 8192, False, True), (3072, 768, 8192, True, False),
+    (768, 768, 32768, True, False), (264, 136, 2048, True, False),
+]
+SHARED_BY_WAVES = [
     (1024, 768, 3072, False, False), (1024, 768, 3072, False, True), (128, 768, 4096, False, True),
-    (3072, 768, 8192, True, False), (768, 768, 32768, True, False), (264, 136, 2048, False, False),
-    (100, 72, 2304, False, True),
+    (264, 136, 2048, False, False), (100, 72, 2304, False, True),
 ]
 
 
 @pytest.mark.parametrize("dtype", HALF)
-@pytest.mark.parametrize("case", SPLITK)
+@pytest.mark.parametrize("case", SPLITK + SHARED_BY_WAVES)
 def test_split_k_matches_float64_and_the_unsplit_kernel(case, dtype):
     m, n, k, ta, tb = case
+    told = _ek().lib().tmb_gemm_layout_workspace_bytes(1, m, n, k, int(ta), int(tb), _ops().code_of(dtype))
+    assert (told > 0) == (case in SPLITK)
     a = seeded((k, m) if ta else (m, k), seed=21, dtype=dtype) * 0.25
     b = seeded((n, k) if tb else (k, n), seed=22, dtype=dtype) * 0.25
     bias = None if ta else seeded((n,), seed=23, dtype=dtype)
@@ -574,8 +584,9 @@ def test_split_k_is_reproducible_and_needs_scratch_only_when_it_pays():
     f32 = _ops().code_of(torch.float32)
     assert lib.tmb_gemm_workspace_bytes(1, 4096, 4096, 4096, f32) == 0       # fp32: plenty of tiles
     assert lib.tmb_gemm_workspace_bytes(1, 1024, 768, 4096, f32) == 0        # fp32: its smaller tiles fill the chip
-    a = _dev(seeded((512, 4096), seed=31, dtype=torch.bfloat16))
-    b = _dev(seeded((4096, 384), seed=32, dtype=torch.bfloat16))
+    assert lib.tmb_gemm_layout_workspace_bytes(1, 512, 384, 8192, 0, 0, code) == 16 * 512 * 384 * 4
+    a = _dev(seeded((512, 8192), seed=31, dtype=torch.bfloat16))
+    b = _dev(seeded((8192, 384), seed=32, dtype=torch.bfloat16))
     first = _ops().gemm(a, b)
     for _ in range(3):
         assert torch.equal(first, _ops().gemm(a, b))
@@ -633,6 +644,7 @@ def test_fp32_split_k_is_reproducible_and_close_to_the_unsplit_kernel():
     m, n, k = 128, 768, 3072
     lib, ek = _ek().lib(), _ek()
     assert lib.tmb_gemm_workspace_bytes(1, m, n, k, ek.F32) == 8 * m * n * 4
+    assert lib.tmb_gemm_layout_workspace_bytes(1, m, n, k, 0, 1, ek.F32) == 8 * m * n * 4
     a = _dev(seeded((m, k), seed=51, dtype=torch.float32))
     w = _dev(seeded((n, k), seed=52, dtype=torch.float32))
     bias = _dev(seeded((n,), seed=53, dtype=torch.float32))
@@ -722,27 +734,45 @@ def test_k64_stream_kernel_bias_broadcast_and_neighbouring_shapes():
 
 
 # ---- operands the matrix-core kernels cannot read as they lie ------------------------------------
-@pytest.mark.parametrize("case", [
-    # (dtype, a shape, a transposed?, b shape, b transposed?)
-    (torch.bfloat16, (700, 1001), False, (1001, 384), False),   # odd K: padded
-    (torch.bfloat16, (1024, 1001), True, (1024, 256), False),   # weight-gradient form, odd M
-    (torch.float16, (700, 1001), False, (384, 1001), True),     # odd K, K-major B
-    (torch.bfloat16, (6, 512, 640), True, (6, 512, 64), False),  # transposed A, 64 columns
-    (torch.float32, (600, 1001), False, (1001, 200), False),    # fp32, K not a multiple of 4
-    (torch.float32, (1024, 1001), True, (1024, 128), False),    # fp32 weight-gradient form, odd M
-])
-def test_large_products_with_awkward_layouts_match_float64(case):
-    """Above the re-layout threshold these run on the matrix-core kernels after one padded or
-    transposed copy; the result is that of the product as given."""
+AWKWARD = [
+    # (dtype, a shape, a transposed?, b shape, b transposed?, padded or transposed copies first?)
+    (torch.bfloat16, (700, 1001), False, (1001, 384), False, False),    # odd K
+    (torch.bfloat16, (1024, 1001), True, (1024, 256), False, False),    # weight-gradient form, odd M
+    (torch.float16, (700, 1001), False, (384, 1001), True, False),      # odd K, K-major B
+    (torch.bfloat16, (6, 512, 640), True, (6, 512, 64), False, False),  # transposed A, 64 columns
+    (torch.float32, (600, 1001), False, (1001, 200), False, False),     # fp32, K not a multiple of 4
+    (torch.float32, (1024, 1001), True, (1024, 128), False, False),     # fp32 weight-gradient form, odd M
+    (torch.bfloat16, (2048, 2049), False, (2049, 2304), False, True),   # odd K: A padded, zero rows below B
+    (torch.bfloat16, (4096, 2049), True, (4096, 2048), False, True),    # odd M: keeps its form, zero columns
+    (torch.float16, (2048, 3073), False, (2304, 3073), True, True),     # odd K, K-major B: both padded
+    (torch.bfloat16, (6, 1024, 2048), True, (6, 2048, 1024), True, True),   # both transposed: A copied row-major
+    (torch.float32, (3072, 97), False, (97, 4096), False, True),        # fp32, short odd K
+    (torch.float32, (97, 3001), True, (97, 3500), False, True),         # fp32, odd M: keeps its form
+    (torch.float32, (4, 96, 2001), True, (4, 96, 2000), False, True),   # fp32, a batch of transposed A
+]
+
+
+def _awkward_operands(case, device):
+    dtype, ashape, ta, bshape, tb, _ = case
+    a = seeded(ashape, seed=41, dtype=dtype).to(device)
+    b = seeded(bshape, seed=42, dtype=dtype).to(device)
+    return a.transpose(-1, -2) if ta else a, b.transpose(-1, -2) if tb else b
+
+
+@pytest.mark.parametrize("case", AWKWARD)
+def test_large_products_with_awkward_layouts_match_float64(case, monkeypatch):
+    """Above the re-layout threshold these run on the matrix-core kernels, some where they lie and some after padded or
+    transposed copies; the result is that of the product as given."""
     from torch_mojo_backend.eager_kernels import hip_ops
-    dtype, ashape, ta, bshape, tb = case
-    a = seeded(ashape, seed=41, dtype=dtype).cuda()
-    b = seeded(bshape, seed=42, dtype=dtype).cuda()
-    av = a.transpose(-1, -2) if ta else a
-    bv = b.transpose(-1, -2) if tb else b
+    dtype, padded = case[0], case[-1]
+    av, bv = _awkward_operands(case, "cuda")
     m, k, n = av.shape[-2], av.shape[-1], bv.shape[-1]
     assert math.prod(av.shape[:-2]) * m * n * k >= hip_ops._RELAYOUT_MIN_WORK
+    relaid = []
+    real = hip_ops._relayout_for_mfma
+    monkeypatch.setattr(hip_ops, "_relayout_for_mfma", lambda *a: (relaid.append(1), real(*a))[1])
     got = hip_ops.gemm(av, bv)
+    assert bool(relaid) == padded
     want = as64(av) @ as64(bv)
     scale = np.abs(want).max()
     tol = {torch.float32: 2e-6, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype]

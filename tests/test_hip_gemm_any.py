@@ -41,7 +41,7 @@ def _check(got, a, b, extra64, what):
 # (m, n, k): the smallest it takes, one per tile, ragged everywhere, K of one slice, K that leaves waves
 # without one, K long enough to be split
 SHAPES = [(8, 8, 8), (9, 15, 11), (1, 67, 129), (17, 33, 65), (40, 3001, 511), (250, 300, 1000), (231, 361, 343),
-          (333, 999, 77), (1999, 1001, 150), (100, 100, 5001), (13, 93, 3075), (65, 129, 63)]
+          (333, 999, 77), (1999, 1001, 150), (100, 100, 5001), (13, 93, 3075), (65, 129, 63), (1999, 1001, 1500)]
 
 
 @pytest.mark.gpu

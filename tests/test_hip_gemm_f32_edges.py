@@ -32,7 +32,7 @@ def _check(got, a, b, extra, what):
 
 # (m, n, k): one per tile (32 x 32 .. 64 x 128), one, two and three elements past a piece, the smallest
 # extents, and runs of K that are split (the last two)
-SHAPES = [(40, 70, 33), (500, 1000, 130), (1332, 770, 770), (750, 2306, 260), (4, 4, 4), (5, 6, 7), (33, 129, 35),
+SHAPES = [(40, 70, 33), (500, 1000, 130), (777, 1025, 259), (1332, 770, 770), (750, 2306, 260), (4, 4, 4), (5, 6, 7), (33, 129, 35),
           (65, 34, 62), (130, 770, 3001), (31, 67, 12565)]
 
 

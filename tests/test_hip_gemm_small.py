@@ -38,7 +38,7 @@ def _check(got, a, b, extra64, what):
 # part of one, K below the waves' share, ragged rows and columns, the most tiles and the longest K
 SHAPES = [(16, 768, 768), (128, 768, 3072), (128, 1024, 1024), (231, 2304, 768), (200, 2304, 768),
           (1024, 1024, 768), (1, 8, 8), (1, 50264, 72), (16, 4104, 4096), (17, 40, 520), (33, 72, 1000),
-          (65, 136, 64), (255, 264, 4096), (1023, 1000, 264)]
+          (65, 136, 64), (255, 264, 4096), (1023, 1000, 264), (300, 768, 4096)]
 
 
 @pytest.mark.parametrize("dtype", HALF)

@@ -287,8 +287,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // row without any key comes out as NaN, as in ATen.
 //
 // What bounds it is how many loads are in flight: WPR waves share a query row (each takes every WPR-th
-// group of four steps, and their results meet in LDS in wave order), chosen so that a few thousand
-// waves run whatever the batch (one wave per row left 32 x 12 heads on 96 workgroups and 12 heads of a
+// group of four steps, and their results meet in LDS in wave order), 16 up to 512 rows and 4 up to 2048,
+// where the keys suffice (one wave per row left 32 x 12 heads on 96 workgroups and 12 heads of a
 // single sequence on three), and a wave requests four steps of K and V at once.
 //
 // APPEND: the keys are a cache [batch, heads, kv_len - 1, D] plus one new row, and the pass that reads
@@ -458,7 +458,10 @@ __global__ __launch_bounds__(WPR < 4 ? 256 : WPR * 64) void attention_decode_ker
   }
 }
 
-// Waves per row: enough that about four thousand run, and at least one group of steps for each.
+// Waves per row: 16 for up to 512 rows of at least eight groups of steps (half of the waves get one then), 4 for up to
+// 2048 rows of at least two, else one, four rows to a workgroup. So 2049 .. rows run a wave each, 513 .. 2048 rows two to
+// eight thousand waves, and fewer rows 16 each: 384 rows, 6144 waves, over 499 keys 73.9 -> 15.1 us against one wave a
+// row, 12 rows only 192 waves, which is as far as a row is cut.
 template <typename T, int D, bool APPEND>
 static int launch_decode(const AttnDecodeArgs& a, hipStream_t s) {
   constexpr int kGroup = 4 * kWave / (D / 8);  // keys a wave requests at once
