@@ -20,8 +20,9 @@ def _exact(q, k, v, scale, causal=False):
 
 
 # (batch, heads, queries, keys): one wave per row (few keys, many rows), four, sixteen; key counts around
-# a wave's 32 (64 at head size 64) and the waves' shares
-CASES = [(1, 12, 1, 31), (1, 12, 1, 33), (1, 12, 1, 300), (2, 12, 3, 1025), (64, 12, 1, 129), (200, 12, 1, 65),
+# a wave's 32 (16 at head size 128) and the waves' shares; keys of one and two steps (8, 4 keys each)
+CASES = [(1, 12, 1, 1), (3, 5, 1, 4), (200, 12, 1, 5), (200, 12, 2, 8), (100, 12, 3, 9), (1, 12, 4, 16), (200, 12, 1, 17),
+         (1, 12, 1, 31), (1, 12, 1, 33), (1, 12, 1, 300), (2, 12, 3, 1025), (64, 12, 1, 129), (200, 12, 1, 65),
          (1, 2, 16, 257), (43, 12, 4, 40)]
 
 
@@ -41,7 +42,7 @@ def test_decode_rows_shared_by_waves(case, dtype, head_dim, causal):
         assert ((got.double() - want).abs() <= ulp * want.abs() + 1e-4).all()
 
 
-@pytest.mark.parametrize("case", [(1, 12, 1), (3, 12, 32), (32, 12, 499), (180, 12, 70), (2, 3, 2000)])
+@pytest.mark.parametrize("case", [(1, 12, 1), (3, 12, 6), (200, 12, 7), (200, 12, 15), (200, 12, 16), (3, 12, 32), (32, 12, 499), (180, 12, 70), (2, 3, 2000)])
 @pytest.mark.parametrize("dtype,head_dim", [(torch.bfloat16, 64), (torch.float16, 128)])
 def test_append_and_attend_in_one_pass(case, dtype, head_dim):
     from torch_mojo_backend.eager_kernels import hip_ops

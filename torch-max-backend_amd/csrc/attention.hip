@@ -289,7 +289,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // What bounds it is how many loads are in flight: WPR waves share a query row (each takes every WPR-th
 // group of four steps, and their results meet in LDS in wave order), 16 up to 512 rows and 4 up to 2048,
 // where the keys suffice (one wave per row left 32 x 12 heads on 96 workgroups and 12 heads of a
-// single sequence on three), and a wave requests four steps of K and V at once.
+// single sequence on three), and a wave requests U steps of K and V at once: four, or one where the keys are
+// one or two steps (a step past the last key is computed and dropped).
 //
 // APPEND: the keys are a cache [batch, heads, kv_len - 1, D] plus one new row, and the pass that reads
 // them writes the grown caches [batch, heads, kv_len, D] on its way: a generation loop that
@@ -319,11 +320,10 @@ struct AttnDecodeArgs {
   int64_t kn_sb, kn_sh, vn_sb, vn_sh;
 };
 
-template <typename T, int D, int WPR, bool APPEND>
+template <typename T, int D, int WPR, int U, bool APPEND>
 __global__ __launch_bounds__(WPR < 4 ? 256 : WPR * 64) void attention_decode_kernel(AttnDecodeArgs a) {
   constexpr int LPK = D / 8;        // lanes per key
   constexpr int KPI = kWave / LPK;  // keys per step of a wave
-  constexpr int U = 4;              // steps in flight
   constexpr int RPB = WPR < 4 ? 4 / WPR : 1;  // rows per workgroup
   __shared__ float merged[WPR > 1 ? RPB * WPR * (D + 2) : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -461,18 +461,22 @@ __global__ __launch_bounds__(WPR < 4 ? 256 : WPR * 64) void attention_decode_ker
 // Waves per row: 16 for up to 512 rows of at least eight groups of steps (half of the waves get one then), 4 for up to
 // 2048 rows of at least two, else one, four rows to a workgroup. So 2049 .. rows run a wave each, 513 .. 2048 rows two to
 // eight thousand waves, and fewer rows 16 each: 384 rows, 6144 waves, over 499 keys 73.9 -> 15.1 us against one wave a
-// row, 12 rows only 192 waves, which is as far as a row is cut.
+// row, 12 rows only 192 waves, which is as far as a row is cut. One step at a time over keys of one or two: 16416 rows x 5
+// keys 13.1 us, 17.6 with four (57280 x 5 35 and 50; from three steps on the two are level).
 template <typename T, int D, bool APPEND>
 static int launch_decode(const AttnDecodeArgs& a, hipStream_t s) {
   constexpr int kGroup = 4 * kWave / (D / 8);  // keys a wave requests at once
   const int64_t groups = (a.kv_len + kGroup - 1) / kGroup;
   const unsigned rows = static_cast<unsigned>(a.rows);
-  if (a.rows > 2048 || groups < 2) {
-    attention_decode_kernel<T, D, 1, APPEND><<<dim3(static_cast<unsigned>((a.rows + 3) / 4)), dim3(256), 0, s>>>(a);
+  const dim3 four_rows(static_cast<unsigned>((a.rows + 3) / 4));
+  if (a.kv_len <= 2 * kGroup / 4) {
+    attention_decode_kernel<T, D, 1, 1, APPEND><<<four_rows, dim3(256), 0, s>>>(a);
+  } else if (a.rows > 2048 || groups < 2) {
+    attention_decode_kernel<T, D, 1, 4, APPEND><<<four_rows, dim3(256), 0, s>>>(a);
   } else if (a.rows > 512 || groups < 8) {
-    attention_decode_kernel<T, D, 4, APPEND><<<dim3(rows), dim3(256), 0, s>>>(a);
+    attention_decode_kernel<T, D, 4, 4, APPEND><<<dim3(rows), dim3(256), 0, s>>>(a);
   } else {
-    attention_decode_kernel<T, D, 16, APPEND><<<dim3(rows), dim3(1024), 0, s>>>(a);
+    attention_decode_kernel<T, D, 16, 4, APPEND><<<dim3(rows), dim3(1024), 0, s>>>(a);
   }
   return check_launch();
 }
