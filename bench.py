@@ -415,7 +415,7 @@ def main() -> int:
         sweep["attention_decode_bf16_512x12x1x208x64"] = {
             "us": round(ms * 1e3, 2), "GB/s": round(dec_bytes / ms / 1e6, 1),
             "frac_hbm": round(dec_bytes / ms / 1e6 / PEAK_HBM_GBS, 4), "bytes": dec_bytes,
-            "note": "one wave per query row, K and V read once (includes the Python wrapper)"}
+            "note": "K and V read once per query row (includes the Python wrapper)"}
         del caches
         # the softmax of the same attention when it runs on its own: [B*H*T, T] scores in,
         # probabilities out; the masked half of every row is not read
