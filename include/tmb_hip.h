@@ -195,7 +195,7 @@ int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, int64_t n, i
 /* fp32 operands that are not whole aligned 16-byte vectors: 1 where zero-padding them into aligned buffers first
  * is faster than multiplying them where they lie, or where only copies reach the matrix cores, else 0. */
 int tmb_gemm_f32_padding_pays(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, int a_aligned,
-                              int b_aligned, int trans_a, int trans_b, int with_residual);
+                              int b_aligned, int trans_a, int trans_b);
 /* The kernels of tmb_gemm*. */
 typedef enum tmb_gemm_kernel {
   TMB_GEMM_SIMT = 0,         /* any layout, vector instructions */
@@ -230,8 +230,9 @@ int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t
  * stream in fp32 (fp32 residual in, fp32 sum out, nothing rounded in between; not together
  * with TMB_EPI_ROUND_LIKE_UNFUSED). TMB_ERR_UNSUPPORTED, after which the caller launches tmb_gemm and
  * adds separately: k == 0, operands with fewer than eight (fp32: four) elements along a contiguous direction,
- * a GELU epilogue unless TMB_EPI_ROUND_LIKE_UNFUSED, and sizes at which the two launches are faster (a large transposed
- * A, short K over many tiles; tmb_gemm_route answers the same).
+ * a GELU epilogue unless TMB_EPI_ROUND_LIKE_UNFUSED, sizes at which the two launches are faster, and, in fp32
+ * and with TMB_EPI_ROUND_LIKE_UNFUSED, products that run on a kernel without a residual step (a large transposed A,
+ * short K over many tiles, fp32 on 128 x 128 tiles; tmb_gemm_route answers the same).
  * Replaces `AddF32Bf16Spec` / the residual add of aten_fast.py:657-687 together with the GEMM
  * in front of it. */
 int tmb_gemm_residual(void* c, const void* a, const void* b, const void* bias,

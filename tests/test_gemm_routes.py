@@ -68,7 +68,7 @@ def test_the_shapes_of_the_gpu_tests_take_every_tile():
         n, batch = (b[-2] if tb else b[-1]), (a[0] if len(a) == 3 else 1)
         form = (batch, m, n, k, m if ta else k, k if tb else n, 1, 1, int(ta), int(tb))
         if dtype.itemsize == 4:
-            assert ek.lib().tmb_gemm_f32_padding_pays(*form, 0) == padded, form
+            assert ek.lib().tmb_gemm_f32_padding_pays(*form) == padded, form
         else:
             assert (ek.lib().tmb_gemm_in_place_workspace_bytes(*form, 1, hip_ops.code_of(dtype)) < 0) == padded, form
 
@@ -125,12 +125,35 @@ def test_a_large_transposed_a_with_a_residual_is_multiplied_and_added():
         large = dict(ta=1, residual=1, epilogue=residual_step, workspace=PLENTY)
         assert route(4096, 4096, 4096, **large) == ek.ERR_UNSUPPORTED
         assert route(50304, 768, 16384, **large) == ek.ERR_UNSUPPORTED
-        assert route(256, 256, 256, **large)[0] == ANY               # one launch instead of two
         assert route(768, 3072, 16384, **large)[0] == SPLITK         # its reduction adds the residual
         assert route(4097, 4096, 4096, **large)[0] == ANY            # the rings do not take it either way
+    assert route(256, 256, 256, ta=1, residual=1)[0] == ANY          # one launch instead of the product and an add in float32
+    assert route(768, 3072, 1024, ta=1, residual=1)[0] == ANY
     rounded = dict(ta=1, residual=1, epilogue=ek.EPI_ROUND_LIKE_UNFUSED)
-    assert route(768, 3072, 1024, **rounded) == ek.ERR_UNSUPPORTED   # one cheap add
-    assert route(768, 3072, 1024, ta=1, residual=1)[0] == ANY        # an add in float32 is four launches
+    assert route(256, 256, 256, **rounded) == ek.ERR_UNSUPPORTED     # (the bits of the rings' product)
+
+
+@pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])
+def test_a_residual_that_is_added_with_the_bits_of_two_operations_is_carried_where_the_product_runs(dtype_name):
+    """fp32, and 16-bit with TMB_EPI_ROUND_LIKE_UNFUSED: the kernel, tile and splits of the product alone, or none; all
+    layouts, alignments, with and without scratch."""
+    ek = _ek()
+    dtype = getattr(ek, dtype_name)
+    carried = apart = 0
+    for batch, m, n, k in itertools.product((1, 5), (8, 100, 768, 4096), (16, 333, 2048), (8, 64, 100, 768, 4096)):
+        for ta, tb, aa, ba, ws in itertools.product((0, 1), repeat=5):
+            form = dict(ta=ta, tb=tb, a_aligned=aa, b_aligned=ba, workspace=ws * PLENTY, batch=batch, dtype=dtype)
+            plain = route(m, n, k, **form)
+            with_it = route(m, n, k, residual=1, epilogue=ek.EPI_ROUND_LIKE_UNFUSED, **form)
+            if plain[0] == STREAM64:
+                assert with_it[0] == RING      # (adds its four steps of K in the same order)
+            elif with_it == ek.ERR_UNSUPPORTED:
+                assert plain[0] in (SIMT, TRANSPOSED_A, F32_WIDE)
+                apart += 1
+            else:
+                assert with_it == plain, (batch, m, n, k, form)
+                carried += 1
+    assert carried > 500 and apart > 100
 
 
 @pytest.mark.gpu
@@ -148,8 +171,7 @@ def test_transposed_a_with_a_residual_matches_float64(mnk):
     # rounded after the product (2^-9 of it) and after the sum
     exact_step = exact + r.double()
     assert ((step.double() - exact_step).abs() <= 2 * slack + 2.0 ** -8 * (exact.abs() + exact_step.abs())).all()
-    if mnk != (256, 256, 256):
-        assert torch.equal(step, plain + r)      # the same product, added apart
+    assert torch.equal(step, plain + r)
     for out_dtype in (None, torch.float32):
         wide = hip_ops.gemm(x.t(), w, bias, residual=r.float(), out_dtype=out_dtype)
         assert ((wide.double() - exact_step).abs() <= 2 * slack + 2.0 ** -8 * (exact.abs() + exact_step.abs())).all()
@@ -277,7 +299,7 @@ def test_fp32_operands_that_no_matrix_kernel_reads_are_padded():
     for m, n, k, ta, tb, extra in itertools.product((3, 4, 64, 65, 5000, 1 << 24, 1 << 25), (3, 4, 128, 129, 8000, 1 << 23),
                                                     (3, 4, 31, 33, 200, 1 << 23, 1 << 26), (0, 1), (0, 1), (0, 1 << 23)):
         lda, ldb = (m if ta else k) + extra, (k if tb else n) + extra
-        pad = _ek().lib().tmb_gemm_f32_padding_pays(1, m, n, k, lda, ldb, 0, 0, ta, tb, 0)
+        pad = _ek().lib().tmb_gemm_f32_padding_pays(1, m, n, k, lda, ldb, 0, 0, ta, tb)
         lines, lanes = (32 if ta else min(m, 64)), (min(n, 128) if tb else 32)
         reach = (1 << 30) - 256
         read = (m if ta else k) >= 4 and (k if tb else n) >= 4 and lda < reach // max(lines - 1, 1) \
@@ -318,7 +340,61 @@ def test_short_k_over_many_tiles_leaves_the_kernels_whose_waves_share_k(dtype_na
             assert route(m, n, k, tb=1, batch=batch, dtype=dtype) == (F32_WIDE, 0, 0)
         assert route(4104, 608, 8, tb=1, batch=48, **off) == _ek().ERR_UNSUPPORTED
         assert route(112, 6216, 8, tb=1, batch=48, residual=1, dtype=dtype) == _ek().ERR_UNSUPPORTED
-        assert route(4096, 4096, 4096, residual=1, dtype=dtype)[0] == F32
+        assert route(4096, 4096, 4096, residual=1, dtype=dtype) == _ek().ERR_UNSUPPORTED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("ta,tb", itertools.product((False, True), repeat=2))
+def test_short_k_over_many_tiles_matches_float64(dtype_name, ta, tb):
+    """Ragged edges of the 64 x 64 and 128 x 128 tiles, with and without a residual, and (fp32, the last two) padded copies."""
+    import torch
+    from torch_mojo_backend.eager_kernels import EPI_GELU_TANH, hip_ops
+    dtype = getattr(torch, dtype_name)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    for batch, m, n, k in ((48, 402, 354, 8), (48, 1100, 17, 9), (1, 6461, 1251, 9), (1, 3001, 3501, 61), (2, 2001, 2000, 97)):
+        rows, cols = ((batch, k, m) if ta else (batch, m, k)), ((batch, n, k) if tb else (batch, k, n))
+        off = torch.randn(batch * m * k + 1, generator=g, device="cuda").to(dtype)[1:].view(rows)
+        a, b = (off.mT if ta else off), torch.randn(cols, generator=g, device="cuda").to(dtype)
+        b = b.mT if tb else b
+        if batch == 1:
+            a, b = a[0], b[0]
+        bias = torch.randn(n, generator=g, device="cuda").to(dtype)
+        r = torch.randn(*a.shape[:-1], n, generator=g, device="cuda").to(dtype)
+        a64, b64 = a.double().contiguous(), b.double().contiguous()
+        exact = a64 @ b64 + bias.double()
+        slack = (k + 2) * 2.0 ** -24 * (a64.abs() @ b64.abs() + exact.abs() + r.double().abs()) + 1e-6
+        ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23}[dtype]
+        plain = hip_ops.gemm(a, b, bias)
+        assert ((plain.double() - exact).abs() <= slack + ulp * exact.abs()).all(), (batch, m, n, k)
+        once = hip_ops.gemm(a, b, bias, residual=r)
+        want = exact + r.double()
+        # (product and sum may be rounded apart)
+        assert ((once.double() - want).abs() <= slack + ulp * (exact.abs() + want.abs())).all(), (batch, m, n, k)
+        assert torch.equal(hip_ops.gemm(a, b, bias, residual=r, round_like_unfused=True), plain + r)
+        if dtype != torch.float32:
+            assert torch.equal(hip_ops.gemm(a, b, bias, epilogue=EPI_GELU_TANH, round_like_unfused=True),
+                               hip_ops.gelu(plain, "tanh"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float32"])
+@pytest.mark.parametrize("form", itertools.product((False, True), (False, True), (0, 1)))
+def test_a_residual_added_like_two_operations_has_their_bits(dtype_name, form):
+    """Whatever the product runs on: small, split, ring, transposed A, any-layout, padded with and without its form, K = 64."""
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    ta, tb, off = form
+    dtype = getattr(torch, dtype_name)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    for m, n, k in ((256, 256, 256), (128, 768, 768), (2000, 768, 3072), (2049, 2048, 4096), (2048, 2304, 2049), (100, 100, 5001),
+                    (4096, 2048, 64), (1999, 1001, 150), (597, 2001, 7235)):
+        a = torch.randn(m * k + off, generator=g, device="cuda").to(dtype)[off:].view((k, m) if ta else (m, k))
+        b = torch.randn((n, k) if tb else (k, n), generator=g, device="cuda").to(dtype)
+        a, b = (a.t() if ta else a), (b.t() if tb else b)
+        bias, r = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((n,), (m, n)))
+        got = hip_ops.gemm(a, b, bias, residual=r, round_like_unfused=True)
+        assert torch.equal(got, hip_ops.gemm(a, b, bias) + r), (m, n, k)
 
 
 def test_the_launcher_pads_fp32_operands_of_short_k(recorded):

@@ -152,17 +152,16 @@ extern "C" int64_t tmb_gemm_in_place_workspace_bytes(int64_t batch, int64_t m, i
 }
 
 extern "C" int tmb_gemm_f32_padding_pays(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
-                                         int a_aligned, int b_aligned, int trans_a, int trans_b, int with_residual) {
+                                         int a_aligned, int b_aligned, int trans_a, int trans_b) {
   using namespace tmb;
   if (batch < 1 || m < 1 || n < 1 || k < 1) return 0;
   GemmArgs g{};
   g.m = m, g.n = n, g.k = k, g.lda = lda, g.ldb = ldb;
   if (!f32_shared_eligible(g, trans_a, trans_b)) return 1;
   const F32Plan plan = f32_plan(batch, m, n, k, true);
-  const double apart = with_residual ? add_apart_cost(g, batch, true) : 0.0;
-  double here = plan.cost + (with_residual ? kF32ResidualPerElement * m * n * batch : 0.0);
-  if (k <= 48 && plan.splits == 0) here = std::fmin(here, simt_cost(true, batch, m, n, k) + apart);
-  return f32_padded_cost(batch, m, n, k, lda, ldb, a_aligned != 0, b_aligned != 0, trans_a, trans_b) + apart < here;
+  double here = plan.cost;
+  if (k <= 48 && plan.splits == 0) here = std::fmin(here, simt_cost(true, batch, m, n, k));
+  return f32_padded_cost(batch, m, n, k, lda, ldb, a_aligned != 0, b_aligned != 0, trans_a, trans_b) < here;
 }
 
 extern "C" int64_t tmb_gemm_route(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,

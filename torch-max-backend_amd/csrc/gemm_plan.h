@@ -156,18 +156,16 @@ static inline double simt_cost(bool f32, int64_t batch, int64_t m, int64_t n, in
   const double many = f32 ? r * (0.038 * k + 0.24 + 1.33 * filled) : r * (0.036 * k + 0.21 + 0.72 * filled);
   return (f32 ? 5.2 : 5.1) + (alone > many ? alone : many);
 }
-// What a product costs beside itself when its residual is added apart: one pass of three tensors, or four launches in
-// float32 when only the sum of 16-bit operands is rounded; 5.8 TB/s.
-constexpr double kF32ResidualPerElement = 2e-6;  // what it costs in the fp32 kernel whose waves share K: about as much
-static inline double add_apart_cost(const GemmArgs& g, int64_t batch, bool f32) {
+// What a 16-bit product costs beside itself when its residual is added apart: one pass of three tensors, or four launches
+// in float32 when only the sum is rounded; 5.8 TB/s.
+static inline double add_apart_cost(const GemmArgs& g, int64_t batch) {
   const double elements = static_cast<double>(g.m) * g.n * batch;
-  if (f32) return 3.0 + elements * 12.0 / 5.8e6;
   return g.round_like_unfused ? 3.0 + elements * 6.0 / 5.8e6 : 12.0 + elements * 30.0 / 5.8e6;
 }
 static inline bool simt_instead_of_any(const GemmArgs& g, int64_t batch, const AnyPlan& plan) {
   if (plan.splits > 0 || g.k > 32) return false;
   const AnyTile& t = kAnyTiles[plan.tile];
-  const double apart = g.residual != nullptr ? add_apart_cost(g, batch, false) : 0.0;
+  const double apart = g.residual != nullptr ? add_apart_cost(g, batch) : 0.0;
   return simt_cost(false, batch, g.m, g.n, g.k) + apart <
          many_tiles_cost(kAnyMany[plan.tile], t.bm, t.bn, batch, g.m, g.n, g.k);
 }
@@ -221,7 +219,7 @@ int gemm_any(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_
 // 193 apart, 768 x 3072 x 1024 24 against 17 and 31, 2048^3 40 against 27 and 46, 1024^3 14 against 15 and 27, 8192 x
 // 8192 x 1024 420 against 204 and 492. The fifth is the models' own error.
 static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, double any_cost) {
-  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add_apart_cost(g, batch, false);
+  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add_apart_cost(g, batch);
 }
 
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
@@ -392,6 +390,16 @@ struct GemmRoute {
 
 static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_a, int trans_b, int epilogue,
                                     size_t workspace_bytes) {
+  if (g.residual != nullptr && g.round_like_unfused) {
+    // the bits of the product alone, rounded, and an add: the kernel, tile and splits that it runs on by itself, or none
+    GemmArgs alone = g;
+    alone.residual = nullptr;
+    GemmRoute r = route_16bit(alone, batch, trans_a, trans_b, epilogue, workspace_bytes);
+    if (r.kernel == TMB_GEMM_STREAM64 && mfma_eligible(g, batch, trans_a, trans_b)) r.kernel = TMB_GEMM_RING;  // (as it adds)
+    if (r.kernel == TMB_GEMM_TRANSPOSED_A || r.kernel == TMB_GEMM_STREAM64 || r.kernel == TMB_GEMM_SIMT)
+      return {TMB_ERR_UNSUPPORTED, 0, 0};
+    return r;
+  }
   const bool aligned = mfma_eligible(g, batch, trans_a, trans_b);
   const bool whole_columns = trans_b || g.n % 8 == 0;
   if (aligned && whole_columns && small_applies(batch, g.m, g.n, g.k))
@@ -424,27 +432,29 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
   return {TMB_GEMM_SIMT, 0, 0};
 }
 
+// A residual is carried where the product alone runs on the kernel whose waves share K, and added by the caller where it
+// does not: the sum has the bits of the two operations, and carrying it saves next to nothing on the others (2 us a
+// million elements there, as much as the add).
 static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
                                   size_t workspace_bytes) {
+  if (g.residual != nullptr) {
+    GemmArgs alone = g;
+    alone.residual = nullptr;
+    const GemmRoute r = route_f32(alone, batch, trans_a, trans_b, workspace_bytes);
+    return r.kernel == TMB_GEMM_F32 ? r : GemmRoute{TMB_ERR_UNSUPPORTED, 0, 0};
+  }
   const bool shared = f32_shared_eligible(g, trans_a, trans_b);
   const bool aligned = f32_mfma_eligible(g, batch, trans_a, trans_b);
-  const bool wide = g.residual == nullptr && aligned;
-  if (!shared && !wide) return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
-  if (wide && f32_wide_pays(batch, g.m, g.n, g.k)) return {TMB_GEMM_F32_WIDE, 0, 0};
+  if (!shared && !aligned) return {TMB_GEMM_SIMT, 0, 0};
+  if (aligned && f32_wide_pays(batch, g.m, g.n, g.k)) return {TMB_GEMM_F32_WIDE, 0, 0};
   F32Plan plan = f32_plan(batch, g.m, g.n, g.k, true);
   if (plan.splits > 0 && (g.m * g.n >= (int64_t{1} << 31) ||
                           workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
     plan = f32_plan(batch, g.m, g.n, g.k, false);
   if (shared) {
     if (plan.splits == 0) {
-      // (neither of the two others carries a residual: the caller adds it then, which has to pay for itself)
-      const double apart = g.residual != nullptr ? add_apart_cost(g, batch, true) : 0.0;
-      const double cost =
-          g.residual != nullptr ? 0.95 * (plan.cost + kF32ResidualPerElement * g.m * g.n * batch) : plan.cost;
-      if (aligned && f32_wide_wins(batch, g.m, g.n, g.k, plan) && f32_wide_cost(batch, g.m, g.n, g.k) + apart < cost)
-        return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_F32_WIDE, 0, 0};
-      if (g.k <= 48 && simt_cost(true, batch, g.m, g.n, g.k) + apart < cost)
-        return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
+      if (aligned && f32_wide_wins(batch, g.m, g.n, g.k, plan)) return {TMB_GEMM_F32_WIDE, 0, 0};
+      if (g.k <= 48 && simt_cost(true, batch, g.m, g.n, g.k) < plan.cost) return {TMB_GEMM_SIMT, 0, 0};
     }
     return {TMB_GEMM_F32, plan.tile, plan.splits};
   }

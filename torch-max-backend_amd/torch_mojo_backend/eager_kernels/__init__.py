@@ -42,7 +42,7 @@ SIGNATURES = {
     "tmb_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _ci]),
     "tmb_gemm_layout_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _ci, _ci, _ci]),
     "tmb_gemm_in_place_workspace_bytes": (_i64, [_i64] * 6 + [_ci] * 6),
-    "tmb_gemm_f32_padding_pays": (_ci, [_i64] * 6 + [_ci] * 5),
+    "tmb_gemm_f32_padding_pays": (_ci, [_i64] * 6 + [_ci] * 4),
     "tmb_gemm_route": (_i64, [_i64] * 8 + [_ci] * 7 + [_sz]),
     "tmb_gemm_ws": (_ci, [_vp, _vp, _vp, _vp] + [_i64] * 10 + [_ci] * 4 + [_vp, _sz, _vp]),
     "tmb_gemm_residual": (_ci, [_vp, _vp, _vp, _vp, _vp] + [_i64] * 12 + [_ci] * 6 + [_vp]),

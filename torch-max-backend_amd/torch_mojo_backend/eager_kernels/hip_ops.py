@@ -251,18 +251,18 @@ def _in_place_workspace(a, b, la, lb, batch, m, n, k, batched, plain) -> Optiona
     return None if ws < 0 else ws
 
 
-def _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched, residual) -> bool:
+def _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched) -> bool:
     """Whether padded copies and the aligned kernel are faster than (or all that multiplies quickly) fp32
     operands that are not whole aligned vectors."""
     one = not (batched and batch > 1)
-    key = (batch, m, n, k, la, lb, residual, a.data_ptr() % 16 == 0 and (one or a.stride(0) % 4 == 0),
+    key = (batch, m, n, k, la, lb, a.data_ptr() % 16 == 0 and (one or a.stride(0) % 4 == 0),
            b.data_ptr() % 16 == 0 and (one or b.stride(0) % 4 == 0))
     pays = _IN_PLACE_WS.get(key)
     if pays is None:   # a pure function of shape, layout and alignment, as the above
         if len(_IN_PLACE_WS) >= 4096:
             _IN_PLACE_WS.clear()
         pays = _IN_PLACE_WS[key] = _ek.lib().tmb_gemm_f32_padding_pays(
-            batch, m, n, k, la[1], lb[1], key[7], key[8], la[0], lb[0], residual)
+            batch, m, n, k, la[1], lb[1], key[6], key[7], la[0], lb[0])
     return bool(pays)
 
 
@@ -355,13 +355,15 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         b = b.contiguous()
         lb = (0, max(n, 1))
     m_given = m
+    # a sum with the bits of the two operations asks where the product alone would run
+    alone = epilogue == _ek.EPI_NONE and (residual is None or round_like_unfused)
     fits = _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE)
-    in_place_ws = None if fits else _in_place_workspace(a, b, la, lb, batch, m, n, k, batched,
-                                                        epilogue == _ek.EPI_NONE and residual is None)
+    in_place_ws = None if fits else _in_place_workspace(a, b, la, lb, batch, m, n, k, batched, alone)
     apart = False
     if not fits and in_place_ws is None and batch * m * n * k >= _RELAYOUT_MIN_WORK and (
-            a.element_size() == 2 or _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched, residual is not None)):
-        apart = residual is not None and a.element_size() == 4   # (the kernel for the copies adds none)
+            a.element_size() == 2 or _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched)):
+        # (the fp32 kernel for the copies adds no residual, nor does the one for a transposed A that stays so)
+        apart = residual is not None and (a.element_size() == 4 or (bool(la[0]) and alone))
         if not apart:
             a, b, la, lb, k, m = _relayout_for_mfma(a, b, la, lb, m, n, k, batched,
                                                     epilogue == _ek.EPI_NONE and residual is None)
@@ -394,7 +396,7 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         return prod + residual
 
     if residual is not None and (apart or (epilogue != _ek.EPI_NONE and not round_like_unfused)):
-        # no kernel has a GELU in front of a float32 add, nor a residual on padded copies of fp32 operands
+        # no kernel has a GELU in front of a float32 add, and some none for these copies
         return unfused_residual()
     if residual is not None:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
