@@ -380,10 +380,10 @@ def test_short_k_over_many_tiles_matches_float64(dtype_name, ta, tb):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float32"])
 @pytest.mark.parametrize("form", itertools.product((False, True), (False, True), (0, 1)))
-def test_a_residual_added_like_two_operations_has_their_bits(dtype_name, form):
+def test_epilogues_rounded_like_separate_operations_have_their_bits(dtype_name, form):
     """Whatever the product runs on: small, split, ring, transposed A, any-layout, padded with and without its form, K = 64."""
     import torch
-    from torch_mojo_backend.eager_kernels import hip_ops
+    from torch_mojo_backend.eager_kernels import EPI_GELU_ERF, EPI_GELU_TANH, hip_ops
     ta, tb, off = form
     dtype = getattr(torch, dtype_name)
     g = torch.Generator(device="cuda").manual_seed(11)
@@ -393,8 +393,13 @@ def test_a_residual_added_like_two_operations_has_their_bits(dtype_name, form):
         b = torch.randn((n, k) if tb else (k, n), generator=g, device="cuda").to(dtype)
         a, b = (a.t() if ta else a), (b.t() if tb else b)
         bias, r = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((n,), (m, n)))
-        got = hip_ops.gemm(a, b, bias, residual=r, round_like_unfused=True)
-        assert torch.equal(got, hip_ops.gemm(a, b, bias) + r), (m, n, k)
+        plain = hip_ops.gemm(a, b, bias)
+        assert torch.equal(hip_ops.gemm(a, b, bias, residual=r, round_like_unfused=True), plain + r), (m, n, k)
+        for epilogue, kind in ((EPI_GELU_TANH, "tanh"), (EPI_GELU_ERF, "none")):
+            got = hip_ops.gemm(a, b, bias, epilogue=epilogue, round_like_unfused=True)
+            assert torch.equal(got, hip_ops.gelu(plain, kind)), (m, n, k, kind)
+            got = hip_ops.gemm(a, b, bias, epilogue=epilogue, residual=r, round_like_unfused=True)
+            assert torch.equal(got, hip_ops.gelu(plain, kind) + r), (m, n, k, kind)
 
 
 def test_the_launcher_pads_fp32_operands_of_short_k(recorded):

@@ -355,12 +355,15 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         b = b.contiguous()
         lb = (0, max(n, 1))
     m_given = m
+    # a 16-bit transposed A has kernels of its own without an epilogue: the bits of product and GELU take both
+    gelu_apart = round_like_unfused and bool(la[0]) and a.element_size() == 2 and k > 0 and \
+        epilogue in (_ek.EPI_GELU_TANH, _ek.EPI_GELU_ERF)
     # a sum with the bits of the two operations asks where the product alone would run
     alone = epilogue == _ek.EPI_NONE and (residual is None or round_like_unfused)
     fits = _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE)
     in_place_ws = None if fits else _in_place_workspace(a, b, la, lb, batch, m, n, k, batched, alone)
     apart = False
-    if not fits and in_place_ws is None and batch * m * n * k >= _RELAYOUT_MIN_WORK and (
+    if not fits and in_place_ws is None and not gelu_apart and batch * m * n * k >= _RELAYOUT_MIN_WORK and (
             a.element_size() == 2 or _f32_padding_pays(a, b, la, lb, batch, m, n, k, batched)):
         # (the fp32 kernel for the copies adds no residual, nor does the one for a transposed A that stays so)
         apart = residual is not None and (a.element_size() == 4 or (bool(la[0]) and alone))
@@ -376,6 +379,9 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
     if wide and round_like_unfused:
         raise ValueError("gemm: a float32 residual or result keeps the epilogue in float32; "
                          "round_like_unfused does not apply")
+    if gelu_apart:
+        out = gelu(gemm(a, b, bias), "tanh" if epilogue == _ek.EPI_GELU_TANH else "none")
+        return out if residual is None else out.add_(residual)
     out = torch.empty(out_shape, dtype=result_dtype, device=a.device)
     if out.numel() == 0:
         return out
