@@ -156,17 +156,10 @@ static inline double simt_cost(bool f32, int64_t batch, int64_t m, int64_t n, in
   const double many = f32 ? r * (0.038 * k + 0.24 + 1.33 * filled) : r * (0.036 * k + 0.21 + 0.72 * filled);
   return (f32 ? 5.2 : 5.1) + (alone > many ? alone : many);
 }
-// What a 16-bit product costs beside itself when its residual is added apart: one pass of three tensors, or four launches
-// in float32 when only the sum is rounded; 5.8 TB/s.
-static inline double add_apart_cost(const GemmArgs& g, int64_t batch) {
-  const double elements = static_cast<double>(g.m) * g.n * batch;
-  return g.round_like_unfused ? 3.0 + elements * 6.0 / 5.8e6 : 12.0 + elements * 30.0 / 5.8e6;
-}
 static inline bool simt_instead_of_any(const GemmArgs& g, int64_t batch, const AnyPlan& plan) {
-  if (plan.splits > 0 || g.k > 32) return false;
+  if (g.residual != nullptr || plan.splits > 0 || g.k > 32) return false;
   const AnyTile& t = kAnyTiles[plan.tile];
-  const double apart = g.residual != nullptr ? add_apart_cost(g, batch) : 0.0;
-  return simt_cost(false, batch, g.m, g.n, g.k) + apart <
+  return simt_cost(false, batch, g.m, g.n, g.k) <
          many_tiles_cost(kAnyMany[plan.tile], t.bm, t.bn, batch, g.m, g.n, g.k);
 }
 // What that kernel asks of its operands: eight elements along each contiguous direction, and lane
@@ -214,12 +207,13 @@ static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k,
 int gemm_any(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, bool bf16, int epilogue,
              hipStream_t stream);
 
-// A transposed A with a residual that the rings would multiply without one: whether the any-layout kernel, which
-// takes the residual along, is faster than their product and the caller's add. 4096^3: 241 us there against 122 and
-// 193 apart, 768 x 3072 x 1024 24 against 17 and 31, 2048^3 40 against 27 and 46, 1024^3 14 against 15 and 27, 8192 x
-// 8192 x 1024 420 against 204 and 492. The fifth is the models' own error.
+// A transposed A with a residual that the rings would multiply without one and that is rounded with the product once:
+// whether the any-layout kernel, which takes the residual along, is faster than their product and the caller's four
+// launches in float32 (5.8 TB/s). 4096^3: 241 us there against 193 apart, 768 x 3072 x 1024 24 against 31, 2048^3 40
+// against 46, 1024^3 14 against 27, 8192 x 8192 x 1024 420 against 492. The fifth is the models' own error.
 static inline bool any_with_residual_pays(const GemmArgs& g, int64_t batch, double any_cost) {
-  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add_apart_cost(g, batch);
+  const double add = 12.0 + static_cast<double>(g.m) * g.n * batch * 30.0 / 5.8e6;
+  return any_cost * 1.2 < ring_cost(batch, g.m, g.n, g.k) + add;
 }
 
 // Split-K: products with few output tiles and a long K (weight gradients, narrow projections)
@@ -423,8 +417,7 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
     if (g.residual != nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue) &&
         !any_with_residual_pays(g, batch, plan.cost))
       return {TMB_ERR_UNSUPPORTED, 0, 0};
-    if (simt_instead_of_any(g, batch, plan))
-      return {g.residual != nullptr ? TMB_ERR_UNSUPPORTED : TMB_GEMM_SIMT, 0, 0};
+    if (simt_instead_of_any(g, batch, plan)) return {TMB_GEMM_SIMT, 0, 0};
     return {TMB_GEMM_ANY, plan.tile, plan.splits};
   }
   if (aligned) return {TMB_GEMM_RING, 0, 0};
