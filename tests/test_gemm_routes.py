@@ -283,8 +283,8 @@ def test_fp32_products_with_long_rows_stay_on_the_matrix_cores():
 
 
 def test_long_runs_of_k_are_padded_for_the_aligned_kernels():
-    """(m, n, k, transposed A, transposed B), A (the first two: and B) off a 16-byte boundary, whose padded copies measured 1.3 .. 1.6 times as fast as
-    the operands where they lie, some of them on a split launch; and a shape that stays."""
+    """(m, n, k, transposed A, transposed B), A (the first two: and B) off a 16-byte boundary, whose padded copies measured
+    1.3 .. 1.6 times as fast as the operands where they lie, some of them on a split launch; and a shape that stays."""
     ek = _ek()
     for m, n, k, ta, tb in ((597, 5159, 7235, 0, 1), (2336, 512, 8672, 0, 1), (192, 7168, 4704, 1, 0)):
         ask = ek.lib().tmb_gemm_in_place_workspace_bytes

@@ -137,9 +137,10 @@ static inline AnyPlan any_plan(int64_t batch, int64_t m, int64_t n, int64_t k, b
 // fp32), so with one slice or less all but one of them idle, and a launch of many tiles takes what a tile's
 // way through LDS takes. The vector kernel's 64 x 64 tiles are then faster (bf16 7309 x 3268 x 2 31 against 70 us, 48 x
 // 402 x 354 x 8 14 against 26; fp32 48 x 5222 x 7 x 5 17 against 55). Microseconds of both, a start and rounds of tiles,
-// fitted to 1200 shapes a type of 2 .. 9000 in each extent, half of them K <= 128, 1 .. 48 batches; 12-17 % (rms). Over
-// those shapes, where one of the two was forced: 97 (fp32: 287) of 1200 were more than a tenth slower than before the
-// kernels whose waves share K, with these rules and f32_padded_cost below 4 (15) are.
+// fitted to 1200 unaligned shapes a type of 2 .. 9000 in each extent, half of them K <= 128, 1 .. 48 batches; 12-17 %
+// (rms; a wave-sharing tile's power law 15-20 % in 16 bits). By the times measured on those shapes with each kernel
+// forced, 97 of 1200 (fp32 287) would take a tenth longer than on the vector kernel or on padded copies if the waves'
+// kernels took them all, and 4 (16) do with the rules here.
 struct ManyTiles {
   double start, per_k, per_tile, power;
 };
@@ -188,7 +189,8 @@ static inline double padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k,
   double cost = ring_cost(batch, m, n, k);
   const int64_t depth = k % 8 == 0 ? k : (k + 63) / 64 * 64;
   const SplitKPlan split = splitk_plan(batch, m, n, depth);
-  if (split.splits > 0 && (trans_a || !small_applies(batch, m, n, depth))) cost = std::fmin(cost, split.cost + 6.0);  // (2336 x 512 x 8672 57 us so, 81 where it lies)
+  if (split.splits > 0 && (trans_a || !small_applies(batch, m, n, depth)))
+    cost = std::fmin(cost, split.cost + 6.0);  // (2336 x 512 x 8672 57 us so, 81 where it lies)
   auto copy = [&](int64_t elements, bool transposing) {
     return 3.0 + static_cast<double>(elements) * batch * 4.0 / (transposing ? 1e6 : 4e6);
   };
@@ -389,7 +391,8 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
     GemmArgs alone = g;
     alone.residual = nullptr;
     GemmRoute r = route_16bit(alone, batch, trans_a, trans_b, epilogue, workspace_bytes);
-    if (r.kernel == TMB_GEMM_STREAM64 && mfma_eligible(g, batch, trans_a, trans_b)) r.kernel = TMB_GEMM_RING;  // (as it adds)
+    if (r.kernel == TMB_GEMM_STREAM64 && mfma_eligible(g, batch, trans_a, trans_b))
+      r.kernel = TMB_GEMM_RING;  // (adds its four steps of K in the same order)
     if (r.kernel == TMB_GEMM_TRANSPOSED_A || r.kernel == TMB_GEMM_STREAM64 || r.kernel == TMB_GEMM_SIMT)
       return {TMB_ERR_UNSUPPORTED, 0, 0};
     return r;
