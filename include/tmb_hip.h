@@ -206,7 +206,7 @@ typedef enum tmb_gemm_kernel {
   TMB_GEMM_ANY = 5,          /* 16-bit, any layout and alignment; tile 0 .. 4 */
   TMB_GEMM_STREAM64 = 6,     /* 16-bit, K = 64 on whole 128 x 128 tiles */
   TMB_GEMM_F32 = 7,          /* fp32, any layout and alignment; tile 0 .. 3 */
-  TMB_GEMM_F32_WIDE = 8      /* fp32, aligned, 128 x 128 tiles */
+  TMB_GEMM_F32_WIDE = 8      /* fp32, 128 x 128 tiles: aligned, or K >= 512 */
 } tmb_gemm_kernel;
 /* What a product of such operands runs on: kernel | tile << 8 | splits << 16 (a tmb_gemm_kernel, an index into
  * its tiles, 0 splits where K is not split), or a negative status where tmb_gemm* answers that. The launch follows

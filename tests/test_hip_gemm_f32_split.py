@@ -1,0 +1,90 @@
+"""fp32 products on the bf16 matrix cores: as exact as fp32 products over the whole range of fp32, infinities and NaN
+where they belong, and every edge of the 128 x 128 kernel (rows, columns, the last stage of K, runs of K split over
+workgroups, operands off 16-byte boundaries)."""
+
+import itertools
+
+import pytest
+import torch
+
+from test_gemm_routes import F32, F32_WIDE, PLENTY, route
+
+
+def _ops():
+    from torch_mojo_backend.eager_kernels import hip_ops
+    return hip_ops
+
+
+def _operand(rows, cols, stored_transposed, seed, offset=0, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    r, c = (cols, rows) if stored_transposed else (rows, cols)
+    buf = torch.full((r * c + offset,), float("nan"), device="cuda")
+    x = buf[offset:].view(r, c)
+    x.copy_(torch.randn(r, c, generator=g, device="cuda").double() * scale)
+    return x.t() if stored_transposed else x
+
+
+def _check(got, a, b, extra=0.0):
+    """|got - exact| <= the a-priori bound of k float32 multiply-adds; among subnormals each of up to 16 partial sums is
+    rounded to a multiple of the smallest one."""
+    a64, b64 = a.double().contiguous(), b.double().contiguous()
+    exact = a64 @ b64 + extra
+    bound = (a.shape[-1] + 2) * 2.0 ** -24 * (a64.abs() @ b64.abs() + exact.abs()) + 8 * 2.0 ** -149
+    assert ((got.double() - exact).abs() <= bound).all()
+
+
+# whole tiles, one row / column past them, K that ends inside a stage or a 16-byte piece; the last two split
+WIDE = [(1408, 2304, 768), (1409, 2433, 772), (2047, 2300, 132), (3001, 1030, 515), (750, 768, 3072), (385, 770, 8201)]
+
+
+def test_the_shapes_reach_the_kernel():
+    from torch_mojo_backend import eager_kernels as ek
+    for m, n, k in WIDE:
+        for ta, tb in itertools.product((0, 1), repeat=2):
+            aligned = (m if ta else k) % 4 == 0 and (k if tb else n) % 4 == 0
+            if aligned or k >= 512:
+                kernel, _, splits = route(m, n, k, ta, tb, ek.F32, a_aligned=aligned, b_aligned=aligned, workspace=PLENTY)
+                assert kernel == F32_WIDE and (splits > 0) == (m < 1000), (m, n, k, ta, tb)
+    assert route(300, 500, 300, dtype=ek.F32, workspace=PLENTY)[0] == F32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", WIDE)
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_edges_of_the_128_tile(mnk, trans_a, trans_b):
+    m, n, k = mnk
+    bias = torch.randn(n, device="cuda")
+    for offset in (0, 1):
+        a, b = _operand(m, k, trans_a, 1, offset), _operand(k, n, trans_b, 2, offset)
+        _check(_ops().gemm(a, b, bias), a, b, bias.double())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(1408, 2304, 768), (300, 500, 300), (64, 128, 2000)])
+@pytest.mark.parametrize("scales", [(2.0 ** -130, 2.0 ** 60), (2.0 ** -118, 2.0 ** -10), (2.0 ** 115, 2.0 ** -60),
+                                    (2.0 ** 100, 2.0 ** 10), (1.0, 2.0 ** -149)])
+def test_the_ends_of_the_range(mnk, scales):
+    """Subnormal operands and results, and operands and results too large for the factor that the split is given room
+    with: as exact as any (operands are rounded to float32 before, so what they are is what is multiplied)."""
+    m, n, k = mnk
+    a, b = _operand(m, k, False, 3, scale=scales[0]), _operand(k, n, True, 4, scale=scales[1])
+    _check(_ops().gemm(a, b), a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(1408, 2304, 768), (300, 500, 300), (64, 128, 2000), (750, 768, 3072)])
+def test_infinities_and_nan(mnk):
+    """Each as in the float64 product of the same operands; rows and columns without them are not touched."""
+    m, n, k = mnk
+    a, b = _operand(m, k, False, 5), _operand(k, n, True, 6)
+    a[3, 7], a[m - 2, 0], a[m // 2, k - 1] = float("inf"), float("nan"), float("-inf")
+    b[k // 2, 5], b[7, n - 1] = float("inf"), 0.0
+    got, exact = _ops().gemm(a, b), a.double() @ b.double().contiguous()
+    assert torch.equal(got.isnan(), exact.isnan()) and torch.equal(got.isinf(), exact.isinf())
+    assert torch.equal(got[got.isinf()], exact[exact.isinf()].float())
+    rows = torch.ones(m, dtype=torch.bool)
+    rows[[3, m - 2, m // 2]] = False
+    columns = torch.ones(n, dtype=torch.bool)
+    columns[5] = False
+    _check(got[rows][:, columns], a[rows], b[:, columns])

@@ -118,7 +118,15 @@ extern "C" size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, 
   using namespace tmb;
   if (dtype != TMB_F32 && dtype != TMB_F16 && dtype != TMB_BF16) return 0;
   if (batch < 1 || m < 1 || n < 1 || k < 1 || m * n >= (int64_t{1} << 31)) return 0;
-  const int splits = dtype == TMB_F32 ? f32_plan(batch, m, n, k, true).splits : splitk_plan(batch, m, n, k).splits;
+  int splits = 0;
+  if (dtype == TMB_F32) {
+    for (int layout = 0; layout < 4; ++layout) {
+      const int here = f32_most_splits(batch, m, n, k, layout >> 1, layout & 1);
+      splits = here > splits ? here : splits;
+    }
+  } else {
+    splits = splitk_plan(batch, m, n, k).splits;
+  }
   return static_cast<size_t>(splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4;
 }
 
@@ -126,8 +134,10 @@ extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int6
                                                   int trans_b, int dtype) {
   // the kernels for small and for wide products need none (operands they cannot take run unsplit then)
   if (dtype == TMB_F32) {
-    if ((trans_a ? m : k) % 4 == 0 && (trans_b ? k : n) % 4 == 0 && tmb::f32_wide_pays(batch, m, n, k)) return 0;
-  } else if (!trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k)) {
+    if (batch < 1 || m < 1 || n < 1 || k < 1 || m * n >= (int64_t{1} << 31)) return 0;
+    return static_cast<size_t>(tmb::f32_most_splits(batch, m, n, k, trans_a, trans_b)) * m * n * 4;
+  }
+  if (!trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k)) {
     return 0;
   }
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
@@ -158,8 +168,9 @@ extern "C" int tmb_gemm_f32_padding_pays(int64_t batch, int64_t m, int64_t n, in
   GemmArgs g{};
   g.m = m, g.n = n, g.k = k, g.lda = lda, g.ldb = ldb;
   if (!f32_shared_eligible(g, trans_a, trans_b)) return 1;
-  const F32Plan plan = f32_plan(batch, m, n, k, true);
+  const F32Plan plan = f32_plan(batch, m, n, k, 16);
   double here = plan.cost;
+  if (k >= kF32WideUnalignedK) here = std::fmin(here, f32_wide_plan(batch, m, n, k, plan).cost);
   if (k <= 48 && plan.splits == 0) here = std::fmin(here, simt_cost(true, batch, m, n, k));
   return f32_padded_cost(batch, m, n, k, lda, ldb, a_aligned != 0, b_aligned != 0, trans_a, trans_b) < here;
 }

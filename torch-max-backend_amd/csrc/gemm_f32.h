@@ -1,25 +1,23 @@
-// fp32 GEMM on the matrix cores (v_mfma_f32_32x32x2_f32: true fp32 products, fp32 accumulation), any
-// of the four operand layouts, any extents and any row pitch.
+// fp32 GEMM on the bf16 matrix cores, any of the four operand layouts, any extents and any row pitch.
+//
+// An fp32 MFMA takes 64 cycles for what a bf16 one does in four. So each operand element is taken apart into three bf16
+// whose sum it is, exactly (F32Pair), and a product is the six of the nine partial products that are above 2^-24 of it,
+// added up in fp32 by v_mfma_f32_16x16x32_bf16: 16 cycles of matrix core instead of 64, and the rounding of a sum once in
+// 32 k instead of at every k. Against 64 bits the results are off by 0.2 .. 0.8 of what fp32 MFMAs (v_mfma_f32_32x32x2)
+// gave, over K 64 .. 50257. 1332 x 768 x 3072 68 -> 51 us, 750 x 3072 x 768 47 -> 36, 4096^3 1110 -> 775 (gemm_f32_wide.h).
 //
 // A workgroup owns a BM x BN tile of C and its WAVES waves share K: wave w multiplies the 32-deep
 // slices w, w + WAVES, ... of the whole tile and the partial tiles meet in LDS once, at the end, where
-// they are added pairwise in wave order (the result depends on the shape only). An fp32 MFMA takes
-// 64 cycles for two 4-byte operands per lane, so the matrix cores bound all but the smallest launches,
-// and what has to be right is the division of the work: tiles small enough to give every CU the same
-// amount (1332 x 3072 x 768 is 264 tiles of 128 x 128, i.e. two rounds of the 256 CUs for 1.03 rounds
-// of work), and no workgroup barrier in the main loop. Sharing K instead of the tile halves what a wave
-// reads from LDS per MFMA against the same tile cut into quarters, and lets a 32 x 32 tile, of which
-// even a small product has hundreds, keep all four SIMDs busy.
+// they are added pairwise in wave order (the result depends on the shape only): no workgroup barrier in the main loop,
+// and tiles small enough to give every CU the same amount. What bounds it is the vector units, which take the operands
+// apart (44 instructions for a fragment of 16 rows, of which two hide behind an MFMA), then the matrix cores.
 //
 // A wave brings a slice in through registers (the next slice travels while this one is multiplied) and
-// a wave-private part of LDS, which works in order per wave. An operand stored with K contiguous
-// (A [M, K], B [N, K]) is kept as lines of 32 floats; a lane takes four consecutive k with one 16-byte
-// read and feeds four MFMAs with them (lanes 0-31 the first four of a group of eight, lanes 32-63 the
-// others: the order in which the k of a slice are added is free as long as A and B agree). An operand
-// stored with its M or N extent contiguous (A [K, M], B [K, N]) is kept as k-rows.
+// a wave-private part of LDS, which works in order per wave; a lane of a fragment takes eight consecutive k of a row.
+// The split of a column block is scheduled between the MFMAs of the block before it.
 //
 // The MFMA gets the B fragment first, so a lane ends up with one row m of C and four consecutive
-// columns per register quad.
+// columns.
 #pragma once
 
 #include "gemm_mfma.h"
@@ -27,6 +25,9 @@
 namespace tmb {
 
 constexpr int kF32KS = 32;  // depth of a slice: one 128-byte line
+// Up to here products are fp32 ones: a wave has a slice or two, and the larger code and register file of the split kernel
+// cost more than its matrix cores save.
+constexpr int64_t kF32SplitK = 128;
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -43,88 +44,209 @@ __device__ __forceinline__ f32x4_t f32_shift(f32x4_t x, int sh) {
   return r;
 }
 
-// One operand's slice: ROWS rows (m or n) by 32 k, as 16-byte pieces along its contiguous direction.
-// A piece that reaches past the operand's edge is read from the last four elements that exist (so at
-// least four must) and moved into place on its way into LDS: no access outside the operand, and no
-// divergent code in the way of the full slices.
+// One operand's slice: ROWS rows (m or n) by 32 k, kept in LDS as lines of 32 k.
+//
+// K contiguous in memory: 16-byte pieces of lines. A piece that reaches past K is read from the last four
+// elements that exist (so at least four must) and moved into place on its way into LDS: no access outside the operand,
+// and no divergent code in the way of the full slices.
 template <int ROWS, bool K_CONTIGUOUS>
 struct F32Slice {
-  // floats per LDS line / k-row: four more than the data keep 16-byte alignment and spread the rows
-  // of a fragment read over the banks
-  static constexpr int PITCH = K_CONTIGUOUS ? kF32KS + 4 : ROWS + 4;
-  static constexpr int FLOATS = K_CONTIGUOUS ? ROWS * PITCH : kF32KS * PITCH;
-  static constexpr int LOADS = ROWS / 8;                   // pieces per lane and slice
-  static constexpr int LPL = K_CONTIGUOUS ? 8 : ROWS / 4;  // lanes per line
+  // floats per LDS line: four more than the data keep 16-byte alignment and spread the rows of a fragment read
+  // over the banks
+  static constexpr int PITCH = kF32KS + 4;
+  static constexpr int FLOATS = ROWS * PITCH;
+  static constexpr int LOADS = ROWS / 8;  // pieces per lane and slice
   f32x4_t v[LOADS];
   uint32_t off[LOADS];  // bytes from four elements in front of the tile's first one (a tile of fewer than
                         // four columns is read from in front of it: offsets stay unsigned that way)
-  int shift;            // how far this lane's pieces reach past the last row (MN-contiguous operands)
 
-  static __device__ __forceinline__ int line_of(int i, int lane) { return i * (64 / LPL) + lane / LPL; }
-  // `rows`: how many of the operand's rows exist from the tile's first one on (lines past the edge of
-  // a K-contiguous operand re-read the last one: computed, never stored)
+  static __device__ __forceinline__ int line_of(int i, int lane) { return i * 8 + lane / 8; }
+  // `rows`: how many of the operand's rows exist from the tile's first one on (lines past the edge re-read the last
+  // one: computed, never stored)
   __device__ __forceinline__ void plan(int64_t ld, int64_t rows, int lane) {
-    const int c = (lane % LPL) * 4;
+    const int c = (lane % 8) * 4;
     const int last = rows > ROWS ? ROWS : static_cast<int>(rows);
-    const int at = K_CONTIGUOUS || c + 4 <= last ? c : last - 4;
-    shift = c - at;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      int line = line_of(i, lane);
-      if constexpr (K_CONTIGUOUS) line = line < last ? line : last - 1;
-      off[i] = static_cast<uint32_t>((line * ld + at + 4) * 4);
+      const int line = line_of(i, lane) < last ? line_of(i, lane) : last - 1;
+      off[i] = static_cast<uint32_t>((line * ld + c + 4) * 4);
     }
   }
   // first: the tile's first row at this slice's first k. `k_left`: how many k exist from there on.
+  __device__ __forceinline__ void load(const char* __restrict__ first, int64_t, int64_t k_left, int lane) {
+    const char* __restrict__ base = first - 16;
+    if (k_left >= kF32KS) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) v[i] = *reinterpret_cast<const f32x4_unaligned_t*>(base + off[i]);
+    } else {
+      const int left = static_cast<int>(k_left), c = (lane % 8) * 4;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        int64_t at = off[i];
+        if (c + 4 > left) at += (left - 4 - c) * 4;
+        v[i] = *reinterpret_cast<const f32x4_unaligned_t*>(base + at);
+      }
+    }
+  }
+  __device__ __forceinline__ void lay_down(float* __restrict__ lds, int64_t k_left, int lane) {
+    const int c = (lane % 8) * 4;
+    if (k_left < kF32KS) {  // wave-uniform
+      const int left = static_cast<int>(k_left);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) v[i] = f32_shift(v[i], c + 4 > left ? c - (left - 4) : 0);
+    }
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) *reinterpret_cast<f32x4_t*>(lds + line_of(i, lane) * PITCH + c) = v[i];
+  }
+  // The eight k that lane quarter `lq` takes of row `row`: 8 * lq .. 8 * lq + 7.
+  static __device__ __forceinline__ void fragment(const float* __restrict__ lds, int row, int lq, f32x4_t (&x)[2]) {
+    const float* p = lds + row * PITCH + lq * 8;
+    x[0] = *reinterpret_cast<const f32x4_t*>(p);
+    x[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
+  }
+};
+// M or N contiguous, 64 rows: a lane is a row and brings its k one by one (the lanes read a k-row's neighbours), so that
+// what it lays down are pieces of lines too: a fragment is two reads instead of eight (4096^3 with both operands so
+// 1030 us, 1190 with the layout below, whose eight fragments at once do not fit the registers).
+template <>
+struct F32Slice<64, false> {
+  static constexpr int ROWS = 64;
+  using Lines = F32Slice<ROWS, true>;
+  static constexpr int FLOATS = Lines::FLOATS, LOADS = Lines::LOADS;
+  f32x4_t v[LOADS];
+  uint32_t off;  // bytes: the lane's row and first k
+
+  static __device__ __forceinline__ int first_k(int lane) { return lane / ROWS * LOADS * 4; }
+  __device__ __forceinline__ void plan(int64_t ld, int64_t rows, int lane) {
+    const int last = rows > ROWS ? ROWS : static_cast<int>(rows), line = lane % ROWS;
+    off = static_cast<uint32_t>((first_k(lane) * ld + (line < last ? line : last - 1)) * 4);
+  }
+  __device__ __forceinline__ void load(const char* __restrict__ first, int64_t ld, int64_t k_left, int lane) {
+    const int64_t step = ld * 4;
+    auto at = [](const char* p) { return *reinterpret_cast<const float*>(p); };
+    if (k_left >= kF32KS) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const char* __restrict__ p = first + 4 * i * step;
+        v[i] = f32x4_t{at(p + off), at(p + step + off), at(p + 2 * step + off), at(p + 3 * step + off)};
+      }
+    } else {  // (k past the last one re-read it)
+      const int most = static_cast<int>(k_left) - 1 - first_k(lane);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const char* __restrict__ p = first + off;
+        auto k = [&](int e) { return (4 * i + e < most ? 4 * i + e : most) * step; };
+        v[i] = f32x4_t{at(p + k(0)), at(p + k(1)), at(p + k(2)), at(p + k(3))};
+      }
+    }
+  }
+  __device__ __forceinline__ void lay_down(float* __restrict__ lds, int64_t k_left, int lane) {
+    if (k_left < kF32KS) {  // wave-uniform
+      const int left = static_cast<int>(k_left) - first_k(lane);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        v[i] = f32x4_t{4 * i < left ? v[i][0] : 0.0f, 4 * i + 1 < left ? v[i][1] : 0.0f, 4 * i + 2 < left ? v[i][2] : 0.0f,
+                       4 * i + 3 < left ? v[i][3] : 0.0f};
+    }
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      *reinterpret_cast<f32x4_t*>(lds + (lane % ROWS) * Lines::PITCH + first_k(lane) + 4 * i) = v[i];
+  }
+  static __device__ __forceinline__ void fragment(const float* __restrict__ lds, int row, int lq, f32x4_t (&x)[2]) {
+    Lines::fragment(lds, row, lq, x);
+  }
+};
+
+// M or N contiguous, 32 rows: 16-byte pieces of k-rows, kept as k-rows. A piece that reaches past the last row is read
+// from the last four that exist and moved into place.
+template <>
+struct F32Slice<32, false> {
+  static constexpr int ROWS = 32;
+  static constexpr int PITCH = ROWS + 4, FLOATS = kF32KS * PITCH, LOADS = ROWS / 8, LPL = ROWS / 4;  // (lanes per k-row)
+  f32x4_t v[LOADS];
+  uint32_t off[LOADS];  // bytes from four elements in front of the tile's first one
+  int shift;            // how far this lane's pieces reach past the last row
+
+  static __device__ __forceinline__ int line_of(int i, int lane) { return i * (64 / LPL) + lane / LPL; }
+  __device__ __forceinline__ void plan(int64_t ld, int64_t rows, int lane) {
+    const int c = (lane % LPL) * 4;
+    const int last = rows > ROWS ? ROWS : static_cast<int>(rows);
+    const int at = c + 4 <= last ? c : last - 4;
+    shift = c - at;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) off[i] = static_cast<uint32_t>((line_of(i, lane) * ld + at + 4) * 4);
+  }
   __device__ __forceinline__ void load(const char* __restrict__ first, int64_t ld, int64_t k_left, int lane) {
     const char* __restrict__ base = first - 16;
     if (k_left >= kF32KS) {  // wave-uniform
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) v[i] = *reinterpret_cast<const f32x4_unaligned_t*>(base + off[i]);
     } else {
-      const int left = static_cast<int>(k_left), c = (lane % LPL) * 4;
+      const int left = static_cast<int>(k_left);
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         int64_t at = off[i];
-        if constexpr (K_CONTIGUOUS) {
-          if (c + 4 > left) at += (left - 4 - c) * 4;
-        } else {
-          const int line = line_of(i, lane);
-          if (line >= left) at -= (line - left + 1) * ld * 4;
-        }
+        const int line = line_of(i, lane);
+        if (line >= left) at -= (line - left + 1) * ld * 4;
         v[i] = *reinterpret_cast<const f32x4_unaligned_t*>(base + at);
       }
     }
   }
-  __device__ __forceinline__ void lay_down(float* __restrict__ lds, int64_t k_left, bool edge, int lane) {
-    const int c = (lane % LPL) * 4;
-    if (K_CONTIGUOUS ? k_left < kF32KS : (edge || k_left < kF32KS)) {  // wave-uniform
-      const int left = k_left < kF32KS ? static_cast<int>(k_left) : kF32KS;
+  __device__ __forceinline__ void lay_down(float* __restrict__ lds, int64_t k_left, int lane) {
+    const int left = k_left < kF32KS ? static_cast<int>(k_left) : kF32KS;
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) {
-        if constexpr (K_CONTIGUOUS) v[i] = f32_shift(v[i], c + 4 > left ? c - (left - 4) : 0);
-        else v[i] = f32_shift(v[i], line_of(i, lane) < left ? shift : 4);
-      }
+    for (int i = 0; i < LOADS; ++i) {
+      const int line = line_of(i, lane);
+      *reinterpret_cast<f32x4_t*>(lds + line * PITCH + (lane % LPL) * 4) = f32_shift(v[i], line < left ? shift : 4);
     }
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) *reinterpret_cast<f32x4_t*>(lds + line_of(i, lane) * PITCH + c) = v[i];
   }
-  // The four k that lane half `lk` takes of group `g` (eight k) in row `row`.
-  static __device__ __forceinline__ f32x4_t fragment(const float* __restrict__ lds, int row, int g, int lk) {
-    if constexpr (K_CONTIGUOUS) {
-      return *reinterpret_cast<const f32x4_t*>(lds + row * PITCH + g * 8 + lk * 4);
-    } else {
-      const float* p = lds + (g * 8 + lk * 4) * PITCH + row;
-      return f32x4_t{p[0], p[PITCH], p[2 * PITCH], p[3 * PITCH]};
+  static __device__ __forceinline__ void fragment(const float* __restrict__ lds, int row, int lq, f32x4_t (&x)[2]) {
+    const float* p = lds + lq * 8 * PITCH + row;
+    x[0] = f32x4_t{p[0], p[PITCH], p[2 * PITCH], p[3 * PITCH]};
+    x[1] = f32x4_t{p[4 * PITCH], p[5 * PITCH], p[6 * PITCH], p[7 * PITCH]};
+  }
+};
+
+// Two fp32 values, times 2^16, as three bf16 each: x = h + m + l with |m| <= 2^-8 |x|, |l| <= 2^-16 |x|. Exact: 24 bits of
+// significand in three times eight, and 2^16 times the smallest fp32 number is the smallest bf16 one. (h is rounded to
+// nearest; what it leaves has at most sixteen bits, which m and l take without rounding.)
+struct F32Pair {
+  uint32_t h, m, l;
+  static constexpr float kUp = 0x1p16f, kDown = 0x1p-16f;  // each operand's factor, and what undoes it
+  static __device__ __forceinline__ F32Pair of(float a, float b) {
+    F32Pair r;
+    a *= kUp;
+    b *= kUp;
+    r.h = pack2<bf16_t>(a, b);
+    a -= __builtin_bit_cast(float, r.h << 16);
+    b -= __builtin_bit_cast(float, r.h & 0xffff0000u);
+    const uint32_t ma = __builtin_bit_cast(uint32_t, a), mb = __builtin_bit_cast(uint32_t, b);
+    r.m = __builtin_amdgcn_perm(mb, ma, 0x07060302u);
+    a -= __builtin_bit_cast(float, ma & 0xffff0000u);
+    b -= __builtin_bit_cast(float, mb & 0xffff0000u);
+    r.l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
+    return r;
+  }
+};
+struct F32Split {
+  u32x4_t h, m, l;
+  __device__ __forceinline__ void of(const f32x4_t (&x)[2]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const F32Pair s = F32Pair::of(x[p >> 1][2 * (p & 1)], x[p >> 1][2 * (p & 1) + 1]);
+      h[p] = s.h;
+      m[p] = s.m;
+      l[p] = s.l;
     }
   }
 };
 
-template <int BM, int BN, int WAVES, int EPI, bool A_MMAJOR, bool B_KMAJOR>
-__global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_kernel(const GemmArgs g) {
+// SPLIT false: fp32 products (short K, kF32SplitK).
+template <int BM, int BN, int WAVES, int EPI, bool A_MMAJOR, bool B_KMAJOR, bool SPLIT>
+__global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) void gemm_f32_kernel(const GemmArgs g) {
   using SliceA = F32Slice<BM, !A_MMAJOR>;
   using SliceB = F32Slice<BN, B_KMAJOR>;
-  constexpr int TM = BM / 32, TN = BN / 32;
+  constexpr int TM = BM / 16, TN = BN / 16;
   constexpr int WAVE_FLOATS = SliceA::FLOATS + SliceB::FLOATS;
   constexpr int RP = BN + 4;  // floats per row of a partial tile
   extern __shared__ __attribute__((aligned(16))) float f32_lds[];
@@ -138,19 +260,13 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
   const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lr = lane & 31, lk = lane >> 5;
+  const int lr = lane & 15, lq = lane >> 4;
   const int64_t M = g.m, N = g.n, K = g.k;
   const float* A = static_cast<const float*>(g.a) + batch * g.stride_a + (A_MMAJOR ? m0 : m0 * g.lda);
   const float* B = static_cast<const float*>(g.b) + batch * g.stride_b + (B_KMAJOR ? n0 * g.ldb : n0);
   const int64_t a_k = A_MMAJOR ? g.lda : 1, b_k = B_KMAJOR ? 1 : g.ldb;  // floats per unit of k
 
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  f32x4v_t acc[TM][TN];
 
   SliceA sa;
   SliceB sb;
@@ -163,48 +279,126 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
     first = slices * split / g.splits;
     slices = slices * (split + 1) / g.splits;
   }
-  const bool a_edge = M - m0 < BM, b_edge = N - n0 < BN;
   auto load = [&](int64_t s) {
     const int64_t k0 = s * kF32KS;
     sa.load(reinterpret_cast<const char*>(A + k0 * a_k), g.lda, K - k0, lane);
     sb.load(reinterpret_cast<const char*>(B + k0 * b_k), g.ldb, K - k0, lane);
   };
-  if (first + wave < slices) load(first + wave);
-  for (int64_t s = first + wave; s < slices; s += WAVES) {
-    sa.lay_down(la, K - s * kF32KS, a_edge, lane);
-    sb.lay_down(lb, K - s * kF32KS, b_edge, lane);
-    wave_lds_point();
-    if (s + WAVES < slices) load(s + WAVES);
+  auto multiply = [&](auto as_bf16) {
 #pragma unroll
-    for (int grp = 0; grp < kF32KS / 8; ++grp) {
-      f32x4_t af[TM], bf[TN];
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = SliceA::fragment(la, i * 32 + lr, grp, lk);
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if (first + wave < slices) load(first + wave);
+    for (int64_t s = first + wave; s < slices; s += WAVES) {
+      sa.lay_down(la, K - s * kF32KS, lane);
+      sb.lay_down(lb, K - s * kF32KS, lane);
+      wave_lds_point();
+      if (s + WAVES < slices) load(s + WAVES);
+      if constexpr (decltype(as_bf16)::value) {
+        F32Split af[TM], bf[2];
+        f32x4v_t t[TM];
+        f32x4_t x[2];
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = SliceB::fragment(lb, j * 32 + lr, grp, lk);
+        for (int i = 0; i < TM; ++i) {
+          SliceA::fragment(la, i * 16 + lr, lq, x);
+          af[i].of(x);
+        }
+        SliceB::fragment(lb, lr, lq, x);
+        bf[0].of(x);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+        for (int j = 0; j < TN; ++j) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (j > 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[i][j - 1][e] += t[i][e];
+          }
+          if (j + 1 < TN) {
+            SliceB::fragment(lb, (j + 1) * 16 + lr, lq, x);
+            bf[(j + 1) & 1].of(x);
+          }
+          const F32Split& b = bf[j & 1];
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.l, af[i].h, f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].l, t[i]);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.m, af[i].m, t[i]);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.m, af[i].h, t[i]);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].m, t[i]);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].h, t[i]);
+          __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // LDS reads
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // vector ALU
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          }
+#pragma unroll
+          for (int i = 0; i < 5 * TM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[j][e], af[i][e], acc[i][j], 0, 0, 0);
+          for (int e = 0; e < 4; ++e) acc[i][TN - 1][e] += t[i][e];
+      } else {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          f32x4_t bf[2];
+          SliceB::fragment(lb, j * 16 + lr, lq, bf);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            f32x4_t af[2];
+            SliceA::fragment(la, i * 16 + lr, lq, af);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[e >> 2][e & 3], af[e >> 2][e & 3], acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+      wave_lds_point();
     }
-    wave_lds_point();
+  };
+  multiply(std::integral_constant<bool, SPLIT>{});
+  float down = 1.0f;
+  if constexpr (SPLIT) {
+    // A sum that is not finite (an operand or a result that is not, or one beyond what the operands' factor leaves room
+    // for) sends the workgroup through its tile again with fp32 products.
+    __shared__ int wave_non_finite[WAVES];
+    float probe = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) probe = __builtin_fmaf(acc[i][j][e], 0.0f, probe);
+    const uint64_t spoiled = __ballot(probe != 0.0f);
+    if (lane == 0) wave_non_finite[wave] = spoiled != 0;
+    __syncthreads();
+    bool again = false;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) again |= wave_non_finite[w] != 0;
+    if (again) multiply(std::false_type{});
+    else down = F32Pair::kDown;  // once per wave, once for their sum: it is rounded once among subnormals, and stays in range
   }
-
-  // Lane holds row lr of each 32 x 32 result and columns 8q + 4 * lk + {0..3}.
   __syncthreads();  // the partial tiles overlay the slices
+
+  // Lane holds row lr of each 16 x 16 result and columns 4 * lq + {0..3}.
   float* part = f32_lds + wave * (BM * RP);
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4_t v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-        *reinterpret_cast<f32x4_t*>(part + (i * 32 + lr) * RP + j * 32 + 8 * q + 4 * lk) = v;
-      }
+      *reinterpret_cast<f32x4_t*>(part + (i * 16 + lr) * RP + j * 16 + 4 * lq) =
+          f32x4_t{acc[i][j][0] * down, acc[i][j][1] * down, acc[i][j][2] * down, acc[i][j][3] * down};
   __syncthreads();
   const float* __restrict__ bias = static_cast<const float*>(g.bias);
   const float* __restrict__ resid = g.residual == nullptr
@@ -231,7 +425,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
     float out[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float x = v[0][e];
+      float x = v[0][e] * down;
       if (bias != nullptr && (whole || col + e < N)) x += bias[col + e];
       x = finish<float, EPI>(x, false);
       if (resid != nullptr && (whole || col + e < N)) x += resid[row * g.ldr + col + e];
@@ -250,7 +444,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 ? 2 : 1) void gemm_f32_
   }
 }
 
-template <int BM, int BN, int WAVES, int EPI>
+template <int BM, int BN, int WAVES, int EPI, bool SPLIT>
 static int launch_f32_tile(const GemmArgs& base, int64_t batch, int trans_a, int trans_b, hipStream_t stream) {
   GemmArgs g = base;
   g.tiles_m = static_cast<int>((g.m + BM - 1) / BM);
@@ -265,7 +459,7 @@ static int launch_f32_tile(const GemmArgs& base, int64_t batch, int trans_a, int
     constexpr int PARTS = WAVES * BM * (BN + 4) * 4;
     constexpr int SMEM = SLICES > PARTS ? SLICES : PARTS;
     static_assert(SMEM <= 160 * 1024, "LDS of one CU");
-    auto kernel = gemm_f32_kernel<BM, BN, WAVES, EPI, AM, BK>;
+    auto kernel = gemm_f32_kernel<BM, BN, WAVES, EPI, AM, BK, SPLIT>;
     static bool configured = false;
     if (!configured) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),

@@ -1,173 +1,301 @@
-// fp32 GEMM on the matrix cores for products of many tiles and for short K (gemm_f32.h holds the one for
-// everything else): a 128 x 128 tile moves half the bytes per product through L1 and LDS that 64 x 64
-// ones do, which is what counts once the tiles fill whole rounds of the CUs.
+// fp32 GEMM on the bf16 matrix cores, for products of many tiles: each fp32 operand element is three bf16
+// (F32Split, gemm_f32.h) and a product is the six of their nine products that reach fp32 accuracy.
 //
-// One workgroup of 2 x 2 waves owns a 128 x 128 tile of C, each wave a 64 x 64 quarter (2 x 2
-// MFMA tiles, 64 accumulator registers). K is walked in stages of 16: stage s+1 travels from
-// global memory into registers (two 16-byte loads per operand and thread) while stage s is
-// multiplied out of LDS, then the registers go to the other LDS buffer and one barrier closes the
-// stage. An fp32 MFMA takes 64 cycles for two 4-byte operands per lane, so LDS bandwidth is far
-// from mattering; the layouts below only keep the 16-byte stores aligned.
+// One workgroup of 2 x 4 waves owns a 128 x 128 tile of C, each wave a 64 x 32 part, and walks K in stages of 32. The workgroup splits each element once, on its way into LDS: stage s + 2
+// travels from global memory into registers while stage s + 1 is taken apart and laid down in one LDS buffer
+// and stage s is multiplied out of the other; one barrier closes the stage. The vector units that
+// do the splitting are the second bound after the matrix cores (five vector instructions hide behind a
+// 32 x 32 x 16 MFMA, two behind a 16 x 16 x 32 one; measured), hence the large tile and the large MFMA.
 //
-// LDS layouts: an operand stored with K contiguous (A [M, K], B [N, K]) is kept [row][16 + 4];
-// an operand stored with its M or N extent contiguous (A [K, M], B [K, N]) is kept [16][128 + 4].
+// 4096^3 1110 -> 775 us (177 TFLOP/s: 1060 of bf16 products, where the clock falls to what the matrix cores' power leaves),
+// 750 x 50257 x 768 520 -> 391, 2048^3 169 -> 100, each against fp32 MFMAs.
 //
-// As in the 16-bit kernels the MFMA gets the B fragment first, so a lane ends up with one row m
-// of C and four consecutive columns per register quad: 16-byte stores after bias and epilogue.
+// LDS: three planes (high, middle, low parts) of four chunks of eight k; a chunk holds 16 bytes per row, so that both the
+// fragment reads (32 rows of one chunk per half wave) and the eight-byte stores run without bank conflicts.
+//
+// The MFMA gets the B fragment first, so a lane ends up with one row m of C and four consecutive
+// columns per register quad: 16-byte stores after bias and epilogue.
 #pragma once
 
-#include "gemm_f32.h"
+#include "gemm_f32_short.h"
 
 namespace tmb {
 
-constexpr int kF32BM = 128, kF32BN = 128, kF32BK = 16;
-constexpr int kF32PitchK = kF32BK + 4;    // floats per tile row, K contiguous
-constexpr int kF32PitchMN = 128 + 4;      // floats per k line, M / N contiguous
+constexpr int kF32Wide = 128, kF32WideThreads = 512;
 
-// One operand's share of a stage: two 16-byte chunks per thread.
+// One operand's share of a stage: 128 rows by 32 k, of which a thread brings four consecutive k of two rows.
 template <bool K_CONTIGUOUS>
-struct F32Stage {
-  f32x4_t v[2];
+struct F32Staged {
+  static constexpr int ROWS = kF32Wide, ITEMS = ROWS / 64;
+  static constexpr int CHUNK = ROWS * 16 + 64;  // bytes; the pad spreads the chunks that a store goes to over the banks
+  static constexpr int PLANE = 4 * CHUNK, BYTES = 3 * PLANE;
+  f32x4_t v[ITEMS];
+  const float* at[ITEMS];  // K-contiguous: this thread's four k of stage 0; otherwise its column in the first k-row
+  int64_t ld;
+  int k4;      // which four of the stage's k
+  int write;   // byte offset of item 0 in a plane
 
-  // base: first element of the operand for this batch. `row0`: first tile row (m or n) of the
-  // tile, `rows`: the operand's extent in that direction, `ld`: leading dimension in floats.
-  __device__ __forceinline__ void load(const float* __restrict__ base, int64_t ld, int64_t row0,
-                                       int64_t rows, int64_t k0, int64_t K, int tid) {
+  // base: the operand's first row of the tile. `rows`: how many rows exist from there on (rows past the edge re-read
+  // the last one: computed, never stored).
+  __device__ __forceinline__ void plan(const float* base, int64_t ld_, int64_t rows, int wave, int lane) {
+    ld = ld_;
+    const int row = K_CONTIGUOUS ? wave * 8 + lane / 8 : lane;
+    k4 = K_CONTIGUOUS ? lane % 8 : wave;
+    write = (k4 >> 1) * CHUNK + row * 16 + (k4 & 1) * 8;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + 256 * i;
-      const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-      if constexpr (K_CONTIGUOUS) {
-        const int r = idx >> 2, kc = idx & 3;
-        int64_t row = row0 + r;
-        row = row < rows ? row : rows - 1;  // rows past the edge are computed and never stored
-        const int64_t gk = k0 + 4 * kc;
-        v[i] = gk < K ? *reinterpret_cast<const f32x4_t*>(base + row * ld + gk) : zero;
-      } else {
-        const int kr = idx >> 5, c4 = idx & 31;
-        const int64_t gk = k0 + kr, col = row0 + 4 * c4;
-        v[i] = (gk < K && col < rows) ? *reinterpret_cast<const f32x4_t*>(base + gk * ld + col)
-                                      : zero;
+    for (int i = 0; i < ITEMS; ++i) {
+      const int64_t r = row + 64 * i < rows ? row + 64 * i : rows - 1;
+      at[i] = K_CONTIGUOUS ? base + r * ld + 4 * k4 : base + r;
+    }
+  }
+  // Item i of a stage that lies inside K and begins at k0.
+  __device__ __forceinline__ void load(int i, int64_t k0) {
+    if constexpr (K_CONTIGUOUS) {
+      v[i] = *reinterpret_cast<const f32x4_unaligned_t*>(at[i] + k0);
+    } else {
+      const float* p = at[i] + (k0 + 4 * k4) * ld;
+      v[i] = f32x4_t{p[0], p[ld], p[2 * ld], p[3 * ld]};
+    }
+  }
+  // Any stage; elements past K are zeros.
+  __device__ __forceinline__ void load_stage(int64_t k0, int64_t K) {
+    if (k0 + 32 <= K) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) load(i, k0);
+    } else {
+      const int64_t left = K - k0 - 4 * k4;
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) {
+        const float* p = K_CONTIGUOUS ? at[i] + k0 : at[i] + (k0 + 4 * k4) * ld;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = e < left ? p[K_CONTIGUOUS ? e : e * ld] : 0.0f;
       }
     }
   }
-
-  __device__ __forceinline__ void store(float* __restrict__ tile, int tid) const {
+  // Half `p` (two k) of item i taken apart, and the whole item laid down.
+  __device__ __forceinline__ void split(int i, int p, u32x2_t& h, u32x2_t& m, u32x2_t& l) const {
+    const F32Pair s = F32Pair::of(v[i][2 * p], v[i][2 * p + 1]);
+    h[p] = s.h;
+    m[p] = s.m;
+    l[p] = s.l;
+  }
+  __device__ __forceinline__ void lay_down(unsigned char* __restrict__ lds, int i, u32x2_t h, u32x2_t m, u32x2_t l) const {
+    unsigned char* dst = lds + write + i * 64 * 16;
+    *reinterpret_cast<u32x2_t*>(dst) = h;
+    *reinterpret_cast<u32x2_t*>(dst + PLANE) = m;
+    *reinterpret_cast<u32x2_t*>(dst + 2 * PLANE) = l;
+  }
+  __device__ __forceinline__ void lay_down_all(unsigned char* __restrict__ lds) const {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int idx = tid + 256 * i;
-      if constexpr (K_CONTIGUOUS) {
-        *reinterpret_cast<f32x4_t*>(tile + (idx >> 2) * kF32PitchK + 4 * (idx & 3)) = v[i];
-      } else {
-        *reinterpret_cast<f32x4_t*>(tile + (idx >> 5) * kF32PitchMN + 4 * (idx & 31)) = v[i];
-      }
+    for (int i = 0; i < ITEMS; ++i) {
+      u32x2_t h, m, l;
+      split(i, 0, h, m, l);
+      split(i, 1, h, m, l);
+      lay_down(lds, i, h, m, l);
     }
   }
-
-  // Element (row r of the tile, k) of the staged tile.
-  static __device__ __forceinline__ float at(const float* __restrict__ tile, int r, int k) {
-    if constexpr (K_CONTIGUOUS) return tile[r * kF32PitchK + k];
-    else return tile[k * kF32PitchMN + r];
+  // The eight k of chunk `chunk` in row `row`, part `part` (0 high, 1 middle, 2 low).
+  static __device__ __forceinline__ u32x4_t fragment(const unsigned char* __restrict__ lds, int part, int row, int chunk) {
+    return *reinterpret_cast<const u32x4_t*>(lds + part * PLANE + chunk * CHUNK + row * 16);
   }
-
-  static constexpr int kFloats = K_CONTIGUOUS ? 128 * kF32PitchK : kF32BK * kF32PitchMN;
 };
 
 template <int EPI, bool A_MMAJOR, bool B_KMAJOR>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const GemmArgs g) {
-  using StageA = F32Stage<!A_MMAJOR>;
-  using StageB = F32Stage<B_KMAJOR>;
-  constexpr int kBuf = StageA::kFloats + StageB::kFloats;
-  __shared__ __align__(16) float lds[2 * kBuf];
+__global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const GemmArgs g) {
+  using StagedA = F32Staged<!A_MMAJOR>;
+  using StagedB = F32Staged<B_KMAJOR>;
+  constexpr int WAVES_N = 4, TM = 2;
+  constexpr int STAGE = StagedA::BYTES + StagedB::BYTES;
+  extern __shared__ __attribute__((aligned(16))) unsigned char f32_wide_lds[];
 
   int tm, tn;
   tile_of_block(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
-  const int64_t batch = blockIdx.y;
-  const float* __restrict__ A = static_cast<const float*>(g.a) + batch * g.stride_a;
-  const float* __restrict__ B = static_cast<const float*>(g.b) + batch * g.stride_b;
-  float* __restrict__ C = static_cast<float*>(g.c) + batch * g.stride_c;
-  const int64_t m0 = static_cast<int64_t>(tm) * kF32BM, n0 = static_cast<int64_t>(tn) * kF32BN;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  // a split launch (g.splits > 0): blockIdx.y is the split, which multiplies its run of stages and
+  // stores fp32 partials [splits][M][N]
+  const int64_t split = g.splits > 0 ? blockIdx.y : 0;
+  const int64_t batch = g.splits > 0 ? 0 : blockIdx.y;
+  const int64_t m0 = static_cast<int64_t>(tm) * kF32Wide, n0 = static_cast<int64_t>(tn) * kF32Wide;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 31, lk = lane >> 5;
+  const int row0 = wave / WAVES_N * 64, col0 = wave % WAVES_N * 32;  // the wave's part of the tile
+  const int64_t M = g.m, N = g.n, K = g.k;
+  const float* A = static_cast<const float*>(g.a) + batch * g.stride_a + (A_MMAJOR ? m0 : m0 * g.lda);
+  const float* B = static_cast<const float*>(g.b) + batch * g.stride_b + (B_KMAJOR ? n0 * g.ldb : n0);
+  int64_t first = 0, last = (K + 31) / 32;
+  if (g.splits > 0) {
+    const int64_t stages = last;
+    first = stages * split / g.splits;
+    last = stages * (split + 1) / g.splits;
+  }
+  StagedA sa;
+  StagedB sb;
+  sa.plan(A, g.lda, M - m0, wave, lane);
+  sb.plan(B, g.ldb, N - n0, wave, lane);
+  f32x16_t acc[TM], t[TM];
 
-  f32x16_t acc[2][2];
+  auto close_stage = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  u32x4_t a[2][TM][3], b[2][3];
+  auto read_b = [&](const unsigned char* stage, int half, int part) {
+    b[half][part] = StagedB::fragment(stage + StagedA::BYTES, part, col0 + lr, 2 * half + lk);
+  };
+  auto read_a = [&](const unsigned char* stage, int half, int i, int part) {
+    a[half][i][part] = StagedA::fragment(stage, part, row0 + i * 32 + lr, 2 * half + lk);
+  };
+  auto read_first_half = [&](const unsigned char* stage) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int part = 0; part < 3; ++part) {
+      read_b(stage, 0, 2 - part);
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int i = 0; i < TM; ++i) read_a(stage, 0, i, part);
+    }
+  };
+  // A stage's products, added to t; one stage's or, where there are 64 and more, four stages' are joined to the sum in
+  // one addition per element: the sum is rounded once in 32 or 128 k (the errors of both levels add up: K = 64 wants
+  // the former, K = 4096 is off by half as much with the latter). A step is two MFMAs, the reading of a fragment that comes later and a share of
+  // the next stage's splitting; nothing moves between steps, so that the vector instructions stand behind the MFMAs.
+  // The barrier that closes the stage is in front of the last steps, which hide the reading of the next stage's first
+  // fragments: by then every wave has read all it needs of this stage and laid down its part of the next.
+  auto multiply = [&](const unsigned char* cur, unsigned char* next, int64_t k_after, auto splits_next) {
+    constexpr bool NEXT = decltype(splits_next)::value;
+    constexpr int STEPS = 12, CLOSE = STEPS - 3, PAIRS = 2 * (StagedA::ITEMS + StagedB::ITEMS);
+    static_assert(PAIRS < CLOSE, "laid down before the barrier");
+    constexpr int kPartA[6] = {0, 2, 1, 0, 1, 0}, kPartB[6] = {2, 0, 1, 1, 0, 0};  // (smallest terms first)
+    u32x2_t h, m, l;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    for (int step = 0; step < STEPS; ++step) {
+      const int half = step / 6, term = step % 6;
+      if (NEXT && step == CLOSE) {
+        close_stage();
+        read_first_half(next);
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        t[i] = Mfma<bf16_t>::run(b[half][kPartB[term]], a[half][i][kPartA[term]], t[i]);
+      }
+      if (half == 0) {
+        if (term < 3) read_b(cur, 1, 2 - term);
+        read_a(cur, 1, term & 1, term >> 1);
+      }
+      if (NEXT && step < PAIRS) {
+        const int item = step >> 1;
+        if (item < StagedA::ITEMS) sa.split(item, step & 1, h, m, l);
+        else sb.split(item - StagedA::ITEMS, step & 1, h, m, l);
+        if ((step & 1) != 0) {
+          if (item < StagedA::ITEMS) {
+            sa.lay_down(next, item, h, m, l);
+            sa.load(item, k_after);
+          } else {
+            sb.lay_down(next + StagedA::BYTES, item - StagedA::ITEMS, h, m, l);
+            sb.load(item - StagedA::ITEMS, k_after);
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto join = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        acc[i][e] += t[i][e];
+        t[i][e] = 0.0f;
+      }
+  };
 
-  StageA sa;
-  StageB sb;
-  const int64_t stages = (g.k + kF32BK - 1) / kF32BK;
-  sa.load(A, g.lda, m0, g.m, 0, g.k, tid);
-  sb.load(B, g.ldb, n0, g.n, 0, g.k, tid);
-  sa.store(lds, tid);
-  sb.store(lds + StageA::kFloats, tid);
-  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = t[i][e] = 0.0f;
+  if (first < last) {
+    sa.load_stage(first * 32, K);
+    sb.load_stage(first * 32, K);
+    sa.lay_down_all(f32_wide_lds);
+    sb.lay_down_all(f32_wide_lds + StagedA::BYTES);
+    if (first + 1 < last) {
+      sa.load_stage((first + 1) * 32, K);
+      sb.load_stage((first + 1) * 32, K);
+    }
+    close_stage();
+    read_first_half(f32_wide_lds);
+    const int joint = last - first >= 64 ? 3 : 0;
+    int buffer = 0;
+    for (int64_t s = first; s + 1 < last; ++s) {
+      // (an element's register is loaded again as soon as it has been taken apart: a stage's time for the way from
+      // memory. Where there is no stage s + 2 or it ends past K, what is loaded is not used.)
+      const bool whole = s + 2 < last && (s + 3) * 32 <= K;
+      multiply(f32_wide_lds + buffer * STAGE, f32_wide_lds + (buffer ^ 1) * STAGE, (whole ? s + 2 : first) * 32,
+               std::true_type{});
+      if (!whole && s + 2 < last) {
+        sa.load_stage((s + 2) * 32, K);
+        sb.load_stage((s + 2) * 32, K);
+      }
+      if (((s - first) & joint) == joint) join();
+      buffer ^= 1;
+    }
+    multiply(f32_wide_lds + buffer * STAGE, nullptr, 0, std::false_type{});
+    join();
+  }
 
-  for (int64_t s = 0; s < stages; ++s) {
-    const float* __restrict__ ta = lds + (s & 1) * kBuf;
-    const float* __restrict__ tb = ta + StageA::kFloats;
-    const bool more = s + 1 < stages;
-    if (more) {
-      sa.load(A, g.lda, m0, g.m, (s + 1) * kF32BK, g.k, tid);
-      sb.load(B, g.ldb, n0, g.n, (s + 1) * kF32BK, g.k, tid);
+  // Sums that are not finite (an operand or a result that is not, or one beyond what the factor leaves room for)
+  // are formed again from fp32 products.
+  float probe = 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) probe = __builtin_fmaf(acc[i][e], 0.0f, probe);
+  float down = F32Pair::kDown * F32Pair::kDown;
+  if (__ballot(probe != 0.0f) != 0) {  // wave-uniform, and each wave's own: no barrier inside
+    down = 1.0f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+    const int64_t end = last * 32 < K ? last * 32 : K;
+    const int64_t c = n0 + col0 + lr < N ? col0 + lr : N - 1 - n0;
+#pragma unroll 1
+    for (int64_t k = first * 32; k < end; k += 2) {
+      const int64_t kk = k + lk < end ? k + lk : end - 1;
+      const float bf = B[B_KMAJOR ? c * g.ldb + kk : kk * g.ldb + c];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int64_t r = m0 + row0 + i * 32 + lr < M ? row0 + i * 32 + lr : M - 1 - m0;
+        const float af = A[A_MMAJOR ? kk * g.lda + r : r * g.lda + kk];
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(k + lk < end ? bf : 0.0f, k + lk < end ? af : 0.0f, acc[i], 0, 0, 0);
+      }
     }
-#pragma unroll
-    for (int ks = 0; ks < kF32BK / 2; ++ks) {
-      float af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = StageA::at(ta, wm * 64 + i * 32 + lr, 2 * ks + lk);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bf[j] = StageB::at(tb, wn * 64 + j * 32 + lr, 2 * ks + lk);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[j], af[i], acc[i][j], 0, 0, 0);
-    }
-    if (more) {
-      float* __restrict__ next = lds + ((s + 1) & 1) * kBuf;
-      sa.store(next, tid);
-      sb.store(next + StageA::kFloats, tid);
-    }
-    __syncthreads();
   }
 
   // Lane holds row lr of each 32 x 32 result and columns 8q + 4 * lk + {0..3}.
   const float* __restrict__ bias = static_cast<const float*>(g.bias);
+  float* __restrict__ C = static_cast<float*>(g.c) + (batch + split) * g.stride_c;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int64_t row = m0 + wm * 64 + i * 32 + lr;
-    if (row >= g.m) continue;
+  for (int i = 0; i < TM; ++i) {
+    const int64_t row = m0 + row0 + i * 32 + lr;
+    if (row >= M) continue;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int q = 0; q < 4; ++q) {
+      const int64_t col = n0 + col0 + 8 * q + 4 * lk;
+      if (col >= N) continue;
+      float* dst = C + row * g.ldc + col;
+      float out[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int64_t col = n0 + wn * 64 + j * 32 + 8 * q + 4 * lk;
-        if (col >= g.n) continue;
-        float* dst = C + row * g.ldc + col;
-        float out[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float v = acc[i][j][4 * q + e];
-          if (bias != nullptr && col + e < g.n) v += bias[col + e];
-          out[e] = finish<float, EPI>(v, false);
-        }
-        if (col + 4 <= g.n) {
-          const f32x4_unaligned_t v = {out[0], out[1], out[2], out[3]};
-          if (g.stream_c) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_unaligned_t*>(dst));
-          else *reinterpret_cast<f32x4_unaligned_t*>(dst) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (col + e < g.n) dst[e] = out[e];
-        }
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[i][4 * q + e] * down;
+        if (bias != nullptr && col + e < N) v += bias[col + e];
+        out[e] = finish<float, EPI>(v, false);
       }
+      if (col + 4 <= N) {
+        const f32x4_unaligned_t v = {out[0], out[1], out[2], out[3]};
+        if (g.stream_c) __builtin_nontemporal_store(v, reinterpret_cast<f32x4_unaligned_t*>(dst));
+        else *reinterpret_cast<f32x4_unaligned_t*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + e < N) dst[e] = out[e];
+      }
+    }
   }
 }
 
@@ -180,25 +308,34 @@ static inline bool f32_mfma_eligible(const GemmArgs& g, int64_t batch, int trans
   if (batch > 1 && (g.stride_a % 4 != 0 || g.stride_b % 4 != 0)) return false;
   if (trans_a ? g.m % 4 != 0 : g.k % 4 != 0) return false;
   if (trans_b ? g.k % 4 != 0 : g.n % 4 != 0) return false;
-  const int64_t tiles_m = (g.m + kF32BM - 1) / kF32BM, tiles_n = (g.n + kF32BN - 1) / kF32BN;
+  const int64_t tiles_m = (g.m + 127) / 128, tiles_n = (g.n + 127) / 128;
   return tiles_m * tiles_n < (int64_t{1} << 30) && tiles_m < (1 << 24) && tiles_n < (1 << 24);
 }
 
 template <int EPI>
-static int launch_f32_mfma(GemmArgs g, int64_t batch, int trans_a, int trans_b,
-                           hipStream_t stream) {
-  g.tiles_m = static_cast<int>((g.m + kF32BM - 1) / kF32BM);
-  g.tiles_n = static_cast<int>((g.n + kF32BN - 1) / kF32BN);
+static int launch_f32_wide(GemmArgs g, int64_t batch, int trans_a, int trans_b, hipStream_t stream) {
+  if (g.k <= kF32SplitK) return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
+  g.tiles_m = static_cast<int>((g.m + kF32Wide - 1) / kF32Wide);
+  g.tiles_n = static_cast<int>((g.n + kF32Wide - 1) / kF32Wide);
   g.stream_c = batch * g.m * g.n * 4 > (int64_t{256} << 20);
   const dim3 grid(static_cast<unsigned>(g.tiles_m * g.tiles_n), static_cast<unsigned>(batch));
-  if (trans_a) {
-    if (trans_b) gemm_f32_mfma_kernel<EPI, true, true><<<grid, 256, 0, stream>>>(g);
-    else gemm_f32_mfma_kernel<EPI, true, false><<<grid, 256, 0, stream>>>(g);
-  } else {
-    if (trans_b) gemm_f32_mfma_kernel<EPI, false, true><<<grid, 256, 0, stream>>>(g);
-    else gemm_f32_mfma_kernel<EPI, false, false><<<grid, 256, 0, stream>>>(g);
-  }
-  return check_launch();
+  auto go = [&](auto a_mmajor, auto b_kmajor) {
+    constexpr bool AM = decltype(a_mmajor)::value, BK = decltype(b_kmajor)::value;
+    constexpr int SMEM = 2 * (F32Staged<!AM>::BYTES + F32Staged<BK>::BYTES);
+    static_assert(SMEM <= 160 * 1024, "LDS of one CU");
+    auto kernel = gemm_f32_wide_kernel<EPI, AM, BK>;
+    static bool configured = false;
+    if (!configured) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+      if (e != hipSuccess) return static_cast<int>(e);
+      configured = true;
+    }
+    kernel<<<grid, kF32WideThreads, SMEM, stream>>>(g);
+    return check_launch();
+  };
+  if (trans_a) return trans_b ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  return trans_b ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 }  // namespace tmb

@@ -263,52 +263,50 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
   return p;
 }
 
-// fp32: tile and split count. A launch of the kernel whose waves share K takes about 7 us (start, first
-// operands, the partial tiles' way through LDS, stores) and, per round of tiles, the matrix cores' time
-// for one (2 FLOP per 256 and cycle at 2.4 GHz) stretched by what L1, L2 and LDS cost at that tile size;
-// 32 x 32 tiles share a CU and are not bound to whole rounds. Within 8-9 % (rms) of 2000 measured
-// shapes (1 .. 4096 rows, 64 .. 4096 columns, K 64 .. 12564, 1 .. 48 batches). A split adds the reduction:
-// a launch and its bytes at 4 TB/s.
+// fp32: tile and split count of the kernel whose waves share K. Microseconds of a launch: a start and, per round of
+// tiles, their way through LDS and the matrix cores; `whole` of a round's time is bound to whole rounds of the 256 CUs.
+// Fitted to 1600 shapes of 8 .. 8192 in each extent, 1 .. 36 batches, in all layouts; 10-13 % (rms) of each tile. A split
+// adds the reduction: a launch and its bytes. A 64 x 64 tile has eight waves where all tiles run at once (two a SIMD to
+// hide each other's waits: 1332 x 768 x 3072 47 us, with four 58), four, two workgroups to a CU, beyond (1332 x 3072 x 768
+// 50 us, with eight 59).
 struct F32Tile {
-  int bm, bn;
-  double stretch, per_tile;
+  int bm, bn, waves;
+  double start, per_k, per_tile, power, whole;
 };
-constexpr F32Tile kF32Tiles[] = {{32, 32, 2.0, 0.5}, {32, 64, 1.6, 1.0}, {64, 64, 1.4, 2.0}, {64, 128, 1.3, 4.0}};
+constexpr F32Tile kF32Tiles[] = {{32, 32, 4, 3.7, 0.00675, 1.1, 0.887, 0.25}, {32, 64, 4, 3.0, 0.0116, 2.5, 0.912, 0.34},
+                                 {64, 64, 4, 1.3, 0.0163, 4.4, 0.919, 0.67}, {64, 64, 8, 4.5, 0.012, 2.7, 1.0, 0.0}};
 constexpr int kF32TileCount = sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
 struct F32Plan {
   int tile;    // index into kF32Tiles
   int splits;  // 0: not split
   double cost;
 };
-constexpr ManyTiles kF32Many[] = {{2.9, 0.0075, 0.90, 0.933}, {2.8, 0.0129, 1.95, 0.939}, {3.6, 0.0211, 3.2, 0.969},
-                                  {0.0, 0.0368, 10.97, 0.953}};
-static inline double f32_cost(const F32Tile& t, double batch, int64_t m, int64_t n, double k) {
-  const double tiles = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * batch;
-  double rounds = std::ceil(tiles / 256.0);
-  if (t.bm * t.bn == 1024) {
-    if (tiles > 1536.0) return 1e30;  // (far slower than the larger tiles there: L1 and L2 traffic)
-    const double r = tiles / 256.0;
-    rounds = r <= 1.0 ? 1.0 : (0.5 + 0.5 * rounds / r) * std::pow(r, 0.9);
+// (the launches of up to kF32SplitK are the fp32 products')
+constexpr ManyTiles kF32Short[] = {{2.9, 0.0075, 0.90, 0.933}, {2.8, 0.0129, 1.95, 0.939}, {3.6, 0.0211, 3.2, 0.969}};
+static inline double f32_cost(int tile, double batch, int64_t m, int64_t n, double k, bool short_k) {
+  const F32Tile& t = kF32Tiles[tile];
+  const double r = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * batch / 256.0;
+  if (short_k) {
+    if (t.waves == 8) return HUGE_VAL;
+    const ManyTiles& s = kF32Short[tile];
+    return s.start + (r <= 1.0 ? 1.0 : std::pow(r, s.power)) * (s.per_k * k + s.per_tile);
   }
-  return 7.0 + rounds * (2.0 * t.bm * t.bn * k / 256.0 / 2400.0 * t.stretch + t.per_tile);
+  if (t.bm == 64 && (r <= 1.0) != (t.waves == 8)) return HUGE_VAL;
+  const double rounds = r <= 1.0 ? 1.0 : std::pow(r, t.power) * (1.0 - t.whole + t.whole * std::ceil(r) / r);
+  return t.start + rounds * (t.per_k * k + t.per_tile);
 }
-static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, bool may_split) {
-  F32Plan p{kF32TileCount - 1, 0, 0.0};
-  double best = 0.0;
+static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, int most_splits) {
+  F32Plan p{0, 0, HUGE_VAL};
   for (int i = 0; i < kF32TileCount; ++i) {
-    const double c = f32_cost(kF32Tiles[i], static_cast<double>(batch), m, n, static_cast<double>(k));
-    if (i == 0 || c < best) {
-      best = c;
-      p.tile = i;
-    }
+    const double c = f32_cost(i, static_cast<double>(batch), m, n, static_cast<double>(k), k <= kF32SplitK);
+    if (c < p.cost) p = F32Plan{i, 0, c};
   }
-  p.cost = many_tiles_cost(kF32Many[p.tile], kF32Tiles[p.tile].bm, kF32Tiles[p.tile].bn, batch, m, n, k);
-  if (batch != 1 || !may_split) return p;
-  best *= 0.92;  // a second launch and a workspace have to pay for themselves
+  if (batch != 1 || m * n >= (int64_t{1} << 31)) return p;
+  double best = p.cost * 0.92;  // a second launch and a workspace have to pay for themselves
   for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
-    if (k < 96 * s) break;
+    if (k < 96 * s || s > most_splits) break;
     for (int i = 0; i < kF32TileCount; ++i) {
-      const double c = f32_cost(kF32Tiles[i], s, m, n, static_cast<double>(k) / s) + 5.5 + 1e-6 * s * m * n;
+      const double c = f32_cost(i, s, m, n, static_cast<double>(k) / s, k <= kF32SplitK) + 5.5 + 1e-6 * s * m * n;
       if (c < best) {
         best = c;
         p = F32Plan{i, s, c};
@@ -317,25 +315,40 @@ static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, b
   }
   return p;
 }
-// The 128 x 128 kernel (16-byte aligned operands): where its tiles fill at least two rounds well (4096^3
-// level, 1332 x 50257 x 768 870 against 930 us, 4096 x 4096 x 768 225 against 248), and short K, whose tiles
-// are all prologue, from 176 of them on (4096 x 768 x 64 15.1 against 17 us).
-static inline bool f32_wide_pays(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = ((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN) * batch;
-  const int64_t slots = (tiles + 255) / 256 * 256;
-  return (tiles >= 512 && tiles * 20 >= slots * 17) || (k <= 256 && tiles >= 176);
+// The kernel of 128 x 128 tiles, fitted with it (10 %). Its bound is the larger of the tiles' time and the stores'.
+static inline double f32_wide_cost(int64_t batch, int64_t m, int64_t n, double k, bool short_k) {
+  const double count = static_cast<double>(((m + 127) / 128) * ((n + 127) / 128)) * batch;
+  const double tiles = short_k  // (gemm_f32_short.h)
+                           ? 3.2 + std::pow(std::ceil(count / 256.0), 0.923) * (0.078 * k + 3.09)
+                           : 0.4 + std::pow(std::ceil(count / 256.0), 1.06) * (0.0355 * k + 4.8 + (count < 128.0 ? count / 80.0 : 1.6));
+  const double stores = 3.2 + static_cast<double>(batch) * m * n * 4.0 / 5.5e6;
+  return tiles > stores ? tiles : stores;
 }
-// Microseconds on that kernel (fitted with the ones above), and whether aligned operands run there: also where these say
-// so (short K on fewer tiles: 7016 x 248 x 12 7 against 13 us, 840 x 3000 x 8 7 against 13; 5 x 1696 x 1848 x 312 122
-// against 159).
-static inline double f32_wide_cost(int64_t batch, int64_t m, int64_t n, int64_t k) {
-  const double rounds = static_cast<double>((((m + kF32BM - 1) / kF32BM) * ((n + kF32BN - 1) / kF32BN) * batch + 255) / 256);
-  const double tiles = std::pow(rounds, 0.923) * (0.078 * k + 3.09);
-  const double stores = static_cast<double>(batch) * m * n * 4.0 / 5.5e6;
-  return 3.2 + (tiles > stores ? tiles : stores);
-}
-static inline bool f32_wide_wins(int64_t batch, int64_t m, int64_t n, int64_t k, const F32Plan& plan) {
-  return f32_wide_pays(batch, m, n, k) || (plan.splits == 0 && f32_wide_cost(batch, m, n, k) < plan.cost);
+// Operands off 16-byte boundaries are as fast there (its loads want none), and run there from this K on; shorter products
+// of such operands are the padded copies', the vector kernel's and the waves-share-K kernel's.
+constexpr int64_t kF32WideUnalignedK = 512;
+struct F32WidePlan {
+  bool taken;  // before the kernel whose waves share K
+  int splits;
+  double cost;
+};
+// Where a product whose operands both take runs on it (`other`: what it runs as otherwise), and with how many splits. Split it is up to 40 tiles only: from 41
+// on the 64 x 64 tiles of the other kernel have most CUs busy without scratch and a second launch (1024 x 768 x 3072
+// 43 us). 750 x 768 x 3072 31 us in 7 splits, 44 there; 750 x 768 x 50257 275 against 470. A split must promise a fifth,
+// twice the models' error.
+static inline F32WidePlan f32_wide_plan(int64_t batch, int64_t m, int64_t n, int64_t k, const F32Plan& other) {
+  F32WidePlan p{false, 0, f32_wide_cost(batch, m, n, static_cast<double>(k), k <= kF32SplitK)};
+  p.taken = p.cost < other.cost;
+  if (batch != 1 || m * n >= (int64_t{1} << 31) || ((m + 127) / 128) * ((n + 127) / 128) > 40) return p;
+  double best = (p.taken ? p.cost : other.cost) * 0.8;
+  for (int s = 2; s <= 16 && k >= 96 * s; ++s) {
+    const double c = f32_wide_cost(s, m, n, static_cast<double>(k) / s, k <= kF32SplitK) + 5.5 + 1e-6 * s * m * n;
+    if (c < best) {
+      best = c;
+      p = F32WidePlan{true, s, c};
+    }
+  }
+  return p;
 }
 // Unaligned operands: the other way is to copy what the 128 x 128 kernel cannot read into padded buffers (8 us a copy
 // with what the host does for it, and the bytes at 5.3 TB/s, 1.3 where it transposes) and to multiply there, a K that is no
@@ -362,8 +375,8 @@ static inline double f32_padded_cost(int64_t batch, int64_t m, int64_t n, int64_
       copy(n * k, !trans_b);
     }
   }
-  if (!f32_wide_wins(batch, m, n, depth, f32_plan(batch, m, n, depth, true))) return HUGE_VAL;
-  return cost + f32_wide_cost(batch, m, n, depth);
+  const F32WidePlan wide = f32_wide_plan(batch, m, n, depth, f32_plan(batch, m, n, depth, 16));
+  return wide.taken && wide.splits == 0 ? cost + wide.cost : HUGE_VAL;
 }
 // What the kernel whose waves share K asks of its operands: at least four elements along each
 // contiguous direction, and lane offsets that fit 32 bits in its largest tile (64 x 128; 32 rows of k for an
@@ -442,22 +455,42 @@ static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a,
   const bool shared = f32_shared_eligible(g, trans_a, trans_b);
   const bool aligned = f32_mfma_eligible(g, batch, trans_a, trans_b);
   if (!shared && !aligned) return {TMB_GEMM_SIMT, 0, 0};
-  if (aligned && f32_wide_pays(batch, g.m, g.n, g.k)) return {TMB_GEMM_F32_WIDE, 0, 0};
-  F32Plan plan = f32_plan(batch, g.m, g.n, g.k, true);
-  if (plan.splits > 0 && (g.m * g.n >= (int64_t{1} << 31) ||
-                          workspace_bytes < static_cast<size_t>(plan.splits) * g.m * g.n * 4))
-    plan = f32_plan(batch, g.m, g.n, g.k, false);
+  auto fits = [&](int splits) {
+    return splits == 0 || workspace_bytes >= static_cast<size_t>(splits) * g.m * g.n * 4;
+  };
   if (shared) {
-    if (plan.splits == 0) {
-      if (aligned && f32_wide_wins(batch, g.m, g.n, g.k, plan)) return {TMB_GEMM_F32_WIDE, 0, 0};
-      if (g.k <= 48 && simt_cost(true, batch, g.m, g.n, g.k) < plan.cost) return {TMB_GEMM_SIMT, 0, 0};
-    }
+    F32Plan plan = f32_plan(batch, g.m, g.n, g.k, 16);
+    const F32WidePlan wide = f32_wide_plan(batch, g.m, g.n, g.k, plan);
+    const bool takes = aligned || g.k >= kF32WideUnalignedK;
+    if (takes && wide.taken && fits(wide.splits)) return {TMB_GEMM_F32_WIDE, 0, wide.splits};
+    // (no more splits than there: the scratch that a caller of known layout is told of does not depend on alignment)
+    if (wide.splits > 0 && plan.splits > wide.splits) plan = f32_plan(batch, g.m, g.n, g.k, wide.splits);
+    if (!fits(plan.splits)) plan = f32_plan(batch, g.m, g.n, g.k, 0);
+    if (takes && plan.splits == 0 && f32_wide_cost(batch, g.m, g.n, static_cast<double>(g.k), g.k <= kF32SplitK) < plan.cost)
+      return {TMB_GEMM_F32_WIDE, 0, 0};
+    if (g.k <= 48 && plan.splits == 0 && simt_cost(true, batch, g.m, g.n, g.k) < plan.cost) return {TMB_GEMM_SIMT, 0, 0};
     return {TMB_GEMM_F32, plan.tile, plan.splits};
   }
+  const F32Plan plan = f32_plan(batch, g.m, g.n, g.k, 16);
   // rows too long for 32-bit offsets: the wide kernel, a split as a batch of equal runs of whole 16-byte pieces
-  int splits = plan.splits;
+  int splits = fits(plan.splits) ? plan.splits : 0;
   while (splits > 0 && (splits == 1 || g.k % (4 * splits) != 0)) --splits;
   return {TMB_GEMM_F32_WIDE, 0, splits};
+}
+
+// The most splits that a product of dense operands in this layout runs with, at any alignment.
+static inline int f32_most_splits(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a, int trans_b) {
+  int most = 0;
+  for (const uintptr_t address : {16, 20}) {  // (never read: only their alignment is looked at)
+    GemmArgs g{};
+    g.a = g.b = reinterpret_cast<const void*>(address);
+    g.m = m, g.n = n, g.k = k;
+    g.lda = trans_a ? m : k, g.ldb = trans_b ? k : n;
+    g.stride_a = m * k, g.stride_b = k * n;
+    const int splits = route_f32(g, batch, trans_a, trans_b, ~size_t{0}).splits;
+    most = splits > most ? splits : most;
+  }
+  return most;
 }
 
 // The typed half of the entry point (gemm_typed.h), one translation unit per storage type.

@@ -216,11 +216,21 @@ static int launch_splitk(const GemmArgs& g, const SplitKPlan& plan, int trans_a,
 
 template <int EPI>
 static int launch_f32_shared(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, hipStream_t stream) {
+  if (g.k <= kF32SplitK) {
+    switch (tile) {
+      case 0: return launch_f32_tile<32, 32, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
+      case 1: return launch_f32_tile<32, 64, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
+      default: return launch_f32_tile<64, 64, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
+    }
+  }
   switch (tile) {
-    case 0: return launch_f32_tile<32, 32, 4, EPI>(g, batch, trans_a, trans_b, stream);
-    case 1: return launch_f32_tile<32, 64, 4, EPI>(g, batch, trans_a, trans_b, stream);
-    case 2: return launch_f32_tile<64, 64, 4, EPI>(g, batch, trans_a, trans_b, stream);
-    default: return launch_f32_tile<64, 128, 4, EPI>(g, batch, trans_a, trans_b, stream);
+    case 0:  // (one workgroup to a CU and slices for all of eight waves: 64 x 768 x 768 7.5 us, with four 8.8)
+      return ((g.m + 31) / 32) * ((g.n + 31) / 32) * batch <= 256 && g.k > 256
+                 ? launch_f32_tile<32, 32, 8, EPI, true>(g, batch, trans_a, trans_b, stream)
+                 : launch_f32_tile<32, 32, 4, EPI, true>(g, batch, trans_a, trans_b, stream);
+    case 1: return launch_f32_tile<32, 64, 4, EPI, true>(g, batch, trans_a, trans_b, stream);
+    case 2: return launch_f32_tile<64, 64, 4, EPI, true>(g, batch, trans_a, trans_b, stream);
+    default: return launch_f32_tile<64, 64, 8, EPI, true>(g, batch, trans_a, trans_b, stream);
   }
 }
 
@@ -249,12 +259,9 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
     const GemmRoute r = route_f32(g, batch, trans_a, trans_b, scratch);
     switch (r.kernel) {
       case TMB_GEMM_F32_WIDE:
-        if (r.splits == 0) return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
-        return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](GemmArgs part) {
-          part.k = g.k / r.splits;
-          part.stride_a = trans_a ? part.k * g.lda : part.k;
-          part.stride_b = trans_b ? part.k : part.k * g.ldb;
-          return launch_f32_mfma<TMB_EPI_NONE>(part, r.splits, trans_a, trans_b, stream);
+        if (r.splits == 0) return launch_f32_wide<EPI>(g, batch, trans_a, trans_b, stream);
+        return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](const GemmArgs& part) {
+          return launch_f32_wide<TMB_EPI_NONE>(part, r.splits, trans_a, trans_b, stream);
         });
       case TMB_GEMM_F32:
         if (r.splits == 0) return launch_f32_shared<EPI>(g, batch, r.tile, trans_a, trans_b, stream);
