@@ -300,6 +300,33 @@ def gemm_if_planned(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tenso
     return out
 
 
+_RESIDUAL_PLANS: dict = {}
+
+
+def _residual_plan_key(a, b, bias, residual, out_dtype, epi_flags, a_ptr, b_ptr):
+    """Everything that `gemm` looks at before it launches a product with a residual."""
+    return (a.shape, a.stride(), b.shape, b.stride(), a.dtype, b.dtype, a.device, b.device, a_ptr & 15, b_ptr & 15,
+            epi_flags, residual.shape, residual.stride(), residual.dtype, residual.device, out_dtype,
+            None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device))
+
+
+def _gemm_residual_if_planned(a, b, bias, residual, out_dtype, epi_flags):
+    """As `gemm_if_planned`, for a product that carries its residual (two of each layer's four)."""
+    a_ptr, b_ptr = a.data_ptr(), b.data_ptr()
+    plan = _RESIDUAL_PLANS.get(_residual_plan_key(a, b, bias, residual, out_dtype, epi_flags, a_ptr, b_ptr))
+    if plan is None:
+        return None
+    out_shape, dtype, dims, ws_bytes = plan
+    out = torch.empty(out_shape, dtype=dtype, device=a.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    rc = _ek.lib().tmb_gemm_residual_ws(
+        out.data_ptr(), a_ptr, b_ptr, None if bias is None else bias.data_ptr(), residual.data_ptr(), *dims,
+        None if ws is None else ws.data_ptr(), ws_bytes, _stream())
+    if rc:
+        _check("tmb_gemm_residual_ws", rc)
+    return out
+
+
 def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
          epilogue: int = _ek.EPI_NONE, residual: Optional[torch.Tensor] = None,
          out_dtype: Optional[torch.dtype] = None, round_like_unfused: bool = False) -> torch.Tensor:
@@ -325,6 +352,10 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         if out is not None:
             return out
         key = True
+    elif residual is not None:
+        out = _gemm_residual_if_planned(a, b, bias, residual, out_dtype, epi_flags)
+        if out is not None:
+            return out
     a_in, b_in, bias_in = a, b, bias
     require_hip(a, b, bias, residual)
     if a.dtype != b.dtype or a.dtype not in FLOAT_DTYPES:
@@ -407,16 +438,23 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
     if residual is not None:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
         res = residual if residual.stride(-1) == 1 and residual.stride(-2) >= n else residual.contiguous()
+        dims = (batch, m, n, k, la[1], lb[1], n, res.stride(-2),
+                a.stride(0) if batched else 0, b.stride(0) if batched else 0, m * n,
+                res.stride(0) if batched else 0,
+                la[0], lb[0], code_of(a.dtype), code_of(res.dtype), code_of(result_dtype), epi_flags)
         rc = lib.tmb_gemm_residual_ws(
             out.data_ptr(), a.data_ptr(), b.data_ptr(), None if bias is None else bias.data_ptr(),
-            res.data_ptr(), batch, m, n, k, la[1], lb[1], n, res.stride(-2),
-            a.stride(0) if batched else 0, b.stride(0) if batched else 0, m * n,
-            res.stride(0) if batched else 0,
-            la[0], lb[0], code_of(a.dtype), code_of(res.dtype), code_of(result_dtype), epi_flags,
-            None if ws is None else ws.data_ptr(), ws_bytes, _stream())
+            res.data_ptr(), *dims, None if ws is None else ws.data_ptr(), ws_bytes, _stream())
         if rc == _ek.ERR_UNSUPPORTED:
             return unfused_residual()
         _check("tmb_gemm_residual_ws", rc)
+        if a is a_in and b is b_in and bias is bias_in and res is residual and not (
+                in_place_ws is not None and a.numel() * 2 >= _PAD_REUSE_MIN_BYTES):
+            # all operands are consumed in place: remember the launch arguments for this layout
+            if len(_RESIDUAL_PLANS) >= 4096:
+                _RESIDUAL_PLANS.clear()
+            _RESIDUAL_PLANS[_residual_plan_key(a, b, bias, residual, out_dtype, epi_flags, a.data_ptr(),
+                                               b.data_ptr())] = (out_shape, result_dtype, dims, ws_bytes)
         return out
     # (an operand that a running graph would pad and share is multiplied in place outside of one only)
     shared = in_place_ws is not None and a.numel() * 2 >= _PAD_REUSE_MIN_BYTES
@@ -502,49 +540,53 @@ def softmax_scaled(x: torch.Tensor, scale: float, causal_q_len: int = 0,
 
 def attention_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """True when `attention` can take these [batch, heads, tokens, 64] tensors as they are."""
+    dtype = q.dtype
     if not (q.is_cuda and k.is_cuda and v.is_cuda):
         return False
-    if q.dtype not in (torch.bfloat16, torch.float16) or k.dtype != q.dtype or v.dtype != q.dtype:
+    if dtype not in (torch.bfloat16, torch.float16) or k.dtype != dtype or v.dtype != dtype:
         return False
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         return False
-    b, h, t, d = q.shape
-    if d != 64 or tuple(k.shape) != (b, h, k.shape[2], 64) or tuple(v.shape) != tuple(k.shape):
+    (b, h, t, d), k_shape = q.shape, k.shape
+    s_len = k_shape[2]
+    if d != 64 or k_shape != (b, h, s_len, 64) or v.shape != k_shape:
         return False
-    if k.shape[2] == 0 or b * h * ((t + 127) // 128) >= 1 << 31 or b * h * t == 0:
+    if s_len == 0 or b * h * ((t + 127) // 128) >= 1 << 31 or b * h * t == 0:
         return False
-    for x in (q, k, v):
-        if x.stride(3) != 1 or any(s % 8 or s < 0 for s in x.stride()[:3]) or x.data_ptr() % 16:
+    for x, tokens in ((q, t), (k, s_len), (v, s_len)):
+        s0, s1, s2, s3 = x.stride()
+        if s3 != 1 or s0 % 8 or s1 % 8 or s2 % 8 or s0 < 0 or s1 < 0 or s2 < 0 or x.data_ptr() % 16:
             return False
-        if (x.shape[2] * x.stride(2) + 64) * 2 >= 1 << 32:
+        if (tokens * s2 + 64) * 2 >= 1 << 32:
             return False
     return True
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, causal: bool,
               round_like_unfused: bool = False, return_lse: bool = False,
-              like_query: bool = False):
+              like_query: bool = False, checked: bool = False):
     """softmax(scale * q k^T [causal]) v for [batch, heads, tokens, 64] tensors (any strides
     `attention_supported` accepts). Returns a [batch, q_len, heads, 64] contiguous tensor, i.e.
     the layout `y.transpose(1, 2).contiguous()` would have produced; with `like_query` a
     [batch, heads, q_len, 64] tensor laid out as `torch.empty_like(q)` (what ATen's fused attention
     ops return). With `return_lse` also the float32 [batch, heads, q_len] log-sum-exp of every
-    query's scores, which `attention_backward` needs."""
-    require_hip(q, k, v)
+    query's scores, which `attention_backward` needs. `checked`: the caller has just seen `attention_supported`
+    accept exactly these operands."""
+    if not checked:
+        require_hip(q, k, v)
     if not (scale > 0.0 and math.isfinite(scale)):
         raise ValueError(f"attention: scale must be positive and finite, got {scale}")
-    if not attention_supported(q, k, v):
+    if not checked and not attention_supported(q, k, v):
         raise ValueError(f"attention: unsupported operands q{tuple(q.shape)} {q.dtype} "
                          f"strides {q.stride()} / k{tuple(k.shape)} / v{tuple(v.shape)}")
     b, h, t, d = q.shape
-    i64x3 = ctypes.c_int64 * 3
-    strides = [i64x3(x.stride(0), x.stride(1), x.stride(2)) for x in (q, k, v)]
+    strides = [_I64X3(*x.stride()[:3]) for x in (q, k, v)]
     if like_query:
         out = _gradient_like(q)
-        o_str = i64x3(out.stride(0), out.stride(1), out.stride(2))
+        o_str = _I64X3(*out.stride()[:3])
     else:
         out = torch.empty((b, t, h, d), dtype=q.dtype, device=q.device)
-        o_str = i64x3(out.stride(0), out.stride(2), out.stride(1))
+        o_str = _I64X3(t * h * d, d, h * d)
     lse = torch.empty((b, h, t), dtype=torch.float32, device=q.device) if return_lse else None
     rc = _ek.lib().tmb_attention_fwd(out.data_ptr(), lse.data_ptr() if return_lse else None,
                                      q.data_ptr(), k.data_ptr(), v.data_ptr(),

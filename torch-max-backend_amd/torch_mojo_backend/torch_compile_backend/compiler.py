@@ -1122,7 +1122,7 @@ def _fused_attention(q, k, v, scale, root, slices):
     s_len = k.shape[2]
     if scale > 0 and hip_ops.attention_supported(q, k, v) and \
             _causal_q_len(root, slices, (t, s_len), check=False) == t:
-        return hip_ops.attention(q, k, v, scale, True)
+        return hip_ops.attention(q, k, v, scale, True, checked=True)
     # the unfused chain, op by op as the graph had it
     flat = lambda x: x.expand(x.shape).clone(memory_format=torch.contiguous_format).view(  # noqa: E731
         b * h, x.shape[2], x.shape[3])
