@@ -88,3 +88,13 @@ def test_infinities_and_nan(mnk):
     columns = torch.ones(n, dtype=torch.bool)
     columns[5] = False
     _check(got[rows][:, columns], a[rows], b[:, columns])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(750, 768, 3072), (385, 770, 8201), (1408, 2304, 768)])
+def test_a_residual_has_the_bits_of_product_and_sum(mnk):
+    """Carried by the reduction of a split launch, added by the caller otherwise."""
+    m, n, k = mnk
+    a, b, bias = _operand(m, k, False, 7), _operand(k, n, True, 8), torch.randn(n, device="cuda")
+    r = _operand(m, n, False, 9)
+    assert torch.equal(_ops().gemm(a, b, bias, residual=r), _ops().gemm(a, b, bias) + r)

@@ -441,16 +441,18 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
   return {TMB_GEMM_SIMT, 0, 0};
 }
 
-// A residual is carried where the product alone runs on the kernel whose waves share K, and added by the caller where it
-// does not: the sum has the bits of the two operations, and carrying it saves next to nothing on the others (2 us a
-// million elements there, as much as the add).
+// A residual is carried where the product alone runs on the kernel whose waves share K or on a split launch, whose
+// reduction adds it, and added by the caller where it does not: the sum has the bits of the two operations, and carrying it
+// saves next to nothing on the others (2 us a million elements there, as much as the add).
 static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a, int trans_b,
                                   size_t workspace_bytes) {
   if (g.residual != nullptr) {
     GemmArgs alone = g;
     alone.residual = nullptr;
     const GemmRoute r = route_f32(alone, batch, trans_a, trans_b, workspace_bytes);
-    return r.kernel == TMB_GEMM_F32 ? r : GemmRoute{TMB_ERR_UNSUPPORTED, 0, 0};
+    const bool carried = r.kernel == TMB_GEMM_F32 ||
+                         (r.kernel == TMB_GEMM_F32_WIDE && r.splits > 0 && f32_shared_eligible(g, trans_a, trans_b));
+    return carried ? r : GemmRoute{TMB_ERR_UNSUPPORTED, 0, 0};
   }
   const bool shared = f32_shared_eligible(g, trans_a, trans_b);
   const bool aligned = f32_mfma_eligible(g, batch, trans_a, trans_b);
