@@ -1,10 +1,10 @@
 // fp32 GEMM on the bf16 matrix cores, for products of many tiles: each fp32 operand element is three bf16
 // (F32Split, gemm_f32.h) and a product is the six of their nine products that reach fp32 accuracy.
 //
-// One workgroup of 2 x 4 waves owns a 128 x 128 tile of C, each wave a 64 x 32 part, and walks K in stages of 32. The workgroup splits each element once, on its way into LDS: stage s + 2
-// travels from global memory into registers while stage s + 1 is taken apart and laid down in one LDS buffer
-// and stage s is multiplied out of the other; one barrier closes the stage. The vector units that
-// do the splitting are the second bound after the matrix cores (five vector instructions hide behind a
+// One workgroup of 2 x 4 waves owns a 128 x 128 tile of C, each wave a 64 x 32 part, and walks K in stages of 32. The
+// workgroup splits each element once, on its way into LDS: stage s + 2 travels from global memory into registers while
+// stage s + 1 is taken apart and laid down in one LDS buffer and stage s is multiplied out of the other; one barrier
+// closes the stage. The vector units that do the splitting are the second bound after the matrix cores (five vector instructions hide behind a
 // 32 x 32 x 16 MFMA, two behind a 16 x 16 x 32 one; measured), hence the large tile and the large MFMA.
 //
 // 4096^3 1110 -> 775 us (177 TFLOP/s: 1060 of bf16 products, where the clock falls to what the matrix cores' power leaves),
