@@ -1,16 +1,20 @@
 // fp32 GEMM on the bf16 matrix cores, any of the four operand layouts, any extents and any row pitch.
 //
 // An fp32 MFMA takes 64 cycles for what a bf16 one does in four. So each operand element is taken apart into three bf16
-// whose sum it is, exactly (F32Pair), and a product is the six of the nine partial products that are above 2^-24 of it,
-// added up in fp32 by v_mfma_f32_16x16x32_bf16: 16 cycles of matrix core instead of 64, and the rounding of a sum once in
-// 32 k instead of at every k. Against 64 bits the results are off by 0.2 .. 0.8 of what fp32 MFMAs (v_mfma_f32_32x32x2)
-// gave, over K 64 .. 50257. 1332 x 768 x 3072 68 -> 51 us, 750 x 3072 x 768 47 -> 36, 4096^3 1110 -> 775 (gemm_f32_wide.h).
+// whose sum it is, exactly (F32Pair), and a product is eight of the nine partial products, all but the one below 2^-33 of
+// it, added up in fp32 by v_mfma_f32_16x16x32_bf16: 21 cycles of matrix core for 64. The large partial products and the
+// small ones are summed apart and joined by a rounded addition: a product that stands alone is off by 1.01 half units at
+// most (with the small ones in one chain, 3.8: the MFMA aligns addends to the largest and cuts), and a sum is rounded once
+// in 32 k instead of at every k. Against fp32 MFMAs the error of dense operands is 0.1 .. 1.0 of what it was over K 129 ..
+// 50257, of rows with a single term the same, of rows with 4 .. 16 terms 0.6 .. 1.2 (each product is rounded before it is
+// added, and the order of the sum is another); operands of exponents 2^-20 .. 2^20 0.3 .. 1.03.
+// 1332 x 768 x 3072 68 -> 57 us, 1332 x 3072 x 768 70 -> 58, 750 x 2304 x 768 36 -> 29.
 //
 // A workgroup owns a BM x BN tile of C and its WAVES waves share K: wave w multiplies the 32-deep
 // slices w, w + WAVES, ... of the whole tile and the partial tiles meet in LDS once, at the end, where
 // they are added pairwise in wave order (the result depends on the shape only): no workgroup barrier in the main loop,
 // and tiles small enough to give every CU the same amount. What bounds it is the vector units, which take the operands
-// apart (44 instructions for a fragment of 16 rows, of which two hide behind an MFMA), then the matrix cores.
+// apart (44 instructions for a fragment of 16 rows, of which two hide behind an MFMA), and the matrix cores.
 //
 // A wave brings a slice in through registers (the next slice travels while this one is multiplied) and
 // a wave-private part of LDS, which works in order per wave; a lane of a fragment takes eight consecutive k of a row.
@@ -207,9 +211,9 @@ struct F32Slice<32, false> {
   }
 };
 
-// Two fp32 values, times 2^16, as three bf16 each: x = h + m + l with |m| <= 2^-8 |x|, |l| <= 2^-16 |x|. Exact: 24 bits of
-// significand in three times eight, and 2^16 times the smallest fp32 number is the smallest bf16 one. (h is rounded to
-// nearest; what it leaves has at most sixteen bits, which m and l take without rounding.)
+// Two fp32 values, times 2^16, as three bf16 each: x = h + m + l with |m| <= 2^-8 |x|, |l| <= 2^-17 |x|. Exact: 24 bits of
+// significand in three times eight, and 2^16 times the smallest fp32 number is the smallest bf16 one. (h and m are rounded
+// to nearest; what h leaves has at most sixteen bits, what m leaves of those at most seven.)
 struct F32Pair {
   uint32_t h, m, l;
   static constexpr float kUp = 0x1p16f, kDown = 0x1p-16f;  // each operand's factor, and what undoes it
@@ -220,10 +224,9 @@ struct F32Pair {
     r.h = pack2<bf16_t>(a, b);
     a -= __builtin_bit_cast(float, r.h << 16);
     b -= __builtin_bit_cast(float, r.h & 0xffff0000u);
-    const uint32_t ma = __builtin_bit_cast(uint32_t, a), mb = __builtin_bit_cast(uint32_t, b);
-    r.m = __builtin_amdgcn_perm(mb, ma, 0x07060302u);
-    a -= __builtin_bit_cast(float, ma & 0xffff0000u);
-    b -= __builtin_bit_cast(float, mb & 0xffff0000u);
+    r.m = pack2<bf16_t>(a, b);
+    a -= __builtin_bit_cast(float, r.m << 16);
+    b -= __builtin_bit_cast(float, r.m & 0xffff0000u);
     r.l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x07060302u);
     return r;
   }
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) v
       if (s + WAVES < slices) load(s + WAVES);
       if constexpr (decltype(as_bf16)::value) {
         F32Split af[TM], bf[2];
-        f32x4v_t t[TM];
+        f32x4v_t t[TM], u[TM];  // the small products' sums, the large ones'
         f32x4_t x[2];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) v
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) acc[i][j - 1][e] += t[i][e];
+              for (int e = 0; e < 4; ++e) acc[i][j - 1][e] += u[i][e] + t[i][e];
           }
           if (j + 1 < TN) {
             SliceB::fragment(lb, (j + 1) * 16 + lr, lq, x);
@@ -321,7 +324,11 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) v
           }
           const F32Split& b = bf[j & 1];
 #pragma unroll
-          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.l, af[i].h, f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f});
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.l, af[i].m, f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.m, af[i].l, t[i]);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.l, af[i].h, t[i]);
 #pragma unroll
           for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].l, t[i]);
 #pragma unroll
@@ -331,24 +338,19 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) v
 #pragma unroll
           for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].m, t[i]);
 #pragma unroll
-          for (int i = 0; i < TM; ++i) t[i] = Mfma16<bf16_t>::run(b.h, af[i].h, t[i]);
+          for (int i = 0; i < TM; ++i) u[i] = Mfma16<bf16_t>::run(b.h, af[i].h, f32x4v_t{0.0f, 0.0f, 0.0f, 0.0f});
           __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // LDS reads
 #pragma unroll
-          for (int i = 0; i < TM; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // vector ALU
+          for (int i = 0; i < 8 * TM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // vector ALU
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-          }
-#pragma unroll
-          for (int i = 0; i < 5 * TM; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][TN - 1][e] += t[i][e];
+          for (int e = 0; e < 4; ++e) acc[i][TN - 1][e] += u[i][e] + t[i][e];
       } else {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {

@@ -1,5 +1,5 @@
 // fp32 GEMM on the bf16 matrix cores, for products of many tiles: each fp32 operand element is three bf16
-// (F32Split, gemm_f32.h) and a product is the six of their nine products that reach fp32 accuracy.
+// (F32Pair, gemm_f32.h) and a product is eight of their nine products.
 //
 // One workgroup of 2 x 4 waves owns a 128 x 128 tile of C, each wave a 64 x 32 part, and walks K in stages of 32. The
 // workgroup splits each element once, on its way into LDS: stage s + 2 travels from global memory into registers while
@@ -7,8 +7,8 @@
 // closes the stage. The vector units that do the splitting are the second bound after the matrix cores (five vector instructions hide behind a
 // 32 x 32 x 16 MFMA, two behind a 16 x 16 x 32 one; measured), hence the large tile and the large MFMA.
 //
-// 4096^3 1110 -> 775 us (177 TFLOP/s: 1060 of bf16 products, where the clock falls to what the matrix cores' power leaves),
-// 750 x 50257 x 768 520 -> 391, 2048^3 169 -> 100, each against fp32 MFMAs.
+// 4096^3 890 us (154 TFLOP/s: 1230 of bf16 products, where the clock falls to what the matrix cores' power leaves), 2048^3
+// 117, 1332 x 50257 x 768 820; fp32 MFMAs took 1110, 169 and 870.
 //
 // LDS: three planes (high, middle, low parts) of four chunks of eight k; a chunk holds 16 bytes per row, so that both the
 // fragment reads (32 rows of one chunk per half wave) and the eight-byte stores run without bank conflicts.
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
   StagedB sb;
   sa.plan(A, g.lda, M - m0, wave, lane);
   sb.plan(B, g.ldb, N - n0, wave, lane);
-  f32x16_t acc[TM], t[TM];
+  f32x16_t acc[TM], t[TM], u[TM];  // the sum; a run of stages' small products, and its large ones
 
   auto close_stage = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   u32x4_t a[2][TM][3], b[2][3];
@@ -150,30 +150,33 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
       for (int i = 0; i < TM; ++i) read_a(stage, 0, i, part);
     }
   };
-  // A stage's products, added to t; one stage's or, where there are 64 and more, four stages' are joined to the sum in
-  // one addition per element: the sum is rounded once in 32 or 128 k (the errors of both levels add up: K = 64 wants
-  // the former, K = 4096 is off by half as much with the latter). A step is two MFMAs, the reading of a fragment that comes later and a share of
+  // A stage's products, added to u (high part times high part) and t (the others, 2^-8 and less of them: in a sum of
+  // their own their bits are not lost to the MFMA's alignment, and a single product is rounded once). A run of stages'
+  // u + t is joined to the sum in one addition per element; runs of about the square root of the stages make the errors of
+  // the two levels least (K = 768, positive operands: 5.0e-8, joined every stage 7.6e-8; K = 6000 7.9e-8 against 1.06e-7
+  // in runs of four). A step is two MFMAs, the reading of a fragment that comes later and a share of
   // the next stage's splitting; nothing moves between steps, so that the vector instructions stand behind the MFMAs.
   // The barrier that closes the stage is in front of the last steps, which hide the reading of the next stage's first
   // fragments: by then every wave has read all it needs of this stage and laid down its part of the next.
   auto multiply = [&](const unsigned char* cur, unsigned char* next, int64_t k_after, auto splits_next) {
     constexpr bool NEXT = decltype(splits_next)::value;
-    constexpr int STEPS = 12, CLOSE = STEPS - 3, PAIRS = 2 * (StagedA::ITEMS + StagedB::ITEMS);
+    constexpr int TERMS = 8, STEPS = 2 * TERMS, CLOSE = STEPS - 3, PAIRS = 2 * (StagedA::ITEMS + StagedB::ITEMS);
     static_assert(PAIRS < CLOSE, "laid down before the barrier");
-    constexpr int kPartA[6] = {0, 2, 1, 0, 1, 0}, kPartB[6] = {2, 0, 1, 1, 0, 0};  // (smallest terms first)
+    constexpr int kPartA[TERMS] = {1, 2, 0, 2, 1, 0, 1, 0}, kPartB[TERMS] = {2, 1, 2, 0, 1, 1, 0, 0};  // (smallest first)
     u32x2_t h, m, l;
 #pragma unroll
     for (int step = 0; step < STEPS; ++step) {
-      const int half = step / 6, term = step % 6;
+      const int half = step / TERMS, term = step % TERMS;
       if (NEXT && step == CLOSE) {
         close_stage();
         read_first_half(next);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        t[i] = Mfma<bf16_t>::run(b[half][kPartB[term]], a[half][i][kPartA[term]], t[i]);
+        f32x16_t& sum = term == TERMS - 1 ? u[i] : t[i];
+        sum = Mfma<bf16_t>::run(b[half][kPartB[term]], a[half][i][kPartA[term]], sum);
       }
-      if (half == 0) {
+      if (half == 0 && term < 6) {
         if (term < 3) read_b(cur, 1, 2 - term);
         read_a(cur, 1, term & 1, term >> 1);
       }
@@ -199,15 +202,15 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        acc[i][e] += t[i][e];
-        t[i][e] = 0.0f;
+        acc[i][e] += u[i][e] + t[i][e];
+        t[i][e] = u[i][e] = 0.0f;
       }
   };
 
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[i][e] = t[i][e] = 0.0f;
+    for (int e = 0; e < 16; ++e) acc[i][e] = t[i][e] = u[i][e] = 0.0f;
   if (first < last) {
     sa.load_stage(first * 32, K);
     sb.load_stage(first * 32, K);
@@ -219,7 +222,8 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
     }
     close_stage();
     read_first_half(f32_wide_lds);
-    const int joint = last - first >= 64 ? 3 : 0;
+    int run = 1;
+    while (run < 16 && 4 * run * run <= last - first) run *= 2;
     int buffer = 0;
     for (int64_t s = first; s + 1 < last; ++s) {
       // (an element's register is loaded again as soon as it has been taken apart: a stage's time for the way from
@@ -231,7 +235,7 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
         sa.load_stage((s + 2) * 32, K);
         sb.load_stage((s + 2) * 32, K);
       }
-      if (((s - first) & joint) == joint) join();
+      if (((s - first) & (run - 1)) == run - 1) join();
       buffer ^= 1;
     }
     multiply(f32_wide_lds + buffer * STAGE, nullptr, 0, std::false_type{});
