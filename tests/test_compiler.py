@@ -741,3 +741,44 @@ def test_layer_norm_backward_takes_the_residual_gradient_and_the_bias_sums_along
             torch.testing.assert_close(g, w, rtol=1e-5, atol=1e-6)
     # the four joins ran inside the fused steps' host route, the four bias sums as well
     assert calls.count("ln_bwd") == 5
+
+
+_FLOATS = torch.arange(24.0).view(4, 6)
+_NAMED = torch.zeros(2, 3).refine_names("a", "b")
+
+
+@pytest.mark.parametrize("name,args", [
+    ("view", (_FLOATS, 6, 4)), ("view", (_FLOATS, 24)), ("view", (_FLOATS, [6, 4])), ("view", (_FLOATS, (6, 4))),
+    ("view", (_FLOATS, torch.int32)), ("view", (_FLOATS, [True, 24])), ("view", (_FLOATS, range(24, 25))),
+    ("view", (_FLOATS, [2.0, 12])), ("view", (_FLOATS, [5, 5])), ("view", (_FLOATS,)), ("view", (None, [1])),
+    ("transpose", (_FLOATS, 0, -1)), ("transpose", (_FLOATS, 0, 2)), ("transpose", (_FLOATS, True, 0)),
+    ("transpose", (_FLOATS, "a", "b")), ("transpose", (_NAMED, "a", "b")), ("transpose", (_NAMED, 0, 1)),
+    ("transpose", (_FLOATS, 0)), ("t", (_FLOATS,)), ("t", (_NAMED,)), ("t", (_FLOATS, 1)), ("t", (_FLOATS[None],))])
+def test_registry_views_take_and_refuse_what_their_operators_do(name, args):
+    op = {"view": torch.ops.aten.view, "transpose": torch.ops.aten.transpose, "t": torch.ops.aten.t.default}[name]
+
+    def answer(fn):
+        try:
+            out = fn(*args)
+            return out.shape, out.dtype, out.stride()
+        except Exception as refused:  # noqa: BLE001 - which one is what is compared
+            return type(refused)
+
+    assert answer(compiler.MAPPING_TORCH_ATEN_TO_MOJO[op]) == answer(op)
+
+
+def test_view_steps_call_the_method_in_the_form_of_the_schema_only(monkeypatch):
+    from torch_mojo_backend import is_running_tests
+
+    monkeypatch.setattr(is_running_tests, "IS_RUNNING_TESTS", False)
+    aten, graph = torch.ops.aten, torch.fx.Graph()
+    x = graph.placeholder("x")
+    viewed = graph.call_function(aten.view.default, (x, [6, 4]))
+    turned = graph.call_function(aten.transpose.int, (viewed, 0, 1))
+    flat = graph.call_function(aten.t.default, (turned,))
+    bits = graph.call_function(aten.view.dtype, (flat, torch.int32))
+    graph.output((bits,))
+    graph.owning_module = torch.nn.Module()
+    steps = compiler._GraphFactory().create_graph(graph).steps
+    assert [s.fn for s in steps[:3]] == [torch.Tensor.view, torch.Tensor.transpose, torch.Tensor.t]
+    assert steps[3].fn is compiler.MAPPING_TORCH_ATEN_TO_MOJO[aten.view]

@@ -519,23 +519,29 @@ def _passthrough(op):
     return run
 
 
-# Every second step of a transformer's graph is one of these; the tensor's own method does the same without
-# the operator packet's search for an overload (1.3 .. 1.6 us a call against 0.4 .. 0.6).
-_METHODS = {"view": torch.Tensor.view, "transpose": torch.Tensor.transpose, "t.default": torch.Tensor.t}
-
-
-def _passthrough_method(op, method):
-    def run(*args, **kwargs):
-        return op(*args, **kwargs) if kwargs else method(*args)
-
-    run.__name__ = run.__qualname__ = _passthrough(op).__name__
-    return run
-
-
 for _name in _PASSTHROUGH:
     _op = _resolve(_name)
     if _op is not None and _op not in MAPPING_TORCH_ATEN_TO_MOJO:
-        map_to(_op)(_passthrough_method(_op, _METHODS[_name]) if _name in _METHODS else _passthrough(_op))
+        map_to(_op)(_passthrough(_op))
+
+# Every second step of a transformer's graph is one of these; a step whose arguments are the schema's own calls the
+# tensor's method, which does the same without the operator packet's search for an overload (1.3 .. 1.6 us a call against
+# 0.4 .. 0.6). Not the registry: the methods also take what the operators refuse (sizes one by one, names of dimensions).
+_BUILTIN_VIEW, _BUILTIN_TRANSPOSE, _BUILTIN_T = (MAPPING_TORCH_ATEN_TO_MOJO[_op]
+                                                 for _op in (aten.view, aten.transpose, aten.t.default))
+
+
+def graph_step_function(fn, args, kwargs):
+    """What a step that computes `fn(*args, **kwargs)` calls (`args` as in the graph: nodes, sizes, dimensions)."""
+    if kwargs or torch_mojo_backend.is_running_tests.IS_RUNNING_TESTS:   # (where calls are counted)
+        return fn
+    if fn is _BUILTIN_VIEW and len(args) == 2 and isinstance(args[1], list):
+        return torch.Tensor.view
+    if fn is _BUILTIN_TRANSPOSE and len(args) == 3 and all(type(dim) is int for dim in args[1:]):
+        return torch.Tensor.transpose
+    if fn is _BUILTIN_T and len(args) == 1:
+        return torch.Tensor.t
+    return fn
 
 if verbose_enabled():
     print(f"Removed {number_of_decompositions_removed}/{original_decomposition_table_size} decompositions.")

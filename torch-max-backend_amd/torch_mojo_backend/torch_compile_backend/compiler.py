@@ -848,6 +848,7 @@ class _GraphFactory:
                 if self.run_device is not None and isinstance(kwargs.get("device"), torch.device) \
                         and kwargs["device"].type in ("cpu", "mojo"):
                     kwargs["device"] = self.run_device
+                fn = aten_functions.graph_step_function(fn, args, kwargs)
                 if fn is _skipped:
                     # no step at all: a fused step later does this node's work
                     self.slots[node.name] = len(self.slots)
