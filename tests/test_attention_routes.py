@@ -161,3 +161,16 @@ def test_a_few_queries_take_the_decode_kernel_where_it_is_the_faster_one(recorde
         assert _took(recorded) == ["tmb_attention_fwd"] and not theirs
     else:
         assert theirs == [1] and _took(recorded) == []
+
+
+@pytest.mark.parametrize("devices", [("cuda:0", "cuda:1", "cuda:0"), ("cuda:0", "cuda:0", "cuda:1"),
+                                     ("cuda:1", "cuda:0", "cuda:0")])
+@pytest.mark.parametrize("checked", [False, True])
+def test_attention_refuses_operands_on_two_devices(devices, checked):
+    """Also where the caller has checked their layout (`attention_supported` looks at each operand by itself): a launch
+    would read another device's memory."""
+    from torch_mojo_backend.eager_kernels import hip_ops
+
+    q, k, v = (types.SimpleNamespace(device=torch.device(d)) for d in devices)
+    with pytest.raises(TypeError, match="different devices"):
+        hip_ops.attention(q, k, v, 0.125, True, checked=checked)

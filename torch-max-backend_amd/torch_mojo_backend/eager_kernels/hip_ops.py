@@ -571,8 +571,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, c
     [batch, heads, q_len, 64] tensor laid out as `torch.empty_like(q)` (what ATen's fused attention
     ops return). With `return_lse` also the float32 [batch, heads, q_len] log-sum-exp of every
     query's scores, which `attention_backward` needs. `checked`: the caller has just seen `attention_supported`
-    accept exactly these operands."""
-    if not checked:
+    accept exactly these operands (which need not lie on one device for that)."""
+    if not checked or k.device != q.device or v.device != q.device:
         require_hip(q, k, v)
     if not (scale > 0.0 and math.isfinite(scale)):
         raise ValueError(f"attention: scale must be positive and finite, got {scale}")
