@@ -131,6 +131,68 @@ def test_infinities_and_nan(mnk):
     _check(got[rows][:, columns], a[rows], b[:, columns])
 
 
+def _spoil(a, b):
+    """Infinities and a NaN in three rows of a, an infinity and a number without room for the factor in two columns of b
+    (2^120: its products, below 2^123 for normal operands, and their sums are finite in float32 too); what is left of rows
+    and columns."""
+    m, k, n = a.shape[-2], a.shape[-1], b.shape[-1]
+    a[..., 3, 7], a[..., m - 2, 0], a[..., m // 2, k - 1] = float("inf"), float("nan"), float("-inf")
+    b[..., k // 2, 5], b[..., k - 2, n - 1] = float("inf"), 2.0 ** 120
+    rows, columns = torch.ones(m, dtype=torch.bool), torch.ones(n, dtype=torch.bool)
+    rows[[3, m - 2, m // 2]] = False
+    columns[[5, n - 1]] = False
+    return rows, columns
+
+
+def _check_spoiled(a, b):
+    clean = _ops().gemm(a, b)
+    rows, columns = _spoil(a, b)
+    got, exact = _ops().gemm(a, b), a.double() @ b.double().contiguous()
+    assert torch.equal(got.isnan(), exact.isnan()) and torch.equal(got.isinf(), exact.isinf())
+    assert torch.equal(got[got.isinf()], exact[exact.isinf()].float())
+    assert torch.equal(got[..., rows, :][..., columns], clean[..., rows, :][..., columns])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", WIDE + SHARED)
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_rows_and_columns_do_not_change_with_what_their_neighbours_hold(mnk, trans_a, trans_b):
+    """Infinities and NaN spread as in the float64 product, whatever the layout and alignment, and rows and columns
+    without them keep their bits."""
+    m, n, k = mnk
+    for offset in (0, 1):
+        _check_spoiled(_operand(m, k, trans_a, 16, offset), _operand(k, n, trans_b, 17, offset))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(3, 700, 1100, 260), (5, 130, 70, 201)])
+def test_batches_do_not_change_with_what_their_neighbours_hold(shape):
+    batch, m, n, k = shape
+    a = torch.stack([_operand(m, k, False, 18 + i) for i in range(batch)])
+    b = torch.stack([_operand(k, n, False, 28 + i) for i in range(batch)])
+    clean = _ops().gemm(a, b)
+    _spoil(a[1], b[1])
+    got = _ops().gemm(a, b)
+    assert torch.equal(got[0], clean[0]) and torch.equal(got[2:], clean[2:])
+    _check_spoiled(a[2:3].clone(), b[2:3].clone())
+    assert torch.equal(_ops().gemm(a[1:2], b[1:2]).isnan(), got[1:2].isnan())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mnk", [(1408, 2304, 768), (300, 500, 300), (64, 128, 2000)])
+def test_results_beyond_the_factors_room_leave_their_neighbours_alone(mnk):
+    """Finite rows of 2^100, whose sums the split has no room for: as exact as any, and other rows keep their bits."""
+    m, n, k = mnk
+    a, b = _operand(m, k, False, 19), _operand(k, n, True, 20)
+    clean = _ops().gemm(a, b)
+    a[5] *= 2.0 ** 100
+    got = _ops().gemm(a, b)
+    _check(got, a, b)
+    others = [r for r in range(m) if r != 5]
+    assert torch.equal(got[others], clean[others])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("mnk", [(750, 768, 3072), (385, 770, 8201), (1408, 2304, 768)])
 def test_a_residual_has_the_bits_of_product_and_sum(mnk):

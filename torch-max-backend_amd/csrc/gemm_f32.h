@@ -370,78 +370,91 @@ __global__ __launch_bounds__(WAVES * 64, BM * BN <= 4096 && WAVES < 8 ? 2 : 1) v
     }
   };
   multiply(std::integral_constant<bool, SPLIT>{});
-  float down = 1.0f;
-  if constexpr (SPLIT) {
-    // A sum that is not finite (an operand or a result that is not, or one beyond what the operands' factor leaves room
-    // for) sends the workgroup through its tile again with fp32 products.
-    __shared__ int wave_non_finite[WAVES];
-    float probe = 0.0f;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) probe = __builtin_fmaf(acc[i][j][e], 0.0f, probe);
-    const uint64_t spoiled = __ballot(probe != 0.0f);
-    if (lane == 0) wave_non_finite[wave] = spoiled != 0;
-    __syncthreads();
-    bool again = false;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) again |= wave_non_finite[w] != 0;
-    if (again) multiply(std::false_type{});
-    else down = F32Pair::kDown;  // once per wave, once for their sum: it is rounded once among subnormals, and stays in range
-  }
   __syncthreads();  // the partial tiles overlay the slices
 
-  // Lane holds row lr of each 16 x 16 result and columns 4 * lq + {0..3}.
-  float* part = f32_lds + wave * (BM * RP);
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      *reinterpret_cast<f32x4_t*>(part + (i * 16 + lr) * RP + j * 16 + 4 * lq) =
-          f32x4_t{acc[i][j][0] * down, acc[i][j][1] * down, acc[i][j][2] * down, acc[i][j][3] * down};
-  __syncthreads();
   const float* __restrict__ bias = static_cast<const float*>(g.bias);
   const float* __restrict__ resid = g.residual == nullptr
                                         ? nullptr
                                         : static_cast<const float*>(g.residual) + batch * g.stride_r;
   float* __restrict__ C = static_cast<float*>(g.c) + (batch + split) * g.stride_c;
+  uint32_t spoiled = 0;  // this thread's elements whose split sum is not finite
+  // Joins the partial tiles and stores what is finite, or (AGAIN) what was not. `down`: what undoes the operands' factors,
+  // once per wave and once for their sum: it is rounded once among subnormals, and stays in range.
+  auto join = [&](auto again, float down) {
+    constexpr bool AGAIN = decltype(again)::value;
+    // Lane holds row lr of each 16 x 16 result and columns 4 * lq + {0..3}.
+    float* part = f32_lds + wave * (BM * RP);
 #pragma unroll
-  for (int p = 0; p < (BM * BN / 4 + WAVES * 64 - 1) / (WAVES * 64); ++p) {
-    const int idx = p * WAVES * 64 + tid;
-    if ((BM * BN / 4) % (WAVES * 64) != 0 && idx >= BM * BN / 4) break;
-    const int r = idx / (BN / 4), c = (idx % (BN / 4)) * 4;
-    const int64_t row = m0 + r, col = n0 + c;
-    if (row >= M || col >= N) continue;
-    f32x4_t v[WAVES];
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) v[w] = *reinterpret_cast<const f32x4_t*>(f32_lds + w * (BM * RP) + r * RP + c);
+      for (int j = 0; j < TN; ++j)
+        *reinterpret_cast<f32x4_t*>(part + (i * 16 + lr) * RP + j * 16 + 4 * lq) =
+            f32x4_t{acc[i][j][0] * down, acc[i][j][1] * down, acc[i][j][2] * down, acc[i][j][3] * down};
+    __syncthreads();
 #pragma unroll
-    for (int step = 1; step < WAVES; step *= 2)
+    for (int p = 0; p < (BM * BN / 4 + WAVES * 64 - 1) / (WAVES * 64); ++p) {
+      const int idx = p * WAVES * 64 + tid;
+      if ((BM * BN / 4) % (WAVES * 64) != 0 && idx >= BM * BN / 4) break;
+      const int r = idx / (BN / 4), c = (idx % (BN / 4)) * 4;
+      const int64_t row = m0 + r, col = n0 + c;
+      if (row >= M || col >= N) continue;
+      f32x4_t v[WAVES];
 #pragma unroll
-      for (int w = 0; w < WAVES; w += 2 * step)
+      for (int w = 0; w < WAVES; ++w) v[w] = *reinterpret_cast<const f32x4_t*>(f32_lds + w * (BM * RP) + r * RP + c);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[w][e] += v[w + step][e];
-    const bool whole = col + 4 <= N;
-    float out[4];
+      for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x = v[0][e] * down;
-      if (bias != nullptr && (whole || col + e < N)) x += bias[col + e];
-      x = finish<float, EPI>(x, false);
-      if (resid != nullptr && (whole || col + e < N)) x += resid[row * g.ldr + col + e];
-      out[e] = x;
+        for (int w = 0; w < WAVES; w += 2 * step)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[w][e] += v[w + step][e];
+      const bool whole = col + 4 <= N;
+      uint32_t mine = 15;
+      if constexpr (SPLIT) {
+        if constexpr (AGAIN) {
+          mine = spoiled >> (4 * p) & 15;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mine &= ~((__builtin_fabsf(v[0][e]) < HUGE_VALF ? 0u : 1u) << e);
+          spoiled |= (mine ^ 15) << (4 * p);
+        }
+      }
+      float out[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x = v[0][e] * down;
+        if (bias != nullptr && (whole || col + e < N)) x += bias[col + e];
+        x = finish<float, EPI>(x, false);
+        if (resid != nullptr && (whole || col + e < N)) x += resid[row * g.ldr + col + e];
+        out[e] = x;
+      }
+      float* dst = C + row * g.ldc + col;
+      if (whole && mine == 15) {
+        const f32x4_unaligned_t o = {out[0], out[1], out[2], out[3]};
+        if (g.stream_c) __builtin_nontemporal_store(o, reinterpret_cast<f32x4_unaligned_t*>(dst));
+        else *reinterpret_cast<f32x4_unaligned_t*>(dst) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + e < N && (mine >> e & 1) != 0) dst[e] = out[e];
+      }
     }
-    float* dst = C + row * g.ldc + col;
-    if (whole) {
-      const f32x4_unaligned_t o = {out[0], out[1], out[2], out[3]};
-      if (g.stream_c) __builtin_nontemporal_store(o, reinterpret_cast<f32x4_unaligned_t*>(dst));
-      else *reinterpret_cast<f32x4_unaligned_t*>(dst) = o;
-    } else {
+  };
+  join(std::false_type{}, SPLIT ? F32Pair::kDown : 1.0f);
+  if constexpr (SPLIT) {
+    // An element whose sum is not finite (an operand or the result is not, or is beyond what the operands' factor leaves
+    // room for) is formed again from fp32 products; its neighbours keep theirs, so a row's bits do not depend on others.
+    // (1332 x 768 x 3072 with a NaN in one row 118 us for 64.)
+    __shared__ int wave_spoiled[WAVES];
+    const uint64_t any = __ballot(spoiled != 0);
+    if (lane == 0) wave_spoiled[wave] = any != 0;
+    __syncthreads();  // (the slices overlay the partial tiles)
+    bool again = false;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (col + e < N) dst[e] = out[e];
+    for (int w = 0; w < WAVES; ++w) again |= wave_spoiled[w] != 0;
+    if (again) {
+      multiply(std::false_type{});
+      __syncthreads();
+      join(std::true_type{}, 1.0f);
     }
   }
 }

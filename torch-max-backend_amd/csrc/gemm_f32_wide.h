@@ -94,6 +94,16 @@ struct F32Staged {
       lay_down(lds, i, h, m, l);
     }
   }
+  // The stage as it is, rows of 32 k (four more floats spread them over the banks), and four k of a row of it.
+  static constexpr int RAW_PITCH = 36, RAW_FLOATS = ROWS * RAW_PITCH;
+  __device__ __forceinline__ void lay_down_raw(float* __restrict__ lds, int wave, int lane) const {
+    const int row = K_CONTIGUOUS ? wave * 8 + lane / 8 : lane;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) *reinterpret_cast<f32x4_t*>(lds + (row + 64 * i) * RAW_PITCH + 4 * k4) = v[i];
+  }
+  static __device__ __forceinline__ f32x4_t raw_fragment(const float* __restrict__ lds, int row, int quad) {
+    return *reinterpret_cast<const f32x4_t*>(lds + row * RAW_PITCH + 4 * quad);
+  }
   // The eight k of chunk `chunk` in row `row`, part `part` (0 high, 1 middle, 2 low).
   static __device__ __forceinline__ u32x4_t fragment(const unsigned char* __restrict__ lds, int part, int row, int chunk) {
     return *reinterpret_cast<const u32x4_t*>(lds + part * PLANE + chunk * CHUNK + row * 16);
@@ -242,33 +252,58 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
     join();
   }
 
-  // Sums that are not finite (an operand or a result that is not, or one beyond what the factor leaves room for)
-  // are formed again from fp32 products.
-  float probe = 0.0f;
+  // Sums that are not finite (an operand or a result that is not, or one beyond what the factor leaves room for) are
+  // formed again from fp32 products; their neighbours keep theirs, so a row's bits do not depend on others. (4096^3 with a NaN
+  // in one row 1630 us for 910, in every row 2020; each wave by itself, two k at a time from memory: 2400 and 6010.)
+  __shared__ int wave_spoiled[kF32WideThreads / 64];
+  uint32_t spoiled = 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) probe = __builtin_fmaf(acc[i][e], 0.0f, probe);
-  float down = F32Pair::kDown * F32Pair::kDown;
-  if (__ballot(probe != 0.0f) != 0) {  // wave-uniform, and each wave's own: no barrier inside
-    down = 1.0f;
+    for (int e = 0; e < 16; ++e) {
+      spoiled |= (__builtin_fabsf(acc[i][e]) < HUGE_VALF ? 0u : 1u) << (16 * i + e);
+      acc[i][e] *= F32Pair::kDown * F32Pair::kDown;
+    }
+  const uint64_t any = __ballot(spoiled != 0);
+  if (lane == 0) wave_spoiled[wave] = any != 0;
+  __syncthreads();
+  bool again = false;
+#pragma unroll
+  for (int w = 0; w < kF32WideThreads / 64; ++w) again |= wave_spoiled[w] != 0;
+  if (again) {
+    float* ra = reinterpret_cast<float*>(f32_wide_lds);
+    float* rb = ra + StagedA::RAW_FLOATS;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-    const int64_t end = last * 32 < K ? last * 32 : K;
-    const int64_t c = n0 + col0 + lr < N ? col0 + lr : N - 1 - n0;
+      for (int e = 0; e < 16; ++e) t[i][e] = 0.0f;
+    sa.load_stage(first * 32, K);
+    sb.load_stage(first * 32, K);
 #pragma unroll 1
-    for (int64_t k = first * 32; k < end; k += 2) {
-      const int64_t kk = k + lk < end ? k + lk : end - 1;
-      const float bf = B[B_KMAJOR ? c * g.ldb + kk : kk * g.ldb + c];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int64_t r = m0 + row0 + i * 32 + lr < M ? row0 + i * 32 + lr : M - 1 - m0;
-        const float af = A[A_MMAJOR ? kk * g.lda + r : r * g.lda + kk];
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(k + lk < end ? bf : 0.0f, k + lk < end ? af : 0.0f, acc[i], 0, 0, 0);
+    for (int64_t s = first; s < last; ++s) {
+      sa.lay_down_raw(ra, wave, lane);
+      sb.lay_down_raw(rb, wave, lane);
+      __syncthreads();
+      if (s + 1 < last) {
+        sa.load_stage((s + 1) * 32, K);
+        sb.load_stage((s + 1) * 32, K);
       }
+#pragma unroll
+      for (int k8 = 0; k8 < 4; ++k8) {
+        const f32x4_t bf = StagedB::raw_fragment(rb, col0 + lr, 2 * k8 + lk);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const f32x4_t af = StagedA::raw_fragment(ra, row0 + i * 32 + lr, 2 * k8 + lk);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) t[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(bf[e], af[e], t[i], 0, 0, 0);
+        }
+      }
+      __syncthreads();
     }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][e] = (spoiled >> (16 * i + e) & 1) != 0 ? t[i][e] : acc[i][e];
   }
 
   // Lane holds row lr of each 32 x 32 result and columns 8q + 4 * lk + {0..3}.
@@ -286,7 +321,7 @@ __global__ __launch_bounds__(kF32WideThreads) void gemm_f32_wide_kernel(const Ge
       float out[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float v = acc[i][4 * q + e] * down;
+        float v = acc[i][4 * q + e];
         if (bias != nullptr && col + e < N) v += bias[col + e];
         out[e] = finish<float, EPI>(v, false);
       }
