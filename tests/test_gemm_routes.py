@@ -441,3 +441,17 @@ def test_fp32_long_rows_match_float64(case):
         size += x.abs() @ y.abs()
     # k roundings in a chain would be k 2^-24 of the sum of magnitudes; runs of at most 2^19 of them are chained
     assert ((got.double() - exact).abs() <= (min(k, 1 << 19) + 40) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("batch,m,n,k,ta,tb,kernel", [
+    (24, 32, 50304, 16, 0, 0, F32_WIDE),     # 77 us, 112 on 32 x 32 tiles
+    (4, 32, 50257, 16, 1, 1, F32_WIDE),      # 20 and 24 (a padded B)
+    (25, 2208, 16, 16, 0, 0, F32_WIDE),      # 6.5 and 8.3
+    (57, 192, 7104, 144, 1, 0, F32_WIDE),    # 358 and 485
+    (13, 160, 50304, 176, 1, 1, F32_WIDE),   # 597 and 648
+    (1, 4560, 50257, 37, 1, 1, SIMT),        # 587 and 826
+    (1, 4528, 50257, 40, 0, 0, SIMT)])       # 576 and 840
+def test_fp32_products_of_short_k_over_many_tiles_run_where_they_are_fastest(batch, m, n, k, ta, tb, kernel):
+    """The many small tiles of the waves-share-K kernel cost as much as their bytes there."""
+    aligned = kernel == F32_WIDE
+    assert route(m, n, k, ta, tb, _ek().F32, batch=batch, a_aligned=aligned, b_aligned=aligned)[0] == kernel

@@ -30,10 +30,13 @@ def _check(got, a, b, extra, what):
     assert ((got.double() - exact).abs() <= bound).all(), what
 
 
-# (m, n, k): one per tile (32 x 32 .. 64 x 128), one, two and three elements past a piece, the smallest
-# extents, and runs of K that are split (the last two)
+# (m, n, k): one, two and three elements past a piece, the smallest extents, runs of K that are split, and (the last seven)
+# one per tile: 32 x 32 with fp32 products over many rounds, 32 x 32 with eight and four waves, 32 x 64, 64 x 64 with four
+# and eight waves, and one of these split
 SHAPES = [(40, 70, 33), (500, 1000, 130), (777, 1025, 259), (1332, 770, 770), (750, 2306, 260), (4, 4, 4), (5, 6, 7), (33, 129, 35),
-          (65, 34, 62), (130, 770, 3001), (31, 67, 12565)]
+          (65, 34, 62), (130, 770, 3001), (31, 67, 12565),
+          (501, 1001, 101), (101, 203, 150), (161, 1367, 133), (877, 573, 683), (1571, 1139, 243), (823, 1135, 163),
+          (37, 2179, 2363)]
 
 
 @pytest.mark.parametrize("mnk", SHAPES)

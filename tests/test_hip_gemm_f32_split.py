@@ -60,10 +60,33 @@ def test_edges_of_the_128_tile(mnk, trans_a, trans_b):
         _check(_ops().gemm(a, b, bias), a, b, bias.double())
 
 
-# the kernel whose waves share K: its tiles, four and eight waves, split and not, and on both sides of the K up to which
-# products are fp32 ones
-SHARED = [(300, 500, 130), (300, 500, 300), (64, 128, 2000), (500, 1000, 100), (1000, 2000, 128), (1000, 1000, 520),
-          (750, 2304, 768), (1332, 768, 1200)]
+# the kernel whose waves share K, at any layout and alignment: fp32 products (K <= 128) in one round of tiles and in several,
+# 32 x 32 tiles with eight waves (one round), split, and with four, 32 x 64, 64 x 64 with four and with eight, split
+SHARED = [(300, 500, 100), (1000, 2000, 128), (300, 500, 300), (64, 128, 2000), (1788, 132, 136), (260, 1764, 680),
+          (1776, 1072, 252), (1040, 936, 152), (132, 1672, 1184)]
+
+
+def _kernels_of(shapes, **alignment):
+    """{(tile, fp32 products, split, all tiles in one round)} of the products on the kernel whose waves share K."""
+    from torch_mojo_backend import eager_kernels as ek
+    took = set()
+    for (m, n, k), ta, tb in itertools.product(shapes, (0, 1), (0, 1)):
+        kernel, tile, splits = route(m, n, k, ta, tb, ek.F32, workspace=PLENTY, **alignment)
+        if kernel == F32:
+            rounds = -(-m // 32) * -(-n // 32) * max(splits, 1) / 256
+            took.add((tile, k <= 128, splits > 0, tile > 0 or rounds <= 1))
+    return took
+
+
+def test_the_shapes_take_every_tile_with_either_product():
+    """A refit of the models' constants must not drop one (32 x 32 tiles have eight waves where they run in one round)."""
+    import test_hip_gemm_f32_edges
+    every = {(0, True, False, True), (0, True, False, False), (0, False, False, True), (0, False, True, True),
+             (0, False, False, False), (1, False, False, True), (2, False, False, True), (3, False, False, True),
+             (3, False, True, True)}
+    unaligned = dict(a_aligned=0, b_aligned=0)
+    assert _kernels_of(SHARED) >= every and _kernels_of(SHARED, **unaligned) >= every
+    assert _kernels_of(test_hip_gemm_f32_edges.SHAPES, **unaligned) >= every
 
 
 @pytest.mark.gpu

@@ -353,9 +353,9 @@ static inline bool f32_mfma_eligible(const GemmArgs& g, int64_t batch, int trans
 
 template <int EPI>
 static int launch_f32_wide(GemmArgs g, int64_t batch, int trans_a, int trans_b, hipStream_t stream) {
-  if (g.k <= kF32SplitK) return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
   g.tiles_m = static_cast<int>((g.m + kF32Wide - 1) / kF32Wide);
   g.tiles_n = static_cast<int>((g.n + kF32Wide - 1) / kF32Wide);
+  if (g.k <= kF32SplitK) return launch_f32_mfma<EPI>(g, batch, trans_a, trans_b, stream);
   g.stream_c = batch * g.m * g.n * 4 > (int64_t{256} << 20);
   const dim3 grid(static_cast<unsigned>(g.tiles_m * g.tiles_n), static_cast<unsigned>(batch));
   auto go = [&](auto a_mmajor, auto b_kmajor) {

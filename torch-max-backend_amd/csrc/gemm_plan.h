@@ -153,9 +153,9 @@ static inline double many_tiles_cost(const ManyTiles& t, int bm, int bn, int64_t
 static inline double simt_cost(bool f32, int64_t batch, int64_t m, int64_t n, int64_t k) {
   const double tiles = static_cast<double>(((m + 63) / 64) * ((n + 63) / 64)) * batch, r = tiles / 256.0;
   const double filled = static_cast<double>(m) * n * batch / (tiles * 4096.0);
-  const double alone = f32 ? 0.17 * k - 1.9 : 0.15 * k - 0.5;
-  const double many = f32 ? r * (0.038 * k + 0.24 + 1.33 * filled) : r * (0.036 * k + 0.21 + 0.72 * filled);
-  return (f32 ? 5.2 : 5.1) + (alone > many ? alone : many);
+  const double alone = f32 ? 0.15 * k - 0.7 : 0.15 * k - 0.5;
+  const double many = f32 ? r * (0.030 * k + 0.31 + 1.21 * filled) : r * (0.036 * k + 0.21 + 0.72 * filled);
+  return (f32 ? 4.8 : 5.1) + (alone > many ? alone : many);
 }
 static inline bool simt_instead_of_any(const GemmArgs& g, int64_t batch, const AnyPlan& plan) {
   if (g.residual != nullptr || plan.splits > 0 || g.k > 32) return false;
@@ -263,50 +263,64 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
   return p;
 }
 
-// fp32: tile and split count of the kernel whose waves share K. Microseconds of a launch: a start and, per round of
-// tiles, their way through LDS and the matrix cores; `whole` of a round's time is bound to whole rounds of the 256 CUs.
-// Fitted to 1600 shapes of 8 .. 8192 in each extent, 1 .. 36 batches, in all layouts; 10-13 % (rms) of each tile. A split
-// adds the reduction: a launch and its bytes. A 64 x 64 tile has eight waves where all tiles run at once (two a SIMD to
-// hide each other's waits: 1332 x 768 x 3072 47 us, with four 58), four, two workgroups to a CU, beyond (1332 x 3072 x 768
-// 50 us, with eight 59).
+// fp32: microseconds of a launch on one of the kernels' tiles: a start and, per round of the 256 CUs, `per_k` for each k of
+// a run and `per_tile` for the tile's way out, `edge` of which is stores that a tile past the matrix's edge leaves out;
+// `whole` of a round's time is bound to whole rounds, and from eight rounds on time is linear in them. No less than all
+// stores at 5.5 TB/s. Fitted to 165000 launches of 28800 shapes: 4 .. 16384 rows and columns, some 50257, K 4 .. 12000, 1 .. 64
+// batches, all layouts. Off by 7 .. 17 % (rms) for each tile, most of which is the layout; what they choose is behind the
+// best tile and split by 1.1 % on average.
 struct F32Tile {
   int bm, bn, waves;
-  double start, per_k, per_tile, power, whole;
+  double start, per_k, per_tile, power, whole, edge;
 };
-constexpr F32Tile kF32Tiles[] = {{32, 32, 4, 3.7, 0.00675, 1.1, 0.887, 0.25}, {32, 64, 4, 3.0, 0.0116, 2.5, 0.912, 0.34},
-                                 {64, 64, 4, 1.3, 0.0163, 4.4, 0.919, 0.67}, {64, 64, 8, 4.5, 0.012, 2.7, 1.0, 0.0}};
+static inline double f32_tile_cost(const F32Tile& t, double copies, int64_t m, int64_t n, double run) {
+  const double tiles = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * copies, r = tiles / 256.0;
+  const double outputs = copies * static_cast<double>(m) * static_cast<double>(n);
+  const double some = r < 8.0 ? r : 8.0;
+  const double rounds = r <= 1.0 ? 1.0 : std::pow(some, t.power) * (r / some) * (1.0 - t.whole + t.whole * std::ceil(r) / r);
+  const double per_tile = t.per_tile * (1.0 - t.edge + t.edge * outputs / (tiles * t.bm * t.bn));
+  return std::fmax(t.start + rounds * (t.per_k * run + per_tile), 3.0 + outputs * 4.0 / 5.5e6);
+}
+// The second launch of a split product.
+static inline double f32_reduction_cost(int64_t m, int64_t n, int splits) {
+  return 3.6 + 0.8e-6 * splits * static_cast<double>(m) * static_cast<double>(n);
+}
+// Of the kernel whose waves share K. A 64 x 64 tile has eight waves where all tiles run at once (two a SIMD to hide each
+// other's waits: 1332 x 768 x 3072 57 us, with four 70), four, two workgroups to a CU, beyond (1332 x 3072 x 768 58 us, with
+// eight 66), and a 32 x 32 tile likewise (64 x 768 x 768 7.9 us, with four 9.2).
+constexpr F32Tile kF32Tiles[] = {{32, 32, 4, 3.28, 0.00836, 0.837, 0.836, 0.49, 0.0}, {32, 64, 4, 3.73, 0.0133, 2.08, 0.885, 0.48, 0.0},
+                                 {64, 64, 4, 4.13, 0.0210, 3.34, 0.879, 0.49, 0.10}, {64, 64, 8, 3.0, 0.0156, 4.2, 1.0, 0.0, 0.12}};
 constexpr int kF32TileCount = sizeof(kF32Tiles) / sizeof(kF32Tiles[0]);
+constexpr F32Tile kF32AllAtOnce = {32, 32, 8, 2.9, 0.0063, 1.2, 1.0, 0.0, 0.35};
+// Short K runs with fp32 products, on 32 x 32 tiles only: 32 x 64 and 64 x 64 ones were faster by more than 3 % in 0.2 and 1 %
+// of 10900 such launches.
+constexpr F32Tile kF32Products = {32, 32, 4, 2.97, 0.00352, 0.746, 1.0, 0.68, 0.10};
 struct F32Plan {
   int tile;    // index into kF32Tiles
   int splits;  // 0: not split
   double cost;
 };
-// (the launches of up to kF32SplitK are the fp32 products')
-constexpr ManyTiles kF32Short[] = {{2.9, 0.0075, 0.90, 0.933}, {2.8, 0.0129, 1.95, 0.939}, {3.6, 0.0211, 3.2, 0.969}};
-static inline double f32_cost(int tile, double batch, int64_t m, int64_t n, double k, bool short_k) {
+static inline double f32_cost(int tile, int64_t batch, int64_t m, int64_t n, int64_t k, int splits) {
+  const double copies = static_cast<double>(splits > 0 ? splits : batch);
+  const double run = static_cast<double>(k) / (splits > 0 ? splits : 1);
   const F32Tile& t = kF32Tiles[tile];
-  const double r = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * batch / 256.0;
-  if (short_k) {
-    if (t.waves == 8) return HUGE_VAL;
-    const ManyTiles& s = kF32Short[tile];
-    return s.start + (r <= 1.0 ? 1.0 : std::pow(r, s.power)) * (s.per_k * k + s.per_tile);
-  }
-  if (t.bm == 64 && (r <= 1.0) != (t.waves == 8)) return HUGE_VAL;
-  const double rounds = r <= 1.0 ? 1.0 : std::pow(r, t.power) * (1.0 - t.whole + t.whole * std::ceil(r) / r);
-  return t.start + rounds * (t.per_k * k + t.per_tile);
+  const bool at_once = static_cast<double>(((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn)) * copies <= 256.0;
+  if (k <= kF32SplitK) return tile == 0 ? f32_tile_cost(kF32Products, copies, m, n, run) : HUGE_VAL;
+  if (t.bm == 64 && at_once != (t.waves == 8)) return HUGE_VAL;
+  return f32_tile_cost(t.bn == 32 && at_once ? kF32AllAtOnce : t, copies, m, n, run);
 }
 static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, int most_splits) {
   F32Plan p{0, 0, HUGE_VAL};
   for (int i = 0; i < kF32TileCount; ++i) {
-    const double c = f32_cost(i, static_cast<double>(batch), m, n, static_cast<double>(k), k <= kF32SplitK);
+    const double c = f32_cost(i, batch, m, n, k, 0);
     if (c < p.cost) p = F32Plan{i, 0, c};
   }
   if (batch != 1 || m * n >= (int64_t{1} << 31)) return p;
-  double best = p.cost * 0.92;  // a second launch and a workspace have to pay for themselves
+  double best = p.cost * 0.95;  // a second launch and a workspace have to pay for themselves
   for (const int s : {2, 3, 4, 6, 8, 12, 16}) {
     if (k < 96 * s || s > most_splits) break;
     for (int i = 0; i < kF32TileCount; ++i) {
-      const double c = f32_cost(i, s, m, n, static_cast<double>(k) / s, k <= kF32SplitK) + 5.5 + 1e-6 * s * m * n;
+      const double c = f32_cost(i, 1, m, n, k, s) + f32_reduction_cost(m, n, s);
       if (c < best) {
         best = c;
         p = F32Plan{i, s, c};
@@ -315,14 +329,13 @@ static inline F32Plan f32_plan(int64_t batch, int64_t m, int64_t n, int64_t k, i
   }
   return p;
 }
-// The kernel of 128 x 128 tiles, fitted with it (10 %). Its bound is the larger of the tiles' time and the stores'.
-static inline double f32_wide_cost(int64_t batch, int64_t m, int64_t n, double k, bool short_k) {
-  const double count = static_cast<double>(((m + 127) / 128) * ((n + 127) / 128)) * batch;
-  const double tiles = short_k  // (gemm_f32_short.h)
-                           ? 3.2 + std::pow(std::ceil(count / 256.0), 0.923) * (0.078 * k + 3.09)
-                           : 0.4 + std::pow(std::ceil(count / 256.0), 1.06) * (0.0355 * k + 4.8 + (count < 128.0 ? count / 80.0 : 1.6));
-  const double stores = 3.2 + static_cast<double>(batch) * m * n * 4.0 / 5.5e6;
-  return tiles > stores ? tiles : stores;
+// The kernel of 128 x 128 tiles, and the one with fp32 products that takes its place at short K.
+constexpr F32Tile kF32WideTile = {128, 128, 8, 2.32, 0.0450, 6.57, 1.07, 1.0, 0.48};
+constexpr F32Tile kF32WideProducts = {128, 128, 4, 1.89, 0.0775, 4.46, 0.869, 0.74, 0.59};
+static inline double f32_wide_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int splits) {
+  const double copies = static_cast<double>(splits > 0 ? splits : batch);
+  return f32_tile_cost(k <= kF32SplitK ? kF32WideProducts : kF32WideTile, copies, m, n,
+                       static_cast<double>(k) / (splits > 0 ? splits : 1));
 }
 // Operands off 16-byte boundaries are as fast there (its loads want none), and run there from this K on; shorter products
 // of such operands are the padded copies', the vector kernel's and the waves-share-K kernel's.
@@ -332,17 +345,17 @@ struct F32WidePlan {
   int splits;
   double cost;
 };
-// Where a product whose operands both take runs on it (`other`: what it runs as otherwise), and with how many splits. Split it is up to 40 tiles only: from 41
-// on the 64 x 64 tiles of the other kernel have most CUs busy without scratch and a second launch (1024 x 768 x 3072
-// 43 us). 750 x 768 x 3072 31 us in 7 splits, 44 there; 750 x 768 x 50257 275 against 470. A split must promise a fifth,
-// twice the models' error.
+// Where a product whose operands both take runs on it (`other`: what it runs as otherwise), and with how many splits. Up to
+// 40 tiles only: callers rely on products that fill most CUs with 64 x 64 tiles to ask for no scratch (1024 x 768 x 3072, 48
+// tiles). Splitting on would pay: 1024 x 768 x 3072 58 us unsplit, 47 in five runs, 2048 x 768 x 3072 99 and 83.
+constexpr int64_t kF32WideSplitTiles = 40;
 static inline F32WidePlan f32_wide_plan(int64_t batch, int64_t m, int64_t n, int64_t k, const F32Plan& other) {
-  F32WidePlan p{false, 0, f32_wide_cost(batch, m, n, static_cast<double>(k), k <= kF32SplitK)};
+  F32WidePlan p{false, 0, f32_wide_cost(batch, m, n, k, 0)};
   p.taken = p.cost < other.cost;
-  if (batch != 1 || m * n >= (int64_t{1} << 31) || ((m + 127) / 128) * ((n + 127) / 128) > 40) return p;
-  double best = (p.taken ? p.cost : other.cost) * 0.8;
+  if (batch != 1 || m * n >= (int64_t{1} << 31) || ((m + 127) / 128) * ((n + 127) / 128) > kF32WideSplitTiles) return p;
+  double best = (p.taken ? p.cost : other.cost) * 0.95;  // (as above)
   for (int s = 2; s <= 16 && k >= 96 * s; ++s) {
-    const double c = f32_wide_cost(s, m, n, static_cast<double>(k) / s, k <= kF32SplitK) + 5.5 + 1e-6 * s * m * n;
+    const double c = f32_wide_cost(1, m, n, k, s) + f32_reduction_cost(m, n, s);
     if (c < best) {
       best = c;
       p = F32WidePlan{true, s, c};
@@ -350,16 +363,17 @@ static inline F32WidePlan f32_wide_plan(int64_t batch, int64_t m, int64_t n, int
   }
   return p;
 }
-// Unaligned operands: the other way is to copy what the 128 x 128 kernel cannot read into padded buffers (8 us a copy
+// Unaligned operands: the other way is to copy what the 128 x 128 kernel cannot read into padded buffers (6 us a copy
 // with what the host does for it, and the bytes at 5.3 TB/s, 1.3 where it transposes) and to multiply there, a K that is no
 // whole number of 16-byte vectors as the next multiple of 64; infinite where the copies would not run on that kernel.
+// 3072 x 4096 x 97 48 us, 58 where it lies; 3072 x 2048 x 97 35 and 29.
 // 7710 x 8280 x 8 60 against 317 us where it lies, 48 x 816 x 3664 x 16 175 against 721, 8051 x 6756 x 172 with a
 // residual 350 against 630.
 static inline double f32_padded_cost(int64_t batch, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb, bool a_ok,
                                      bool b_ok, int trans_a, int trans_b) {
   double cost = 0.0;
   auto copy = [&](int64_t elements, bool transposing) {
-    cost += 8.0 + static_cast<double>(elements) * batch * 8.0 / (transposing ? 1.3e6 : 5.3e6);
+    cost += 6.0 + static_cast<double>(elements) * batch * 8.0 / (transposing ? 1.3e6 : 5.3e6);
   };
   int64_t depth = k;
   const bool b_fits = b_ok && ldb % 4 == 0;
@@ -468,7 +482,7 @@ static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a,
     // (no more splits than there: the scratch that a caller of known layout is told of does not depend on alignment)
     if (wide.splits > 0 && plan.splits > wide.splits) plan = f32_plan(batch, g.m, g.n, g.k, wide.splits);
     if (!fits(plan.splits)) plan = f32_plan(batch, g.m, g.n, g.k, 0);
-    if (takes && plan.splits == 0 && f32_wide_cost(batch, g.m, g.n, static_cast<double>(g.k), g.k <= kF32SplitK) < plan.cost)
+    if (takes && plan.splits == 0 && f32_wide_cost(batch, g.m, g.n, g.k, 0) < plan.cost)
       return {TMB_GEMM_F32_WIDE, 0, 0};
     if (g.k <= 48 && plan.splits == 0 && simt_cost(true, batch, g.m, g.n, g.k) < plan.cost) return {TMB_GEMM_SIMT, 0, 0};
     return {TMB_GEMM_F32, plan.tile, plan.splits};

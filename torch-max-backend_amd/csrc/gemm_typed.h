@@ -216,16 +216,10 @@ static int launch_splitk(const GemmArgs& g, const SplitKPlan& plan, int trans_a,
 
 template <int EPI>
 static int launch_f32_shared(const GemmArgs& g, int64_t batch, int tile, int trans_a, int trans_b, hipStream_t stream) {
-  if (g.k <= kF32SplitK) {
-    switch (tile) {
-      case 0: return launch_f32_tile<32, 32, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
-      case 1: return launch_f32_tile<32, 64, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
-      default: return launch_f32_tile<64, 64, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
-    }
-  }
+  if (g.k <= kF32SplitK) return launch_f32_tile<32, 32, 4, EPI, false>(g, batch, trans_a, trans_b, stream);
   switch (tile) {
-    case 0:  // (one workgroup to a CU and slices for all of eight waves: 64 x 768 x 768 7.5 us, with four 8.8)
-      return ((g.m + 31) / 32) * ((g.n + 31) / 32) * batch <= 256 && g.k > 256
+    case 0:
+      return ((g.m + 31) / 32) * ((g.n + 31) / 32) * batch <= 256
                  ? launch_f32_tile<32, 32, 8, EPI, true>(g, batch, trans_a, trans_b, stream)
                  : launch_f32_tile<32, 32, 4, EPI, true>(g, batch, trans_a, trans_b, stream);
     case 1: return launch_f32_tile<32, 64, 4, EPI, true>(g, batch, trans_a, trans_b, stream);
