@@ -276,6 +276,9 @@ def test_fp32_products_with_long_rows_stay_on_the_matrix_cores():
     kernel, _, splits = route(64, 64, 1 << 25, tb=1, **f32)
     assert kernel == F32_WIDE and splits > 1 and (1 << 25) % (4 * splits) == 0
     assert route(64, 64, (1 << 25) + 4, tb=1, **f32)[0] == F32_WIDE
+    for k in (4096, 3004):           # (runs of K need not come out even)
+        dense = route(64, 60, k, tb=1, dtype=f32["dtype"], workspace=PLENTY, a_aligned=0)
+        assert route(64, 60, k, tb=1, lda=1 << 25, **f32) == (F32_WIDE, 0, dense[2]) and dense[2] > 1
     assert route(64, 64, 1 << 25, tb=1, dtype=_ek().F32) == (F32_WIDE, 0, 0)
     assert route(1 << 26, 64, 64, ta=1, **f32)[0] == F32_WIDE
     assert route(64, 64, 1 << 25, tb=1, residual=1, **f32) == _ek().ERR_UNSUPPORTED
@@ -417,7 +420,8 @@ def test_the_launcher_pads_fp32_operands_of_short_k(recorded):
 @pytest.mark.parametrize("case", [
     # (m, n, k, pitch of A, A stored [K, M])
     (4, 8, (1 << 23) + 1, None, False),      # long rows, few of them
-    (64, 60, 4096, 1 << 25, False),          # rows out of reach: the wide kernel, K split as a batch
+    (64, 60, 4096, 1 << 25, False),          # rows out of reach: the wide kernel, K split
+    (64, 60, 3004, 1 << 25, False),          # and in runs that do not come out even
     (130, 60, 100, 35651584, True)])         # k-rows out of reach
 def test_fp32_long_rows_match_float64(case):
     import torch

@@ -132,14 +132,12 @@ extern "C" size_t tmb_gemm_workspace_bytes(int64_t batch, int64_t m, int64_t n, 
 
 extern "C" size_t tmb_gemm_layout_workspace_bytes(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a,
                                                   int trans_b, int dtype) {
-  // the kernels for small and for wide products need none (operands they cannot take run unsplit then)
   if (dtype == TMB_F32) {
     if (batch < 1 || m < 1 || n < 1 || k < 1 || m * n >= (int64_t{1} << 31)) return 0;
     return static_cast<size_t>(tmb::f32_most_splits(batch, m, n, k, trans_a, trans_b)) * m * n * 4;
   }
-  if (!trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k)) {
-    return 0;
-  }
+  // the kernel for small products needs none (operands it cannot take run unsplit then)
+  if (!trans_a && (trans_b || n % 8 == 0) && k % 8 == 0 && tmb::small_applies(batch, m, n, k)) return 0;
   return tmb_gemm_workspace_bytes(batch, m, n, k, dtype);
 }
 

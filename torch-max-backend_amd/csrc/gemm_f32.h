@@ -119,14 +119,13 @@ struct F32Slice<64, false> {
   using Lines = F32Slice<ROWS, true>;
   static constexpr int FLOATS = Lines::FLOATS, LOADS = Lines::LOADS;
   f32x4_t v[LOADS];
-  uint32_t off;  // bytes: the lane's row and first k
+  uint32_t off;  // bytes: the lane's row
 
-  static __device__ __forceinline__ int first_k(int lane) { return lane / ROWS * LOADS * 4; }
-  __device__ __forceinline__ void plan(int64_t ld, int64_t rows, int lane) {
-    const int last = rows > ROWS ? ROWS : static_cast<int>(rows), line = lane % ROWS;
-    off = static_cast<uint32_t>((first_k(lane) * ld + (line < last ? line : last - 1)) * 4);
+  __device__ __forceinline__ void plan(int64_t, int64_t rows, int lane) {
+    const int last = rows > ROWS ? ROWS : static_cast<int>(rows);
+    off = static_cast<uint32_t>((lane < last ? lane : last - 1) * 4);
   }
-  __device__ __forceinline__ void load(const char* __restrict__ first, int64_t ld, int64_t k_left, int lane) {
+  __device__ __forceinline__ void load(const char* __restrict__ first, int64_t ld, int64_t k_left, int) {
     const int64_t step = ld * 4;
     auto at = [](const char* p) { return *reinterpret_cast<const float*>(p); };
     if (k_left >= kF32KS) {  // wave-uniform
@@ -136,7 +135,7 @@ struct F32Slice<64, false> {
         v[i] = f32x4_t{at(p + off), at(p + step + off), at(p + 2 * step + off), at(p + 3 * step + off)};
       }
     } else {  // (k past the last one re-read it)
-      const int most = static_cast<int>(k_left) - 1 - first_k(lane);
+      const int most = static_cast<int>(k_left) - 1;
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         const char* __restrict__ p = first + off;
@@ -147,7 +146,7 @@ struct F32Slice<64, false> {
   }
   __device__ __forceinline__ void lay_down(float* __restrict__ lds, int64_t k_left, int lane) {
     if (k_left < kF32KS) {  // wave-uniform
-      const int left = static_cast<int>(k_left) - first_k(lane);
+      const int left = static_cast<int>(k_left);
 #pragma unroll
       for (int i = 0; i < LOADS; ++i)
         v[i] = f32x4_t{4 * i < left ? v[i][0] : 0.0f, 4 * i + 1 < left ? v[i][1] : 0.0f, 4 * i + 2 < left ? v[i][2] : 0.0f,
@@ -155,7 +154,7 @@ struct F32Slice<64, false> {
     }
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-      *reinterpret_cast<f32x4_t*>(lds + (lane % ROWS) * Lines::PITCH + first_k(lane) + 4 * i) = v[i];
+      *reinterpret_cast<f32x4_t*>(lds + lane * Lines::PITCH + 4 * i) = v[i];
   }
   static __device__ __forceinline__ void fragment(const float* __restrict__ lds, int row, int lq, f32x4_t (&x)[2]) {
     Lines::fragment(lds, row, lq, x);

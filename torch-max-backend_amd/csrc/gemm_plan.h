@@ -392,8 +392,8 @@ static inline double f32_padded_cost(int64_t batch, int64_t m, int64_t n, int64_
   const F32WidePlan wide = f32_wide_plan(batch, m, n, depth, f32_plan(batch, m, n, depth, 16));
   return wide.taken && wide.splits == 0 ? cost + wide.cost : HUGE_VAL;
 }
-// What the kernel whose waves share K asks of its operands: at least four elements along each
-// contiguous direction, and lane offsets that fit 32 bits in its largest tile (64 x 128; 32 rows of k for an
+// What the kernel whose waves share K asks of its operands: at least four elements along each contiguous direction, and
+// lane offsets that fit 32 bits in its largest tile (64 x 64, of which B is held to twice the rows; 32 rows of k for an
 // operand stored K-outer).
 static inline bool f32_shared_eligible(const GemmArgs& g, int trans_a, int trans_b) {
   if (g.m < 1 || g.n < 1 || g.k < 1) return false;
@@ -487,11 +487,9 @@ static inline GemmRoute route_f32(const GemmArgs& g, int64_t batch, int trans_a,
     if (g.k <= 48 && plan.splits == 0 && simt_cost(true, batch, g.m, g.n, g.k) < plan.cost) return {TMB_GEMM_SIMT, 0, 0};
     return {TMB_GEMM_F32, plan.tile, plan.splits};
   }
-  const F32Plan plan = f32_plan(batch, g.m, g.n, g.k, 16);
-  // rows too long for 32-bit offsets: the wide kernel, a split as a batch of equal runs of whole 16-byte pieces
-  int splits = fits(plan.splits) ? plan.splits : 0;
-  while (splits > 0 && (splits == 1 || g.k % (4 * splits) != 0)) --splits;
-  return {TMB_GEMM_F32_WIDE, 0, splits};
+  // rows too long for 32-bit offsets: the wide kernel, which addresses in 64 bits, split as far as the other one would be
+  const int splits = f32_plan(batch, g.m, g.n, g.k, 16).splits;
+  return {TMB_GEMM_F32_WIDE, 0, fits(splits) ? splits : 0};
 }
 
 // The most splits that a product of dense operands in this layout runs with, at any alignment.
