@@ -232,7 +232,7 @@ int tmb_gemm_ws(void* c, const void* a, const void* b, const void* bias, int64_t
  * adds separately: k == 0, operands with fewer than eight (fp32: four) elements along a contiguous direction,
  * a GELU epilogue unless TMB_EPI_ROUND_LIKE_UNFUSED, sizes at which the two launches are faster, and, in fp32
  * and with TMB_EPI_ROUND_LIKE_UNFUSED, products that run on a kernel without a residual step (a large transposed A,
- * short K over many tiles, fp32 on 128 x 128 tiles; tmb_gemm_route answers the same).
+ * short K over many tiles, fp32 on 128 x 128 tiles unless K is split; tmb_gemm_route answers the same).
  * Replaces `AddF32Bf16Spec` / the residual add of aten_fast.py:657-687 together with the GEMM
  * in front of it. */
 int tmb_gemm_residual(void* c, const void* a, const void* b, const void* bias,

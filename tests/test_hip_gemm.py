@@ -615,7 +615,7 @@ def test_fp32_mfma_all_layouts_match_float64(case):
     a64 = as64(a).T if ta else as64(a)
     b64 = as64(b).T if tb else as64(b)
     want = a64 @ b64 + as64(bias)
-    # fp32 products are exact in the accumulator's input; k additions round at 2^-24 each
+    # a product is off by 2^-24 of it, once, and no more than k additions round at 2^-24 each
     bound = k * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64) + np.abs(as64(bias)))
     assert_close64(got, want, extra_abs=bound, what=f"fp32 gemm {case}")
     assert rel_frobenius(got, want) <= 2e-6

@@ -2,11 +2,11 @@
 //
 // An fp32 MFMA takes 64 cycles for what a bf16 one does in four. So each operand element is taken apart into three bf16
 // whose sum it is, exactly (F32Pair), and a product is eight of the nine partial products, all but the one below 2^-33 of
-// it, added up in fp32 by v_mfma_f32_16x16x32_bf16: 21 cycles of matrix core for 64. The large partial products and the
+// it, added up in fp32 by v_mfma_f32_16x16x32_bf16: 32 cycles of matrix core for 64. The large partial products and the
 // small ones are summed apart and joined by a rounded addition: a product that stands alone is off by 1.01 half units at
 // most (with the small ones in one chain, 3.8: the MFMA aligns addends to the largest and cuts), and a sum is rounded once
 // in 32 k instead of at every k. Against fp32 MFMAs the error of dense operands is 0.1 .. 1.0 of what it was over K 129 ..
-// 50257, of rows with a single term the same, of rows with 4 .. 16 terms 0.6 .. 1.2 (each product is rounded before it is
+// 50257, of rows with a single term the same, of rows with 4 .. 16 terms 0.6 .. 1.13 (each product is rounded before it is
 // added, and the order of the sum is another); operands of exponents 2^-20 .. 2^20 0.3 .. 1.03.
 // 1332 x 768 x 3072 68 -> 57 us, 1332 x 3072 x 768 70 -> 58, 750 x 2304 x 768 36 -> 29.
 //
