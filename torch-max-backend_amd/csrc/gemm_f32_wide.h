@@ -4,8 +4,9 @@
 // One workgroup of 2 x 4 waves owns a 128 x 128 tile of C, each wave a 64 x 32 part, and walks K in stages of 32. The
 // workgroup splits each element once, on its way into LDS: stage s + 2 travels from global memory into registers while
 // stage s + 1 is taken apart and laid down in one LDS buffer and stage s is multiplied out of the other; one barrier
-// closes the stage. The vector units that do the splitting are the second bound after the matrix cores (five vector instructions hide behind a
-// 32 x 32 x 16 MFMA, two behind a 16 x 16 x 32 one; measured), hence the large tile and the large MFMA.
+// closes the stage. The vector units that do the splitting are the second bound after the matrix cores (five vector
+// instructions hide behind a 32 x 32 x 16 MFMA, two behind a 16 x 16 x 32 one; measured), hence the large tile and the
+// large MFMA.
 //
 // 4096^3 890 us (154 TFLOP/s: 1230 of bf16 products, where the clock falls to what the matrix cores' power leaves), 2048^3
 // 117, 1332 x 50257 x 768 820; fp32 MFMAs took 1110, 169 and 870.
