@@ -202,7 +202,7 @@ typedef enum tmb_gemm_kernel {
   TMB_GEMM_RING = 1,         /* 16-bit, aligned, A row-major: direct-to-LDS rings and register-staged tiles */
   TMB_GEMM_TRANSPOSED_A = 2, /* 16-bit, aligned, A stored [K, M] and B [K, N] */
   TMB_GEMM_SPLITK = 3,       /* the two above with K split over workgroups; tile 0: 128 x 128, 1: 256 x 256 */
-  TMB_GEMM_SMALL = 4,        /* 16-bit, aligned, few tiles: waves share K; tile 0 .. 5 (5 of a K-major B: a ring) */
+  TMB_GEMM_SMALL = 4,        /* 16-bit, aligned, few tiles: waves share K; tile 0 .. 5 */
   TMB_GEMM_ANY = 5,          /* 16-bit, any layout and alignment; tile 0 .. 4 */
   TMB_GEMM_STREAM64 = 6,     /* 16-bit, K = 64 on whole 128 x 128 tiles */
   TMB_GEMM_F32 = 7,          /* fp32, any layout and alignment; tile 0 .. 3 */

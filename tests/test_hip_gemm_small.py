@@ -89,3 +89,14 @@ def test_small_epilogues(mnk, dtype):
         exact = torch.nn.functional.gelu(a.double() @ b.double().contiguous() + bias.double(), approximate=approximate)
         slack = 1.2 * k * 2.0 ** -24 * (a.double().abs() @ b.double().abs().contiguous()) + 4e-6
         assert ((once.double() - exact).abs() <= slack + (ULP[dtype] + 1e-5) * exact.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", HALF)
+@pytest.mark.parametrize("mnk", [(231, 3072, 768), (300, 2304, 768), (1025, 1000, 256), (960, 776, 3072)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_a_16_bit_result_is_the_float32_result_rounded(mnk, dtype, trans_b):
+    """The largest tile: the type of the result chooses neither the kernel nor the order of its sums."""
+    a, b, bias, _ = _inputs(*mnk, dtype, trans_b)
+    zero = torch.zeros(*mnk[:2], device="cuda")
+    wide = _ops().gemm(a, b, bias, residual=zero, out_dtype=torch.float32)
+    assert torch.equal(_ops().gemm(a, b, bias), wide.to(dtype))

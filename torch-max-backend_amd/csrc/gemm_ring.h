@@ -98,10 +98,9 @@ constexpr bool kRingPersistent = ring_waves_per_simd(BM, BN, BK, WAVES, R) <= 2;
 // MI16_: multiply with v_mfma_f32_16x16x32 instead of v_mfma_f32_32x32x16.
 // K_TAIL: K may end inside a stage (a multiple of 8). The lanes of the last stage whose k lies past the end fetch zeros.
 // SHORT_CHAINS: every 512 of K the accumulators are added to a second set and start from zero. These tiles took over products
-// of split launches and of the kernel whose waves share K, whose float32 sums (a float32 residual stream keeps them) are
-// off by 1.5e-7 .. 2e-7 of the result (rms, K = 2304 and 3072) where one chain of additions is by 2.9e-7 .. 3.4e-7. Each
-// addition waits for the matrix pipes, 0.15 us; a float32 result of 64 x 64 tiles, which the waves' kernel summed to within
-// 1.2e-7 (K = 3072), takes chains of 256. Below K = 2048 the larger tiles took over from other rings: one chain, and the same bits.
+// of split launches, whose float32 sums (a float32 residual stream keeps them) are off by 1.5e-7 .. 2e-7 of the result
+// (rms, K = 2304 and 3072) where one chain of additions is by 2.9e-7 .. 3.4e-7. Each addition waits for the matrix pipes,
+// 0.15 us. Below K = 2048 the larger tiles took over from other rings: one chain, and the same bits.
 template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int R, bool B_KMAJOR, int EPI,
           bool A_MMAJOR = false, bool OUT_F32 = false, bool MI16_ = (BK == 64), bool SHORT_CHAINS = false,
           bool K_TAIL = false>
@@ -752,7 +751,7 @@ static int launch_ring(const GemmArgs& base, int64_t batch, hipStream_t stream) 
   g.tiles_m = static_cast<int>((g.m + BM - 1) / BM);
   g.tiles_n = static_cast<int>((g.n + BN - 1) / BN);
   g.stream_c = g.m * g.n * batch * (g.out_f32 ? 4 : 2) >= (int64_t{256} << 20);
-  g.chain_mask = BM * BN == 64 * 64 ? (g.out_f32 ? 3 : 7) : g.k < 2048 ? 0x3fffffff : 7;
+  g.chain_mask = BM * BN != 64 * 64 && g.k < 2048 ? 0x3fffffff : 7;
   const int64_t tiles = static_cast<int64_t>(g.tiles_m) * g.tiles_n;
   if (tiles >= (int64_t{1} << 31) || batch > 65535) return TMB_ERR_UNSUPPORTED;
   // as many workgroups as the device holds at once (a multiple of the 8 XCDs), shared between

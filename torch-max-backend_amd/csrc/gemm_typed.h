@@ -299,13 +299,7 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
     constexpr bool BF16 = __is_same(T, bf16_t);
     const GemmRoute r = route_16bit(g, batch, trans_a, trans_b, EPI, scratch);
     switch (r.kernel) {
-      case TMB_GEMM_SMALL:
-        // (64 x 64 tiles of a K-major B, whole stages: from a ring, 900 x 768 x 768 8.7 -> 6.7 us, 1300 x 768 x 3072
-        // 16.7 -> 14.3; the ring's swizzle of an N-major B needs 128 columns. A float32 result of shorter K is summed a little
-        // more accurately by the waves' kernel: K = 768 7.2e-8 against 8.2e-8 of the result, 3072 1.17e-7 against 1.09e-7.)
-        if (r.tile == 5 && trans_b && g.k % 64 == 0 && g.k >= 256 && (!g.out_f32 || g.k >= 2560))
-          return launch_ring<T, 64, 64, 64, 2, 2, 4, true, EPI, false, false, true, true>(g, batch, stream);
-        return gemm_small(g, batch, r.tile, trans_b, BF16, EPI, stream);
+      case TMB_GEMM_SMALL: return gemm_small(g, batch, r.tile, trans_b, BF16, EPI, stream);
       case TMB_GEMM_SPLITK:
         return launch_splitk<T, EPI>(g, SplitKPlan{r.splits, r.tile == 1 ? 256 : 128, 0.0}, trans_a, trans_b,
                                      static_cast<float*>(workspace), stream);
