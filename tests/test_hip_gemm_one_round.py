@@ -15,7 +15,7 @@ def _ek():
 
 # (m, n, k): 64 x 128 tiles in one round (two of them with one row or column past a tile), 128 x 128 in one round, 64 x 128
 # two to a CU in one round and in more, products that no longer split, runs of a split on eight waves, narrow outputs of few
-# and many rows, and the 64 x 64 tiles of a K-major B
+# and many rows, and 64 x 64 tiles whose waves share K
 ROW_MAJOR = [(2049, 768, 256), (2048, 776, 320), (4096, 1024, 256), (3400, 1160, 320), (5400, 768, 256), (6785, 776, 320),
              (2113, 768, 2304), (2700, 768, 3072), (520, 1096, 8192), (300, 64, 4160), (32768, 48, 256), (32709, 56, 320),
              (1025, 1000, 256), (960, 776, 3072)]
@@ -73,3 +73,14 @@ def test_k_that_ends_inside_a_stage(mnk, dtype, trans_b):
     a[7] = a[11] = 0
     bias64[7] = bias64[11] = 0
     _check(got, a, b, bias64, mnk)
+
+
+@pytest.mark.parametrize("dtype", HALF)
+@pytest.mark.parametrize("k", [2048, 2496, 4096])
+def test_transposed_products_are_summed_in_short_chains(k, dtype):
+    """2^29 first and its negative last, ones between. Float32 numbers of 2^29 lie 64 apart, more than what an MFMA adds at a
+    time: one chain over K loses all the ones, chains of 512 lose those of the first and the last."""
+    a, b = (torch.ones(k, n, device="cuda", dtype=dtype) for n in (3072, 768))
+    a[0], a[-1], b[0], b[-1] = 2.0 ** 15, -2.0 ** 15, 2.0 ** 14, 2.0 ** 14
+    got = _ops().gemm(a.t(), b)
+    assert got.min() >= (k - 1024) * (1 - 2.0 ** -8) and got.max() <= k

@@ -177,7 +177,7 @@ static inline bool any_eligible(int64_t m, int64_t n, int64_t k, int64_t lda, in
 // only: a 64-wide A stored [K, M] has too few 16-byte chunks a row for its swizzle) and 128 x 128. What bounds them is the
 // wait for a stage, which two waves a SIMD cover and four did not: bf16, the 128 x 128 x 32 tiles of four waves
 // that ran before against these, microseconds: 2100 x 768 x 768 11.9 and 8.2, 3400 x 768 x 768 12.1 and 10.2, 2700 x
-// 768 x 3072 33.5 (split) and 24.5, dy^T x 3072 x 768 x 2048 27.1 (split) and 18.4. Beyond one round 64 x 128 tiles,
+// 768 x 3072 33.5 (split) and 24.5, dy^T x 3072 x 768 x 2048 27.5 (split) and 19.3. Beyond one round 64 x 128 tiles,
 // two workgroups to a CU, of three stages: 5400 x 768 x 768 17.5 and 12.1, 5400 x 768 x 3072 50.4 and 42.8.
 enum { kRing64x128 = 1, kRing128x128 = 2 };
 static inline int ring_one_round(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a) {
@@ -298,7 +298,7 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
 }
 // The same, or no split where one round of the tiles above is faster (the model's costs are 4.5 us under the measured ones):
 // A row-major 2100 x 768 x 3072 30.0 us split and 18.7, 4300 x 768 x 3072 45.2 and 33.7; A stored [K, M] 3072 x 768 x 2048
-// 27.1 and 18.4, x 4096 45.1 and 35.9, with half of the CUs idle level (2304 x 768 x 3072 24 both) or behind (224 x 7464 x
+// 27.5 and 19.3, x 4096 46 and 34, with half of the CUs idle level (2304 x 768 x 3072 24 both) or behind (224 x 7464 x
 // 3008 29 and 35). A row-major product that fills three quarters of the chip or less stays split from K = 3072 on, and any
 // from 4096 on: there the line could lie higher (2000 x 768 x 3072 27.5 and 17, 3072 x 768 x 4096 44 and 36), but callers
 // size their scratch by the plans of those shapes.

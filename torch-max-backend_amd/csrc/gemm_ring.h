@@ -99,7 +99,8 @@ constexpr bool kRingPersistent = ring_waves_per_simd(BM, BN, BK, WAVES, R) <= 2;
 // K_TAIL: K may end inside a stage (a multiple of 8). The lanes of the last stage whose k lies past the end fetch zeros.
 // SHORT_CHAINS: every 512 of K the accumulators are added to a second set and start from zero. These tiles took over products
 // of split launches, whose float32 sums (a float32 residual stream keeps them) are off by 1.5e-7 .. 2e-7 of the result
-// (rms, K = 2304 and 3072) where one chain of additions is by 2.9e-7 .. 3.4e-7. Each addition waits for the matrix pipes,
+// (rms, K = 2304 and 3072) where one chain of additions is by 2.9e-7 .. 3.4e-7 (a transposed A of K 2048 .. 4096: split
+// 1.4e-7 .. 2.0e-7, one chain 2.7e-7 .. 4.0e-7, chains of 512 1.3e-7 .. 1.4e-7). Each addition waits for the matrix pipes,
 // 0.15 us. Below K = 2048 the larger tiles took over from other rings: one chain, and the same bits.
 template <typename T, int BM, int BN, int BK, int WAVES_M, int WAVES_N, int R, bool B_KMAJOR, int EPI,
           bool A_MMAJOR = false, bool OUT_F32 = false, bool MI16_ = (BK == 64), bool SHORT_CHAINS = false,
