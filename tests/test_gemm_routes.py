@@ -133,6 +133,18 @@ def test_a_large_transposed_a_with_a_residual_is_multiplied_and_added():
     assert route(256, 256, 256, **rounded) == ek.ERR_UNSUPPORTED     # (the bits of the rings' product)
 
 
+def test_a_transposed_a_with_a_gelu_runs_split_where_one_round_takes_the_product_alone():
+    """The reduction of a split launch evaluates it; the rings take such a product without one only, and the any-layout
+    kernel is 1.5 times as long on it."""
+    ek = _ek()
+    for m, n, k in ((3072, 768, 2048), (2304, 768, 2048), (2304, 1024, 3072), (3072, 768, 4096)):
+        plain = dict(ta=1, workspace=PLENTY)
+        for step in (0, ek.EPI_ROUND_LIKE_UNFUSED):
+            assert route(m, n, k, epilogue=step, **plain)[0] == TRANSPOSED_A, (m, n, k)
+            for gelu in (ek.EPI_GELU_TANH, ek.EPI_GELU_ERF):
+                assert route(m, n, k, epilogue=gelu | step, **plain)[0] == SPLITK, (m, n, k)
+
+
 @pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])
 def test_a_residual_that_is_added_with_the_bits_of_two_operations_is_carried_where_the_product_runs(dtype_name):
     """fp32, and 16-bit with TMB_EPI_ROUND_LIKE_UNFUSED: the kernel, tile and splits of the product alone, or none; all

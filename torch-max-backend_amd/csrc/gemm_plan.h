@@ -483,9 +483,10 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
   if (aligned && whole_columns && small_applies(batch, g.m, g.n, g.k))
     return {TMB_GEMM_SMALL, small_tile(batch, g.m, g.n, g.k), 0};
   if (workspace_bytes > 0) {
-    // (a transposed A with a residual: the reduction adds it, the ring would not)
-    const SplitKPlan plan = trans_a && g.residual != nullptr ? splitk_plan(batch, g.m, g.n, g.k)
-                                                             : splitk_or_whole(batch, g.m, g.n, g.k, trans_a);
+    // (a transposed A with a residual or a GELU: the reduction takes them along, the ring would not)
+    const bool split_only = trans_a && (g.residual != nullptr || epilogue != TMB_EPI_NONE);
+    const SplitKPlan plan = split_only ? splitk_plan(batch, g.m, g.n, g.k)
+                                       : splitk_or_whole(batch, g.m, g.n, g.k, trans_a);
     const bool operands_ok = trans_a ? mfma_transposed_a_eligible(g, batch, trans_a, trans_b, TMB_EPI_NONE)
                                      : aligned && whole_columns;
     if (plan.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
