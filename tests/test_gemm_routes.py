@@ -145,6 +145,41 @@ def test_a_transposed_a_with_a_gelu_runs_split_where_one_round_takes_the_product
                 assert route(m, n, k, epilogue=gelu | step, **plain)[0] == SPLITK, (m, n, k)
 
 
+ONE_ROUND = [(3072, 768, 2048), (3064, 776, 2304), (3072, 768, 4096)]    # (m, n, k) of a transposed A, else split
+
+
+def test_a_residual_on_a_transposed_a_is_carried_where_a_split_launch_carried_it():
+    ek = _ek()
+    for m, n, k in ONE_ROUND:
+        told = ek.lib().tmb_gemm_layout_workspace_bytes(1, m, n, k, 1, 0, ek.BF16)
+        rounded = dict(ta=1, residual=1, epilogue=ek.EPI_ROUND_LIKE_UNFUSED)
+        assert route(m, n, k, ta=1, workspace=told) == (TRANSPOSED_A, 0, 0)
+        assert route(m, n, k, workspace=told, **rounded) == (TRANSPOSED_A, 0, 0)
+        assert route(m, n, k, **rounded) == ek.ERR_UNSUPPORTED       # without the scratch, as ever
+        assert route(m, n, k, ta=1, residual=1, workspace=told)[0] == SPLITK
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
+@pytest.mark.parametrize("mnk", ONE_ROUND)
+def test_that_residual_has_the_bits_of_two_operations(mnk, dtype_name):
+    import torch
+    from torch_mojo_backend.eager_kernels import hip_ops
+    m, n, k = mnk
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x, w, bias, r = (torch.randn(*s, generator=g, device="cuda").to(getattr(torch, dtype_name))
+                     for s in ((k, m), (k, n), (n,), (m, n)))
+    out, ws = torch.empty_like(r), torch.empty(128 << 20, dtype=torch.uint8, device="cuda")
+    ek = _ek()
+    code = hip_ops.code_of(r.dtype)
+    for b in (None, bias):
+        assert ek.lib().tmb_gemm_residual_ws(
+            out.data_ptr(), x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), r.data_ptr(), 1, m, n, k, m, n,
+            n, n, 0, 0, 0, 0, 1, 0, code, code, code, ek.EPI_ROUND_LIKE_UNFUSED, ws.data_ptr(), ws.numel(),
+            torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(out, hip_ops.gemm(x.t(), w, b) + r)
+
+
 @pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])
 def test_a_residual_that_is_added_with_the_bits_of_two_operations_is_carried_where_the_product_runs(dtype_name):
     """fp32, and 16-bit with TMB_EPI_ROUND_LIKE_UNFUSED: the kernel, tile and splits of the product alone, or none; all

@@ -474,6 +474,12 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
     GemmRoute r = route_16bit(alone, batch, trans_a, trans_b, epilogue, workspace_bytes);
     if (r.kernel == TMB_GEMM_STREAM64 && mfma_eligible(g, batch, trans_a, trans_b))
       r.kernel = TMB_GEMM_RING;  // (adds its four steps of K in the same order)
+    // (a transposed A that one round of the rings takes in place of a split launch: added where that launch's reduction did,
+    // by the tiles' way out)
+    if (r.kernel == TMB_GEMM_TRANSPOSED_A) {
+      const int splits = splitk_plan(batch, g.m, g.n, g.k).splits;
+      if (splits > 0 && workspace_bytes >= static_cast<size_t>(splits) * g.m * g.n * 4) return r;
+    }
     if (r.kernel == TMB_GEMM_TRANSPOSED_A || r.kernel == TMB_GEMM_STREAM64 || r.kernel == TMB_GEMM_SIMT)
       return {TMB_ERR_UNSUPPORTED, 0, 0};
     return r;
