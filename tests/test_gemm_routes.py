@@ -133,16 +133,18 @@ def test_a_large_transposed_a_with_a_residual_is_multiplied_and_added():
     assert route(256, 256, 256, **rounded) == ek.ERR_UNSUPPORTED     # (the bits of the rings' product)
 
 
-def test_a_transposed_a_with_a_gelu_runs_split_where_one_round_takes_the_product_alone():
-    """The reduction of a split launch evaluates it; the rings take such a product without one only, and the any-layout
-    kernel is 1.5 times as long on it."""
+def test_a_transposed_a_with_a_gelu_does_not_fall_back_where_one_round_takes_the_product_alone():
+    """The reduction of a split launch evaluates it, or, where it is to have the bits of two operations, the tiles that the
+    product alone runs on; the any-layout kernel is 1.5 times as long."""
     ek = _ek()
     for m, n, k in ((3072, 768, 2048), (2304, 768, 2048), (2304, 1024, 3072), (3072, 768, 4096)):
         plain = dict(ta=1, workspace=PLENTY)
         for step in (0, ek.EPI_ROUND_LIKE_UNFUSED):
             assert route(m, n, k, epilogue=step, **plain)[0] == TRANSPOSED_A, (m, n, k)
-            for gelu in (ek.EPI_GELU_TANH, ek.EPI_GELU_ERF):
-                assert route(m, n, k, epilogue=gelu | step, **plain)[0] == SPLITK, (m, n, k)
+        for gelu in (ek.EPI_GELU_TANH, ek.EPI_GELU_ERF):
+            assert route(m, n, k, epilogue=gelu, **plain)[0] == SPLITK, (m, n, k)
+            assert route(m, n, k, epilogue=gelu | ek.EPI_ROUND_LIKE_UNFUSED, **plain)[0] == TRANSPOSED_A, (m, n, k)
+            assert route(m, n, k, epilogue=gelu | ek.EPI_ROUND_LIKE_UNFUSED, ta=1)[0] == ANY
 
 
 ONE_ROUND = [(3072, 768, 2048), (3064, 776, 2304), (3072, 768, 4096)]    # (m, n, k) of a transposed A, else split
@@ -162,7 +164,7 @@ def test_a_residual_on_a_transposed_a_is_carried_where_a_split_launch_carried_it
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype_name", ["bfloat16", "float16"])
 @pytest.mark.parametrize("mnk", ONE_ROUND)
-def test_that_residual_has_the_bits_of_two_operations(mnk, dtype_name):
+def test_that_residual_and_a_gelu_have_the_bits_of_two_operations(mnk, dtype_name):
     import torch
     from torch_mojo_backend.eager_kernels import hip_ops
     m, n, k = mnk
@@ -177,7 +179,14 @@ def test_that_residual_has_the_bits_of_two_operations(mnk, dtype_name):
             out.data_ptr(), x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), r.data_ptr(), 1, m, n, k, m, n,
             n, n, 0, 0, 0, 0, 1, 0, code, code, code, ek.EPI_ROUND_LIKE_UNFUSED, ws.data_ptr(), ws.numel(),
             torch.cuda.current_stream().cuda_stream) == 0
-        assert torch.equal(out, hip_ops.gemm(x.t(), w, b) + r)
+        plain = hip_ops.gemm(x.t(), w, b)
+        assert torch.equal(out, plain + r)
+        for gelu, approximate in ((ek.EPI_GELU_TANH, "tanh"), (ek.EPI_GELU_ERF, "none")):
+            assert ek.lib().tmb_gemm_ws(
+                out.data_ptr(), x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), 1, m, n, k, m, n, n, 0, 0,
+                0, 1, 0, code, gelu | ek.EPI_ROUND_LIKE_UNFUSED, ws.data_ptr(), ws.numel(),
+                torch.cuda.current_stream().cuda_stream) == 0
+            assert torch.equal(out, hip_ops.gelu(plain, approximate))
 
 
 @pytest.mark.parametrize("dtype_name", ["BF16", "F16", "F32"])

@@ -489,15 +489,19 @@ static inline GemmRoute route_16bit(const GemmArgs& g, int64_t batch, int trans_
   if (aligned && whole_columns && small_applies(batch, g.m, g.n, g.k))
     return {TMB_GEMM_SMALL, small_tile(batch, g.m, g.n, g.k), 0};
   if (workspace_bytes > 0) {
-    // (a transposed A with a residual or a GELU: the reduction takes them along, the ring would not)
-    const bool split_only = trans_a && (g.residual != nullptr || epilogue != TMB_EPI_NONE);
-    const SplitKPlan plan = split_only ? splitk_plan(batch, g.m, g.n, g.k)
-                                       : splitk_or_whole(batch, g.m, g.n, g.k, trans_a);
+    // (a transposed A with a residual or a GELU: the reduction takes them along, the rings do not, but for a GELU that is to
+    // have the bits of two operations, on the tiles that the product alone runs on)
+    const bool gelu_after = trans_a && epilogue != TMB_EPI_NONE;
+    const bool split_only = trans_a && (g.residual != nullptr || (gelu_after && !g.round_like_unfused));
+    const SplitKPlan split = splitk_plan(batch, g.m, g.n, g.k);
+    const SplitKPlan plan = split_only ? split : splitk_or_whole(batch, g.m, g.n, g.k, trans_a);
     const bool operands_ok = trans_a ? mfma_transposed_a_eligible(g, batch, trans_a, trans_b, TMB_EPI_NONE)
                                      : aligned && whole_columns;
-    if (plan.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
-        workspace_bytes >= static_cast<size_t>(plan.splits) * g.m * g.n * 4)
-      return {TMB_GEMM_SPLITK, plan.tile == 256 ? 1 : 0, plan.splits};
+    if (split.splits > 0 && operands_ok && g.m * g.n < (int64_t{1} << 31) &&
+        workspace_bytes >= static_cast<size_t>(split.splits) * g.m * g.n * 4) {
+      if (plan.splits > 0) return {TMB_GEMM_SPLITK, plan.tile == 256 ? 1 : 0, plan.splits};
+      if (gelu_after) return {TMB_GEMM_TRANSPOSED_A, 0, 0};
+    }
   }
   if (g.residual == nullptr && mfma_transposed_a_eligible(g, batch, trans_a, trans_b, epilogue))
     return {TMB_GEMM_TRANSPOSED_A, 0, 0};

@@ -305,7 +305,10 @@ static int gemm_typed(const GemmArgs& g, int64_t batch, int trans_a, int trans_b
       case TMB_GEMM_SPLITK:
         return launch_splitk<T, EPI>(g, SplitKPlan{r.splits, r.tile == 1 ? 256 : 128, 0.0}, trans_a, trans_b,
                                      static_cast<float*>(workspace), stream);
-      case TMB_GEMM_TRANSPOSED_A: return mfma_transposed_a<T>(g, batch, stream);
+      case TMB_GEMM_TRANSPOSED_A:
+        if constexpr (EPI == TMB_EPI_NONE) return mfma_transposed_a<T>(g, batch, stream);
+        // (the tile of one round, K >= 2048: no other form is asked for a GELU)
+        else return launch_ring<T, 128, 128, 64, 4, 2, 3, false, EPI, true, false, false, true>(g, batch, stream);
       case TMB_GEMM_ANY:
         if (r.splits == 0) return gemm_any(g, batch, r.tile, trans_a, trans_b, BF16, EPI, stream);
         return launch_split<T, EPI>(g, r.splits, stream, workspace, [&](const GemmArgs& part) {
