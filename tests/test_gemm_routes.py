@@ -296,6 +296,19 @@ def test_the_launch_of_an_epilogue_does_not_depend_on_the_plain_product_before(r
         assert _launch(recorded, a, b, **gelu) == alone and _launch(recorded, a, b) == plain
 
 
+def test_a_product_that_runs_whole_is_given_no_scratch(recorded):
+    """A transposed A: one round of whole tiles takes the first, a split launch the second."""
+    import torch
+    for m, n, k, pitch in ((3072, 768, 2048, 3072), (3000, 768, 2048, 3072), (768, 768, 16384, 768)):
+        a, b = torch.zeros(k, pitch).bfloat16()[:, :m].t(), torch.zeros(k, n).bfloat16()
+        splits = route(m, n, k, ta=1, lda=pitch, workspace=PLENTY)[2]
+        (name, _, scratch), = _launch(recorded, a, b)
+        assert scratch == splits * m * n * 4 and (name == "tmb_gemm_ws") == (splits > 0), (m, n, k)
+        residual = torch.zeros(m, n).bfloat16()
+        (name, _, _), = _launch(recorded, a, b, residual=residual)
+        assert name == "tmb_gemm_residual_ws"
+
+
 def test_products_of_depth_64_stay_on_their_kernel_beyond_four_gigabytes():
     """It addresses a tile at a time; the rings' 32-bit offsets from the base end there."""
     for m in (8192, (1 << 25) - 128, 1 << 25, 1 << 26):

@@ -445,11 +445,17 @@ def gemm(a: torch.Tensor, b: torch.Tensor, bias: Optional[torch.Tensor] = None,
         return out
     lib = _ek.lib()
     # few output tiles and a long K: the library splits K when it is handed scratch memory
-    key = (batch, m, n, k, la[0], lb[0], a.dtype)
+    # (a transposed A by itself may run whole where the library, which is not told of residuals, names the split's scratch)
+    alone_t = bool(la[0]) and residual is None and a.element_size() == 2 and \
+        _mfma_layouts_ok(a, b, la, lb, m, n, k, batched, epilogue == _ek.EPI_NONE)
+    key = (batch, m, n, k, la[0], lb[0], a.dtype, (la[1], lb[1]) if alone_t else None)
     ws_bytes = _GEMM_WS_BYTES.get(key) if in_place_ws is None else in_place_ws
     if ws_bytes is None:  # a pure function of shape and layout: asked once for each
-        ws_bytes = _GEMM_WS_BYTES[key] = lib.tmb_gemm_layout_workspace_bytes(batch, m, n, k, la[0], lb[0],
-                                                                             code_of(a.dtype))
+        ws_bytes = lib.tmb_gemm_layout_workspace_bytes(batch, m, n, k, la[0], lb[0], code_of(a.dtype))
+        if ws_bytes and alone_t and lib.tmb_gemm_route(batch, m, n, k, la[1], lb[1], 0, 0, 1, 1, la[0], lb[0],
+                                                       code_of(a.dtype), epi_flags, 0, ws_bytes) >> 16 == 0:
+            ws_bytes = 0
+        _GEMM_WS_BYTES[key] = ws_bytes
 
     def unfused_residual():
         # no kernel carries this epilogue for these operands: product first, then the add.
