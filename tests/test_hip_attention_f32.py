@@ -102,3 +102,14 @@ def test_a_float32_graph_runs_one_fused_attention_per_block(monkeypatch):
         torch.compile(blind, backend=mojo_backend, fullgraph=True)(idx.cuda())
     assert len(calls) == 2
     torch.testing.assert_close(got.cpu().double(), want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("scale", [0.1, 0.3, 1.0 / 7.0])
+def test_the_backward_has_the_probabilities_of_the_forward(scale):
+    """One key: its probability is exp(0) / 1, exactly, where the backward rounds the scaled score as the forward did whose
+    maximum it takes off. (Scores of 1e6: their rounding is some hundredths.)"""
+    q, k, v, dout = (seeded((2, 3, 1, 64), seed=i, scale=200.0 if i < 2 else 1.0).cuda() for i in range(4))
+    ops = _ops()
+    out, stats = ops.attention_f32(q, k, v, scale, True, return_stats=True)
+    _, _, dv = ops.attention_f32_backward(dout, q, k, v, out.transpose(1, 2), stats, scale, True)
+    assert torch.equal(out.transpose(1, 2), v) and torch.equal(dv, dout)

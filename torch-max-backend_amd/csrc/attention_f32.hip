@@ -93,6 +93,12 @@ __device__ __forceinline__ float f32_exp_nonpositive(float x) {
   return __builtin_fmaf(e, lo * kLn2, e);
 }
 
+// A scaled score, rounded by itself wherever it is formed: the backward takes the forward's maximum off the same number
+__device__ __forceinline__ float f32_scaled(float score, float scale) {
+#pragma clang fp contract(off)
+  return score * scale;
+}
+
 __device__ __forceinline__ void f32_clear(af32x16_t& x) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) x[i] = 0.0f;
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     f32_load_row(kf, kr, next * kF32Block, lane);  // arrives while the values are multiplied
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] *= a.scale;
+    for (int r = 0; r < 16; ++r) s[r] = f32_scaled(s[r], a.scale);
     if ((a.causal && k0 + kF32Block - 1 > q0) || k0 + kF32Block > a.kv_len) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      s[r] = f32_exp_nonpositive(s[r] * a.scale - m) * inv_l * (dp[r] - delta) * a.scale;
+      s[r] = f32_exp_nonpositive(f32_scaled(s[r], a.scale) - m) * inv_l * (dp[r] - delta) * a.scale;
     if ((a.causal && k0 + kF32Block - 1 > q0) || k0 + kF32Block > a.kv_len) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -491,7 +497,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const af32x4_t st = row_stats[wave][8 * (r >> 2) + 4 * half + (r & 3)];
-      s[r] = f32_exp_nonpositive(s[r] * a.scale - st[0]) * st[1];
+      s[r] = f32_exp_nonpositive(f32_scaled(s[r], a.scale) - st[0]) * st[1];
       ds[r] = s[r] * (ds[r] - st[2]) * a.scale;
       if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (all the statistics at once would be 64 registers)
     }
