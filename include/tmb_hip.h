@@ -302,7 +302,9 @@ int tmb_attention_bwd(void* dq, void* dk, void* dv, const void* dout, const void
  * Strides are in elements, multiples of 4, a token's below 2^30 / (tokens + 32), bases 16-byte aligned (`stats`: 8). `workspace` is device memory of
  * tmb_attention_f32_bwd_workspace_bytes(batch, heads, q_len) bytes, 16-byte aligned, that the backward
  * overwrites. Same status codes as the 16-bit entry points; less than 2^24 blocks of 32 queries
- * (keys) over all heads. Replaces the bmm, mul, masked_fill, _softmax, bmm chain of
+ * (keys) over all heads. An infinite or NaN row that the causal mask hides from a query (key) does not reach it, but for
+ * those of one aligned block of 32 with one that sees it, which may get NaN (0 * infinity, which a product with the whole
+ * score matrix gives to all). Replaces the bmm, mul, masked_fill, _softmax, bmm chain of
  * aten_functions.py:443-677 in float32 graphs. */
 int tmb_attention_f32_fwd(void* out, void* stats, const void* q, const void* k, const void* v, int64_t batch,
                           int64_t heads, int64_t q_len, int64_t kv_len, int64_t head_dim, const int64_t* q_strides,

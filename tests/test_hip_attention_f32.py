@@ -83,6 +83,31 @@ def test_attention_f32_with_scores_far_apart_infinite_and_nan():
     torch.testing.assert_close(got[1:40].double(), want[1:40], rtol=0, atol=2 * 40 * 66 * EPS * 500)
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_f32_with_values_that_are_not_finite(bad):
+    """Row 70 of one operand, in the third block of 32 of five: what sees it is not finite, what does not and shares no
+    block with what does has the bits that it has without."""
+    q, k, v, dout = (seeded((1, 2, 150, 64), seed=i).cuda() for i in range(4))
+    ops = _ops()
+
+    def run(q, k, v, dout):
+        out, stats = ops.attention_f32(q, k, v, 0.125, True, return_stats=True)
+        return out.transpose(1, 2), *ops.attention_f32_backward(dout, q, k, v, out.transpose(1, 2), stats, 0.125, True)
+
+    def spoilt(x):
+        x = x.clone()
+        x[:, :, 70] = bad
+        return x
+
+    clean = run(q, k, v, dout)
+    out, dq, dk, dv = run(q, k, spoilt(v), dout)
+    assert not out[:, :, 70:].isfinite().any() and not dq[:, :, 70:].isfinite().any()
+    assert torch.equal(out[:, :, :64], clean[0][:, :, :64]) and torch.equal(dq[:, :, :64], clean[1][:, :, :64])
+    _, _, dk, dv = run(q, k, v, spoilt(dout))       # query 70 sees keys 0 .. 70
+    assert not dk[:, :, :71].isfinite().any() and not dv[:, :, :71].isfinite().any()
+    assert torch.equal(dk[:, :, 96:], clean[2][:, :, 96:]) and torch.equal(dv[:, :, 96:], clean[3][:, :, 96:])
+
+
 def test_a_float32_graph_runs_one_fused_attention_per_block(monkeypatch):
     from demo_scripts.gpt2 import build_gpt2_small, seeded_tokens
     from torch_mojo_backend import mojo_backend

@@ -31,6 +31,11 @@
 //
 // Scores are rounded to float32 before and after the scale, as a product and a multiplication store them, and the
 // exponential is exp_f32 of the difference to the row's maximum: what a separate softmax computes.
+//
+// Infinities and NaN: what a query sees reaches it as through a softmax and two products. What the mask hides from it is
+// multiplied by its probability of 0 only within its own block of 32, by the MFMAs: an infinite or NaN value (in dq: key;
+// in dk, dv: query, dout) that is hidden from all of a block does not reach the block, where a product with the whole
+// score matrix would give NaN, and one that part of a block sees leaves NaN in the rest of that block too.
 #include "tmb_common.h"
 
 namespace tmb {
