@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 CHECKS = ["gpt2_training_step_gradients_match_cpu", "training_graph_runs_the_fused_attention_forward_and_backward",
           "float32_training_graph_runs_the_fused_attention_forward_and_backward",
+          "float32_graphs_over_host_tensors_keep_the_separate_ops",
           "attention_backward_follows_the_route_the_forward_took",
           "sdpa_training_graph_runs_the_fused_forward_and_backward",
           "one_sgd_step_lowers_the_loss",

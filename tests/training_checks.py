@@ -128,6 +128,31 @@ def float32_training_graph_runs_the_fused_attention_forward_and_backward():
         torch._dynamo.reset()
 
 
+def float32_graphs_over_host_tensors_keep_the_separate_ops():
+    """Training and evaluation of one model on host tensors run the same attention, op by op: the same logits."""
+    from demo_scripts.gpt2 import build_gpt2_small, seeded_tokens
+    from torch_mojo_backend import mojo_backend
+    from torch_mojo_backend.eager_kernels import hip_ops
+
+    calls = []
+    for name in ("attention_f32", "attention_f32_backward"):
+        real = getattr(hip_ops, name)
+        setattr(hip_ops, name, lambda *a, _real=real, _name=name, **k: (calls.append(_name), _real(*a, **k))[1])
+    idx, targets = seeded_tokens(2, 77, seed=0), seeded_tokens(2, 77, seed=1)
+    ref, model = build_gpt2_small(seed=0, n_layer=2).double(), build_gpt2_small(seed=0, n_layer=2)
+    compiled = torch.compile(model, backend=mojo_backend)
+    with torch.no_grad():
+        evaluated, _ = compiled(idx)
+    logits, _ = compiled(idx)
+    assert torch.equal(logits.detach(), evaluated)
+    F.cross_entropy(logits.view(-1, logits.shape[-1]), targets.view(-1)).backward()
+    assert calls == []
+    _loss(ref, idx, targets).backward()
+    for (name, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
+        scale = q.grad.abs().max().item() + 1e-12
+        assert (p.grad.double() - q.grad).abs().max().item() <= 2e-4 * scale, name
+
+
 def attention_backward_follows_the_route_the_forward_took():
     """The mask buffer edited between forward and backward: the backward step takes the route the
     forward recorded in its log-sum-exp (all values: fused; no elements: op by op) and never
