@@ -5,7 +5,7 @@ check_functions_are_equivalent, torch_mojo_backend/testing.py:139-166)."""
 import pytest
 import torch
 
-from demo_scripts.gpt2 import build_gpt2_small, seeded_tokens
+from demo_scripts.gpt2 import GPT, GPTConfig, build_gpt2_small, seeded_tokens
 from helpers import seeded
 
 pytestmark = pytest.mark.gpu
@@ -18,10 +18,23 @@ def _hot_counts():
                                                af.aten_argmax, af.aten_gelu)}
 
 
-def test_gpt2_small_fp32_batch1_seq128_matches_cpu_eager():
+def _counted(monkeypatch, *names):
+    """name -> calls of these launchers so far."""
+    from torch_mojo_backend.eager_kernels import hip_ops
+    calls = dict.fromkeys(names, 0)
+    for name in names:
+        def counting(*a, _real=getattr(hip_ops, name), _name=name, **kw):
+            calls[_name] += 1
+            return _real(*a, **kw)
+        monkeypatch.setattr(hip_ops, name, counting)
+    return calls
+
+
+def test_gpt2_small_fp32_batch1_seq128_matches_cpu_eager(monkeypatch):
     """Workload: 12 layers, d 768, 12 heads, B=1, T=128, float32, seed 0."""
     from torch_mojo_backend import mojo_backend
 
+    launched = _counted(monkeypatch, "attention_f32", "softmax_scaled")
     model = build_gpt2_small(seed=0)
     idx = seeded_tokens(1, 128, seed=0)
     with torch.no_grad():
@@ -33,13 +46,14 @@ def test_gpt2_small_fp32_batch1_seq128_matches_cpu_eager():
         logits, nxt = compiled(idx.to("cuda"))
     after = _hot_counts()
     assert logits.shape == (1, 128, 50257) and logits.dtype == torch.float32
-    # every hot op of the graph went through the HIP mapping functions
+    # every hot op of the graph went through the HIP mapping functions or the launchers of the fused steps
     # (of the 48 addmm, c_fc's 12 run fused with their gelu and the 24 projections in front of a
     # residual add run fused with that add; those steps launch the GEMM kernel directly)
     assert after["aten_addmm"] - before["aten_addmm"] == 12
-    assert after["aten_bmm"] - before["aten_bmm"] == 24
-    # mul + masked_fill + _softmax run as one fused step that launches the kernel directly
+    # bmm + mul + masked_fill + _softmax + bmm run as one fused step a layer that launches the kernel directly
+    assert after["aten_bmm"] - before["aten_bmm"] == 0
     assert after["aten__softmax"] - before["aten__softmax"] == 0
+    assert launched == {"attention_f32": 12, "softmax_scaled": 0}
     assert after["aten_native_layer_norm"] - before["aten_native_layer_norm"] == 25
     assert after["aten_mm"] - before["aten_mm"] == 1
     assert after["aten_argmax"] - before["aten_argmax"] == 1
@@ -51,6 +65,24 @@ def test_gpt2_small_fp32_batch1_seq128_matches_cpu_eager():
     top2 = want_logits[:, -1, :].topk(2, dim=-1).values
     if (top2[:, 0] - top2[:, 1]).min() > 2e-4:
         assert torch.equal(nxt.cpu(), want_next)
+
+
+def test_float32_heads_of_another_width_run_op_by_op(monkeypatch):
+    """24 heads of 32, which the fused attention does not take: two bmm and a masked softmax a layer."""
+    from torch_mojo_backend import mojo_backend
+
+    launched = _counted(monkeypatch, "attention_f32", "softmax_scaled")
+    idx = seeded_tokens(2, 77, seed=0)
+    with torch.no_grad():
+        torch.manual_seed(0)
+        model = GPT(GPTConfig(n_layer=2, n_head=24)).eval()
+        want, _ = model(idx)
+        compiled = torch.compile(model.to("cuda"), backend=mojo_backend)
+        before = _hot_counts()
+        got, _ = compiled(idx.to("cuda"))
+    assert _hot_counts()["aten_bmm"] - before["aten_bmm"] == 4
+    assert launched == {"attention_f32": 0, "softmax_scaled": 2}
+    torch.testing.assert_close(got.cpu(), want, rtol=1e-4, atol=1e-4)
 
 
 def test_gpt2_small_bf16_logits_vs_fp32_oracle():

@@ -8,6 +8,7 @@ the process's accelerator and its autograd engine can no longer run a backward p
 tensors (internal assert in torch/csrc/autograd/engine.cpp), so these checks must not share a
 process with the eager-device tests."""
 
+import copy
 import sys
 
 import torch
@@ -20,32 +21,47 @@ def _loss(model, idx, targets):
 
 
 def gpt2_training_step_gradients_match_cpu():
-    from demo_scripts.gpt2 import build_gpt2_small, seeded_tokens
+    """Heads of 64, whose attention and its gradient are a fused step each, and of 32, which run op by op."""
+    from demo_scripts.gpt2 import GPT, GPTConfig, seeded_tokens
     from torch_mojo_backend import MAPPING_TORCH_ATEN_TO_MOJO as mapping
     from torch_mojo_backend import mojo_backend
+    from torch_mojo_backend.eager_kernels import hip_ops
 
-    idx, targets = seeded_tokens(2, 32, seed=0), seeded_tokens(2, 32, seed=1)
-    ref = build_gpt2_small(seed=0, n_layer=2)
-    ref_loss = _loss(ref, idx, targets)
-    ref_loss.backward()
-
-    model = build_gpt2_small(seed=0, n_layer=2).cuda()
-    compiled = torch.compile(model, backend=mojo_backend)
+    fused = []
+    for entry in ("attention_f32", "attention_f32_backward"):
+        real = getattr(hip_ops, entry)
+        setattr(hip_ops, entry, lambda *a, _real=real, _name=entry, **k: (fused.append(_name), _real(*a, **k))[1])
     aten = torch.ops.aten
-    watched = (aten.gelu_backward, aten._softmax_backward_data, aten.native_layer_norm_backward,
-               aten.mm)
-    before = {op: mapping[op].call_count for op in watched}
-    loss = _loss(compiled, idx.cuda(), targets.cuda())
-    loss.backward()
-    torch.testing.assert_close(loss.cpu(), ref_loss, rtol=1e-5, atol=1e-5)
-    for (name, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
-        assert p.grad is not None, name
-        scale = q.grad.abs().max().item() + 1e-12
-        assert (p.grad.cpu() - q.grad).abs().max().item() <= 2e-4 * scale, name
-    grew = {op for op in watched if mapping[op].call_count > before[op]}
-    # 2 layers: a GELU, a softmax and two layer norms per block plus the final layer norm, and
-    # the weight / input gradient GEMMs
-    assert grew == set(watched), f"not every backward twin ran: {grew}"
+    idx, targets = seeded_tokens(2, 32, seed=0), seeded_tokens(2, 32, seed=1)
+    for heads in (12, 24):
+        torch.manual_seed(0)
+        ref = GPT(GPTConfig(n_layer=2, n_head=heads)).eval()
+        model = copy.deepcopy(ref).cuda()
+        ref_loss = _loss(ref, idx, targets)
+        ref_loss.backward()
+
+        compiled = torch.compile(model, backend=mojo_backend)
+        watched = (aten.gelu_backward, aten._softmax_backward_data, aten.bmm, aten.native_layer_norm_backward,
+                   aten.mm)
+        before = {op: mapping[op].call_count for op in watched}
+        fused.clear()
+        loss = _loss(compiled, idx.cuda(), targets.cuda())
+        loss.backward()
+        torch.testing.assert_close(loss.cpu(), ref_loss, rtol=1e-5, atol=1e-5)
+        for (name, p), (_, q) in zip(model.named_parameters(), ref.named_parameters()):
+            assert p.grad is not None, name
+            scale = q.grad.abs().max().item() + 1e-12
+            assert (p.grad.cpu() - q.grad).abs().max().item() <= 2e-4 * scale, (heads, name)
+        grew = {op: mapping[op].call_count - before[op] for op in watched}
+        # 2 layers: a GELU and two layer norms per block plus the final layer norm, and the weight / input gradient
+        # GEMMs; attention as one launch each way, or as a softmax backward and six products
+        assert grew[aten.gelu_backward] == 2 and grew[aten.native_layer_norm_backward] == 5 and grew[aten.mm] > 0, grew
+        if heads == 12:
+            assert fused == ["attention_f32"] * 2 + ["attention_f32_backward"] * 2, fused
+            assert grew[aten._softmax_backward_data] == grew[aten.bmm] == 0, grew
+        else:
+            assert fused == [] and grew[aten._softmax_backward_data] == 2 and grew[aten.bmm] == 12, (fused, grew)
+        torch._dynamo.reset()
 
 
 def training_graph_runs_the_fused_attention_forward_and_backward():
