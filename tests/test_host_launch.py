@@ -148,6 +148,13 @@ def test_a_plan_is_not_used_where_layout_or_arguments_differ():
     assert not torch.equal(a, b)
     assert ops.layer_norm(x, [96], g, None, 1e-5, need_stats=False)[1] is None
 
+    # a number in a tensor may have changed since the call that left a plan
+    for number in (torch.tensor(1e-5), torch.tensor(1e-5).numpy()):
+        for value in (1e-5, 10.0, 1e-5):
+            number[...] = value
+            got = [ops.layer_norm(x, [96], g, None, number)[0] for _ in range(2)]
+            assert torch.equal(got[0], b if value > 1 else a) and torch.equal(got[1], got[0])
+
     class Wrapped(torch.Tensor):
         pass
 

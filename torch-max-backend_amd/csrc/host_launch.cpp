@@ -10,8 +10,8 @@
 // A plan's key is everything the launcher looks at: per tensor type, device, sizes, strides and the address modulo 16,
 // and the call's other arguments. Addresses are not part of it: every call passes those of its own tensors, and
 // allocates results and scratch of its own on PyTorch's allocator. Calls this file does not take (a subclass, a tensor without
-// plain storage, an unknown layout) return None and run in Python. All state is guarded by the interpreter lock, which
-// is given up during the launch, as ctypes does.
+// plain storage, an argument that is no constant, an unknown layout) return None and run in Python. All state is guarded by
+// the interpreter lock, which is given up during the launch, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -115,6 +115,18 @@ bool usable(const at::Tensor& t) {
   return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(odd) && t.has_storage();
 }
 
+// What a plan may hold on to of a call's other arguments: values that nobody can change. (A 0-dimensional tensor given for a
+// number equals itself whatever it holds by then.)
+bool constant(PyObject* o, int depth = 0) {
+  if (o == Py_None || PyBool_Check(o) || PyLong_CheckExact(o) || PyFloat_CheckExact(o) || PyUnicode_CheckExact(o) ||
+      THPDtype_Check(o))
+    return true;
+  if (!PyTuple_CheckExact(o) || depth > 1) return false;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(o); ++i)
+    if (!constant(PyTuple_GET_ITEM(o, i), depth + 1)) return false;
+  return true;
+}
+
 struct Call {
   std::vector<int64_t> key;
   std::vector<Py_hash_t> hashes;
@@ -164,8 +176,9 @@ bool read_call(PyObject* const* args, Py_ssize_t nargs, Call& c) {
   auto mix = [&](uint64_t v) { h = (h ^ v) * 1099511628211ull, h ^= h >> 29; };
   for (const int64_t v : c.key) mix(static_cast<uint64_t>(v));
   for (Py_ssize_t i = 0; i < c.extra_count; ++i) {
+    if (!constant(c.extras[i])) return false;
     const Py_hash_t v = PyObject_Hash(c.extras[i]);
-    if (v == -1) {  // (not hashable)
+    if (v == -1) {
       PyErr_Clear();
       return false;
     }
