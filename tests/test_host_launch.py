@@ -167,3 +167,23 @@ def test_a_plan_is_not_used_where_layout_or_arguments_differ():
         out = ops.gelu(ops.gelu(x, "tanh"), "tanh")
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(out, ops.gelu(ops.gelu(x, "tanh"), "tanh"))
+
+
+@pytest.mark.gpu
+def test_plans_in_use_outlast_the_plans_of_many_layouts():
+    """As many layouts as three tables hold: the plan that every few of them use is there throughout, the first ones go."""
+    from torch_mojo_backend import eager_kernels as ek
+
+    host, x = _host(), torch.ones(4, 4, device="cuda")
+    host.forget()
+    spec = ("tmb_gelu", ek.address("tmb_gelu"), (("o", 0), ("t", 0), 16, ek.F32, 0, "stream"),
+            (((4, 4), None, torch.float32),), 0, 0)
+    assert host.keep(spec, 901, 1, x, "often") is True and host.planned(901, 1, x, "often") is not None
+    for i in range(3 * 8192):
+        assert host.keep(spec, 900, 1, x, i) is True
+        if i % 1000 == 0:
+            assert host.planned(901, 1, x, "often") is not None, i
+    assert host.planned(900, 1, x, 0) is None and host.planned(900, 1, x, 8192) is None
+    assert host.planned(900, 1, x, 3 * 8192 - 1) is not None and host.planned(900, 1, x, 2 * 8192 + 9) is not None
+    host.forget()
+    assert host.planned(901, 1, x, "often") is None

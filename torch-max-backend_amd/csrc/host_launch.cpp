@@ -21,6 +21,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
+#include <deque>
 #include <memory>
 #include <string>
 #include <unordered_map>
@@ -95,6 +97,8 @@ struct Plan {
   int64_t scratch = 0;
   bool single = true;
   std::vector<int> results;  // output numbers; -1: None
+  uint64_t hash = 0;
+  bool used = false;  // since it last stood in front of g_order
   ~Plan() {
     for (PyObject* o : extras) Py_DECREF(o);
   }
@@ -102,7 +106,10 @@ struct Plan {
 // (never destroyed: at the end of the process the interpreter that owns the plans' objects is gone)
 std::unordered_map<uint64_t, std::vector<std::shared_ptr<Plan>>>& g_plans =
     *new std::unordered_map<uint64_t, std::vector<std::shared_ptr<Plan>>>;
-size_t g_plan_count = 0;
+// The plans in the order in which they may go once there are kMostPlans: from the front, and one that has been used since
+// it last stood there goes to the back instead. A generation loop leaves a plan for every length of its cache; those of
+// its other launches stay. (Some 2 KB each.)
+std::deque<std::shared_ptr<Plan>>& g_order = *new std::deque<std::shared_ptr<Plan>>;
 constexpr size_t kMostPlans = 8192;
 PyObject* g_check = nullptr;  // check(name, status): raises
 
@@ -202,9 +209,26 @@ std::shared_ptr<Plan> find(const Call& c) {
       if (equal < 0) PyErr_Clear();
       same = equal == 1;
     }
-    if (same) return plan;
+    if (same) {
+      plan->used = true;
+      return plan;
+    }
   }
   return nullptr;
+}
+
+void drop_one() {
+  while (g_order.front()->used) {  // (ends: each one passed is marked unused)
+    g_order.front()->used = false;
+    g_order.push_back(std::move(g_order.front()));
+    g_order.pop_front();
+  }
+  const std::shared_ptr<Plan> plan = std::move(g_order.front());
+  g_order.pop_front();
+  const auto at = g_plans.find(plan->hash);
+  auto& same_hash = at->second;
+  same_hash.erase(std::find(same_hash.begin(), same_hash.end(), plan));
+  if (same_hash.empty()) g_plans.erase(at);
 }
 
 PyObject* launch(const Plan& plan, const Call& c) {
@@ -362,19 +386,17 @@ PyObject* keep(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     plan->extras.push_back(c.extras[i]);
   }
   if (find(c) != nullptr) Py_RETURN_FALSE;
-  if (g_plan_count >= kMostPlans) {
-    g_plans.clear();
-    g_plan_count = 0;
-  }
+  if (g_order.size() >= kMostPlans) drop_one();
+  plan->hash = c.hash;
+  g_order.push_back(plan);
   g_plans[c.hash].push_back(std::move(plan));
-  ++g_plan_count;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
 
 PyObject* forget(PyObject*, PyObject*) {
   g_plans.clear();
-  g_plan_count = 0;
+  g_order.clear();
   Py_RETURN_NONE;
 }
 
