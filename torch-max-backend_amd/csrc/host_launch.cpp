@@ -423,8 +423,9 @@ struct Step {
 };
 struct Program {
   std::vector<Step> steps;
-  PyObject* materialize;
-  PyObject* current_node;  // the context variable that names the running step's node
+  size_t most_arguments = 0;  // of one step
+  PyObject* materialize = nullptr;
+  PyObject* current_node = nullptr;  // the context variable that names the running step's node
   ~Program() {
     for (Step& s : steps) {
       Py_DECREF(s.function);
@@ -440,6 +441,7 @@ constexpr const char* kProgram = "tmb_program";
 void free_program(PyObject* capsule) { delete static_cast<Program*>(PyCapsule_GetPointer(capsule, kProgram)); }
 
 PyObject* program(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
   PyObject *steps, *materialize, *current_node;
   if (!PyArg_ParseTuple(args, "O!OO", &PyList_Type, &steps, &materialize, &current_node)) return nullptr;
   auto p = std::make_unique<Program>();
@@ -470,6 +472,7 @@ PyObject* program(PyObject*, PyObject* args) {
         Py_INCREF(PyTuple_GET_ITEM(part, j));
         s.arguments.push_back(PyTuple_GET_ITEM(part, j));
       }
+    p->most_arguments = std::max(p->most_arguments, s.arguments.size());
     s.flat = from != Py_None;
     if (s.flat) {
       if (!PyTuple_Check(from)) {
@@ -492,12 +495,16 @@ PyObject* program(PyObject*, PyObject* args) {
       if (PyErr_Occurred()) return nullptr;
     }
   }
-  return PyCapsule_New(p.release(), kProgram, free_program);
+  PyObject* capsule = PyCapsule_New(p.get(), kProgram, free_program);
+  if (capsule != nullptr) p.release();
+  return capsule;
+  END_HANDLE_TH_ERRORS
 }
 
 // run(program, env, failed): the steps in order, results into the list `env`. A step that raises leaves its number in
 // `failed`.
 PyObject* run(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
   PyObject *capsule, *env, *failed;
   if (!PyArg_ParseTuple(args, "OO!O!", &capsule, &PyList_Type, &env, &PyList_Type, &failed)) return nullptr;
   auto* p = static_cast<Program*>(PyCapsule_GetPointer(capsule, kProgram));
@@ -512,6 +519,7 @@ PyObject* run(PyObject*, PyObject* args) {
     return PyList_SetItem(env, slot, value) == 0;
   };
   std::vector<PyObject*> stack;
+  stack.reserve(p->most_arguments + 1);  // (no allocation, and so nothing that throws, between a step's own actions)
   for (size_t i = 0; i < p->steps.size(); ++i) {
     const Step& s = p->steps[i];
     PyObject* token = PyContextVar_Set(p->current_node, s.node);
@@ -565,6 +573,7 @@ PyObject* run(PyObject*, PyObject* args) {
     }
   }
   Py_RETURN_NONE;
+  END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef kMethods[] = {
