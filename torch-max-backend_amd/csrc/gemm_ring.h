@@ -55,7 +55,7 @@ __device__ __forceinline__ int ring_swizzle(int row) {
 }
 
 // What a lane fetches in place of operands past the end of K.
-static __device__ const uint32_t kRingZeros[4] = {0u, 0u, 0u, 0u};
+alignas(16) static __device__ const uint32_t kRingZeros[4] = {0u, 0u, 0u, 0u};
 
 template <int... Is, typename F>
 __device__ __forceinline__ void static_for_impl(std::integer_sequence<int, Is...>, F&& f) {
