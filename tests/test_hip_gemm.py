@@ -530,10 +530,11 @@ def test_mm_transposed_a_batched_and_strided():
 # ---- split-K (few output tiles, long K) ----------------------------------------------------------
 # (m, n, k, trans_a, trans_b): row-major A with both layouts of B and transposed A, on both tiles of the split launch
 # (test_gemm_routes.py checks that), ragged rows and columns, the fewest and the most splits; the rest are products whose
-# K the waves of one small tile share (the comparison with the unsplit kernel is one of a kernel with itself there)
+# K the waves of one small tile share, or that run whole in one round of ring tiles (the comparison with the unsplit kernel
+# is one of a kernel with itself there)
 SPLITK = [
-    (2000, 768, 3072, False, False), (2000, 768, 3072, False, True), (512, 2048, 8192, False, True),
-    (768, 3072, 4096, False, False), (3072, 768, 4096, False, True), (1800, 768, 8192, False, False),
+    (2000, 768, 5120, False, False), (2000, 768, 5120, False, True), (512, 2048, 8192, False, True),
+    (768, 3072, 5120, False, False), (3072, 768, 5120, False, True), (1800, 768, 8192, False, False),
     (264, 136, 4160, False, False), (100, 72, 8192, False, True), (3072, 768, 8192, True, False),
     (768, 768, 32768, True, False), (264, 136, 2048, True, False),
 ]
@@ -541,10 +542,14 @@ SHARED_BY_WAVES = [
     (1024, 768, 3072, False, False), (1024, 768, 3072, False, True), (128, 768, 4096, False, True),
     (264, 136, 2048, False, False), (100, 72, 2304, False, True),
 ]
+ONE_ROUND = [
+    (2000, 768, 3072, False, False), (2000, 768, 3072, False, True), (768, 3072, 4096, False, False),
+    (3072, 768, 4096, False, True),
+]
 
 
 @pytest.mark.parametrize("dtype", HALF)
-@pytest.mark.parametrize("case", SPLITK + SHARED_BY_WAVES)
+@pytest.mark.parametrize("case", SPLITK + SHARED_BY_WAVES + ONE_ROUND)
 def test_split_k_matches_float64_and_the_unsplit_kernel(case, dtype):
     m, n, k, ta, tb = case
     told = _ek().lib().tmb_gemm_layout_workspace_bytes(1, m, n, k, int(ta), int(tb), _ops().code_of(dtype))

@@ -64,9 +64,10 @@ def test_small_products_ragged_columns_batches_and_row_pitches(dtype):
 
 
 @pytest.mark.parametrize("dtype", HALF)
-@pytest.mark.parametrize("mnk", [(5, 1001, 768), (100, 768, 3072), (130, 768, 768), (300, 768, 4096), (2000, 768, 3072)])
+@pytest.mark.parametrize("mnk", [(5, 1001, 768), (100, 768, 3072), (130, 768, 768), (300, 768, 4096), (2000, 768, 3072),
+                                 (2000, 768, 5120)])
 def test_small_epilogues(mnk, dtype):
-    """Residual (storage type and float32) and GELU; the last shape runs split along K."""
+    """Residual (storage type and float32) and GELU; the last two shapes run in one round of ring tiles and split along K."""
     m, n, k = mnk
     a, b, bias, g = _inputs(m, n, k, dtype, True)
     b = (b * 0.1)

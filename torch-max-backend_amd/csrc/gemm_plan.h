@@ -296,20 +296,19 @@ static inline SplitKPlan splitk_plan(int64_t batch, int64_t m, int64_t n, int64_
   if (model != nullptr) *model = best;
   return p;
 }
-// The same, or no split where one round of the tiles above is faster (the model's costs are 4.5 us under the measured ones):
-// A row-major 2100 x 768 x 3072 30.0 us split and 18.7, 4300 x 768 x 3072 45.2 and 33.7; A stored [K, M] 3072 x 768 x 2048
-// 27.5 and 19.3, x 4096 46 and 34, with half of the CUs idle level (2304 x 768 x 3072 24 both) or behind (224 x 7464 x
-// 3008 29 and 35). A row-major product that fills three quarters of the chip or less stays split from K = 3072 on, and any
-// from 4096 on: there the line could lie higher (2000 x 768 x 3072 27.5 and 17, 3072 x 768 x 4096 44 and 36), but callers
-// size their scratch by the plans of those shapes.
+// The same, or no split where one round of the tiles above is faster (the model's costs are 4.5 us under the measured ones).
+// A row-major up to K = 4096, as far as their cost was fitted: 2100 x 768 x 3072 30.0 us split and 18.7, 4300 x 768 x 3072
+// 45.2 and 33.7, 2000 x 768 x 3072 27.7 and 17.1, 3072 x 768 x 4096 42.4 and 32.3; 70 shapes of K 3072 .. 4096 take 0.79 of
+// the time (geometric mean, worst 1.05). Beyond, the costs of both choose no better than the split (0.97 of the time, worst
+// 1.16, over 350 shapes of K 4160 .. 8192). A stored [K, M] 3072 x 768 x 2048 27.5 and 19.3, x 4096 46 and 34, with half of
+// the CUs idle level (2304 x 768 x 3072 24 both) or behind (224 x 7464 x 3008 29 and 35).
 static inline SplitKPlan splitk_or_whole(int64_t batch, int64_t m, int64_t n, int64_t k, int trans_a) {
   double split_cost = 0.0;
   const SplitKPlan p = splitk_plan(batch, m, n, k, &split_cost);
   const int form = ring_one_round(batch, m, n, k, trans_a);
   if (p.splits == 0 || form == 0) return p;
   const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128);
-  const bool whole = trans_a ? k < 2560 || (k <= 4096 && t128 > 128)
-                             : k < 3072 || (k < 4096 && ((m + 63) / 64) * ((n + 127) / 128) > 192);
+  const bool whole = trans_a ? k < 2560 || (k <= 4096 && t128 > 128) : k <= 4096;
   return whole && one_round_cost(form, t128, k) < split_cost + 4.5 ? SplitKPlan{0, 0, 0.0} : p;
 }
 
